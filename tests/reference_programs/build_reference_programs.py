@@ -331,7 +331,7 @@ def build_suite(verbose=False):
 
 
 def build_all(verbose=False):
-    if not os.path.isdir(REFERENCE):
+    if not os.path.isdir(os.path.join(REFERENCE, "benchmarks")):
         if verbose:
             print("[reference programs] %s is absent: nothing built" % REFERENCE)
         return False
