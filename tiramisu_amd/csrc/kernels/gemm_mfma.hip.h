@@ -457,7 +457,12 @@ __device__ __forceinline__ void tile_epilogue(const accumulators<CFG> &acc, int 
 // elements load and store in turn pays a round trip to memory per element.  Here the values of a group of
 // accumulator tiles (64 elements per lane: what the loads of the first pass may keep in registers) are all
 // computed before the group's first store is issued: one round trip per group.
-template <class CFG, class VALUE, class STORE>
+// EDGE: an element outside C takes its value at the nearest element of C (the loads of the first pass then need no
+// branch and are all in flight together: guarded one by one, every element of a tile waited for its own load) and only
+// its store is skipped: 1000 x 750 x 500 24.3 -> 19.3 us in fp32, 22.0 -> 16.9 with bf16 inputs, a convolution of 8 images
+// of 112 x 112 from 3 to 64 channels 21.3 -> 12.4.  PURE false: value() writes something itself and is called for
+// elements of C only.
+template <class CFG, bool PURE = true, class VALUE, class STORE>
 __device__ __forceinline__ void tile_epilogue(accumulators<CFG> &acc, int M, int N, int m0, int n0, VALUE value, STORE store) {
     const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) % (CFG::WGM * CFG::WGN);
     const int wm = wave / CFG::WGN, wn = wave % CFG::WGN;
@@ -474,9 +479,13 @@ __device__ __forceinline__ void tile_epilogue(accumulators<CFG> &acc, int M, int
                     const int i = g / CFG::TN, j = g % CFG::TN;
                     const int row = m0 + wm * CFG::WM + i * 32 + 8 * (r / 4) + 4 * h + (r % 4);
                     const int col = n0 + wn * CFG::WN + j * 32 + l32;
-                    if (!CFG::EDGE || (row < M && col < N)) {
-                        if (pass == 0) acc.t[i][j][r] = value(row, col, acc.t[i][j][r]);
-                        else store(row, col, acc.t[i][j][r]);
+                    const bool inside = !CFG::EDGE || (row < M && col < N);
+                    if (pass == 1) {
+                        if (inside) store(row, col, acc.t[i][j][r]);
+                    } else if (CFG::EDGE && PURE) {
+                        acc.t[i][j][r] = value(row < M ? row : M - 1, col < N ? col : N - 1, acc.t[i][j][r]);
+                    } else if (inside) {
+                        acc.t[i][j][r] = value(row, col, acc.t[i][j][r]);
                     }
                 }
 }

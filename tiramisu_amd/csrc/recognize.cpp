@@ -1669,7 +1669,8 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         body << window_call_head << epi_args << ");\n";
     } else {
         if (WGK > 1) body << "    if (tgemm::tile_reduce_k<CFG>(_acc, _lds))\n    ";
-        body << "    tgemm::tile_epilogue<CFG>(_acc, _M, _N, _tm * CFG::BM, _tn * CFG::BN, " << epi_args << ");\n";
+        // the value of a tile that a consumer takes over is also written to LDS
+        body << "    tgemm::tile_epilogue<CFG" << (with_consumer && two_pass ? ", false" : "") << ">(_acc, _M, _N, _tm * CFG::BM, _tn * CFG::BN, " << epi_args << ");\n";
     }
     body << consumer_text.str();
 
