@@ -133,3 +133,28 @@ def test_gpu_large_tiles_short_k(M, N, K):
     exact = 1.5 * (from_bf16(A).astype(np.float64) @ from_bf16(B).astype(np.float64)) + 0.5 * C
     out = run_gpu(M, N, K, scal, A, B, C.copy())
     assert np.max(np.abs(out - exact)) <= 1e-5 * np.max(np.abs(exact))
+
+
+EDGES = [(4002, 3998, 500, "tile 256x256x32, guarded edges"), (2000, 1500, 1006, "tile 128x128x32, guarded edges"),
+         (70, 66, 130, "tile 64x64x64, guarded edges"), (66, 2, 6, "tile 64x64x64, guarded edges"),
+         (2001, 1501, 1001, "tile 128x128x64, guarded edges"), (65, 67, 193, "tile 64x64x64, guarded edges"),
+         (64, 65, 63, "tile 64x64x64, guarded edges"), (33, 3, 65, "tile 64x64x64, guarded edges")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,what", EDGES)
+def test_gpu_sizes_that_end_inside_a_tile(M, N, K, what, programs_dir):
+    """Small integers: every sum is exact.  The first elements of A's rows are infinite in every other row: a row read past
+    its last k goes on into them, and must not use them."""
+    import json
+    from gpu_util import DeviceArray
+    how = json.load(open(os.path.join(programs_dir, "build", name_of(M, N, K) + ".o.json")))["kernels"][0]["how"]
+    assert what in how and ("straight into LDS" in how) == (K % 2 == 0 and N % 2 == 0)
+    rng = np.random.RandomState(M + N + K)
+    A, B = rng.randint(-3, 4, (M, K)).astype(np.float32), rng.randint(1, 4, (K, N)).astype(np.float32)
+    A[1::2, 0] = np.inf
+    C = rng.randint(-8, 9, (M, N)).astype(np.float32)
+    exact = 2.0 * (A @ B) + 0.5 * C            # sums of at most 1006 products below 10: exact in float32 in any order
+    d = [DeviceArray(a) for a in (to_bf16(A), to_bf16(B), C)]
+    runtime.load(programs_dir, name_of(M, N, K))(np.array([2.0, 0.5], np.float32), *[x.buffer() for x in d])
+    assert np.array_equal(d[2].download(), exact)

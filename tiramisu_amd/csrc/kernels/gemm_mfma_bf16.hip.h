@@ -15,11 +15,13 @@
 //     write every fourth column) and keeps the reads conflict-free.
 //   * Row m of k-group kq of A sits at position m ^ swz(kq) for the same reason (the lanes that
 //     store the k-groups of one row are 4096 bytes apart).
-// With EDGE the tile may hang over the M x N x K problem and rows need not be aligned: loads outside
-// read as zero (element loads where a 16-byte / 8-byte piece is not whole or not aligned), and the
-// epilogue skips elements outside.  Without it: M % BM == 0, N % BN == 0, K % BK == 0, rows of A 16-byte
-// and rows of B 8-byte aligned (the emitter checks).  Large tiles use the second variant further down
-// (tile_accumulate_bf16_direct: slices loaded straight into an LDS ring); this one serves 64x64 tiles.
+// With EDGE the tile may hang over the M x N x K problem and rows need not be aligned, and the epilogue skips elements
+// outside.  Without it: M % BM == 0, N % BN == 0, K % BK == 0, rows of A 16-byte and rows of B 8-byte aligned (the emitter
+// checks).  This variant serves rows of an odd number of elements (16-byte loads of any alignment cost little: the same
+// 64 x 64 tiles take 17.4 us for 2000 x 1500 x 1000 and 21.0 for 2001 x 1501 x 1001; guarded element by element, where
+// loads of such rows were and of every piece at an edge, 48.7 us), sizes known at run time only and operands of 2 GiB and
+// more.  Rows of an even number of elements use the second variant further down (tile_accumulate_bf16_direct: slices
+// loaded straight into an LDS ring).
 #ifndef TIRAMISU_AMD_GEMM_MFMA_BF16_HIP_H
 #define TIRAMISU_AMD_GEMM_MFMA_BF16_HIP_H
 #include "gemm_mfma.hip.h"
@@ -29,6 +31,8 @@ namespace tgemm {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));   // rows of an odd number of elements
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
 
 template <int BM_, int BN_, int BK_, int WGM_, int WGN_, bool EDGE_ = false>
 struct config_bf16 {
@@ -51,9 +55,6 @@ template <class CFG>
 __device__ __forceinline__ void tile_accumulate_bf16(accumulators<CFG> &acc, const uint16_t *__restrict__ A, long lda,
                                                      const uint16_t *__restrict__ B, long ldb, int M, int N, int K, int m0, int n0,
                                                      uint32_t *lds) {
-    // whole 16-byte pieces of A / 8-byte pieces of B may be loaded as such
-    const bool vec_a = !CFG::EDGE || ((lda % 8 == 0) && ((uintptr_t)A % 16 == 0));
-    const bool vec_b = !CFG::EDGE || ((ldb % 4 == 0) && ((uintptr_t)B % 8 == 0));
     constexpr int TM = CFG::TM, TN = CFG::TN, BK = CFG::BK, BM = CFG::BM, BN = CFG::BN, NT = CFG::NT;
     constexpr int NVA = CFG::NVA, NVB = CFG::NVB;
     constexpr int Q = BK / 16;                      // MFMA steps (fragment sets) per slice
@@ -72,38 +73,59 @@ __device__ __forceinline__ void tile_accumulate_bf16(accumulators<CFG> &acc, con
     // (4096 bytes apart) then hit different 16-byte bank groups
     auto swz = [](int kq) -> int { return (BK / 8 >= 8) ? (kq & 7) : 2 * (kq & 3); };
 
-    auto load_a = [&](int k0) {
+    // A slice's global loads.  LAST: the slice may reach behind the last k, where both operands have to be zero.  Rows of A and
+    // columns of B outside the problem only reach elements of C that nobody stores: their loads are moved onto the last row
+    // and the last four columns instead of being guarded (the columns that exist end up in their place by a shift), so that
+    // the loads of all slices but the last have no branch.
+    const uint16_t *pa[NVA], *pb[NVB];
+    int shift_b[NVB];
+    const bool narrow = CFG::EDGE && N < 4;         // no four columns to move onto: B element by element
+#pragma unroll
+    for (int v = 0; v < NVA; v++) {
+        const int idx = t + NT * v, kq = idx % (BK / 8), m = m0 + idx / (BK / 8);
+        pa[v] = A + (long)(CFG::EDGE && m >= M ? M - 1 : m) * lda + 8 * kq;
+    }
+#pragma unroll
+    for (int v = 0; v < NVB; v++) {
+        const int idx = t + NT * v, n = n0 + 4 * (idx % (BN / 4)), kq = idx / (BN / 4), in = CFG::EDGE && !narrow && n > N - 4 ? N - 4 : n;
+        pb[v] = B + (long)(8 * kq) * ldb + in;
+        shift_b[v] = 16 * (n - in < 3 ? n - in : 3);
+    }
+    auto load_a = [&](int k0, auto last_c) {
 #pragma unroll
         for (int v = 0; v < NVA; v++) {
-            const int idx = t + NT * v, kq = idx % (BK / 8), m = idx / (BK / 8);
-            const uint16_t *p = A + (long)(m0 + m) * lda + k0 + 8 * kq;
-            if (!CFG::EDGE || (vec_a && m0 + m < M && k0 + 8 * kq + 7 < K)) {
-                ra[v] = *reinterpret_cast<const u32x4 *>(p);
+            const int kq = (t + NT * v) % (BK / 8);
+            if (!CFG::EDGE) {
+                ra[v] = *reinterpret_cast<const u32x4 *>(pa[v] + k0);
+            } else if (!decltype(last_c)::value || k0 + 8 * kq + 7 < K) {
+                ra[v] = *reinterpret_cast<const u32x4_any *>(pa[v] + k0);
             } else {
                 uint16_t e[8];
 #pragma unroll
-                for (int i = 0; i < 8; i++) e[i] = (m0 + m < M && k0 + 8 * kq + i < K) ? p[i] : (uint16_t)0;
+                for (int i = 0; i < 8; i++) e[i] = k0 + 8 * kq + i < K ? pa[v][k0 + i] : (uint16_t)0;
                 ra[v] = u32x4{e[0] | ((uint32_t)e[1] << 16), e[2] | ((uint32_t)e[3] << 16), e[4] | ((uint32_t)e[5] << 16), e[6] | ((uint32_t)e[7] << 16)};
             }
         }
     };
     auto col_pos = [](int n) -> int { return n ^ ((n >> 3) & 7); };
-    auto load_b = [&](int k0) {
+    auto load_b = [&](int k0, auto last_c) {
 #pragma unroll
         for (int v = 0; v < NVB; v++) {
-            const int idx = t + NT * v, n4 = idx % (BN / 4), kq = idx / (BN / 4);
-            if (CFG::UNITS_B % NT == 0 || idx < CFG::UNITS_B) {
-                const uint16_t *p = B + (long)(k0 + 8 * kq) * ldb + n0 + 4 * n4;
+            const int kq = (t + NT * v) / (BN / 4);
+            if (CFG::UNITS_B % NT == 0 || t + NT * v < CFG::UNITS_B) {
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
-                    if (!CFG::EDGE || (vec_b && k0 + 8 * kq + i < K && n0 + 4 * n4 + 3 < N)) {
-                        rb[v][i] = *reinterpret_cast<const u32x2 *>(p + i * ldb);
-                    } else {
+                    const uint16_t *p = pb[v] + (long)(k0 + i) * ldb;
+                    if (!CFG::EDGE) rb[v][i] = *reinterpret_cast<const u32x2 *>(p);
+                    else if (narrow) {
+                        const int n = n0 + 4 * ((t + NT * v) % (BN / 4));
                         uint16_t e[4];
 #pragma unroll
-                        for (int c = 0; c < 4; c++) e[c] = (k0 + 8 * kq + i < K && n0 + 4 * n4 + c < N) ? p[i * ldb + c] : (uint16_t)0;
+                        for (int c = 0; c < 4; c++) e[c] = k0 + 8 * kq + i < K && n + c < N ? p[c] : (uint16_t)0;
                         rb[v][i] = u32x2{e[0] | ((uint32_t)e[1] << 16), e[2] | ((uint32_t)e[3] << 16)};
                     }
+                    else if (!decltype(last_c)::value || k0 + 8 * kq + i < K) rb[v][i] = *reinterpret_cast<const u32x2_any *>(p);
+                    else rb[v][i] = u32x2{0u, 0u};
                 }
             }
         }
@@ -120,6 +142,13 @@ __device__ __forceinline__ void tile_accumulate_bf16(accumulators<CFG> &acc, con
         for (int v = 0; v < NVB; v++) {
             const int idx = t + NT * v, n4 = idx % (BN / 4), kq = idx / (BN / 4);
             if (CFG::UNITS_B % NT == 0 || idx < CFG::UNITS_B) {
+                if (CFG::EDGE) {
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const uint64_t w = (((uint64_t)rb[v][i][1] << 32) | rb[v][i][0]) >> shift_b[v];
+                        rb[v][i] = u32x2{(uint32_t)w, (uint32_t)(w >> 32)};
+                    }
+                }
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
                     // word p of column c = (row 2p, row 2p+1) as (low, high) halves
@@ -163,20 +192,20 @@ __device__ __forceinline__ void tile_accumulate_bf16(accumulators<CFG> &acc, con
     // cover the first fragment reads of the next slice.  Memory instructions are dealt out between
     // the matrix instructions with scheduling groups.
     const int KT = CFG::EDGE ? (K + BK - 1) / BK : K / BK;
-    load_a(0);
-    load_b(0);
+    load_a(0, std::true_type());
+    load_b(0, std::true_type());
     store_a(0);
     store_b(0);
     if (KT > 1) {
-        load_a(BK);
-        load_b(BK);
+        load_a(BK, std::true_type());
+        load_b(BK, std::true_type());
     }
     __syncthreads();
     read_frags(0, 0, 0);
 
     constexpr int MFMAS = TM * TN;
     constexpr int FRAG_READS = TM + TN;             // LDS read instructions per set
-    auto slice = [&](int kt, auto more_c, auto load_c) {
+    auto slice = [&](int kt, auto more_c, auto load_c, auto last_c) {
         constexpr bool MORE = decltype(more_c)::value, LOAD = decltype(load_c)::value;
         const int cur = kt & 1;
 #pragma unroll
@@ -184,11 +213,11 @@ __device__ __forceinline__ void tile_accumulate_bf16(accumulators<CFG> &acc, con
             const int buf = q & 1;
             if (q == 0 && MORE) {
                 store_a(cur ^ 1);
-                if (LOAD) load_a((kt + 2) * BK);
+                if (LOAD) load_a((kt + 2) * BK, last_c);
             }
             if (q == (Q > 2 ? 1 : 0) && MORE) {
                 store_b(cur ^ 1);
-                if (LOAD) load_b((kt + 2) * BK);
+                if (LOAD) load_b((kt + 2) * BK, last_c);
             }
             if (q + 1 < Q) {
                 read_frags(cur, q + 1, buf ^ 1);
@@ -213,9 +242,10 @@ __device__ __forceinline__ void tile_accumulate_bf16(accumulators<CFG> &acc, con
         }
     };
     int kt = 0;
-    for (; kt + 2 < KT; kt++) slice(kt, std::true_type(), std::true_type());
-    if (kt + 1 < KT) { slice(kt, std::true_type(), std::false_type()); kt++; }
-    if (kt < KT) slice(kt, std::false_type(), std::false_type());
+    for (; kt + 2 + (CFG::EDGE ? 1 : 0) < KT; kt++) slice(kt, std::true_type(), std::true_type(), std::false_type());
+    if (CFG::EDGE && kt + 2 < KT) { slice(kt, std::true_type(), std::true_type(), std::true_type()); kt++; }
+    if (kt + 1 < KT) { slice(kt, std::true_type(), std::false_type(), std::true_type()); kt++; }
+    if (kt < KT) slice(kt, std::false_type(), std::false_type(), std::true_type());
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -233,14 +263,21 @@ __device__ __forceinline__ void tile_accumulate_bf16(accumulators<CFG> &acc, con
 //     (k0 .. k0 + 3, column n0 + L).
 //   * The swizzles keep the reads free of bank conflicts whether the LDS serves 128 bytes (8 lanes of
 //     a 16-byte read, 16 of a transposing one) or 256 bytes per cycle: swzA spreads 8 and 16
-//     consecutive rows, swzB (0, 4, 10, 14 for k % 4) the four rows of a transposing read, over
+//     consecutive rows, swzB (0, 4, 10, 14 for k % 4; 0, 2, 4, 6 with rows of 64 columns) the four rows of a transposing read, over
 //     distinct 16-byte bank groups in both cases (measured: SQ_LDS_BANK_CONFLICT = 0).
 // A call ends with a barrier (every wave is past its last read), so it may be repeated for a second
-// pair of operands.  Rows of A and of B must be 16-byte aligned.
-template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int STAGES_>
+// pair of operands.  Rows of A and of B must be 4-byte aligned.
+// With EDGE the tiles may hang over the problem and K need not be a multiple of the slice.  What a load finds there needs
+// no guard: behind the last row of A and of B the buffer descriptor ends and reads give zero (it is checked dword by
+// dword, so the last row itself is whole); columns of B behind N are the start of the next row and only reach columns of C
+// that nobody stores; so do rows of A behind M.  Only k behind the last one has to be zero: rows of B there are (behind
+// the end), and A, whose row simply goes on into the next, is masked in registers in the last slice.
+// (2000 x 1500 x 1000: 15.7 us with 128 x 128 tiles against 48.7 with guarded 64 x 64 tiles staged through registers;
+// 300 x 260 x 3000: 16.9 us with 64 x 128 tiles against 99.8.)
+template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int STAGES_, bool EDGE_ = false>
 struct config_bf16_direct {
     static constexpr int BM = BM_, BN = BN_, BK = BK_, WGM = WGM_, WGN = WGN_, STAGES = STAGES_;
-    static constexpr bool EDGE = false;
+    static constexpr bool EDGE = EDGE_;
     static constexpr int NW = WGM * WGN, NT = 64 * NW;
     static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
     static constexpr int GA = BK / 8, GB = BN / 8;          // 16-byte granules per row of the A / B slice
@@ -249,7 +286,7 @@ struct config_bf16_direct {
     static constexpr int LA = BM * GA / 64 / NW, LB = BK * GB / 64 / NW;   // wave-wide loads per wave and slice
     static_assert(BK == 32 || BK == 64, "slices of 32 or 64 k");
     static_assert(BM * GA % (64 * NW) == 0 && BK * GB % (64 * NW) == 0, "slices must split evenly over the waves");
-    static_assert(GB >= 16 && (GB & (GB - 1)) == 0, "row of B: a power of two of 128 columns or more (the swizzle spans 16 granules)");
+    static_assert(GB >= 8 && (GB & (GB - 1)) == 0, "row of B: a power of two of 64 columns or more (the swizzle spans 8 or 16 granules)");
     static_assert(STAGES >= 2, "the ring needs two stages or more");
 };
 
@@ -269,7 +306,7 @@ __device__ __forceinline__ void tile_accumulate_bf16_direct(accumulators<CFG> &a
     const int l32 = lane & 31, h = lane >> 5;
     lds_char *const base = (lds_char *)lds;
     auto swzA = [](int m) -> int { return GA == 8 ? ((m ^ (m >> 3)) & 7) : (((m >> 2) & 1) | ((((m >> 1) ^ (m >> 3)) & 1) << 1)); };
-    auto swzB = [](int k) -> int { return ((k & 1) << 2) | ((k & 2) ? 10 : 0); };   // 0, 4, 10, 14
+    auto swzB = [](int k) -> int { return GB == 8 ? 2 * (k & 3) : ((k & 1) << 2) | ((k & 2) ? 10 : 0); };   // 0, 2, 4, 6 or 0, 4, 10, 14
 
     // The loads are buffer loads (base in a resource descriptor, 32-bit byte offset per lane, one
     // scalar offset per operand that advances by a slice): no 64-bit address arithmetic in the loop,
@@ -338,6 +375,15 @@ __device__ __forceinline__ void tile_accumulate_bf16_direct(accumulators<CFG> &a
             if (half) fbh[buf][j] = v; else fbl[buf][j] = v;
         }
     };
+    // EDGE, last slice: the part of a lane's fragment of step s that lies behind the last k is set to zero
+    auto mask_tail = [&](int kt, int s, int buf) {
+        const int rest = K - (kt * BK + 16 * s + 8 * h);
+        u32x4 keep;
+#pragma unroll
+        for (int w = 0; w < 4; w++) keep[w] = rest >= 2 * w + 2 ? 0xffffffffu : rest == 2 * w + 1 ? 0x0000ffffu : 0u;
+#pragma unroll
+        for (int i = 0; i < TM; i++) fa[buf][i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, fa[buf][i]) & keep);
+    };
     auto mfma_one = [&](int buf, int idx) {
         const int i = idx / TN, j = idx % TN;
         const s16x8 both = __builtin_shufflevector(fbl[buf][j], fbh[buf][j], 0, 1, 2, 3, 4, 5, 6, 7);
@@ -354,9 +400,9 @@ __device__ __forceinline__ void tile_accumulate_bf16_direct(accumulators<CFG> &a
     // instructions, with large wave tiles one read each, so that a fragment is requested at least seven
     // matrix instructions before its use and the compiler's waits count exactly (buffer loads, unlike
     // global or flat ones, do not make it wait for every outstanding LDS access).
-    const int KT = K / BK;
+    const int KT = CFG::EDGE ? (K + BK - 1) / BK : K / BK;
     constexpr int PER = LA + LB;                    // loads per wave and slice
-    constexpr int PRE = MFMAS >= 16 ? 4 : 1;        // matrix instructions of the last step ahead of the barrier
+    constexpr int PRE = MFMAS >= 16 ? 4 : MFMAS > 1 ? 1 : 0;        // matrix instructions of the last step ahead of the barrier
     static_assert((ST - 1) * PER <= 63, "the load counter holds 63");
     constexpr int SLOTS = READS < MFMAS ? (READS > MFMAS - 4 ? READS : MFMAS - 4) : MFMAS;   // matrix instructions of a step that are followed by reads
 #pragma unroll
@@ -374,6 +420,7 @@ __device__ __forceinline__ void tile_accumulate_bf16_direct(accumulators<CFG> &a
 #pragma unroll
         for (int q = 0; q < Q; q++) {
             const int buf = q & 1;
+            if (CFG::EDGE && !MORE && K % BK != 0) mask_tail(KT - 1, q, buf);
             if (q + 1 < Q) {
 #pragma unroll
                 for (int idx = 0; idx < MFMAS; idx++) {

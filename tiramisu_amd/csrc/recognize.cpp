@@ -1182,37 +1182,41 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     if (const char *e = backend_option("TIRAMISU_MFMA_DEPTH")) DEPTH = std::atoi(e);
     if (const char *e = backend_option("TIRAMISU_MFMA_PAD")) PADX = std::atoi(e);
     if (const char *e = backend_option("TIRAMISU_MFMA_WGK")) WGK = std::atoi(e);
-    bool bf16_edge = false;
+    bool bf16_edge = false, bf16_direct = false;
+    int bf16_stages = 2;                 // of the LDS ring
     if (bf16) {
-        // 256x256 when that fills the chip, else 128x128 (both load their slices straight into LDS and want whole
-        // tiles, 16-byte aligned rows and operands below 2 GiB), else 64x64 -- with guarded loads when tiles hang
-        // over the problem, sizes are known at run time only, or rows are not aligned
+        // the tile whose launch is modelled fastest (kernels/target_gfx950.h); rows of an even number of elements are
+        // loaded straight into LDS (32-bit offsets: operands below 2 GiB), others, and sizes known at run time only,
+        // through registers (guarded 64x64 tiles in the latter case)
         for (auto &o : operands)
             if (!o.first.linear || !o.second.linear || !o.first.kmajor || o.second.kmajor) return reject(25);
-        bool aligned = true, small_enough = true;
+        bool aligned = true, dword_rows = true, small_enough = true;
         for (auto &o : operands) {
             long v;
-            for (const operand_info *g : {&o.first, &o.second})
+            for (const operand_info *g : {&o.first, &o.second}) {
                 if (!literal_value(g->ld, v) || v % 8 != 0 || !multiple_of(g->base, 8)) aligned = false;
+                if (!literal_value(g->ld, v) || v % 2 != 0 || !multiple_of(g->base, 2)) dword_rows = false;
+            }
             long lda = 0, ldb = 0;
             if (lit && literal_value(o.first.ld, lda) && literal_value(o.second.ld, ldb)) {
-                if ((double)Ml * lda * 2 >= 2147483648.0 || (double)Kl * ldb * 2 >= 2147483648.0) small_enough = false;
+                // (a tile's rows and slices may reach behind the operand: their offsets must not wrap either)
+                if ((double)(Ml + 256) * lda * 2 >= 2147483648.0 || (double)(Kl + 256) * ldb * 2 >= 2147483648.0) small_enough = false;
             } else {
                 small_enough = false;
             }
         }
-        WGM = WGN = 2;
-        if (lit && aligned && small_enough && (Ml / 256) * (Nl / 256) >= 3 * ttarget::COMPUTE_UNITS / 4 && Ml % 256 == 0 && Nl % 256 == 0 && Kl % 32 == 0) { BM = BN = 256; BK = 32; }
-        else if (lit && aligned && small_enough && Ml % 128 == 0 && Nl % 128 == 0 && Kl % 32 == 0 && (Ml / 128) * (Nl / 128) >= 3 * ttarget::COMPUTE_UNITS / 16) { BM = BN = 128; BK = 32; }
-        else {
-            BM = BN = 64;
-            BK = 64;
-            bf16_edge = !(lit && aligned && Ml % 64 == 0 && Nl % 64 == 0 && Kl % 64 == 0);
-        }
+        bf16_direct = lit && dword_rows && small_enough;
+        const ttarget::bf16_tile tile = lit ? ttarget::bf16_tile_for(Ml, Nl, Kl, bf16_direct) : ttarget::BF16_TILE_ANY_SIZE;
+        BM = BN = tile.edge;
+        BK = tile.k;
+        WGM = tile.waves_m;
+        WGN = tile.waves_n;
+        bf16_stages = tile.stages;
+        bf16_edge = !(lit && (bf16_direct || aligned) && Ml % BM == 0 && Nl % BN == 0 && Kl % BK == 0);
     }
     bool edge = !(lit && Ml % BM == 0 && Nl % BN == 0 && Kl % BK == 0);
     if (bf16) edge = bf16_edge;
-    for (auto &o : operands)
+    else for (auto &o : operands)
         for (const operand_info *g : {&o.first, &o.second}) {
             long v;
             if (g->linear && (!literal_value(g->ld, v) || v % 4 != 0)) edge = true;
@@ -1487,8 +1491,8 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     const int NT = 64 * WGM * WGN * WGK;
     if (bf16) {
         body << "    extern __shared__ __attribute__((aligned(16))) uint32_t _lds[];\n";
-        // large tiles: slices go straight from global memory into a four-stage LDS ring
-        if (BM >= 128) body << "    typedef tgemm::config_bf16_direct<" << BM << ", " << BN << ", " << BK << ", " << WGM << ", " << WGN << ", 4> CFG;\n";
+        // slices go straight from global memory into an LDS ring where they can
+        if (bf16_direct) body << "    typedef tgemm::config_bf16_direct<" << BM << ", " << BN << ", " << BK << ", " << WGM << ", " << WGN << ", " << bf16_stages << (edge ? ", true" : ", false") << "> CFG;\n";
         else body << "    typedef tgemm::config_bf16<" << BM << ", " << BN << ", " << BK << ", " << WGM << ", " << WGN << ", " << (edge ? "true" : "false") << "> CFG;\n";
     } else {
         body << "    extern __shared__ __attribute__((aligned(16))) float _lds[];\n";
@@ -1508,7 +1512,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         if (bf16) {
             used_buffers.insert(o.first.buf->get_name());
             used_buffers.insert(o.second.buf->get_name());
-            body << "        tgemm::tile_accumulate_bf16" << (BM >= 128 ? "_direct" : "") << "<CFG>(_acc, " << o.first.buf->get_name() << " + (" << dev.print(o.first.base) << "), "
+            body << "        tgemm::tile_accumulate_bf16" << (bf16_direct ? "_direct" : "") << "<CFG>(_acc, " << o.first.buf->get_name() << " + (" << dev.print(o.first.base) << "), "
                  << dev.print(o.first.ld) << ", " << o.second.buf->get_name() << " + (" << dev.print(o.second.base) << "), " << dev.print(o.second.ld)
                  << ", _M, _N, _K, _tm * CFG::BM, _tn * CFG::BN, _lds);\n    }\n";
             term++;
@@ -1678,7 +1682,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     k.name = kname;
     bool any_gather = false;
     for (auto &o : operands) any_gather = any_gather || !o.first.linear || !o.second.linear;
-    k.how = std::string("mfma-contraction: ") + (bf16 ? (BM >= 128 ? "v_mfma_f32_32x32x16_bf16, slices loaded straight into LDS, " : "v_mfma_f32_32x32x16_bf16, ") : "v_mfma_f32_32x32x2_f32, ") + (windowed ? "implicit GEMM, sliding window of " + std::to_string(win_taps) + " taps staged in LDS by blocks of " + std::to_string(win_cb) + " channels, " :
+    k.how = std::string("mfma-contraction: ") + (bf16 ? (bf16_direct ? "v_mfma_f32_32x32x16_bf16, slices loaded straight into LDS, " : "v_mfma_f32_32x32x16_bf16, ") : "v_mfma_f32_32x32x2_f32, ") + (windowed ? "implicit GEMM, sliding window of " + std::to_string(win_taps) + " taps staged in LDS by blocks of " + std::to_string(win_cb) + " channels, " :
                                                                                       any_gather ? "implicit GEMM (gathered operand), " : "") + "M " +
             std::to_string(Mg.size()) + " dim(s) x N " + std::to_string(Ng.size()) + " x K " + std::to_string(Kg.size()) + ", tile " +
             std::to_string(BM) + "x" + std::to_string(BN) + "x" + std::to_string(BK) + (edge ? ", guarded edges" : ", whole tiles") + ", " +
@@ -1759,7 +1763,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         const int rowA = operands[0].first.kmajor ? (BK / 4) * (BM + PADX) * 4 : BK * BM;
         const int rowB = operands[0].second.kmajor ? (BK / 4) * (BN + PADX) * 4 : BK * BN;
         k.lds_bytes = std::to_string(2 * (rowA + rowB) * 4);
-        if (bf16) k.lds_bytes = std::to_string((BM >= 128 ? 4 : 2) * (BK / 8) * (BM + BN) * 4 * 4);   // four-stage ring for the large tiles
+        if (bf16) k.lds_bytes = std::to_string(bf16_stages * (BK / 8) * (BM + BN) * 4 * 4);
         else if (ktab_words) k.lds_bytes = std::to_string(2 * (rowA + rowB) * 4 + ktab_words * 4);
         if (with_consumer) k.lds_bytes = std::to_string(std::stol(k.lds_bytes) + BM * (BN + 1) * 4);
         if (windowed) k.lds_bytes = std::to_string(2 * ((long)win_cb * (win_taps * BM + 32) + (long)win_cb * win_floats) * 4);
