@@ -143,3 +143,13 @@ def test_gpu_full_size():
     assert_fp32_parity(out, exact, "conv2d vs float64 restatement", RTOL)
     # linearity in the input away from the clamp: conv(2x) - 2 conv(x) + bias term
     assert np.count_nonzero(out) > 0.3 * out.size
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("s", [(2, 5, 7, 9), (1, 3, 33, 10), (3, 9, 17, 20), (2, 31, 64, 33), (1, 64, 50, 12)])
+def test_gpu_sizes_that_no_tile_divides(s, programs_dir):
+    from gpu_util import DeviceArray
+    xp, w, b = make_inputs(s, sum(s), integer=True)
+    d = [DeviceArray(a) for a in (xp, w, b, np.full((s[0], s[2], s[3], s[3]), np.nan, np.float32))]
+    runtime.load(programs_dir, name_of(s))(*[q.buffer() for q in d])
+    assert np.array_equal(d[3].download(), ref.conv2d_bias_relu(xp, w, b))      # integers: exact

@@ -67,6 +67,30 @@ def test_transposed_operands_padding_and_offsets(tA, tB):
     run(50, 30, 20, 1.0, 0.0, tA=tA, tB=tB, pad=3, off=5)
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 35, 9), (65, 130, 33), (129, 67, 130), (64, 70, 64), (300, 260, 2051)])
+@pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_sizes_that_end_inside_a_tile(M, N, K, tA, tB, pad):
+    """Operands that begin and end with their allocations but for NaN around them and between their rows, which must not
+    reach the result; the rows of C keep what lies between them."""
+    import torch
+    rng = np.random.RandomState(M + N + K + pad)
+
+    def surrounded(rows, cols):
+        flat = np.full(5 + rows * (cols + pad) + 4, np.nan, np.float32)
+        inside = flat[5:5 + rows * (cols + pad)].reshape(rows, cols + pad)[:, :cols]
+        inside[:] = rng.randint(-3, 4, (rows, cols))
+        return torch.from_numpy(flat).cuda(), inside.astype(np.float64), cols + pad
+
+    (dA, a, ldA), (dB, b, ldB), (dC, c, ldC) = [surrounded(*v) for v in ((K, M) if tA else (M, K), (N, K) if tB else (K, N), (M, N))]
+    before = dC.cpu().numpy()
+    torch.cuda.synchronize()
+    runtime.wrappers().tiramisu_hip_sgemm(dA.data_ptr(), dB.data_ptr(), dC.data_ptr(), M, N, K, 2.0, 3.0, ldA, ldB, ldC, 5, 5, 5, tA, tB)
+    runtime.wrappers().tiramisu_hip_stream_synchronize(0)
+    before[5:5 + M * ldC].reshape(M, ldC)[:, :N] = 2.0 * ((a.T if tA else a) @ (b.T if tB else b)) + 3.0 * c     # integers: exact
+    assert np.array_equal(dC.cpu().numpy(), before, equal_nan=True)
+
+
 def test_seeded_sweep_of_shapes():
     # 80 shapes up to 300 in each dimension, every transposition, with and without padding / offsets
     rng = np.random.RandomState(2026)

@@ -131,3 +131,14 @@ def test_gpu_full_size_matches_oracle():
     y0 = run_gpu(s, w0, b, x)
     assert np.max(np.abs(y0 - ref.lstm(w0, b, x))) <= 1e-6
     assert np.all(np.abs(y0 - y0[:, :1, :]) == 0)   # no dependence on the sample
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("s", [(2, 5, 33, 3), (1, 35, 18, 2), (2, 14, 129, 3), (3, 33, 160, 2), (1, 70, 288, 2)])
+def test_gpu_sizes_that_no_tile_divides(s, programs_dir):
+    from gpu_util import DeviceArray, assert_fp32_parity
+    w, b, x = make_inputs(s, 3 + sum(s))
+    d = [DeviceArray(a) for a in (w, b, x, np.full((s[3], s[1], s[2]), np.nan, np.float32))]
+    runtime.load(programs_dir, name_of(s))(*[q.buffer() for q in d])
+    # fp32 sums of at most 576 products below 0.08: 1e-6 apart in another order, and expf / tanhf a few ulps
+    assert_fp32_parity(d[3].download(), ref.lstm(w, b, x), "lstm %s vs numpy oracle" % (s,), 1e-5)

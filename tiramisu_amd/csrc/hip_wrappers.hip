@@ -163,16 +163,16 @@ thread_local int active_batch_count = 0;
 
 template <class CFG>
 void launch_mfma(const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc,
-                 float alpha, float beta, bool vec_ok) {
+                 float alpha, float beta) {
     const int tiles = ((M + CFG::BM - 1) / CFG::BM) * ((N + CFG::BN - 1) / CFG::BN);
     if (active_batch) {
         hipLaunchKernelGGL((tgemm::sgemm_batched_kernel<CFG>), dim3(tiles, 1, active_batch_count), dim3(CFG::NT), CFG::LDS_BYTES, current_stream,
-                           *active_batch, M, N, K, lda, ldb, ldc, alpha, beta, vec_ok ? 1 : 0);
+                           *active_batch, M, N, K, lda, ldb, ldc, alpha, beta);
         check(hipGetLastError(), "tiramisu_hip_sgemm");
         return;
     }
     hipLaunchKernelGGL((tgemm::sgemm_kernel<CFG>), dim3(tiles), dim3(CFG::NT), CFG::LDS_BYTES, current_stream, A, B, C,
-                       M, N, K, lda, ldb, ldc, alpha, beta, vec_ok ? 1 : 0);
+                       M, N, K, lda, ldb, ldc, alpha, beta);
     check(hipGetLastError(), "tiramisu_hip_sgemm");
 }
 
@@ -181,18 +181,18 @@ int tile_for(int M, int N) { return ttarget::square_tile_for(M, N); }
 
 template <bool AK, bool BK_, bool EDGE>
 void dispatch_tile(const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc,
-                   float alpha, float beta, bool vec_ok) {
+                   float alpha, float beta) {
     const int bm = tile_for(M, N);
     if constexpr (!EDGE) {
         if (bm == 256)
-            return launch_mfma<tgemm::config<256, 256, 16, 2, 2, AK, BK_, false, 0>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, vec_ok);
+            return launch_mfma<tgemm::config<256, 256, 16, 2, 2, AK, BK_, false, 0>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
         if (bm == 192)
-            return launch_mfma<tgemm::config<192, 192, 16, 2, 2, AK, BK_, false>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, vec_ok);
+            return launch_mfma<tgemm::config<192, 192, 16, 2, 2, AK, BK_, false>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     }
     if (bm == 128)
-        launch_mfma<tgemm::config<128, 128, 16, 2, 2, AK, BK_, EDGE>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, vec_ok);
+        launch_mfma<tgemm::config<128, 128, 16, 2, 2, AK, BK_, EDGE>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     else
-        launch_mfma<tgemm::config<64, 64, 32, 2, 2, AK, BK_, EDGE>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, vec_ok);
+        launch_mfma<tgemm::config<64, 64, 32, 2, 2, AK, BK_, EDGE>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
 
 // Few C tiles but a long reduction (a batch of 64 rows against wide weights, as in recurrent
@@ -207,12 +207,12 @@ void dispatch_skinny(const float *A, const float *B, float *C, int M, int N, int
                      float alpha, float beta) {
     // K = 512 (the recurrent product of a 512-unit cell): four groups of wavefronts, 64-k slices, one slice ahead
     // (9.2 us per call against 10.9 us for the eight-group form below)
-    if (K == 512) return launch_mfma<tgemm::config<64, 32, 64, 2, 1, true, BK_, false, 0, 4, 1>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, true);
+    if (K == 512) return launch_mfma<tgemm::config<64, 32, 64, 2, 1, true, BK_, false, 0, 4, 1>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     switch (std::min(4, K / 128 - 1)) {
-    case 1: return launch_mfma<tgemm::config<64, 32, 128, 2, 1, true, BK_, false, 0, 8, 1>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, true);
-    case 2: return launch_mfma<tgemm::config<64, 32, 128, 2, 1, true, BK_, false, 0, 8, 2>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, true);
-    case 3: return launch_mfma<tgemm::config<64, 32, 128, 2, 1, true, BK_, false, 0, 8, 3>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, true);
-    default: return launch_mfma<tgemm::config<64, 32, 128, 2, 1, true, BK_, false, 0, 8, 4>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, true);
+    case 1: return launch_mfma<tgemm::config<64, 32, 128, 2, 1, true, BK_, false, 0, 8, 1>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    case 2: return launch_mfma<tgemm::config<64, 32, 128, 2, 1, true, BK_, false, 0, 8, 2>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    case 3: return launch_mfma<tgemm::config<64, 32, 128, 2, 1, true, BK_, false, 0, 8, 3>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    default: return launch_mfma<tgemm::config<64, 32, 128, 2, 1, true, BK_, false, 0, 8, 4>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     }
 }
 
@@ -230,7 +230,7 @@ constexpr uint64_t SPLITK_COUNTER_BYTES = SPLITK_MAX_TILES * sizeof(unsigned);
 template <class CFG>
 __global__ void __launch_bounds__(CFG::NT) sgemm_splitk_kernel(const float *__restrict__ A, const float *__restrict__ B,
                                                                 float *__restrict__ C, int M, int N, int K, long lda, long ldb,
-                                                                long ldc, float alpha, float beta, int vec_ok, int chunk,
+                                                                long ldc, float alpha, float beta, int chunk,
                                                                 float *__restrict__ partial, unsigned *__restrict__ counters) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ unsigned ticket;
@@ -243,8 +243,8 @@ __global__ void __launch_bounds__(CFG::NT) sgemm_splitk_kernel(const float *__re
     const int k0 = z * chunk, kc = min(chunk, K - k0);
     tgemm::accumulators<CFG> acc;
     acc.clear();
-    tgemm::linear_source<CFG::A_KMAJOR, CFG::EDGE> sa{A + (CFG::A_KMAJOR ? (long)k0 : (long)k0 * lda), lda, M, kc, vec_ok != 0};
-    tgemm::linear_source<CFG::B_KMAJOR, CFG::EDGE> sb{B + (CFG::B_KMAJOR ? (long)k0 : (long)k0 * ldb), ldb, N, kc, vec_ok != 0};
+    tgemm::linear_source<CFG::A_KMAJOR, CFG::EDGE> sa{A + (CFG::A_KMAJOR ? (long)k0 : (long)k0 * lda), lda, M, kc};
+    tgemm::linear_source<CFG::B_KMAJOR, CFG::EDGE> sb{B + (CFG::B_KMAJOR ? (long)k0 : (long)k0 * ldb), ldb, N, kc};
     tgemm::tile_accumulate<CFG>(acc, sa, sb, kc, tm * CFG::BM, tn * CFG::BN, lds);
     tgemm::f32x4 *mine = reinterpret_cast<tgemm::f32x4 *>(partial) + ((long)blockIdx.x * Z + z) * 4 * CFG::NT;
 #pragma unroll
@@ -309,22 +309,22 @@ splitk_plan plan_splitk(int M, int N, int K, uint64_t max_bytes) {
 
 template <bool AK, bool BK_, bool EDGE>
 void launch_splitk(const splitk_plan &p, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc,
-                   float alpha, float beta, bool vec_ok, void *scratch) {
+                   float alpha, float beta, void *scratch) {
     typedef tgemm::config<SPLITK_TILE, SPLITK_TILE, 32, 2, 2, AK, BK_, EDGE> CFG;
     static_assert(CFG::NT == SPLITK_THREADS, "scratch layout assumes 256 threads");
     unsigned *counters = reinterpret_cast<unsigned *>(scratch);
     float *partial = reinterpret_cast<float *>(reinterpret_cast<char *>(scratch) + SPLITK_COUNTER_BYTES);
     hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(SPLITK_MAX_TILES), 0, current_stream, counters, p.tiles);
     hipLaunchKernelGGL((sgemm_splitk_kernel<CFG>), dim3(p.tiles, p.chunks), dim3(CFG::NT), CFG::LDS_BYTES, current_stream, A, B, C,
-                       M, N, K, lda, ldb, ldc, alpha, beta, vec_ok ? 1 : 0, p.chunk, partial, counters);
+                       M, N, K, lda, ldb, ldc, alpha, beta, p.chunk, partial, counters);
     check(hipGetLastError(), "tiramisu_hip_sgemm");
 }
 
 void dispatch_splitk(const splitk_plan &p, bool tA, bool tB, bool edge, const float *A, const float *B, float *C, int M, int N, int K,
-                     long lda, long ldb, long ldc, float alpha, float beta, bool vec_ok, void *scratch) {
+                     long lda, long ldb, long ldc, float alpha, float beta, void *scratch) {
 #define SPLITK_CASE(AK, BKM)                                                                                              \
-    if (edge) launch_splitk<AK, BKM, true>(p, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, vec_ok, scratch);              \
-    else launch_splitk<AK, BKM, false>(p, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, vec_ok, scratch)
+    if (edge) launch_splitk<AK, BKM, true>(p, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, scratch);              \
+    else launch_splitk<AK, BKM, false>(p, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, scratch)
     if (!tA && !tB) { SPLITK_CASE(true, false); }
     else if (!tA && tB) { SPLITK_CASE(true, true); }
     else if (tA && !tB) { SPLITK_CASE(false, false); }
@@ -365,9 +365,9 @@ void *static_scratch_here() {
 
 template <bool AK, bool BK_>
 void dispatch_edge(bool edge, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb,
-                   long ldc, float alpha, float beta, bool vec_ok) {
-    if (edge) dispatch_tile<AK, BK_, true>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, vec_ok);
-    else dispatch_tile<AK, BK_, false>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta, vec_ok);
+                   long ldc, float alpha, float beta) {
+    if (edge) dispatch_tile<AK, BK_, true>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else dispatch_tile<AK, BK_, false>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
 
 template <class S, bool A_KFAST, bool B_NFAST>
@@ -580,16 +580,16 @@ static int sgemm_impl(const char *fn, bool static_scratch, float *A, float *B, f
             ws = block.ptr;
         }
         const bool edge = !(vec_ok && m % SPLITK_TILE == 0 && n % SPLITK_TILE == 0 && plan.chunk % 32 == 0 && k % plan.chunk == 0);
-        dispatch_splitk(plan, transposeA, transposeB, edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta, vec_ok, ws);
+        dispatch_splitk(plan, transposeA, transposeB, edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta, ws);
         return 0;
     }
     const int bm = tile_for(m, n);
     const bool edge = !(vec_ok && m % bm == 0 && n % bm == 0 && k % (bm == 64 ? 32 : 16) == 0);   // K-slice of the tile
     // A is K-contiguous unless transposed; B is K-contiguous only when transposed.
-    if (!transposeA && !transposeB) dispatch_edge<true, false>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta, vec_ok);
-    else if (!transposeA && transposeB) dispatch_edge<true, true>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta, vec_ok);
-    else if (transposeA && !transposeB) dispatch_edge<false, false>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta, vec_ok);
-    else dispatch_edge<false, true>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta, vec_ok);
+    if (!transposeA && !transposeB) dispatch_edge<true, false>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
+    else if (!transposeA && transposeB) dispatch_edge<true, true>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
+    else if (transposeA && !transposeB) dispatch_edge<false, false>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
+    else dispatch_edge<false, true>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
     return 0;
 }
 

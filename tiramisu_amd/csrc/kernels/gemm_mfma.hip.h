@@ -82,28 +82,69 @@ __device__ __forceinline__ void handed_over_loads_begin() {
 #endif
 }
 
+// Elements s .. s + 3 of the four given, zeros behind them (s >= 0).
+__device__ __forceinline__ f32x4 shifted_down(f32x4 v, int s) {
+    const f32x4 one = {v[1], v[2], v[3], 0.f};
+    v = (s & 1) ? one : v;
+    const f32x4 two = {v[2], v[3], 0.f, 0.f};
+    v = (s & 2) ? two : v;
+    const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+    return s > 3 ? none : v;
+}
+
 // An operand stored with one unit stride: element (x, k) lives at base[x*ld + k] (KMAJOR) or
-// base[k*ld + x].  With EDGE, elements outside XE x KE read as zero and rows need not be
-// 16-byte aligned (vec_ok false).
+// base[k*ld + x].  A source is read in two steps, so that nothing waits for a load where it is issued:
+//   load4(x, k, tail)      the 16 bytes at (x, k) as they come from memory,
+//   finish4(v, x, k, tail) the four elements from them, when they are stored to LDS.
+// Without EDGE all of the operand is there and 16-byte aligned.  With EDGE a tile may hang over XE, the last slice
+// (tail = std::true_type; all others lie within KE) over KE, and rows may start at any element.  Behind KE a source gives
+// zeros; what it gives behind XE only reaches elements of C that nobody stores.  No load is guarded and none is
+// taken apart: it is moved to the nearest place that holds four elements (16-byte loads need not be aligned), and
+// finish4 shifts the elements that exist into theirs.  A slice that is not the last has another row behind its own, so
+// that four elements from any x of the operand on exist there.
+// (Guarded element by element, every element of a slice waited for its own load.  1000 x 750 x 500 24.3 us before, 13.1 now,
+// 2001 x 1501 x 1001 96 and 56, 3001 x 2900 x 2803 with B transposed 727 and 429 (0.73 of the fp32 matrix rate), a step of an
+// LSTM of 320 units and 33 samples 29 and 19, a convolution of 30 images of 100 x 100 from 61 to 50 channels 258 and 187.)
 template <bool KMAJOR, bool EDGE>
 struct linear_source {
+    static constexpr bool SEAM = false;         // (of concat_k)
     const float *__restrict__ base;
     long ld;
     int XE, KE;
-    bool vec_ok;
-    __device__ __forceinline__ f32x4 load4(int x, int k) const {
-        const long off = KMAJOR ? (long)x * ld + k : (long)k * ld + x;
-        if (!EDGE) return *reinterpret_cast<const f32x4 *>(base + off);
-        const bool full = KMAJOR ? (x < XE && k + 3 < KE) : (k < KE && x + 3 < XE);
-        if (full && vec_ok) return *reinterpret_cast<const f32x4 *>(base + off);
-        f32x4 r = {0.f, 0.f, 0.f, 0.f};
+    template <class TAIL>
+    __device__ __forceinline__ f32x4 load4(int x, int k, TAIL) const {
+        if (!EDGE) return *reinterpret_cast<const f32x4 *>(base + (KMAJOR ? (long)x * ld + k : (long)k * ld + x));
+        f32x4_u v = {0.f, 0.f, 0.f, 0.f};
+        if (KMAJOR) {
+            const float *row = base + (long)(x < XE ? x : XE - 1) * ld;
+            if (!TAIL::value || KE >= 4) {
+                v = *reinterpret_cast<const f32x4_u *>(row + (!TAIL::value || k < KE - 4 ? k : KE - 4));
+            } else {
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int xx = KMAJOR ? x : x + e, kk = KMAJOR ? k + e : k;
-            if (xx < XE && kk < KE) r[e] = base[KMAJOR ? (long)xx * ld + kk : (long)kk * ld + xx];
+                for (int e = 0; e < 3; e++)
+                    if (e < KE) v[e] = row[e];
+            }
+        } else {
+            const float *row = base + (long)(!TAIL::value || k < KE ? k : KE - 1) * ld;
+            if (whole_loads()) {
+                const int last = TAIL::value ? XE - 4 : XE - 1;
+                v = *reinterpret_cast<const f32x4_u *>(row + (x < last ? x : last));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = row[x + e < XE ? x + e : XE - 1];
+            }
         }
-        return r;
+        return f32x4{v[0], v[1], v[2], v[3]};
     }
+    template <class TAIL>
+    __device__ __forceinline__ f32x4 finish4(f32x4 v, int x, int k, TAIL) const {
+        if (!EDGE || !TAIL::value) return v;
+        if (KMAJOR) return shifted_down(v, KE < 4 ? (k < KE ? 0 : 4) : k < KE - 4 ? 0 : k - (KE - 4));
+        const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+        return k < KE ? shifted_down(v, !whole_loads() || x < XE - 4 ? 0 : x - (XE - 4)) : none;
+    }
+    // (x contiguous) rows that hold four elements, and whose next row holds those that a load reads behind the end
+    __device__ __forceinline__ bool whole_loads() const { return XE >= 4 && ld >= 4; }
 };
 
 // Columns of C (rows x of the B operand) dealt to tiles in groups: the operand's XE-long x range is
@@ -111,27 +152,44 @@ struct linear_source {
 // consecutive units u out of every one of the G groups -- tile position x' stands for
 //     x = (x' % BN / UB) * UE + (x' / BN) * UB + x' % UB.
 // A workgroup then owns all G columns of its units, which is what an epilogue that combines them
-// (the gates of a recurrent cell) needs.  UB must be a multiple of 4 for operands whose x is contiguous.
+// (the gates of a recurrent cell) needs.  UB must be a multiple of 4 for operands whose x is contiguous.  Units of the last
+// tile behind the last one stand for the last one (operands whose x is contiguous: UE is a multiple of UB).
 template <int BN, int UB>
 __device__ __forceinline__ int regrouped_index(int x, int UE) {
-    return ((x % BN) / UB) * UE + (x / BN) * UB + (x % UB);
+    const int u = (x / BN) * UB + (x % UB);
+    return ((x % BN) / UB) * UE + (u < UE ? u : UE - 1);
 }
 template <class SRC, int BN, int UB>
 struct regrouped_rows {
+    static constexpr bool SEAM = SRC::SEAM;
     SRC src;
     int UE;
-    __device__ __forceinline__ auto load4(int x, int k) const { return src.load4(regrouped_index<BN, UB>(x, UE), k); }
+    template <class TAIL>
+    __device__ __forceinline__ f32x4 load4(int x, int k, TAIL tail) const { return src.load4(regrouped_index<BN, UB>(x, UE), k, tail); }
+    template <class TAIL>
+    __device__ __forceinline__ f32x4 finish4(f32x4 v, int x, int k, TAIL tail) const { return src.finish4(v, regrouped_index<BN, UB>(x, UE), k, tail); }
 };
 
 // Two operands behind one another along k: k < K1 reads the first, the rest the second (from its own
 // k = 0).  Lets several product terms that feed the same accumulators run as one pipelined loop;
-// K1 must be a multiple of 4 (a 16-byte load along k never straddles the seam).
-template <class S1, class S2>
+// K1 must be a multiple of 4 (a 16-byte load along k never straddles the seam).  RAGGED: the operands' own K is not K1 but
+// less (the first one's zeros fill up to K1), or rows of the first end where a load could reach behind it: every slice
+// is treated as a last one.
+template <class S1, class S2, bool RAGGED>
 struct concat_k {
+    static constexpr bool SEAM = RAGGED;
     S1 first;
     S2 second;
     int K1;
-    __device__ __forceinline__ f32x4 load4(int x, int k) const { return k < K1 ? first.load4(x, k) : second.load4(x, k - K1); }
+    template <class TAIL>
+    __device__ __forceinline__ f32x4 load4(int x, int k, TAIL tail) const {
+        return k < K1 ? first.load4(x, k, tail) : second.load4(x, k - K1, tail);
+    }
+    template <class TAIL>
+    __device__ __forceinline__ f32x4 finish4(f32x4 v, int x, int k, TAIL tail) const {
+        if (!TAIL::value) return v;
+        return k < K1 ? first.finish4(v, x, k, tail) : second.finish4(v, x, k - K1, tail);
+    }
 };
 
 // One operand tile of X x BK elements (X = BM for A, BN for B).
@@ -146,10 +204,10 @@ struct operand_tile {
 
     static __device__ __forceinline__ int swizzle(int x, int kq) { return x ^ (2 * (kq & 3)); }
 
-    // SRC::load4(x, k) returns 4 consecutive elements along the operand's contiguous direction:
-    // (x, k..k+3) for a K-major operand, (x..x+3, k) otherwise.
-    template <class SRC>
-    static __device__ __forceinline__ void load_global(const SRC &src, int x0, int k0, f32x4 (&regs)[NV]) {
+    // SRC::load4(x, k, tail) and finish4 give 4 consecutive elements along the operand's contiguous direction:
+    // (x, k..k+3) for a K-major operand, (x..x+3, k) otherwise.  The slice that was loaded is finished with the same `tail`.
+    template <class SRC, class TAIL>
+    static __device__ __forceinline__ void load_global(const SRC &src, int x0, int k0, f32x4 (&regs)[NV], TAIL tail) {
         const int t = threadIdx.x;
 #pragma unroll
         for (int v = 0; v < NV; v++) {
@@ -158,11 +216,12 @@ struct operand_tile {
             int x, k;
             if (KMAJOR) { k = 4 * (idx % (BK / 4)); x = idx / (BK / 4); }
             else        { x = 4 * (idx % (X / 4));  k = idx / (X / 4); }
-            regs[v] = src.load4(x0 + x, k0 + k);
+            regs[v] = src.load4(x0 + x, k0 + k, tail);
         }
     }
 
-    static __device__ __forceinline__ void store_lds(float *lds, const f32x4 (&regs)[NV]) {
+    template <class SRC, class TAIL>
+    static __device__ __forceinline__ void store_lds(float *lds, const f32x4 (&regs)[NV], const SRC &src, int x0, int k0, TAIL tail) {
         const int t = threadIdx.x;
 #pragma unroll
         for (int v = 0; v < NV; v++) {
@@ -170,10 +229,10 @@ struct operand_tile {
             if (PARTIAL && idx >= UNITS) break;
             if (KMAJOR) {
                 const int kq = idx % (BK / 4), x = idx / (BK / 4);
-                *reinterpret_cast<f32x4 *>(lds + kq * ROW + swizzle(x, kq) * 4) = regs[v];
+                *reinterpret_cast<f32x4 *>(lds + kq * ROW + swizzle(x, kq) * 4) = src.finish4(regs[v], x0 + x, k0 + 4 * kq, tail);
             } else {
                 const int xq = idx % (X / 4), k = idx / (X / 4);
-                *reinterpret_cast<f32x4 *>(lds + k * ROW + 4 * xq) = regs[v];
+                *reinterpret_cast<f32x4 *>(lds + k * ROW + 4 * xq) = src.finish4(regs[v], x0 + 4 * xq, k0 + k, tail);
             }
         }
     }
@@ -284,16 +343,28 @@ __device__ __forceinline__ void tile_accumulate(accumulators<CFG> &acc, const SR
     // instructions the memory instructions are dealt out one per matrix instruction (scheduling
     // group barriers below); the steady-state slice is branch-free so that this is one scheduling
     // region, and the last two slices are peeled.
+    // With EDGE the last slice (sources with a seam: every one) may reach behind K and is loaded and stored as such.
+    constexpr bool ALL_TAILS = CFG::EDGE && (SRCA::SEAM || SRCB::SEAM);
+    typedef std::integral_constant<bool, ALL_TAILS> inner_t;
+    typedef std::integral_constant<bool, CFG::EDGE> last_t;
     const int KT = (K + BK - 1) / BK;
-    opA::load_global(A, m0, 0, ra[0]);
-    opB::load_global(B, n0, 0, rb[0]);
-    opA::store_lds(stage_a(0), ra[0]);
-    opB::store_lds(stage_b(0), rb[0]);
+    if (CFG::EDGE && KT <= 0) return;
+    auto load = [&](int s, int slot, auto tail) {
+        opA::load_global(A, m0, s * BK, ra[slot], tail);
+        opB::load_global(B, n0, s * BK, rb[slot], tail);
+    };
+    auto store = [&](int s, int slot, auto tail) {
+        opA::store_lds(stage_a(s & 1), ra[slot], A, m0, s * BK, tail);
+        opB::store_lds(stage_b(s & 1), rb[slot], B, n0, s * BK, tail);
+    };
+    constexpr bool ONE_KIND = inner_t::value == last_t::value;
+    if (ONE_KIND || KT > 1) { load(0, 0, inner_t()); store(0, 0, inner_t()); }
+    else { load(0, 0, last_t()); store(0, 0, last_t()); }
 #pragma unroll
     for (int s = 1; s <= D; s++)
         if (s < KT) {
-            opA::load_global(A, m0, s * BK, ra[s % D]);
-            opB::load_global(B, n0, s * BK, rb[s % D]);
+            if (ONE_KIND || s + 1 < KT) load(s, s % D, inner_t());
+            else load(s, s % D, last_t());
         }
     __syncthreads();
     read_frags(0, 0, 0);
@@ -310,20 +381,16 @@ __device__ __forceinline__ void tile_accumulate(accumulators<CFG> &acc, const SR
     constexpr int MFMAS = 4 * TM * TN;                                   // per fragment set
     constexpr int FRAG_READS = TM + (CFG::B_KMAJOR ? TN : 2 * TN) + (CFG::A_KMAJOR ? 0 : TM);  // LDS read instructions per set (approx.)
     // one slice; MORE: another slice follows (in register slot `slot`); LOAD: the slice D after that
-    // one exists and takes its place in the slot
-    auto slice = [&](int kt, int slot, auto more_c, auto load_c) {
+    // one exists and takes its place in the slot; STORED, LOADED: whether those two are inner slices or the last one
+    auto slice = [&](int kt, int slot, auto more_c, auto load_c, auto stored_c, auto loaded_c) {
         constexpr bool MORE = decltype(more_c)::value, LOAD = decltype(load_c)::value;
         const int cur = kt & 1;
 #pragma unroll
         for (int q = 0; q < Q; q++) {
             const int buf = q & 1;
             if (q == 0 && MORE) {
-                opA::store_lds(stage_a(cur ^ 1), ra[slot]);
-                opB::store_lds(stage_b(cur ^ 1), rb[slot]);
-                if (LOAD) {
-                    opA::load_global(A, m0, (kt + 1 + D) * BK, ra[slot]);
-                    opB::load_global(B, n0, (kt + 1 + D) * BK, rb[slot]);
-                }
+                store(kt + 1, slot, stored_c);
+                if (LOAD) load(kt + 1 + D, slot, loaded_c);
             }
             if (q + 1 < Q) {
                 read_frags(cur, q + 1, buf ^ 1);
@@ -368,21 +435,26 @@ __device__ __forceinline__ void tile_accumulate(accumulators<CFG> &acc, const SR
             else { if (MFMAS > FRAG_READS) __builtin_amdgcn_sched_group_barrier(0x008, REST_MID, 0); }
         }
     };
+    typedef std::true_type yes;
+    typedef std::false_type no;
     if (D == 1) {
         int kt = 0;
-        for (; kt + 2 < KT; kt++) slice(kt, 0, std::true_type(), std::true_type());
-        if (kt + 1 < KT) { slice(kt, 0, std::true_type(), std::false_type()); kt++; }
-        if (kt < KT) slice(kt, 0, std::false_type(), std::false_type());
+        for (; kt + 2 + (ONE_KIND ? 0 : 1) < KT; kt++) slice(kt, 0, yes(), yes(), inner_t(), inner_t());
+        if (!ONE_KIND && kt + 2 < KT) { slice(kt, 0, yes(), yes(), inner_t(), last_t()); kt++; }
+        if (kt + 1 < KT) { slice(kt, 0, yes(), no(), last_t(), last_t()); kt++; }
+        if (kt < KT) slice(kt, 0, no(), no(), last_t(), last_t());
     } else {
         // unrolled by D so that every register slot index is a constant
         for (int kt0 = 0; kt0 < KT; kt0 += D) {
 #pragma unroll
             for (int d = 0; d < D; d++) {
-                const int kt = kt0 + d;
+                const int kt = kt0 + d, slot = (d + 1) % D;
                 if (kt >= KT) break;
-                if (kt + 1 + D < KT) slice(kt, (d + 1) % D, std::true_type(), std::true_type());
-                else if (kt + 1 < KT) slice(kt, (d + 1) % D, std::true_type(), std::false_type());
-                else slice(kt, (d + 1) % D, std::false_type(), std::false_type());
+                if (kt + 1 + D + (ONE_KIND ? 0 : 1) < KT) slice(kt, slot, yes(), yes(), inner_t(), inner_t());
+                else if (!ONE_KIND && kt + 1 + D < KT) slice(kt, slot, yes(), yes(), inner_t(), last_t());
+                else if (kt + 1 + (ONE_KIND ? 0 : 1) < KT) slice(kt, slot, yes(), no(), inner_t(), inner_t());
+                else if (!ONE_KIND && kt + 1 < KT) slice(kt, slot, yes(), no(), last_t(), last_t());
+                else slice(kt, slot, no(), no(), last_t(), last_t());
             }
         }
     }
@@ -492,12 +564,12 @@ __device__ __forceinline__ void tile_epilogue(accumulators<CFG> &acc, int M, int
 
 template <class CFG, class VALUE, class STORE>
 __device__ __forceinline__ void tile_mainloop(const float *__restrict__ A, long lda, const float *__restrict__ B,
-                                              long ldb, int M, int N, int K, int m0, int n0, bool vec_ok,
+                                              long ldb, int M, int N, int K, int m0, int n0,
                                               float *lds, VALUE value, STORE store) {
     accumulators<CFG> acc;
     acc.clear();
-    linear_source<CFG::A_KMAJOR, CFG::EDGE> sa{A, lda, M, K, vec_ok};
-    linear_source<CFG::B_KMAJOR, CFG::EDGE> sb{B, ldb, N, K, vec_ok};
+    linear_source<CFG::A_KMAJOR, CFG::EDGE> sa{A, lda, M, K};
+    linear_source<CFG::B_KMAJOR, CFG::EDGE> sb{B, ldb, N, K};
     tile_accumulate<CFG>(acc, sa, sb, K, m0, n0, lds);
     if (tile_reduce_k<CFG>(acc, lds)) tile_epilogue<CFG>(acc, M, N, m0, n0, value, store);
 }
@@ -520,11 +592,11 @@ struct axpby_store {
 template <class CFG>
 __global__ void __launch_bounds__(CFG::NT) sgemm_kernel(const float *__restrict__ A, const float *__restrict__ B,
                                                          float *__restrict__ C, int M, int N, int K, long lda, long ldb,
-                                                         long ldc, float alpha, float beta, int vec_ok) {
+                                                         long ldc, float alpha, float beta) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     int tm, tn;
     tile_of_block((M + CFG::BM - 1) / CFG::BM, (N + CFG::BN - 1) / CFG::BN, tm, tn);
-    tile_mainloop<CFG>(A, lda, B, ldb, M, N, K, tm * CFG::BM, tn * CFG::BN, vec_ok != 0, lds, axpby_value{C, ldc, alpha, beta},
+    tile_mainloop<CFG>(A, lda, B, ldb, M, N, K, tm * CFG::BM, tn * CFG::BN, lds, axpby_value{C, ldc, alpha, beta},
                        axpby_store{C, ldc});
 }
 
@@ -538,13 +610,13 @@ struct sgemm_batch {
 
 template <class CFG>
 __global__ void __launch_bounds__(CFG::NT) sgemm_batched_kernel(const sgemm_batch batch, int M, int N, int K, long lda, long ldb,
-                                                                 long ldc, float alpha, float beta, int vec_ok) {
+                                                                 long ldc, float alpha, float beta) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     int tm, tn;
     tile_of_block((M + CFG::BM - 1) / CFG::BM, (N + CFG::BN - 1) / CFG::BN, tm, tn);
     const float *A = batch.A[blockIdx.z], *B = batch.B[blockIdx.z];
     float *C = batch.C[blockIdx.z];
-    tile_mainloop<CFG>(A, lda, B, ldb, M, N, K, tm * CFG::BM, tn * CFG::BN, vec_ok != 0, lds, axpby_value{C, ldc, alpha, beta},
+    tile_mainloop<CFG>(A, lda, B, ldb, M, N, K, tm * CFG::BM, tn * CFG::BN, lds, axpby_value{C, ldc, alpha, beta},
                        axpby_store{C, ldc});
 }
 

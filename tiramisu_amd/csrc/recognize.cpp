@@ -1505,8 +1505,13 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     const std::string kname = "_kernel_" + std::to_string(ctx.next_kernel_id());
     // several product terms over plain operands: one pipelined loop over the concatenated reduction ranges
     // (a call per term would drain and refill the pipeline between the terms)
-    bool merge_terms = !bf16 && operands.size() > 1 && lit && Kl % 4 == 0 && !backend_option("TIRAMISU_MFMA_SEPARATE_TERMS");
+    bool merge_terms = !bf16 && operands.size() > 1 && lit && !backend_option("TIRAMISU_MFMA_SEPARATE_TERMS");
     for (auto &o : operands) merge_terms = merge_terms && o.first.linear && o.second.linear;
+    // a range that is not a multiple of a 16-byte load is followed by zeros up to one; an operand with k outermost may not be
+    // read behind its last row, which lies inside the joint range
+    const std::string K1_text = std::to_string((Kl + 3) / 4 * 4);
+    bool ragged_terms = lit && Kl % 4 != 0;
+    for (auto &o : operands) ragged_terms = ragged_terms || (edge && !(o.first.kmajor && o.second.kmajor));
     for (auto &o : operands) {
         if (!merge_terms || term == 0) body << "    {\n";
         if (bf16) {
@@ -1547,8 +1552,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
                 body << "        const float *" << nm << "p = " << g->buf->get_name() << " + (" << dev.print(g->base) << ");\n";
                 body << "        const long " << nm << "ld = " << dev.print(g->ld) << ";\n";
                 body << "        const tgemm::linear_source<" << (g->kmajor ? "true" : "false") << ", " << (edge ? "true" : "false") << "> " << nm
-                     << "{" << nm << "p, " << nm << "ld, " << (which == 0 ? "_M" : "_N") << ", _K, (" << nm << "ld % 4 == 0) && ((uintptr_t)" << nm
-                     << "p % 16 == 0)};\n";
+                     << "{" << nm << "p, " << nm << "ld, " << (which == 0 ? "_M" : "_N") << ", _K};\n";
             } else {
                 // gather source: offsets are separable sums over the digits of the row and k indices
                 const std::string sname = kname + "_src" + std::to_string(term) + (which == 0 ? "a" : "b");
@@ -1579,14 +1583,20 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
                     body << "        for (int _k = threadIdx.x; _k < _K; _k += CFG::NT) _ktab[_k] = " << sname << "::koff(_k);\n";
                     body << "        __syncthreads();\n";
                 }
-                pre << "    __device__ __forceinline__ tgemm::f32x4 load4(int x, int k) const {\n";
-                const char *full = g->gather_kdir ? "(x < XE && k + 3 < KE)" : "(k < KE && x + 3 < XE)";
-                if (g->gather_vec)
-                    pre << "        if (" << (edge ? full : "true") << ") { tgemm::f32x4_u v = *reinterpret_cast<const tgemm::f32x4_u *>(base + offset(x, k)); "
-                           "return tgemm::f32x4{v[0], v[1], v[2], v[3]}; }\n";
-                pre << "        tgemm::f32x4 r = {0.f, 0.f, 0.f, 0.f};\n";
-                pre << "        for (int e = 0; e < 4; e++) {\n            const int xx = " << (g->kmajor ? "x" : "x + e") << ", kk = " << (g->kmajor ? "k + e" : "k")
-                    << ";\n            if (xx < XE && kk < KE) r[e] = base[offset(xx, kk)];\n        }\n        return r;\n    }\n};\n";
+                // as linear_source: what lies behind the ends is loaded from the nearest place inside, and zero behind the
+                // last k when it is stored (where four elements are contiguous the extent is a multiple of four)
+                pre << "    static constexpr bool SEAM = false;\n";
+                pre << "    template <class TAIL> __device__ __forceinline__ tgemm::f32x4 load4(int x, int k, TAIL) const {\n";
+                if (g->gather_vec) {
+                    if (edge) pre << "        x = min(x, XE - " << (g->gather_kdir ? 1 : 4) << ");\n        if (TAIL::value) k = min(k, KE - " << (g->gather_kdir ? 4 : 1) << ");\n";
+                    pre << "        const tgemm::f32x4_u v = *reinterpret_cast<const tgemm::f32x4_u *>(base + offset(x, k));\n"
+                           "        return tgemm::f32x4{v[0], v[1], v[2], v[3]};\n    }\n";
+                } else {
+                    if (edge) pre << "        if (TAIL::value) k = min(k, KE - 1);\n";
+                    pre << "        tgemm::f32x4 r;\n        for (int e = 0; e < 4; e++) r[e] = base[offset(" << (edge ? "min(x + e, XE - 1)" : "x + e") << ", k)];\n        return r;\n    }\n";
+                }
+                pre << "    template <class TAIL> __device__ __forceinline__ tgemm::f32x4 finish4(tgemm::f32x4 v, int, int k, TAIL) const {\n"
+                       "        const tgemm::f32x4 none = {0.f, 0.f, 0.f, 0.f};\n        return !TAIL::value || k < KE ? v : none;\n    }\n};\n";
                 body << "        const " << sname << " " << nm << "{" << g->buf->get_name() << " + (" << dev.print(g->base) << "), " << (which == 0 ? "_M" : "_N")
                      << ", _K, " << (tabulate ? "_ktab" : "nullptr") << "};\n";
             }
@@ -1601,11 +1611,11 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
             for (int t = 1; t < term; t++) {
                 for (std::string *nm : {&a_name, &b_name}) {
                     const std::string next = std::string(nm == &a_name ? "_A" : "_B") + std::to_string(t), cat = *nm + "c";
-                    body << "        const tgemm::concat_k<decltype(" << *nm << "), decltype(" << next << ")> " << cat << "{" << *nm << ", " << next << ", " << t << " * _K};\n";
+                    body << "        const tgemm::concat_k<decltype(" << *nm << "), decltype(" << next << "), " << (ragged_terms ? "true" : "false") << "> " << cat << "{" << *nm << ", " << next << ", " << t << " * " << K1_text << "};\n";
                     *nm = cat;
                 }
             }
-            k_text = std::to_string(term) + " * _K";
+            k_text = std::to_string(term - 1) + " * " + K1_text + " + _K";
         }
         if (with_consumer) {
             body << "        const tgemm::regrouped_rows<decltype(" << b_name << "), CFG::BN, " << UB << "> _Bq{" << b_name << ", " << UE << "};\n";
