@@ -9,7 +9,9 @@ It contains no compute of its own and has no CPU fallback: loading fails loudly 
 HIP libraries were not built.
 """
 import ctypes
+import math
 import os
+import struct
 
 import numpy as np
 
@@ -33,6 +35,15 @@ class halide_buffer_t(ctypes.Structure):
 
 
 _TYPE_CODES = {"i": 0, "u": 1, "f": 2, "b": 1}
+_DIMENSIONS_OF = ctypes.POINTER(halide_dimension_t)
+_tensor_types = {}                                            # torch's element types as numpy's
+
+
+def _tensor_type(t):
+    if t not in _tensor_types:
+        import torch
+        _tensor_types[t] = np.dtype(np.uint16) if t == torch.bfloat16 else np.dtype(str(t).replace("torch.", ""))
+    return _tensor_types[t]
 
 
 class Buffer:
@@ -42,23 +53,25 @@ class Buffer:
     (M, N) has dim[0] = N (stride 1) and dim[1] = M (stride N)."""
 
     def __init__(self, shape, dtype, host_ptr=0, device_ptr=0, keepalive=None):
+        # (every argument of every call that is given as a tensor or an array passes here: structures are filled in one
+        # go, without an object per dimension)
         dtype = np.dtype(dtype)
         self.keepalive = keepalive
-        self.shape, self.dtype, self.on_device = tuple(int(v) for v in shape), dtype, bool(device_ptr)
-        nd = len(shape)
+        self.shape, self.dtype, self.on_device = tuple([int(v) for v in shape]), dtype, bool(device_ptr)
+        nd = len(self.shape)
         self.dims = (halide_dimension_t * max(nd, 1))()
-        stride = 1
-        for i, extent in enumerate(reversed(shape)):
-            self.dims[i] = halide_dimension_t(0, int(extent), stride, 0)
-            stride *= int(extent)
-        self.raw = halide_buffer_t()
-        self.raw.device = device_ptr
-        self.raw.device_interface = None
-        self.raw.host = host_ptr
-        self.raw.flags = 0
-        self.raw.type = halide_type_t(_TYPE_CODES[dtype.kind], dtype.itemsize * 8, 1)
-        self.raw.dimensions = nd
-        self.raw.dim = ctypes.cast(self.dims, ctypes.POINTER(halide_dimension_t))
+        stride, numbers = 1, []
+        for extent in reversed(self.shape):
+            numbers += (0, extent, stride, 0)
+            stride *= extent
+        self.elements = stride
+        try:
+            struct.pack_into("=%di" % len(numbers), self.dims, 0, *numbers)
+        except struct.error:                    # beyond 31 bits: the fields hold the low 32 of them
+            for i in range(nd):
+                self.dims[i] = halide_dimension_t(*numbers[4 * i:4 * i + 4])
+        self.raw = halide_buffer_t(device_ptr, None, host_ptr, 0, (_TYPE_CODES[dtype.kind], dtype.itemsize * 8, 1), nd,
+                                   _DIMENSIONS_OF.from_buffer(ctypes.c_void_p(ctypes.addressof(self.dims))))
 
     @staticmethod
     def from_numpy(a):
@@ -76,16 +89,12 @@ class Buffer:
         """A ``torch.Tensor`` as an argument, without a copy: a tensor on the GPU describes a buffer tagged
         tag_gpu_global() (its storage is the device pointer), a CPU tensor a host buffer.  bfloat16 tensors
         are the 16-bit storage of p_bfloat16 buffers.  The tensor stays referenced while the buffer lives."""
-        import torch
         if not t.is_contiguous():
             raise ValueError("Tiramisu buffers are dense row-major: pass a contiguous tensor")
-        if t.dtype == torch.bfloat16:
-            dtype = np.dtype(np.uint16)
-        else:
-            dtype = np.dtype(str(t.dtype).replace("torch.", ""))
+        dtype = _tensor_type(t.dtype)
         if t.is_cuda:
-            return Buffer(tuple(t.shape), dtype, device_ptr=t.data_ptr(), keepalive=t)
-        return Buffer(tuple(t.shape), dtype, host_ptr=t.data_ptr(), keepalive=t)
+            return Buffer(t.shape, dtype, device_ptr=t.data_ptr(), keepalive=t)
+        return Buffer(t.shape, dtype, host_ptr=t.data_ptr(), keepalive=t)
 
     def pointer(self):
         return ctypes.byref(self.raw)
@@ -168,6 +177,8 @@ class Program:
     type, constant extents, host or device memory): a wrong buffer would otherwise be a
     out-of-bounds access on the GPU."""
 
+    expected = None          # _expected_arguments(), from the first check on
+
     def __init__(self, library_path, function_name, needs_gpu_runtime=True):
         if not os.path.exists(library_path):
             raise RuntimeError("%s is missing: run __graft_entry__.build() first" % library_path)
@@ -179,23 +190,32 @@ class Program:
         self.name = function_name
         self.manifest = manifest_of(library_path, function_name) if needs_gpu_runtime else None
 
-    def check(self, bufs):
-        expected = self.manifest["arguments"]
-        if len(bufs) != len(expected):
-            raise ValueError("%s takes %d buffers, %d given" % (self.name, len(expected), len(bufs)))
-        for b, e in zip(bufs, expected):
-            if np.dtype(_C_TYPES.get(e["type"], b.dtype)) != b.dtype:
-                raise ValueError("%s: buffer %s holds %s, %s given" % (self.name, e["name"], e["type"], b.dtype))
-            if (e["memory"] == "device") != b.on_device:
-                raise ValueError("%s: buffer %s lives in %s memory" % (self.name, e["name"], e["memory"]))
+    def _expected_arguments(self):
+        """What check() compares: (description, element type, on the device, number of elements) of every argument,
+        None where anything will do."""
+        out = []
+        for e in self.manifest["arguments"]:
             # a host input may be declared larger than what the program reads of it (the reference's
             # sgemm generators declare their two scalars over the row range); anything the GPU
             # touches, and every output, must have the declared number of elements
             strict = e["memory"] == "device" or e["kind"] != "input"
-            if strict and all(isinstance(v, int) for v in e["shape"]):
-                want = int(np.prod(e["shape"])) if e["shape"] else 1
-                if int(np.prod(b.shape)) != want:
-                    raise ValueError("%s: buffer %s has shape %s, %s given" % (self.name, e["name"], e["shape"], list(b.shape)))
+            constant = strict and all(isinstance(v, int) for v in e["shape"])
+            out.append((e, np.dtype(_C_TYPES[e["type"]]) if e["type"] in _C_TYPES else None, e["memory"] == "device",
+                        math.prod(e["shape"]) if constant else None))
+        return out
+
+    def check(self, bufs):
+        if self.expected is None:
+            self.expected = self._expected_arguments()
+        if len(bufs) != len(self.expected):
+            raise ValueError("%s takes %d buffers, %d given" % (self.name, len(self.expected), len(bufs)))
+        for b, (e, dtype, on_device, elements) in zip(bufs, self.expected):
+            if dtype is not None and dtype != b.dtype:
+                raise ValueError("%s: buffer %s holds %s, %s given" % (self.name, e["name"], e["type"], b.dtype))
+            if on_device != b.on_device:
+                raise ValueError("%s: buffer %s lives in %s memory" % (self.name, e["name"], e["memory"]))
+            if elements is not None and b.elements != elements:
+                raise ValueError("%s: buffer %s has shape %s, %s given" % (self.name, e["name"], e["shape"], list(b.shape)))
 
     def __call__(self, *args):
         """Arguments: ``Buffer`` objects, numpy arrays (host buffers) or torch tensors (host or GPU buffers by where
