@@ -109,7 +109,13 @@ def test_seeded_sweep_of_shapes():
 DOUBLE_CASES = [(70, 50, 30, False, False), (64, 96, 128, True, False), (33, 65, 17, False, True), (128, 128, 64, True, True),
                 # enough 128 x 128 tiles for the large-tile kernel, ragged in M, N and K, all four transposition cases
                 (1500, 1430, 250, False, False), (1500, 1430, 250, True, False), (1500, 1430, 250, False, True), (1411, 1600, 77, True, True),
-                (1, 1, 1, False, False), (17, 3000, 5, False, False)]
+                (1, 1, 1, False, False), (17, 3000, 5, False, False),
+                # the other tiles: 96 x 96 and 128 x 128 with a last slice of 1 and of 15 k, 64 x 64 whose groups of wavefronts share
+                # a slice (last one of 1 and 63 k), 32 x 32 with and without shared slices, 16 x 16 (last slice 1 and 127 of 128 k)
+                (1999, 1101, 673, False, True), (1999, 1101, 687, True, False), (2047, 2033, 257, False, False), (2047, 2033, 271, True, True),
+                (1001, 999, 961, False, False), (1023, 1001, 1023, True, True), (301, 1799, 97, True, False), (301, 1799, 3, False, True),
+                (499, 511, 513, False, True), (511, 499, 575, True, False), (15, 17, 1921, False, False), (33, 31, 2047, True, True),
+                (16, 16, 128, False, True), (5, 7, 127, True, False)]
 
 
 @pytest.mark.parametrize("M,N,K,tA,tB", DOUBLE_CASES)
