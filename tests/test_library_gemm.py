@@ -36,7 +36,8 @@ def run(M, N, K, alpha, beta, tA=False, tB=False, pad=0, off=0, seed=0):
 
 
 @pytest.mark.parametrize("M,N,K", [(64, 64, 64), (64, 64, 48), (100, 70, 50), (640, 2048, 512), (2048, 2048, 48),
-                                   (3072, 3072, 32), (4096, 4096, 64), (33, 17, 9), (8, 8, 4)])
+                                   (3072, 3072, 32), (4096, 4096, 64), (33, 17, 9), (8, 8, 4),
+                                   (512, 512, 512), (1024, 768, 192)])
 def test_square_tiles(M, N, K):
     run(M, N, K, 1.0, 0.0)
     run(M, N, K, 3.0, 2.0, seed=1)
@@ -67,7 +68,9 @@ def test_transposed_operands_padding_and_offsets(tA, tB):
     run(50, 30, 20, 1.0, 0.0, tA=tA, tB=tB, pad=3, off=5)
 
 
-@pytest.mark.parametrize("M,N,K", [(33, 35, 9), (65, 130, 33), (129, 67, 130), (64, 70, 64), (300, 260, 2051)])
+@pytest.mark.parametrize("M,N,K", [(33, 35, 9), (65, 130, 33), (129, 67, 130), (64, 70, 64), (300, 260, 2051),
+                                   # 64 x 32 tiles; thin ones: 32 x 32 tiles of which a row or column of C is a part
+                                   (1000, 1500, 65), (1, 700, 40), (700, 3, 67), (17, 31, 2100), (5, 6, 9), (1, 1, 64)])
 @pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("pad", [0, 3])
 def test_sizes_that_end_inside_a_tile(M, N, K, tA, tB, pad):

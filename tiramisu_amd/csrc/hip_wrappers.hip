@@ -195,6 +195,14 @@ void dispatch_tile(const float *A, const float *B, float *C, int M, int N, int K
         launch_mfma<tgemm::config<64, 64, 32, 2, 2, AK, BK_, EDGE>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
 
+// 64 x 32 and 32 x 32 tiles: slices of 64 k, shared by four groups of wavefronts
+template <bool AK, bool BK_, int BM, int BN>
+void launch_small(bool edge, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc, float alpha, float beta) {
+    constexpr int WGM = BM / 32, WGN = BN / 32;
+    if (edge) launch_mfma<tgemm::config<BM, BN, 64, WGM, WGN, AK, BK_, true, 1, 4>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else launch_mfma<tgemm::config<BM, BN, 64, WGM, WGN, AK, BK_, false, 1, 4>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+}
+
 // Few C tiles but a long reduction (a batch of 64 rows against wide weights, as in recurrent
 // cells): 64x32 tiles, 8 groups of wavefronts share the K range of each tile and reduce through
 // LDS, and up to four K-slices are requested ahead (the launch is latency-bound).
@@ -364,8 +372,16 @@ void *static_scratch_here() {
 }
 
 template <bool AK, bool BK_>
-void dispatch_edge(bool edge, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb,
+void dispatch_edge(bool vec_ok, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb,
                    long ldc, float alpha, float beta) {
+    const int bm = tile_for(M, N);
+    const bool edge = !(vec_ok && M % bm == 0 && N % bm == 0 && K % (bm == 64 ? 32 : 16) == 0);   // K-slice of the tile
+    if (bm == 64 || M < 32 || N < 32) {
+        const ttarget::small_tile t = ttarget::small_tile_for(M, N, K, active_batch ? active_batch_count : 1, !edge);
+        const bool slices = vec_ok && K % 64 == 0;
+        if (t == ttarget::TILE_64x32) return launch_small<AK, BK_, 64, 32>(!(slices && M % 64 == 0 && N % 32 == 0), A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+        if (t == ttarget::TILE_32) return launch_small<AK, BK_, 32, 32>(!(slices && M % 32 == 0 && N % 32 == 0), A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    }
     if (edge) dispatch_tile<AK, BK_, true>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     else dispatch_tile<AK, BK_, false>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
@@ -532,11 +548,13 @@ static int sgemm_impl(const char *fn, bool static_scratch, float *A, float *B, f
     }
     const int m = (int)M, n = (int)N, k = (int)K;
     const bool vec_ok = (ldA % 4 == 0) && (ldB % 4 == 0) && ((uintptr_t)a % 16 == 0) && ((uintptr_t)b % 16 == 0);
-    const bool small = (m < 32 || n < 32 || k < 8);
+    // Products of a few k are one thread per element.  Thin ones (a dimension of C below a tile's 32) are one row or column of
+    // 32 x 32 tiles, without scratch: guarded, the rest of the tile is work for nothing, but one thread per element walked K alone.
+    const bool small = k < 8, thin = m < 32 || n < 32;
     if (batch_open && !static_scratch) {
         // inside a batch scope: remember the call; tiramisu_hip_batch_end launches it, together with the calls of
         // the same shape that follow it
-        const bool to_mfma = !small && (skinny(m, n, k, vec_ok, transposeA) || plan_splitk(m, n, k, SPLITK_WORKSPACE_LIMIT).chunks <= 1);
+        const bool to_mfma = !small && !thin && (skinny(m, n, k, vec_ok, transposeA) || plan_splitk(m, n, k, SPLITK_WORKSPACE_LIMIT).chunks <= 1);
         batch_calls.push_back({a, b, c, M, N, K, alpha, beta, ldA, ldB, ldC, transposeA, transposeB, vec_ok, to_mfma});
         return 0;
     }
@@ -555,7 +573,7 @@ static int sgemm_impl(const char *fn, bool static_scratch, float *A, float *B, f
         return 0;
     }
     // few tiles, deep reduction: K split over workgroups through a scratch buffer
-    const splitk_plan plan = plan_splitk(m, n, k, SPLITK_WORKSPACE_LIMIT);
+    const splitk_plan plan = thin ? splitk_plan() : plan_splitk(m, n, k, SPLITK_WORKSPACE_LIMIT);
     if (plan.chunks > 1) {
         void *ws;
         if (static_scratch) {
@@ -583,13 +601,11 @@ static int sgemm_impl(const char *fn, bool static_scratch, float *A, float *B, f
         dispatch_splitk(plan, transposeA, transposeB, edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta, ws);
         return 0;
     }
-    const int bm = tile_for(m, n);
-    const bool edge = !(vec_ok && m % bm == 0 && n % bm == 0 && k % (bm == 64 ? 32 : 16) == 0);   // K-slice of the tile
     // A is K-contiguous unless transposed; B is K-contiguous only when transposed.
-    if (!transposeA && !transposeB) dispatch_edge<true, false>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
-    else if (!transposeA && transposeB) dispatch_edge<true, true>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
-    else if (transposeA && !transposeB) dispatch_edge<false, false>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
-    else dispatch_edge<false, true>(edge, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
+    if (!transposeA && !transposeB) dispatch_edge<true, false>(vec_ok, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
+    else if (!transposeA && transposeB) dispatch_edge<true, true>(vec_ok, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
+    else if (transposeA && !transposeB) dispatch_edge<false, false>(vec_ok, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
+    else dispatch_edge<false, true>(vec_ok, a, b, c, m, n, k, ldA, ldB, ldC, alpha, beta);
     return 0;
 }
 

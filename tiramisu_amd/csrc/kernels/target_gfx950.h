@@ -32,6 +32,30 @@ inline int square_tile_for(long M, long N) {
     return edge;
 }
 
+// Where 64 x 64 is the square tile chosen and its tiles are few, smaller ones whose four groups of wavefronts share a slice's k: the
+// launch is bound by the chain of a tile's slices, not by the matrix cores.  Modelled like the fp64 tiles: `fixed` microseconds and,
+// per k, `first` for a round of tiles over the compute units, `further` for each of several, whichever is more; 64 x 64 is faster
+// per k where no tile hangs over the operands.  Fits to whole launches at sizes that no tile divides (measured / modelled, us):
+// 700 x 900 x 1000 26.3 / 26.5 with 64 x 64, 26.4 / 25.8 with 64 x 32, 23.2 / 22.5 with 32 x 32; 1100 x 1300 x 2000 82 / 80, 69 / 71,
+// 76 / 81; 2001 x 1501 x 1001 60 / 61, 67 / 71, 72 / 81; 400 x 400 x 500 14.5 / 14.8, 9.7 / 9.3, 8.1 / 7.5.
+enum small_tile { TILE_64, TILE_64x32, TILE_32 };
+inline small_tile small_tile_for(long M, long N, long K, long problems, bool whole) {
+    if (M < 32 || N < 32) return TILE_32;
+    static const struct { int m, n; double fixed, first, further; } model[3] = {
+        {64, 64, 3.0, 0.0235, 0.0193}, {64, 32, 3.2, 0.0122, 0.0113}, {32, 32, 3.0, 0.009, 0.0065}};
+    int best = 0;
+    double best_cost = 0;
+    for (int i = 0; i < 3; i++) {
+        const long tiles = ((M + model[i].m - 1) / model[i].m) * ((N + model[i].n - 1) / model[i].n) * problems;
+        const double rounds = (double)((tiles + ttarget::COMPUTE_UNITS - 1) / ttarget::COMPUTE_UNITS);
+        const bool whole_64 = i == 0 && whole;
+        const double first = whole_64 ? 0.0165 : model[i].first, further = rounds * (whole_64 ? 0.0155 : model[i].further);
+        const double cost = model[i].fixed + K * (first > further ? first : further);
+        if (i == 0 || cost < best_cost) { best = i; best_cost = cost; }
+    }
+    return (small_tile)best;
+}
+
 // C tiles of the bf16-input kernels.  A launch is modelled to take `fixed` microseconds (start, first slices, epilogue) plus,
 // for every 32 k, `first` for the first round of tiles over the compute units and `further` for each round after it.  The
 // figures are fits to whole launches of 100 ... 4096 k with a tenth of the chip's tiles up to sixteen rounds (measured /
