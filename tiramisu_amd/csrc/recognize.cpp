@@ -1166,6 +1166,20 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         // (4-layer LSTM cell, 64x2048x1024 per layer: 1.30 ms per pass against 1.55 ms)
         if ((long)products.size() * Kl >= 1024) { BK = 64; WGK = 4; DEPTH = 1; }
     }
+    // a plain product of few 64x64 tiles: smaller tiles whose groups of wavefronts share each slice, where they are modelled faster
+    // (kernels/target_gfx950.h)
+    bool plain = lit && !bf16 && !with_consumer && !batched && BM == 64 && BN == 64 && WGK == 1 && operands.size() == 1;
+    for (auto &o : operands) plain = plain && o.first.linear && o.second.linear;
+    for (const char *forced : {"TIRAMISU_MFMA_BM", "TIRAMISU_MFMA_BN", "TIRAMISU_MFMA_BK", "TIRAMISU_MFMA_WGM", "TIRAMISU_MFMA_WGN",
+                               "TIRAMISU_MFMA_WGK", "TIRAMISU_MFMA_NO_SPLITK"})
+        if (backend_option(forced)) plain = false;        // (they change the 64x64 tile's own figures)
+    if (plain) {
+        const ttarget::small_tile t = ttarget::small_tile_for(Ml, Nl, Kl, 1, Ml % 64 == 0 && Nl % 64 == 0 && Kl % 32 == 0);
+        if (t != ttarget::TILE_64) {
+            BM = t == ttarget::TILE_64x32 ? 64 : 32;
+            BN = 32; BK = 64; WGM = BM / 32; WGN = 1; WGK = 4;
+        }
+    }
     // at most one 64x64 tile per compute unit and a long reduction: two groups of wavefronts share each
     // (64-k) slice, so that every SIMD has two wavefronts to alternate between (1024^3: 20.6 us against 21.9)
     if (lit && !bf16 && BM == 64 && BN == 64 && WGK == 1 && Ml % 64 == 0 && Nl % 64 == 0 && Kl % 64 == 0 && Kl >= 512 &&
