@@ -158,3 +158,36 @@ def test_gpu_sizes_that_end_inside_a_tile(M, N, K, what, programs_dir):
     d = [DeviceArray(a) for a in (to_bf16(A), to_bf16(B), C)]
     runtime.load(programs_dir, name_of(M, N, K))(np.array([2.0, 0.5], np.float32), *[x.buffer() for x in d])
     assert np.array_equal(d[2].download(), exact)
+
+
+VIEWS = [("a_backwards", 200, 150, 100), ("b_backwards", 200, 150, 100), ("a_backwards_whole", 128, 192, 128), ("b_backwards_whole", 128, 192, 128),
+         ("b_overlapping", 66, 30, 50)]
+
+
+@pytest.mark.parametrize("form", [v[0] for v in VIEWS])
+def test_operands_walked_backwards_or_overlapping_are_not_loaded_straight_into_lds(form, programs_dir):
+    """Those loads address an operand by 32-bit offsets from its first row and rely on what follows its last row reading as zero."""
+    import json
+    kernels = json.load(open(os.path.join(programs_dir, "build", "sgemm_bf16_%s.o.json" % form)))["kernels"]
+    assert len(kernels) == 1 and "v_mfma_f32_32x32x16_bf16" in kernels[0]["how"] and "straight into LDS" not in kernels[0]["how"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,M,N,K", VIEWS)
+def test_gpu_operands_walked_backwards_or_overlapping(form, M, N, K, programs_dir):
+    from gpu_util import DeviceArray
+    rng = np.random.RandomState(M + N + K)
+    A, B = rng.randint(-3, 4, (M, K)).astype(np.float32), rng.randint(-3, 4, (K, N)).astype(np.float32)
+    C = rng.randint(-8, 9, (M, N)).astype(np.float32)
+    stored_a, stored_b = A, B
+    if form.startswith("a_"):
+        stored_a = A[::-1]
+    elif form != "b_overlapping":
+        stored_b = B[::-1]
+    else:                                       # row k begins at element 2 k: what lies behind the last row must not be used
+        stored_b = np.full((K, N + 2 * K), np.inf, np.float32)
+        stored_b[0, :2 * (K - 1) + N] = rng.randint(-3, 4, 2 * (K - 1) + N)
+        B = np.stack([stored_b[0, 2 * k:2 * k + N] for k in range(K)])
+    d = [DeviceArray(a) for a in (to_bf16(stored_a), to_bf16(stored_b), C)]
+    runtime.load(programs_dir, "sgemm_bf16_" + form)(*[x.buffer() for x in d])
+    assert np.array_equal(d[2].download(), A @ B + C)       # integers: exact

@@ -1200,11 +1200,12 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     int bf16_stages = 2;                 // of the LDS ring
     if (bf16) {
         // the tile whose launch is modelled fastest (kernels/target_gfx950.h); rows of an even number of elements are
-        // loaded straight into LDS (32-bit offsets: operands below 2 GiB), others, and sizes known at run time only,
-        // through registers (guarded 64x64 tiles in the latter case)
+        // loaded straight into LDS (32-bit offsets from an operand's first row: operands below 2 GiB, walked forwards; rows
+        // of B that do not overlap, so that what follows the last one lies behind the operand), others, and sizes known
+        // at run time only, through registers (guarded 64x64 tiles in the latter case)
         for (auto &o : operands)
             if (!o.first.linear || !o.second.linear || !o.first.kmajor || o.second.kmajor) return reject(25);
-        bool aligned = true, dword_rows = true, small_enough = true;
+        bool aligned = true, dword_rows = true, small_enough = true, forwards = true;
         for (auto &o : operands) {
             long v;
             for (const operand_info *g : {&o.first, &o.second}) {
@@ -1215,11 +1216,12 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
             if (lit && literal_value(o.first.ld, lda) && literal_value(o.second.ld, ldb)) {
                 // (a tile's rows and slices may reach behind the operand: their offsets must not wrap either)
                 if ((double)(Ml + 256) * lda * 2 >= 2147483648.0 || (double)(Kl + 256) * ldb * 2 >= 2147483648.0) small_enough = false;
+                if (lda <= 0 || ldb < Nl) forwards = false;
             } else {
                 small_enough = false;
             }
         }
-        bf16_direct = lit && dword_rows && small_enough;
+        bf16_direct = lit && dword_rows && small_enough && forwards;
         const ttarget::bf16_tile tile = lit ? ttarget::bf16_tile_for(Ml, Nl, Kl, bf16_direct) : ttarget::BF16_TILE_ANY_SIZE;
         BM = BN = tile.edge;
         BK = tile.k;
