@@ -50,6 +50,9 @@ int main()
     generate({"b_backwards", 200, 150, 100, 100, 150, 1, 0, -1, 99});
     generate({"a_backwards_whole", 128, 192, 128, 128, 192, -1, 127, 1, 0});
     generate({"b_backwards_whole", 128, 192, 128, 128, 192, 1, 0, -1, 127});
+    generate({"odd_k", 200, 150, 101, 102, 150, 1, 0, 1, 0});
+    generate({"odd_n", 200, 149, 100, 100, 150, 1, 0, 1, 0});
+    generate({"odd_k_and_n", 129, 257, 33, 36, 258, 1, 0, 1, 0});
     generate({"b_overlapping", 66, 30, 50, 50, 130, 1, 0, 0, 0}, true);
     return 0;
 }

@@ -191,3 +191,20 @@ def test_gpu_operands_walked_backwards_or_overlapping(form, M, N, K, programs_di
     d = [DeviceArray(a) for a in (to_bf16(stored_a), to_bf16(stored_b), C)]
     runtime.load(programs_dir, "sgemm_bf16_" + form)(*[x.buffer() for x in d])
     assert np.array_equal(d[2].download(), A @ B + C)       # integers: exact
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,M,N,K,lda,ldb", [("odd_k", 200, 150, 101, 102, 150), ("odd_n", 200, 149, 100, 100, 150),
+                                                ("odd_k_and_n", 129, 257, 33, 36, 258)])
+def test_gpu_odd_parts_of_rows_of_an_even_number_of_elements(form, M, N, K, lda, ldb, programs_dir):
+    """The last element of the last row is the first half of a dword whose second half is not part of the operand."""
+    import json
+    from gpu_util import DeviceArray
+    assert "straight into LDS" in json.load(open(os.path.join(programs_dir, "build", "sgemm_bf16_%s.o.json" % form)))["kernels"][0]["how"]
+    rng = np.random.RandomState(M + N + K)
+    A, B = np.full((M, lda), np.inf, np.float32), np.full((K, ldb), np.inf, np.float32)
+    A[:, :K], B[:, :N] = rng.randint(1, 4, (M, K)), rng.randint(1, 4, (K, N))        # no zeros: a lost element shows
+    C = rng.randint(-8, 9, (M, N)).astype(np.float32)
+    d = [DeviceArray(a) for a in (to_bf16(A), to_bf16(B), C)]
+    runtime.load(programs_dir, "sgemm_bf16_" + form)(*[x.buffer() for x in d])
+    assert np.array_equal(d[2].download(), A[:, :K] @ B[:, :N] + C)       # integers: exact

@@ -310,9 +310,12 @@ __device__ __forceinline__ void tile_accumulate_bf16_direct(accumulators<CFG> &a
 
     // The loads are buffer loads (base in a resource descriptor, 32-bit byte offset per lane, one
     // scalar offset per operand that advances by a slice): no 64-bit address arithmetic in the loop,
-    // and an address past the operand reads as zero instead of faulting.
-    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, (int)((((long)M - 1) * lda + K) * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, (int)((((long)K - 1) * ldb + N) * 2), 0x00020000);
+    // and an address past the operand reads as zero instead of faulting.  The descriptor ends with a whole dword: one that
+    // begins inside and ends outside reads as zero, and an operand that ends with its first half (an odd part of rows of an
+    // even number of elements) would lose its last element.  The second half is padding of that row, or in the same dword
+    // behind it: masked behind K, or of a column that nobody stores.
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, (int)(((((long)M - 1) * lda + K + 1) & ~1L) * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, (int)(((((long)K - 1) * ldb + N + 1) & ~1L) * 2), 0x00020000);
     int va[LA], vb[LB];                              // per-lane byte offsets of this wave's loads within a slice
 #pragma unroll
     for (int v = 0; v < LA; v++) {
