@@ -208,3 +208,29 @@ def test_gpu_odd_parts_of_rows_of_an_even_number_of_elements(form, M, N, K, lda,
     d = [DeviceArray(a) for a in (to_bf16(A), to_bf16(B), C)]
     runtime.load(programs_dir, "sgemm_bf16_" + form)(*[x.buffer() for x in d])
     assert np.array_equal(d[2].download(), A[:, :K] @ B[:, :N] + C)       # integers: exact
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(200, 150, 100), (128, 192, 128), (1024, 1280, 512), (2000, 1500, 1006), (66, 2, 6)])
+@pytest.mark.parametrize("odd_a,odd_b", [(True, False), (False, True), (True, True)])
+def test_gpu_operands_that_begin_at_an_odd_element(M, N, K, odd_a, odd_b, programs_dir):
+    """Contiguous parts of larger tensors: the loads straight into LDS want multiples of four bytes, so another kernel serves
+    these addresses.  Infinities around the operands must not be used."""
+    import torch
+    rng = np.random.RandomState(M + N + K)
+
+    def part(rows, cols, odd):
+        flat = torch.full((rows * cols + 9,), float("inf"), dtype=torch.bfloat16)
+        values = rng.randint(-3, 4, (rows, cols)).astype(np.float32)
+        first = 7 if odd else 4
+        flat[first:first + rows * cols] = torch.from_numpy(values).flatten()
+        view = flat.cuda()[first:first + rows * cols].view(rows, cols)
+        assert view.data_ptr() % 4 == (2 if odd else 0)
+        return view, values
+
+    (dA, A), (dB, B) = part(M, K, odd_a), part(K, N, odd_b)
+    C = rng.randint(-8, 9, (M, N)).astype(np.float32)
+    dC = torch.from_numpy(C).cuda()
+    directory = PROGRAMS if os.path.exists(os.path.join(PROGRAMS, "build", name_of(M, N, K) + ".o.json")) else programs_dir
+    runtime.load(directory, name_of(M, N, K))(np.array([2.0, 0.5], np.float32), dA, dB, dC)
+    assert np.array_equal(dC.cpu().numpy(), 2.0 * (A @ B) + 0.5 * C)       # sums of at most 1006 products up to 9: exact in float32

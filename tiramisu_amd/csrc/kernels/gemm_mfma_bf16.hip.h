@@ -19,9 +19,10 @@
 // outside.  Without it: M % BM == 0, N % BN == 0, K % BK == 0, rows of A 16-byte and rows of B 8-byte aligned (the emitter
 // checks).  This variant serves rows of an odd number of elements (16-byte loads of any alignment cost little: the same
 // 64 x 64 tiles take 17.4 us for 2000 x 1500 x 1000 and 21.0 for 2001 x 1501 x 1001; guarded element by element, where
-// loads of such rows were and of every piece at an edge, 48.7 us), sizes known at run time only and operands of 2 GiB and
-// more.  Rows of an even number of elements use the second variant further down (tile_accumulate_bf16_direct: slices
-// loaded straight into an LDS ring).
+// loads of such rows were and of every piece at an edge, 48.7 us), sizes known at run time only, operands of 2 GiB and
+// more, walked backwards or with overlapping rows of B, and the calls that bring an operand at an odd element's address.
+// Other rows of an even number of elements use the second variant further down (tile_accumulate_bf16_direct: slices loaded
+// straight into an LDS ring).
 #ifndef TIRAMISU_AMD_GEMM_MFMA_BF16_HIP_H
 #define TIRAMISU_AMD_GEMM_MFMA_BF16_HIP_H
 #include "gemm_mfma.hip.h"
@@ -266,7 +267,8 @@ __device__ __forceinline__ void tile_accumulate_bf16(accumulators<CFG> &acc, con
 //     consecutive rows, swzB (0, 4, 10, 14 for k % 4; 0, 2, 4, 6 with rows of 64 columns) the four rows of a transposing read, over
 //     distinct 16-byte bank groups in both cases (measured: SQ_LDS_BANK_CONFLICT = 0).
 // A call ends with a barrier (every wave is past its last read), so it may be repeated for a second
-// pair of operands.  Rows of A and of B must be 4-byte aligned.
+// pair of operands.  Rows of A and of B must be 4-byte aligned (the emitted call looks at the operands' addresses), lda
+// positive and ldb at least N.
 // With EDGE the tiles may hang over the problem and K need not be a multiple of the slice.  What a load finds there needs
 // no guard: behind the last row of A and of B the buffer descriptor ends and reads give zero (it is checked dword by
 // dword, so the last row itself is whole); columns of B behind N are the start of the next row and only reach columns of C

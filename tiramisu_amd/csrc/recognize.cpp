@@ -1505,11 +1505,17 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
                             std::to_string(WGM) + ", " + std::to_string(WGN) + ", " + (operands[0].first.kmajor ? "true" : "false") + ", " +
                             (operands[0].second.kmajor ? "true" : "false") + ", " + (edge ? "true" : "false") + ", " + std::to_string(PADX) + ", " + std::to_string(WGK) + ", " + std::to_string(DEPTH) + ">";
     const int NT = 64 * WGM * WGN * WGK;
+    auto bf16_config_text = [](bool direct, int tile, int k, int waves_m, int waves_n, int stages, bool guarded) {
+        std::ostringstream os;
+        os << "    typedef tgemm::config_bf16" << (direct ? "_direct<" : "<") << tile << ", " << tile << ", " << k << ", " << waves_m << ", " << waves_n;
+        if (direct) os << ", " << stages;
+        os << (guarded ? ", true" : ", false") << "> CFG;\n";
+        return os.str();
+    };
     if (bf16) {
         body << "    extern __shared__ __attribute__((aligned(16))) uint32_t _lds[];\n";
         // slices go straight from global memory into an LDS ring where they can
-        if (bf16_direct) body << "    typedef tgemm::config_bf16_direct<" << BM << ", " << BN << ", " << BK << ", " << WGM << ", " << WGN << ", " << bf16_stages << (edge ? ", true" : ", false") << "> CFG;\n";
-        else body << "    typedef tgemm::config_bf16<" << BM << ", " << BN << ", " << BK << ", " << WGM << ", " << WGN << ", " << (edge ? "true" : "false") << "> CFG;\n";
+        body << bf16_config_text(bf16_direct, BM, BK, WGM, WGN, bf16_stages, edge);
     } else {
         body << "    extern __shared__ __attribute__((aligned(16))) float _lds[];\n";
         body << "    typedef " << cfg << " CFG;\n";
@@ -1708,7 +1714,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     k.name = kname;
     bool any_gather = false;
     for (auto &o : operands) any_gather = any_gather || !o.first.linear || !o.second.linear;
-    k.how = std::string("mfma-contraction: ") + (bf16 ? (bf16_direct ? "v_mfma_f32_32x32x16_bf16, slices loaded straight into LDS, " : "v_mfma_f32_32x32x16_bf16, ") : "v_mfma_f32_32x32x2_f32, ") + (windowed ? "implicit GEMM, sliding window of " + std::to_string(win_taps) + " taps staged in LDS by blocks of " + std::to_string(win_cb) + " channels, " :
+    k.how = std::string("mfma-contraction: ") + (bf16 ? (bf16_direct ? "v_mfma_f32_32x32x16_bf16, slices loaded straight into LDS (through registers where an operand begins at an odd element), " : "v_mfma_f32_32x32x16_bf16, ") : "v_mfma_f32_32x32x2_f32, ") + (windowed ? "implicit GEMM, sliding window of " + std::to_string(win_taps) + " taps staged in LDS by blocks of " + std::to_string(win_cb) + " channels, " :
                                                                                       any_gather ? "implicit GEMM (gathered operand), " : "") + "M " +
             std::to_string(Mg.size()) + " dim(s) x N " + std::to_string(Ng.size()) + " x K " + std::to_string(Kg.size()) + ", tile " +
             std::to_string(BM) + "x" + std::to_string(BN) + "x" + std::to_string(BK) + (edge ? ", guarded edges" : ", whole tiles") + ", " +
@@ -1796,21 +1802,52 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     }
     std::ostringstream src;
     src << pre.str();
-    src << "extern \"C\" __global__ void __launch_bounds__(" << NT;
-    if (windowed && win_resident > 1) src << ", " << win_resident * (NT / 64) / 4;       // waves per SIMD: bounds the registers
-    src << ") " << k.name << "(";
-    for (size_t i = 0; i < k.params.size(); i++) {
-        auto &p = k.params[i];
-        src << (i ? ", " : "");
-        if (p.is_buffer) src << primitive_c_name(p.type) << " *__restrict__ " << p.name;
-        else src << "const " << primitive_c_name(p.type) << " " << p.name;
+    auto print_kernel = [&](const kernel &which, const std::string &text) {
+        src << "extern \"C\" __global__ void __launch_bounds__(" << which.block[0];
+        if (windowed && win_resident > 1) src << ", " << win_resident * (NT / 64) / 4;       // waves per SIMD: bounds the registers
+        src << ") " << which.name << "(";
+        for (size_t i = 0; i < which.params.size(); i++) {
+            auto &p = which.params[i];
+            src << (i ? ", " : "");
+            if (p.is_buffer) src << primitive_c_name(p.type) << " *__restrict__ " << p.name;
+            else src << "const " << primitive_c_name(p.type) << " " << p.name;
+        }
+        src << ")\n{\n" << batch_prologue.str() << text << "}\n";
+    };
+    print_kernel(k, body.str());
+    // Loads straight into LDS want operands at multiples of four bytes, which a buffer need not begin at (a part of a larger one,
+    // from an odd element on): the call looks at the addresses and has a kernel that loads through registers for the others.
+    kernel unaligned;
+    std::string addresses;
+    if (bf16_direct) {
+        const ttarget::bf16_tile t = ttarget::bf16_tile_for(Ml, Nl, Kl, false);
+        unaligned = k;
+        unaligned.name = kname + "_unaligned";
+        unaligned.grid[0] = std::to_string(((Ml + t.edge - 1) / t.edge) * ((Nl + t.edge - 1) / t.edge));
+        unaligned.block[0] = std::to_string(64 * t.waves_m * t.waves_n);
+        unaligned.lds_bytes = std::to_string(t.stages * (t.k / 8) * 2 * t.edge * 4 * 4);
+        std::string text = body.str();
+        auto replace_all = [&](const std::string &from, const std::string &to) {
+            for (size_t at = text.find(from); at != std::string::npos; at = text.find(from, at + to.size())) text.replace(at, from.size(), to);
+        };
+        replace_all(bf16_config_text(true, BM, BK, WGM, WGN, bf16_stages, edge), bf16_config_text(false, t.edge, t.k, t.waves_m, t.waves_n, t.stages, true));
+        replace_all("tile_accumulate_bf16_direct<CFG>", "tile_accumulate_bf16<CFG>");
+        print_kernel(unaligned, text);
+        std::set<std::string> operand_buffers;
+        for (auto &o : operands)
+            for (const operand_info *g : {&o.first, &o.second}) operand_buffers.insert(g->buf->get_name());
+        for (auto &nm : operand_buffers) addresses += (addresses.empty() ? "(uintptr_t)" : " | (uintptr_t)") + nm;
     }
-    src << ")\n{\n" << batch_prologue.str() << body.str() << "}\n";
     k.source = src.str();
     add_include_once(ctx, "#include \"gemm_mfma.hip.h\"");
     if (bf16) add_include_once(ctx, "#include \"gemm_mfma_bf16.hip.h\"");
     if (windowed) add_include_once(ctx, "#include \"gemm_mfma_window.hip.h\"");
-    host << launch_text(k, "        ") << "    }\n";
+    if (bf16_direct) {
+        host << "        if ((" << addresses << ") % 4 == 0) {\n" << launch_text(k, "            ") << "        } else {\n"
+             << launch_text(unaligned, "            ") << "        }\n    }\n";
+    } else {
+        host << launch_text(k, "        ") << "    }\n";
+    }
     plan.kernels.push_back(k);
     plan.host_code = host.str();
     return true;
