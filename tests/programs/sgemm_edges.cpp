@@ -15,5 +15,6 @@ int main()
     generate(9, 3, 66);           // fewer columns than a 16-byte load
     generate(37, 70, 3);          // fewer k than one
     generate(70, 45, 64);         // whole slices
+    generate(96, 96, 64);         // whole 32x32 tiles
     return 0;
 }

@@ -152,3 +152,27 @@ def test_gpu_sizes_that_end_inside_a_tile(M, N, K, programs_dir):
     d = [DeviceArray(a) for a in (A, B, C)]
     runtime.load(programs_dir, name)(np.array([2.0, 0.5], np.float32), *[x.buffer() for x in d])
     assert np.array_equal(d[2].download(), exact)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,what", [(96, 96, 64, "tile 32x32x64, whole tiles"), (70, 45, 64, "guarded edges"), (65, 67, 33, "guarded edges")])
+@pytest.mark.parametrize("first", [1, 2, 3])
+def test_gpu_operands_that_begin_at_any_element(M, N, K, what, first, programs_dir):
+    """Contiguous parts of larger tensors, at addresses that are not multiples of 16 bytes, with infinities around them."""
+    import json
+    import torch
+    name = name_of(M, N, K)
+    assert what in json.load(open(os.path.join(programs_dir, "build", name + ".o.json")))["kernels"][0]["how"]
+    rng = np.random.RandomState(M + N + K + first)
+
+    def part(rows, cols):
+        flat = torch.full((rows * cols + 8,), float("inf"))
+        values = rng.randint(-3, 4, (rows, cols)).astype(np.float32)
+        flat[first:first + rows * cols] = torch.from_numpy(values).flatten()
+        view = flat.cuda()[first:first + rows * cols].view(rows, cols)
+        assert view.data_ptr() % 16 == 4 * first
+        return view, values
+
+    (dA, A), (dB, B), (dC, C) = part(M, K), part(K, N), part(M, N)
+    runtime.load(programs_dir, name)(np.array([2.0, 0.5], np.float32), dA, dB, dC)
+    assert np.array_equal(dC.cpu().numpy(), 2.0 * (A @ B) + 0.5 * C)       # integers: exact

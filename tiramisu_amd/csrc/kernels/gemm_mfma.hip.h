@@ -96,7 +96,8 @@ __device__ __forceinline__ f32x4 shifted_down(f32x4 v, int s) {
 // base[k*ld + x].  A source is read in two steps, so that nothing waits for a load where it is issued:
 //   load4(x, k, tail)      the 16 bytes at (x, k) as they come from memory,
 //   finish4(v, x, k, tail) the four elements from them, when they are stored to LDS.
-// Without EDGE all of the operand is there and 16-byte aligned.  With EDGE a tile may hang over XE, the last slice
+// Without EDGE all of the operand is there; its rows are multiples of 16 bytes, but need not begin at one (the same 16-byte load
+// instruction serves any 4-byte aligned address).  With EDGE a tile may hang over XE, the last slice
 // (tail = std::true_type; all others lie within KE) over KE, and rows may start at any element.  Behind KE a source gives
 // zeros; what it gives behind XE only reaches elements of C that nobody stores.  No load is guarded and none is
 // taken apart: it is moved to the nearest place that holds four elements (16-byte loads need not be aligned), and
@@ -113,8 +114,11 @@ struct linear_source {
     int XE, KE;
     template <class TAIL>
     __device__ __forceinline__ f32x4 load4(int x, int k, TAIL) const {
-        if (!EDGE) return *reinterpret_cast<const f32x4 *>(base + (KMAJOR ? (long)x * ld + k : (long)k * ld + x));
         f32x4_u v = {0.f, 0.f, 0.f, 0.f};
+        if (!EDGE) {
+            v = *reinterpret_cast<const f32x4_u *>(base + (KMAJOR ? (long)x * ld + k : (long)k * ld + x));
+            return f32x4{v[0], v[1], v[2], v[3]};
+        }
         if (KMAJOR) {
             const float *row = base + (long)(x < XE ? x : XE - 1) * ld;
             if (!TAIL::value || KE >= 4) {
