@@ -16,5 +16,8 @@ int main()
     generate(37, 70, 3);          // fewer k than one
     generate(70, 45, 64);         // whole slices
     generate(96, 96, 64);         // whole 32x32 tiles
+    generate(224, 160, 32);       // whole 32x32 tiles, slices of 32 k
+    generate(416, 2592, 31);      // guarded slices of 32 k
+    generate(130, 95, 9);
     return 0;
 }

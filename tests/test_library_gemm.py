@@ -70,7 +70,11 @@ def test_transposed_operands_padding_and_offsets(tA, tB):
 
 @pytest.mark.parametrize("M,N,K", [(33, 35, 9), (65, 130, 33), (129, 67, 130), (64, 70, 64), (300, 260, 2051),
                                    # 64 x 32 tiles; thin ones: 32 x 32 tiles of which a row or column of C is a part
-                                   (1000, 1500, 65), (1, 700, 40), (700, 3, 67), (17, 31, 2100), (5, 6, 9), (1, 1, 64)])
+                                   (1000, 1500, 65), (1, 700, 40), (700, 3, 67), (17, 31, 2100), (5, 6, 9), (1, 1, 64),
+                                   # the smaller tiles with slices of 32 k: one k less than, as many as and one more than a slice; a
+                                   # few k and a few rows or columns, one thread per element or not
+                                   (129, 335, 31), (96, 1184, 32), (700, 96, 33), (640, 1600, 17), (3, 900, 11), (900, 4, 8), (4, 65, 12),
+                                   (5, 65, 11)])
 @pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("pad", [0, 3])
 def test_sizes_that_end_inside_a_tile(M, N, K, tA, tB, pad):

@@ -137,7 +137,7 @@ def test_gpu_4096_closed_form_and_sampled_rows():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(300, 260, 1001), (130, 4098, 131), (2001, 1501, 37), (65, 67, 33), (14, 1732, 433), (9, 3, 66), (37, 70, 3),
-                                   (70, 45, 64)])
+                                   (70, 45, 64), (224, 160, 32), (416, 2592, 31), (130, 95, 9)])
 def test_gpu_sizes_that_end_inside_a_tile(M, N, K, programs_dir):
     """Small integers: every sum is exact.  A row of A read past its last k goes on into the next one's first element, and a row
     of B past its last column likewise: infinite in every other row, they must not be used there."""

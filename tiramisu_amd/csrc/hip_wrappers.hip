@@ -195,12 +195,20 @@ void dispatch_tile(const float *A, const float *B, float *C, int M, int N, int K
         launch_mfma<tgemm::config<64, 64, 32, 2, 2, AK, BK_, EDGE>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
 
-// 64 x 32 and 32 x 32 tiles: slices of 64 k, shared by four groups of wavefronts
+// 64 x 32 and 32 x 32 tiles: slices of 64 k shared by four groups of wavefronts, of 32 k shared by two where there are no more
+// (ttarget::small_tile_slice)
+template <bool AK, bool BK_, int BM, int BN, int SLICE>
+void launch_small_slice(bool edge, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc, float alpha, float beta) {
+    constexpr int WGM = BM / 32, WGN = BN / 32, WGK = SLICE / 16;
+    if (edge) launch_mfma<tgemm::config<BM, BN, SLICE, WGM, WGN, AK, BK_, true, 1, WGK>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else launch_mfma<tgemm::config<BM, BN, SLICE, WGM, WGN, AK, BK_, false, 1, WGK>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+}
 template <bool AK, bool BK_, int BM, int BN>
-void launch_small(bool edge, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc, float alpha, float beta) {
-    constexpr int WGM = BM / 32, WGN = BN / 32;
-    if (edge) launch_mfma<tgemm::config<BM, BN, 64, WGM, WGN, AK, BK_, true, 1, 4>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    else launch_mfma<tgemm::config<BM, BN, 64, WGM, WGN, AK, BK_, false, 1, 4>>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+void launch_small(bool vec_ok, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc, float alpha, float beta) {
+    const int slice = ttarget::small_tile_slice(K);
+    const bool edge = !(vec_ok && M % BM == 0 && N % BN == 0 && K % slice == 0);
+    if (slice == 32) launch_small_slice<AK, BK_, BM, BN, 32>(edge, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else launch_small_slice<AK, BK_, BM, BN, 64>(edge, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
 
 // Few C tiles but a long reduction (a batch of 64 rows against wide weights, as in recurrent
@@ -378,9 +386,8 @@ void dispatch_edge(bool vec_ok, const float *A, const float *B, float *C, int M,
     const bool edge = !(vec_ok && M % bm == 0 && N % bm == 0 && K % (bm == 64 ? 32 : 16) == 0);   // K-slice of the tile
     if (bm == 64 || M < 32 || N < 32) {
         const ttarget::small_tile t = ttarget::small_tile_for(M, N, K, active_batch ? active_batch_count : 1, !edge);
-        const bool slices = vec_ok && K % 64 == 0;
-        if (t == ttarget::TILE_64x32) return launch_small<AK, BK_, 64, 32>(!(slices && M % 64 == 0 && N % 32 == 0), A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-        if (t == ttarget::TILE_32) return launch_small<AK, BK_, 32, 32>(!(slices && M % 32 == 0 && N % 32 == 0), A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+        if (t == ttarget::TILE_64x32) return launch_small<AK, BK_, 64, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+        if (t == ttarget::TILE_32) return launch_small<AK, BK_, 32, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     }
     if (edge) dispatch_tile<AK, BK_, true>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     else dispatch_tile<AK, BK_, false>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);

@@ -56,6 +56,12 @@ inline small_tile small_tile_for(long M, long N, long K, long problems, bool who
     return (small_tile)best;
 }
 
+// The k of a slice of those smaller tiles: 64, dealt to four groups of wavefronts by sixteen k each; 32 and two groups where K
+// holds no more, so that no half of a slice is padding.  The partial sums are the same ones.  us of a call before (with 64 x 64
+// tiles), with slices of 64 and of 32: 384 x 3104 x 32 6.1, 8.5, 6.0; 480 x 5216 x 32 8.3, 12.1, 8.3; 1696 x 3168 x 20 13.7, 24.6,
+// 14.4; with one row 1 x 142339 x 20 17.8 (one thread per element), 18.2, 10.2.
+inline int small_tile_slice(long K) { return K <= 32 ? 32 : 64; }
+
 // C tiles of the bf16-input kernels.  A launch is modelled to take `fixed` microseconds (start, first slices, epilogue) plus,
 // for every 32 k, `first` for the first round of tiles over the compute units and `further` for each round after it.  The
 // figures are fits to whole launches of 100 ... 4096 k with a tenth of the chip's tiles up to sixteen rounds (measured /

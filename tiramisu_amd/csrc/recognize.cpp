@@ -1177,7 +1177,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         const ttarget::small_tile t = ttarget::small_tile_for(Ml, Nl, Kl, 1, Ml % 64 == 0 && Nl % 64 == 0 && Kl % 32 == 0);
         if (t != ttarget::TILE_64) {
             BM = t == ttarget::TILE_64x32 ? 64 : 32;
-            BN = 32; BK = 64; WGM = BM / 32; WGN = 1; WGK = 4;
+            BN = 32; BK = ttarget::small_tile_slice(Kl); WGM = BM / 32; WGN = 1; WGK = BK / 16;
         }
     }
     // at most one 64x64 tile per compute unit and a long reduction: two groups of wavefronts share each
