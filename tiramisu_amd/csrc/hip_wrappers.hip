@@ -555,9 +555,13 @@ static int sgemm_impl(const char *fn, bool static_scratch, float *A, float *B, f
     }
     const int m = (int)M, n = (int)N, k = (int)K;
     const bool vec_ok = (ldA % 4 == 0) && (ldB % 4 == 0) && ((uintptr_t)a % 16 == 0) && ((uintptr_t)b % 16 == 0);
-    // Products of a few k are one thread per element.  Thin ones (a dimension of C below a tile's 32) are one row or column of
-    // 32 x 32 tiles, without scratch: guarded, the rest of the tile is work for nothing, but one thread per element walked K alone.
-    const bool small = k < 8, thin = m < 32 || n < 32;
+    // Products of a few k are one thread per element: of fewer than 8, and of fewer than 12 where C is at most four rows, or
+    // columns whose threads read neighbouring elements of both operands (us with one thread per element / with tiles, 8 and
+    // 12 k: 1 x 65536 4.4 / 5.7, 4.7 / 5.6; 4 x 300000 11.2 / 18.6, 19.1 / 18.5; 1000000 x 4 61 / 58, 75 / 59, with A transposed
+    // 84 / 55).  Other thin ones (a dimension of C below a tile's 32) are one row or column of 32 x 32 tiles, without
+    // scratch: guarded, the rest of the tile is work for nothing, but one thread per element walked K alone.
+    const bool narrow = m <= 4 || (!transposeA && (n == 1 || (n <= 4 && !transposeB)));
+    const bool small = k < (narrow ? 12 : 8), thin = m < 32 || n < 32;
     if (batch_open && !static_scratch) {
         // inside a batch scope: remember the call; tiramisu_hip_batch_end launches it, together with the calls of
         // the same shape that follow it
