@@ -122,7 +122,10 @@ DOUBLE_CASES = [(70, 50, 30, False, False), (64, 96, 128, True, False), (33, 65,
                 (1999, 1101, 673, False, True), (1999, 1101, 687, True, False), (2047, 2033, 257, False, False), (2047, 2033, 271, True, True),
                 (1001, 999, 961, False, False), (1023, 1001, 1023, True, True), (301, 1799, 97, True, False), (301, 1799, 3, False, True),
                 (499, 511, 513, False, True), (511, 499, 575, True, False), (15, 17, 1921, False, False), (33, 31, 2047, True, True),
-                (16, 16, 128, False, True), (5, 7, 127, True, False)]
+                (16, 16, 128, False, True), (5, 7, 127, True, False),
+                # at most 32 k: 32 x 32 and 16 x 16 tiles whose slices two groups share
+                (434, 564, 15, False, False), (1184, 160, 32, True, False), (345, 533, 17, False, True), (345, 533, 33, True, True),
+                (47, 628, 31, True, True), (96, 160, 32, False, True), (5, 7, 1, True, False)]
 
 
 @pytest.mark.parametrize("M,N,K,tA,tB", DOUBLE_CASES)

@@ -738,13 +738,16 @@ int tiramisu_hip_dgemm(double *A, double *B, double *C, uint64_t M, uint64_t N, 
     // element (m, k) of op(A) and (k, n) of op(B) through two strides each
     const long sam = transposeA ? 1L : (long)ldA, sak = transposeA ? (long)ldA : 1L;
     const long sbk = transposeB ? 1L : (long)ldB, sbn = transposeB ? (long)ldB : 1L;
+    auto launch = [&](auto shape) {
+        launch_dgemm<decltype(shape)>(transposeA, transposeB, a, b, c, (int)M, (int)N, (int)K, sam, sak, sbk, sbn, (long)ldC, alpha, beta);
+    };
     switch (tgemm64::tile_for((long)M, (long)N, (long)K)) {
-    case tgemm64::TILE_128: launch_dgemm<tgemm64::shape_128>(transposeA, transposeB, a, b, c, (int)M, (int)N, (int)K, sam, sak, sbk, sbn, (long)ldC, alpha, beta); break;
-    case tgemm64::TILE_96: launch_dgemm<tgemm64::shape_96>(transposeA, transposeB, a, b, c, (int)M, (int)N, (int)K, sam, sak, sbk, sbn, (long)ldC, alpha, beta); break;
-    case tgemm64::TILE_64: launch_dgemm<tgemm64::shape_64>(transposeA, transposeB, a, b, c, (int)M, (int)N, (int)K, sam, sak, sbk, sbn, (long)ldC, alpha, beta); break;
-    case tgemm64::TILE_32: launch_dgemm<tgemm64::shape_32>(transposeA, transposeB, a, b, c, (int)M, (int)N, (int)K, sam, sak, sbk, sbn, (long)ldC, alpha, beta); break;
-    case tgemm64::TILE_32_SHARED: launch_dgemm<tgemm64::shape_32_shared>(transposeA, transposeB, a, b, c, (int)M, (int)N, (int)K, sam, sak, sbk, sbn, (long)ldC, alpha, beta); break;
-    default: launch_dgemm<tgemm64::shape_16>(transposeA, transposeB, a, b, c, (int)M, (int)N, (int)K, sam, sak, sbk, sbn, (long)ldC, alpha, beta); break;
+    case tgemm64::TILE_128: launch(tgemm64::shape_128()); break;
+    case tgemm64::TILE_96: launch(tgemm64::shape_96()); break;
+    case tgemm64::TILE_64: launch(tgemm64::shape_64()); break;
+    case tgemm64::TILE_32: launch(tgemm64::shape_32()); break;
+    case tgemm64::TILE_32_SHARED: K <= 32 ? launch(tgemm64::shape_32_short()) : launch(tgemm64::shape_32_shared()); break;
+    default: K <= 32 ? launch(tgemm64::shape_16_short()) : launch(tgemm64::shape_16()); break;
     }
     return 0;
 }

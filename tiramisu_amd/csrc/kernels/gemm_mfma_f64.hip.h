@@ -50,8 +50,8 @@ struct shape {
 // The tiles, and the one whose launch is modelled fastest: `fixed` microseconds (start, the last store), `round` for every round of
 // tiles over the compute units (first slice, epilogue), and per k `first` for a round that a compute unit has to itself or
 // `further` for each of several, whichever is more.  Fits to whole launches of 16 ... 2048 in each size (measured / modelled:
-// 1500 x 1430 x 250 32.5 / 34.1 with 32 x 32, 34.3 / 34.4 with 96 x 96, 46 / 47 with 128 x 128; x 1000 114 / 120, 107 / 108,
-// 155 / 156; 1000^3 48 / 46 with 64 x 64, 55 / 55 with 32 x 32; 700 x 900 x 1000 45.5 / 42.1 without and 42.4 / 41.9 with
+// 1500 x 1430 x 250 32.5 / 34.1 with 32 x 32, 34.3 / 34.7 with 96 x 96, 46 / 47 with 128 x 128; x 1000 114 / 120, 107 / 108,
+// 155 / 155; 2080 x 4832 x 32 25 / 29, 30 / 29, 27 / 29; 1000^3 48 / 46 with 64 x 64, 55 / 55 with 32 x 32; 700 x 900 x 1000 45.5 / 42.1 without and 42.4 / 41.9 with
 // shared slices; 200 x 300 x 1000 9.7 / 8.6 with 16 x 16, 18.6 / 18 with 32 x 32).
 enum tile { TILE_128, TILE_96, TILE_64, TILE_32, TILE_32_SHARED, TILE_16, TILES };
 typedef shape<4, 2, 2, 4, 16> shape_128;             // 2 x 4 wavefronts: two per SIMD cover each other's waits
@@ -60,10 +60,15 @@ typedef shape<2, 2, 2, 2, 64, 4> shape_64;
 typedef shape<1, 1, 2, 2, 16> shape_32;              // eight workgroups to a compute unit: short reductions, many tiles
 typedef shape<1, 1, 2, 2, 64, 4> shape_32_shared;
 typedef shape<1, 1, 1, 1, 128, 8> shape_16;
+// For at most 32 k, which two groups hold sixteen each of, as in the slices above (the sums are the same ones): the other groups'
+// wavefronts only cost their start.  us of a call with 32 x 32 tiles without shared slices, with all groups, with two:
+// 384 x 512 x 32 3.9, 4.2, 3.9; 345 x 533 x 11 3.8, 4.3, 4.0; 1184 x 160 x 32 3.8, 4.3, 3.9.
+typedef shape<1, 1, 2, 2, 32, 2> shape_32_short;
+typedef shape<1, 1, 1, 1, 32, 2> shape_16_short;
 
 inline tile tile_for(long M, long N, long K) {
     static const struct { int edge; double fixed, round, first, further; } model[TILES] = {
-        {128, 9.0, 2.0, 0.1445, 0.14}, {96, 9.0, 1.0, 0.0975, 0.084}, {64, 1.3, 5.0, 0.0395, 0.0395},
+        {128, 8.0, 2.5, 0.1445, 0.14}, {96, 9.0, 1.3, 0.0975, 0.084}, {64, 1.3, 5.0, 0.0395, 0.0395},
         {32, 3.3, 0.25, 0.0235, 0.0127}, {32, 2.6, 0.9, 0.0145, 0.0122}, {16, 2.2, 0.9, 0.0055, 0.0052}};
     int best = TILE_128;
     double best_cost = 0;
