@@ -15,5 +15,6 @@ int main()
     generate(65, 67, 193);        // 64x64 through registers, one k in the last slice
     generate(64, 65, 63);         // odd rows, a single partial slice
     generate(33, 3, 65);          // fewer than four columns
+    generate(640, 704, 64);       // whole tiles, for the order of the instructions behind them
     return 0;
 }

@@ -60,6 +60,28 @@ def test_every_shape_gets_the_bf16_mfma_kernel(M, N, K, what):
     assert len(kernels) == 1 and "v_mfma_f32_32x32x16_bf16" in kernels[0]["how"] and what in kernels[0]["how"]
 
 
+@pytest.mark.parametrize("M,N,K", [(640, 704, 64), (70, 66, 130), (2000, 1500, 1006)])
+def test_loads_of_the_epilogue_are_in_flight_together(M, N, K, programs_dir, tmp_path):
+    """In the instructions of the kernel, the loads of C are not waited for one by one, each before the next is issued."""
+    import subprocess
+    from tiramisu_amd import build
+    text = str(tmp_path / "kernel.s")
+    subprocess.run([build.HIPCC] + build.HIP_FLAGS + ["--cuda-device-only", "-S", "-I" + os.path.join(build.CSRC, "kernels"), "-o", text,
+                    os.path.join(programs_dir, "build", name_of(M, N, K) + ".o.hip")], check=True, stderr=subprocess.DEVNULL)
+    loads, alone, last = 0, 0, ""
+    for line in open(text):
+        words = line.split()
+        if words[:1] == ["s_endpgm"]:
+            break                               # of the kernel for operands at multiples of four bytes
+        if words and words[0] in ("global_load_dword", "global_store_dword"):
+            loads += words[0] == "global_load_dword"
+            last = words[0]
+        elif words[:2] == ["s_waitcnt", "vmcnt(0)"]:
+            alone += last == "global_load_dword"
+            last = ""
+    assert loads >= 16 and alone <= loads // 8, "%d of %d loads waited for one by one" % (alone, loads)
+
+
 @pytest.mark.parametrize("M,N,K", SMALL)
 def test_cpu_generated_code_matches_float64(M, N, K):
     rng = np.random.RandomState(M + K)
