@@ -139,12 +139,18 @@ def test_gpu_4096_sampled_rows():
     assert np.array_equal(out[rows], exact.astype(np.float32))
 
 
+def how(directory, name):
+    import json
+    return json.load(open(os.path.join(directory, "build", name + ".o.json")))["kernels"][0]["how"]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(4096, 3072, 32), (3072, 4096, 160)])
 def test_gpu_large_tiles_short_k(M, N, K):
-    """256x256 tiles (slices loaded straight into the four-stage LDS ring) with one and five K-slices:
+    """128x128 tiles (slices loaded straight into the four-stage LDS ring) with one and five K-slices:
     the ring's start-up, a single steady-state turn and the drain, every element checked, with the
     alpha / beta epilogue."""
+    assert "straight into LDS" in how(PROGRAMS, name_of(M, N, K)) and "tile 128x128x32, whole tiles" in how(PROGRAMS, name_of(M, N, K))
     rng = np.random.RandomState(M + K)
     scal = np.array([1.5, 0.5], np.float32)
     A, B = to_bf16(rng.randint(-4, 5, (M, K)).astype(np.float32)), to_bf16(rng.randint(-4, 5, (K, N)).astype(np.float32))

@@ -62,12 +62,16 @@ inline small_tile small_tile_for(long M, long N, long K, long problems, bool who
 // 14.4; with one row 1 x 142339 x 20 17.8 (one thread per element), 18.2, 10.2.
 inline int small_tile_slice(long K) { return K <= 32 ? 32 : 64; }
 
-// C tiles of the bf16-input kernels.  A launch is modelled to take `fixed` microseconds (start, first slices, epilogue) plus,
-// for every 32 k, `first` for the first round of tiles over the compute units and `further` for each round after it.  The
-// figures are fits to whole launches of 100 ... 4096 k with a tenth of the chip's tiles up to sixteen rounds (measured /
-// modelled: 300 x 260 x 3000 12.8 / 14.2 us with 64 x 64, 1000 x 750 x 500 5.3 / 4.7, 2000 x 1500 x 1000 15.4 / 9.3 with
-// 128 x 128 against 17.8 / 14.3 with 64 x 64, 3000 x 2700 x 4000 82 / 78 with 256 x 256 against 109 / 165 with 128 x 128).
-// Direct tiles load their slices straight into LDS; the others serve rows of an odd number of elements.
+// C tiles of the bf16-input kernels.  What the loops over K of a launch take is modelled as `fixed` microseconds (start, first
+// slices) plus, for every 32 k of whole slices, `first` for the first round of tiles over the compute units and `further` for
+// each round after it.  Reading and writing C is left out: it takes every tile the same (64 MiB in and out at 4096 x 4096 20 us),
+// so the model only orders the tiles.  It is fitted to whole launches of 32 ... 4096 k with a tenth of the chip's tiles up to
+// sixteen rounds: 300 x 260 x 3000 takes 13.0 us with 64 x 64 (14.1 modelled) and 21.6 with 128 x 128 (19.9), 1000 x 750 x 500
+// 5.6 and 8.0 (4.7, 6.6), 2000 x 1500 x 1000 15.6 with 128 x 128 and 18.0 with 64 x 64 (9.3, 14.3), 3000 x 2700 x 4000 82 with
+// 256 x 256 and 109 with 128 x 128 (78, 95), 4096 x 3072 x 32, half of a slice of the 64 x 64 tiles, 17.3 with 128 x 128 and
+// 20.5 with 64 x 64 (4.6, 5.7).
+// Direct tiles load their slices straight into LDS; the others serve rows of an odd number of elements and other operands that
+// those loads cannot address.
 struct bf16_tile {
     int edge, k, waves_m, waves_n, stages;
     bool direct;
@@ -84,7 +88,7 @@ inline bf16_tile bf16_tile_for(long M, long N, long K, bool direct) {
     for (const bf16_tile &c : BF16_TILES) {
         if (c.direct != direct) continue;
         const long tiles = ((M + c.edge - 1) / c.edge) * ((N + c.edge - 1) / c.edge), rounds = (tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS;
-        const double cost = c.fixed + ((K + 31) / 32) * (c.first + (rounds - 1) * c.further);
+        const double cost = c.fixed + ((K + c.k - 1) / c.k * c.k / 32) * (c.first + (rounds - 1) * c.further);
         if (!best || cost < best_cost) { best = &c; best_cost = cost; }
     }
     return *best;

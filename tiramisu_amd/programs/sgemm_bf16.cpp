@@ -73,8 +73,8 @@ int main(int argc, char **argv)
     tiramisu::backend_options_from_command_line(argc, argv);
     generate(4096, 4096, 4096);   // benchmark configuration 3, bf16-input variant
     if (std::getenv("SGEMM_BF16_ONLY_FULL")) return 0;   // for sweeps over the emitter's knobs
-    generate(4096, 3072, 32);     // 256x256 tiles, a single K-slice
-    generate(3072, 4096, 160);    // 256x256 tiles, five K-slices: one steady-state turn of the four-stage ring, then the drain
+    generate(4096, 3072, 32);     // 128x128 tiles, a single K-slice
+    generate(3072, 4096, 160);    // 128x128 tiles, five K-slices: one steady-state turn of the four-stage ring, then the drain
     generate(1024, 1280, 512);    // 128x128 tiles
     generate(128, 192, 128);      // whole 64x64x64 tiles: MFMA path
     generate(48, 40, 24);         // one ragged 64x64 tile: MFMA path with guarded loads
