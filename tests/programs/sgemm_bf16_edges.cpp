@@ -15,6 +15,9 @@ int main()
     generate(65, 67, 193);        // 64x64 through registers, one k in the last slice
     generate(64, 65, 63);         // odd rows, a single partial slice
     generate(33, 3, 65);          // fewer than four columns
+    generate(20480, 20480, 32);   // 256x256 tiles with one slice, three (fewer than the LDS ring has stages) and five
+    generate(8192, 12288, 96);
+    generate(8192, 8192, 160);
     generate(640, 704, 64);       // whole tiles, for the order of the instructions behind them
     return 0;
 }

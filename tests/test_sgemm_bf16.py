@@ -163,6 +163,25 @@ def test_gpu_large_tiles_short_k(M, N, K):
     assert np.max(np.abs(out - exact)) <= 1e-5 * np.max(np.abs(exact))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(20480, 20480, 32), (8192, 12288, 96), (8192, 8192, 160)])
+def test_gpu_largest_tiles_short_k(M, N, K, programs_dir):
+    """256x256 tiles, which the model takes for large planes where K is short, with one, three and five K-slices of the four-stage
+    ring: every element against torch's fp32 product, exact for small integers."""
+    import torch
+    name = name_of(M, N, K)
+    assert "straight into LDS" in how(programs_dir, name) and "tile 256x256x32, whole tiles" in how(programs_dir, name)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + K)
+    A, B = (torch.randint(-4, 5, s, generator=g, device="cuda").float() for s in ((M, K), (K, N)))
+    C = torch.randint(-8, 9, (M, N), generator=g, device="cuda", dtype=torch.int8).float()
+    exact = torch.addmm(C, A, B, beta=0.5, alpha=2.0)
+    runtime.load(programs_dir, name)(np.array([2.0, 0.5], np.float32), A.to(torch.bfloat16), B.to(torch.bfloat16), C)
+    assert torch.equal(C, exact)
+    del A, B, C, exact
+    torch.cuda.empty_cache()
+
+
 EDGES = [(4002, 3998, 500, "tile 256x256x32, guarded edges"), (2000, 1500, 1006, "tile 128x128x32, guarded edges"),
          (70, 66, 130, "tile 64x64x64, guarded edges"), (66, 2, 6, "tile 64x64x64, guarded edges"),
          (2001, 1501, 1001, "tile 128x128x64, guarded edges"), (65, 67, 193, "tile 64x64x64, guarded edges"),
