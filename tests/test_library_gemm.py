@@ -78,13 +78,17 @@ def test_transposed_operands_padding_and_offsets(tA, tB):
 @pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("pad", [0, 3])
 def test_sizes_that_end_inside_a_tile(M, N, K, tA, tB, pad):
+    surrounded_by_nan(M, N, K, tA, tB, pad, np.float32)
+
+
+def surrounded_by_nan(M, N, K, tA, tB, pad, dtype):
     """Operands that begin and end with their allocations but for NaN around them and between their rows, which must not
     reach the result; the rows of C keep what lies between them."""
     import torch
     rng = np.random.RandomState(M + N + K + pad)
 
     def surrounded(rows, cols):
-        flat = np.full(5 + rows * (cols + pad) + 4, np.nan, np.float32)
+        flat = np.full(5 + rows * (cols + pad) + 4, np.nan, dtype)
         inside = flat[5:5 + rows * (cols + pad)].reshape(rows, cols + pad)[:, :cols]
         inside[:] = rng.randint(-3, 4, (rows, cols))
         return torch.from_numpy(flat).cuda(), inside.astype(np.float64), cols + pad
@@ -92,8 +96,10 @@ def test_sizes_that_end_inside_a_tile(M, N, K, tA, tB, pad):
     (dA, a, ldA), (dB, b, ldB), (dC, c, ldC) = [surrounded(*v) for v in ((K, M) if tA else (M, K), (N, K) if tB else (K, N), (M, N))]
     before = dC.cpu().numpy()
     torch.cuda.synchronize()
-    runtime.wrappers().tiramisu_hip_sgemm(dA.data_ptr(), dB.data_ptr(), dC.data_ptr(), M, N, K, 2.0, 3.0, ldA, ldB, ldC, 5, 5, 5, tA, tB)
-    runtime.wrappers().tiramisu_hip_stream_synchronize(0)
+    w = runtime.wrappers()
+    call = w.tiramisu_hip_sgemm if dtype == np.float32 else w.tiramisu_hip_dgemm
+    call(dA.data_ptr(), dB.data_ptr(), dC.data_ptr(), M, N, K, 2.0, 3.0, ldA, ldB, ldC, 5, 5, 5, tA, tB)
+    w.tiramisu_hip_stream_synchronize(0)
     before[5:5 + M * ldC].reshape(M, ldC)[:, :N] = 2.0 * ((a.T if tA else a) @ (b.T if tB else b)) + 3.0 * c     # integers: exact
     assert np.array_equal(dC.cpu().numpy(), before, equal_nan=True)
 
@@ -145,6 +151,15 @@ def test_double_precision(M, N, K, tA, tB):
     dA, dB, dC = DeviceArray(A), DeviceArray(B), DeviceArray(C)
     runtime.wrappers().tiramisu_hip_dgemm(dA.ptr, dB.ptr, dC.ptr, M, N, K, 2.0, 0.0, 0, 0, 0, 0, 0, 0, tA, tB)
     assert np.array_equal(dC.download(), 2.0 * ((A.T if tA else A) @ (B.T if tB else B)))
+
+
+@pytest.mark.parametrize("M,N,K", [(2047, 2033, 257), (1999, 1101, 673), (1001, 999, 961), (301, 1799, 97), (499, 511, 513),
+                                   (434, 564, 31), (33, 31, 2047), (47, 628, 17), (5, 7, 127), (5, 6, 1)])
+@pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_double_precision_inside_larger_allocations(M, N, K, tA, tB, pad):
+    # one size for each of the tiles: 128, 96, 64, 32 without and with shared slices (of 64 and of 32 k), 16 (of 128 and of 32 k)
+    surrounded_by_nan(M, N, K, tA, tB, pad, np.float64)
 
 
 def test_double_precision_leading_dimensions_and_offsets():
@@ -212,6 +227,33 @@ def test_deep_reductions_on_two_streams_of_one_thread_use_separate_scratch():
             d.free()
     for s in streams:
         w.tiramisu_hip_stream_destroy(s)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 290, 130), (256, 256, 64), (130, 96, 20)])
+def test_batches_of_more_calls_than_a_launch_holds(M, N, K):
+    """Ten calls of one shape on the smaller tiles go as launches of eight and of two, whose tiles may differ (the sums' order, and
+    so the last bits of the results, depends on how many calls a launch covers): exact on small integers either way, and close
+    on uniform data."""
+    from gpu_util import DeviceArray
+    w = runtime.wrappers()
+    rng = np.random.RandomState(M + K)
+    for integer in (True, False):
+        jobs = []
+        for i in range(10):
+            values = [(rng.randint(-3, 4, s) if integer else rng.uniform(-1, 1, s)).astype(np.float32) for s in ((M, K), (K, N), (M, N))]
+            jobs.append(values + [DeviceArray(v) for v in values])
+        assert w.tiramisu_hip_batch_begin() == 0
+        for A, B, C, dA, dB, dC in jobs:
+            assert w.tiramisu_hip_sgemm(dA.ptr, dB.ptr, dC.ptr, M, N, K, 2.0, 0.5, 0, 0, 0, 0, 0, 0, False, False) == 0
+        assert w.tiramisu_hip_batch_end() == 0
+        for A, B, C, dA, dB, dC in jobs:
+            exact = 2.0 * (A.astype(np.float64) @ B.astype(np.float64)) + 0.5 * C
+            if integer:
+                assert np.array_equal(dC.download(), exact)
+            else:                              # K sums of at most K, each rounded by 2^-24 of it, times alpha
+                assert np.max(np.abs(dC.download() - exact)) <= 2.0 * K * K * 2.0 ** -24
+            for d in (dA, dB, dC):
+                d.free()
 
 
 def test_calls_gathered_in_a_batch_scope_give_the_results_of_separate_calls():

@@ -139,19 +139,25 @@ def test_gpu_4096_closed_form_and_sampled_rows():
 @pytest.mark.parametrize("M,N,K", [(300, 260, 1001), (130, 4098, 131), (2001, 1501, 37), (65, 67, 33), (14, 1732, 433), (9, 3, 66), (37, 70, 3),
                                    (70, 45, 64), (224, 160, 32), (416, 2592, 31), (130, 95, 9)])
 def test_gpu_sizes_that_end_inside_a_tile(M, N, K, programs_dir):
-    """Small integers: every sum is exact.  A row of A read past its last k goes on into the next one's first element, and a row
-    of B past its last column likewise: infinite in every other row, they must not be used there."""
+    """Small integers: every sum is exact.  First all finite, so that every element counts; then with the first elements of A's
+    even rows, of its odd ones, and of every other row of B infinite: a row read past its end goes on into the next one's, which
+    must not be used (where they belong, they make a row or the first column of the result infinite)."""
     from gpu_util import DeviceArray
     name = name_of(M, N, K)
     assert "v_mfma_f32" in open(os.path.join(programs_dir, "build", name + ".o.hip")).read()
     rng = np.random.RandomState(M + N + K)
-    A, B = rng.randint(-3, 4, (M, K)).astype(np.float32), rng.randint(1, 4, (K, N)).astype(np.float32)
-    C = rng.randint(-8, 9, (M, N)).astype(np.float32)
-    A[1::2, 0] = np.inf
-    exact = 2.0 * (A @ B) + 0.5 * C            # sums of at most 1001 products below 10: exact in float32 in any order
-    d = [DeviceArray(a) for a in (A, B, C)]
-    runtime.load(programs_dir, name)(np.array([2.0, 0.5], np.float32), *[x.buffer() for x in d])
-    assert np.array_equal(d[2].download(), exact)
+    for infinite in ("nothing", "even rows of A", "odd rows of A", "rows of B"):
+        A, B = rng.randint(-3, 4, (M, K)).astype(np.float32), rng.randint(1, 4, (K, N)).astype(np.float32)
+        if infinite.endswith("A"):
+            A[infinite.startswith("odd")::2, 0] = np.inf
+        elif infinite.endswith("B"):
+            B[1::2, 0] = np.inf
+        C = rng.randint(-8, 9, (M, N)).astype(np.float32)
+        with np.errstate(invalid="ignore"):
+            exact = 2.0 * (A @ B) + 0.5 * C        # sums of at most 1001 products below 10: exact in float32 in any order
+        d = [DeviceArray(a) for a in (A, B, C)]
+        runtime.load(programs_dir, name)(np.array([2.0, 0.5], np.float32), *[x.buffer() for x in d])
+        assert np.array_equal(d[2].download(), exact, equal_nan=True), infinite
 
 
 @pytest.mark.gpu

@@ -191,20 +191,25 @@ EDGES = [(4002, 3998, 500, "tile 256x256x32, guarded edges"), (2000, 1500, 1006,
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,what", EDGES)
 def test_gpu_sizes_that_end_inside_a_tile(M, N, K, what, programs_dir):
-    """Small integers: every sum is exact.  The first elements of A's rows are infinite in every other row: a row read past
-    its last k goes on into them, and must not use them."""
-    import json
+    """Small integers: every sum is exact.  First all finite, so that every element counts; then with the first elements of A's
+    even rows, of its odd ones, and of every other row of B infinite: a row read past its end goes on into the next one's, which
+    must not be used (where they belong, they make a row or the first column of the result infinite)."""
     from gpu_util import DeviceArray
-    how = json.load(open(os.path.join(programs_dir, "build", name_of(M, N, K) + ".o.json")))["kernels"][0]["how"]
-    assert what in how and ("straight into LDS" in how) == (K % 2 == 0 and N % 2 == 0)
+    tile = how(programs_dir, name_of(M, N, K))
+    assert what in tile and ("straight into LDS" in tile) == (K % 2 == 0 and N % 2 == 0)
     rng = np.random.RandomState(M + N + K)
-    A, B = rng.randint(-3, 4, (M, K)).astype(np.float32), rng.randint(1, 4, (K, N)).astype(np.float32)
-    A[1::2, 0] = np.inf
-    C = rng.randint(-8, 9, (M, N)).astype(np.float32)
-    exact = 2.0 * (A @ B) + 0.5 * C            # sums of at most 1006 products below 10: exact in float32 in any order
-    d = [DeviceArray(a) for a in (to_bf16(A), to_bf16(B), C)]
-    runtime.load(programs_dir, name_of(M, N, K))(np.array([2.0, 0.5], np.float32), *[x.buffer() for x in d])
-    assert np.array_equal(d[2].download(), exact)
+    for infinite in ("nothing", "even rows of A", "odd rows of A", "rows of B"):
+        A, B = rng.randint(-3, 4, (M, K)).astype(np.float32), rng.randint(1, 4, (K, N)).astype(np.float32)
+        if infinite.endswith("A"):
+            A[infinite.startswith("odd")::2, 0] = np.inf
+        elif infinite.endswith("B"):
+            B[1::2, 0] = np.inf
+        C = rng.randint(-8, 9, (M, N)).astype(np.float32)
+        with np.errstate(invalid="ignore"):
+            exact = 2.0 * (A @ B) + 0.5 * C        # sums of at most 1006 products below 10: exact in float32 in any order
+        d = [DeviceArray(a) for a in (to_bf16(A), to_bf16(B), C)]
+        runtime.load(programs_dir, name_of(M, N, K))(np.array([2.0, 0.5], np.float32), *[x.buffer() for x in d])
+        assert np.array_equal(d[2].download(), exact, equal_nan=True), infinite
 
 
 VIEWS = [("a_backwards", 200, 150, 100), ("b_backwards", 200, 150, 100), ("a_backwards_whole", 128, 192, 128), ("b_backwards_whole", 128, 192, 128),
@@ -214,9 +219,8 @@ VIEWS = [("a_backwards", 200, 150, 100), ("b_backwards", 200, 150, 100), ("a_bac
 @pytest.mark.parametrize("form", [v[0] for v in VIEWS])
 def test_operands_walked_backwards_or_overlapping_are_not_loaded_straight_into_lds(form, programs_dir):
     """Those loads address an operand by 32-bit offsets from its first row and rely on what follows its last row reading as zero."""
-    import json
-    kernels = json.load(open(os.path.join(programs_dir, "build", "sgemm_bf16_%s.o.json" % form)))["kernels"]
-    assert len(kernels) == 1 and "v_mfma_f32_32x32x16_bf16" in kernels[0]["how"] and "straight into LDS" not in kernels[0]["how"]
+    tile = how(programs_dir, "sgemm_bf16_" + form)
+    assert "v_mfma_f32_32x32x16_bf16" in tile and "straight into LDS" not in tile
 
 
 @pytest.mark.gpu
@@ -245,9 +249,8 @@ def test_gpu_operands_walked_backwards_or_overlapping(form, M, N, K, programs_di
                                                 ("odd_k_and_n", 129, 257, 33, 36, 258)])
 def test_gpu_odd_parts_of_rows_of_an_even_number_of_elements(form, M, N, K, lda, ldb, programs_dir):
     """The last element of the last row is the first half of a dword whose second half is not part of the operand."""
-    import json
     from gpu_util import DeviceArray
-    assert "straight into LDS" in json.load(open(os.path.join(programs_dir, "build", "sgemm_bf16_%s.o.json" % form)))["kernels"][0]["how"]
+    assert "straight into LDS" in how(programs_dir, "sgemm_bf16_" + form)
     rng = np.random.RandomState(M + N + K)
     A, B = np.full((M, lda), np.inf, np.float32), np.full((K, ldb), np.inf, np.float32)
     A[:, :K], B[:, :N] = rng.randint(1, 4, (M, K)), rng.randint(1, 4, (K, N))        # no zeros: a lost element shows
