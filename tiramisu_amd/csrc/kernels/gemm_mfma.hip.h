@@ -156,12 +156,11 @@ struct linear_source {
 // consecutive units u out of every one of the G groups -- tile position x' stands for
 //     x = (x' % BN / UB) * UE + (x' / BN) * UB + x' % UB.
 // A workgroup then owns all G columns of its units, which is what an epilogue that combines them
-// (the gates of a recurrent cell) needs.  UB must be a multiple of 4 for operands whose x is contiguous.  Units of the last
-// tile behind the last one stand for the last one (operands whose x is contiguous: UE is a multiple of UB).
+// (the gates of a recurrent cell) needs.  UB must be a multiple of 4 for operands whose x is contiguous, UE one of UB (no
+// tile hangs over the units).
 template <int BN, int UB>
 __device__ __forceinline__ int regrouped_index(int x, int UE) {
-    const int u = (x / BN) * UB + (x % UB);
-    return ((x % BN) / UB) * UE + (u < UE ? u : UE - 1);
+    return ((x % BN) / UB) * UE + (x / BN) * UB + (x % UB);
 }
 template <class SRC, int BN, int UB>
 struct regrouped_rows {
