@@ -57,7 +57,7 @@ int tiramisu_hip_dgemm(double *A, double *B, double *C, uint64_t M, uint64_t N, 
 /* tiramisu_hip_sgemm for callers that cannot allocate device memory (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments,
  * same kernels, bit-identical results; the difference is where deep reductions (at most 128 tiles of
- * 64x64 and K >= 2048, whose K range is split over workgroups) keep their partial tiles and per-tile
+ * 64x64, no dimension of C below 32, K >= 2048: their K range is split over workgroups) keep their partial tiles and per-tile
  * counters: tiramisu_hip_sgemm takes them from a per-thread workspace that it allocates and grows with
  * hipMalloc, this entry point from a 4 MiB (+512 B of counters) array that lives in the library's code
  * object, one copy per GPU, held until the process ends.  It calls no hipMalloc / hipFree.  A problem
@@ -73,7 +73,9 @@ int tiramisu_hip_sgemm_static_scratch(float *A, float *B, float *C, uint64_t M, 
  * calls are gathered instead of launched; _end launches them in call order, runs of calls of one shape (sizes,
  * leading dimensions, transposition, alpha, beta) as ONE launch with a problem per blockIdx.z (up to 8 per launch).
  * The gathered calls must be independent of one another: generated code opens a scope around the GEMM call of a
- * statement that it runs for all iterations of a host loop tagged parallel.  Scopes do not nest (_begin inside a
+ * statement that it runs for all iterations of a host loop tagged parallel.  The tile of a small product, and with it
+ * the order of its sums, depends on how many calls share its launch (the last bits of the results may differ from
+ * those of separate calls).  Scopes do not nest (_begin inside a
  * scope and _end outside one return 1); tiramisu_hip_sgemm_static_scratch and tiramisu_hip_dgemm are not gathered. */
 int tiramisu_hip_batch_begin(void);
 int tiramisu_hip_batch_end(void);

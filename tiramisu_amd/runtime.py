@@ -241,8 +241,8 @@ class Program:
         if torch_stream is None:
             rc = self.fn(*[b.pointer() for b in bufs])
         elif torch_stream == 0:
-            # torch's default stream is the device's null stream, which the runtime has no handle for: order the
-            # call by waiting on both sides instead
+            # torch's default stream is the device's null stream, and its handle, 0, means the calling thread's own
+            # default stream to tiramisu_hip_set_stream: the call is ordered by waiting on both sides instead
             import torch
             torch.cuda.current_stream().synchronize()
             rc = self.fn(*[b.pointer() for b in bufs])
