@@ -36,6 +36,7 @@ struct shape {
     static constexpr int TM = TM_, TN = TN_, WGM = WGM_, WGN = WGN_, BK = BK_, WGK = WGK_;
     static constexpr int NT = 64 * WGM * WGN * WGK;
     static constexpr int RESIDENT = WGK == 1 ? 2 : 1;                        // workgroups that share a compute unit
+    static constexpr int WAVES_PER_SIMD = NT * RESIDENT >= 256 ? NT * RESIDENT / 256 : 1;
     static constexpr int BM = 16 * TM * WGM, BN = 16 * TN * WGN;
     static constexpr int A_ROW = BM + PAD, B_ROW = BN + PAD;                 // doubles per k row of a stage
     static constexpr int STAGE = BK * (A_ROW + B_ROW);
@@ -86,7 +87,7 @@ inline tile tile_for(long M, long N, long K) {
 // compute unit: at 136 registers instead of 128 a single workgroup is resident and the kernel is a quarter slower.
 // A_KFAST: consecutive k of A are adjacent in memory (stride_ak == 1), else consecutive m are; likewise B_NFAST.
 template <class S, bool A_KFAST, bool B_NFAST>
-__global__ void __launch_bounds__(S::NT, S::NT * S::RESIDENT / 256) dgemm_kernel(const double *__restrict__ A, const double *__restrict__ B, double *__restrict__ C, int M, int N,
+__global__ void __launch_bounds__(S::NT, S::WAVES_PER_SIMD) dgemm_kernel(const double *__restrict__ A, const double *__restrict__ B, double *__restrict__ C, int M, int N,
                                                    int K, long stride_am, long stride_ak, long stride_bk, long stride_bn, long ldc, double alpha,
                                                    double beta) {
     constexpr int TM = S::TM, TN = S::TN, NT = S::NT, BK = S::BK;
