@@ -1,0 +1,161 @@
+"""fp32 products whose operands are split into bf16 parts (kernels/gemm_mfma_split.hip.h): the rule that picks them on the CPU,
+and on the GPU every tile, whole and guarded, in every layout, through the library call and the programs.
+
+Exactness: products and sums of small whole numbers are exact.  Accuracy: with uniform operands a sum of K products rounds its
+accumulator once per matrix instruction, six per sixteen k, each time by at most 2^-24 of the sum of the magnitudes so far; the
+products left out are at most 2^-25 of theirs.  |error| <= (6/16 K 2^-24 / 2 + 2^-25) sum |a b| therefore bounds every element (on
+average half the accumulator's final value is there when it is rounded), with a few more roundings for partial sums, alpha and beta."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from tiramisu_amd import build, runtime
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PROGRAMS = os.path.join(ROOT, "tests", "programs")
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    """split_tile_for of kernels/target_gfx950.h, preceded by the fp32 tile that the library call would take."""
+    d = tmp_path_factory.mktemp("rule")
+    (d / "rule.cpp").write_text('''#include "%s"
+extern "C" int fp32_tile(long M, long N, long K, int *m, int *n) {
+    const int bm = ttarget::square_tile_for(M, N);
+    bool edge = !(M %% bm == 0 && N %% bm == 0 && K %% (bm == 64 ? 32 : 16) == 0);
+    *m = *n = bm;
+    if (bm == 64 || M < 32 || N < 32) {
+        const ttarget::small_tile t = ttarget::small_tile_for(M, N, K, 1, !edge);
+        if (t != ttarget::TILE_64) { *m = t == ttarget::TILE_64x32 ? 64 : 32; *n = 32; edge = !(M %% *m == 0 && N %% *n == 0 && K %% ttarget::small_tile_slice(K) == 0); }
+    }
+    return edge;
+}
+extern "C" int split_tile(long M, long N, long K) {
+    int m, n;
+    const int edge = fp32_tile(M, N, K, &m, &n);
+    return ttarget::split_tile_for(M, N, K, 1, m, n, edge);
+}
+''' % os.path.join(build.CSRC, "kernels", "target_gfx950.h"))
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-o", str(d / "rule.so"), str(d / "rule.cpp")], check=True)
+    lib = ctypes.CDLL(str(d / "rule.so"))
+    for f in (lib.split_tile, lib.fp32_tile):
+        f.argtypes = [ctypes.c_long] * 3 + ([ctypes.POINTER(ctypes.c_int)] * 2 if f is lib.fp32_tile else [])
+    return lib
+
+
+def test_rule(rule):
+    for M, N, K, edge in ((4096, 4096, 4096, 256), (2048, 2048, 2048, 128), (1024, 1024, 1024, 64), (4096, 4096, 95, 0), (63, 4096, 4096, 0),
+                          (4096, 63, 4096, 0), (512, 512, 512, 0), (64, 64, 4096, 0), (4097, 4096, 96, 256)):
+        assert rule.split_tile(M, N, K) == edge, (M, N, K)
+    m, n = ctypes.c_int(), ctypes.c_int()
+    rng = np.random.RandomState(1)
+    for _ in range(3000):
+        M, N, K = (int(v) for v in np.exp(rng.uniform(np.log(16), np.log(5000), 3)))
+        if rng.rand() < 0.5:
+            M, N, K = (max(64, v // 64 * 64) for v in (M, N, K))
+        edge = rule.split_tile(M, N, K)
+        rule.fp32_tile(M, N, K, m, n)
+        if edge:      # sizes that the kernels' loads require; as many partial sums as the fp32 tile's four, or more
+            assert min(M, N) >= 64 and K >= 96 and (n.value != 32 or edge == 64)
+            assert edge != 64 or (M % 64 == 0 and N % 64 == 0 and K % 16 == 0)
+
+
+def bound(A, B, K):
+    return (6 / 16 * K / 2 + 24) * 2.0 ** -24 * (np.abs(A) @ np.abs(B)) + 2.0 ** -25 * (np.abs(A) @ np.abs(B))
+
+
+def operands(rng, M, N, K, tA, tB, pad, kind):
+    def one(rows, cols):
+        full = np.full((rows, cols + pad), np.nan, np.float32)       # what lies between the rows must not matter
+        full[:, :cols] = rng.randint(-8, 9, (rows, cols)) if kind == "whole" else rng.uniform(-1, 1, (rows, cols))
+        return full
+    return one(*((K, M) if tA else (M, K))), one(*((N, K) if tB else (K, N)))
+
+
+def call(A, B, C, M, N, K, alpha, beta, tA, tB, offset=0):
+    from gpu_util import DeviceArray
+    dA, dB, dC = (DeviceArray(np.concatenate([np.zeros(offset, np.float32), x.ravel()])) for x in (A, B, C))
+    rc = runtime.wrappers().tiramisu_hip_sgemm(dA.ptr, dB.ptr, dC.ptr, M, N, K, alpha, beta, A.shape[1], B.shape[1], C.shape[1], offset, offset, offset, tA, tB)
+    assert rc == 0
+    return dC.download()[offset:].reshape(C.shape)
+
+
+SIZES = [(704, 1088, 528, 64), (1408, 2560, 416, 128), (1219, 2747, 611, 128), (1300, 2690, 450, 128), (2560, 3584, 208, 256), (2701, 3915, 99, 256)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K,edge", SIZES)
+def test_library_call(rule, M, N, K, edge, tA, tB):
+    assert rule.split_tile(M, N, K) == edge
+    rng = np.random.RandomState(M + K)
+    for kind, pad, offset, alpha, beta in (("whole", 0, 0, 2.0, 3.0), ("uniform", 3 if edge != 64 else 4, 1 if M % 2 else 4, 1.0, 0.0)):
+        A, B = operands(rng, M, N, K, tA, tB, pad, kind)
+        a = A[:, :M].T if tA else A[:, :K]
+        b = B[:, :K].T if tB else B[:, :N]
+        C = rng.randint(-8, 9, (M, N + pad)).astype(np.float32)
+        out = call(A, B, C, M, N, K, alpha, beta, tA, tB, offset)
+        a, b = a.astype(np.float64), b.astype(np.float64)
+        expected = alpha * (a @ b) + beta * C[:, :N]
+        assert np.array_equal(out[:, N:], C[:, N:])
+        if kind == "whole":
+            assert np.array_equal(out[:, :N], expected)
+        else:
+            assert np.all(np.abs(out[:, :N] - expected) <= bound(a, b, K))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [s[:3] for s in SIZES if s[0] != 1300])
+def test_program(M, N, K):
+    name = "sgemm_%dx%dx%d" % (M, N, K)
+    p = runtime.load(PROGRAMS, name)
+    assert any("three bf16 parts" in k["how"] for k in p.manifest["kernels"])
+    from gpu_util import DeviceArray
+    rng = np.random.RandomState(K)
+    A, B, C = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32), rng.uniform(-1, 1, (M, N)).astype(np.float32)
+    d = [DeviceArray(x) for x in (A, B, C)]
+    p(np.array([1.5, 0.5], np.float32), *[x.buffer() for x in d])
+    a, b = A.astype(np.float64), B.astype(np.float64)
+    assert np.all(np.abs(d[2].download() - (1.5 * (a @ b) + 0.5 * C)) <= 1.5 * bound(a, b, K) + 2.0 ** -23)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(704, 1088, 528), (1219, 2747, 611), (2560, 3584, 208)])
+def test_numbers_that_three_parts_do_not_hold(M, N, K):
+    rng = np.random.RandomState(5)
+    A, B = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N)))
+    A[3, 5], A[M - 1, K - 1], A[70, 0], B[7, 9] = np.inf, np.nan, 2.0 ** 120, -np.inf
+    A[130] *= np.float32(2.0 ** 115)                        # a row of large numbers: beyond the scale, their sums well within range
+    B[:, 200] *= np.float32(2.0 ** -100)
+    A[131] = np.float32(2.0 ** -120) * A[131]               # products down to 2^-240: zero or subnormal
+    A[132] *= np.float32(2.0 ** -126)                       # subnormal numbers, against columns of ordinary ones
+    with np.errstate(all="ignore"):
+        expected = A.astype(np.float64) @ B.astype(np.float64)
+        fp32 = expected.astype(np.float32)
+        out = call(A, B, np.zeros((M, N), np.float32), M, N, K, 1.0, 0.0, False, False)
+        assert np.array_equal(np.isnan(out), np.isnan(fp32))
+        # (a sum of fp32 numbers may overflow where the exact one does not: only near the largest number, which no element is)
+        assert np.array_equal(np.isinf(out), np.isinf(fp32)) and np.array_equal(np.sign(out[np.isinf(out)]), np.sign(fp32[np.isinf(out)]))
+        fine = np.isfinite(fp32)
+        finite = lambda x: np.where(np.isfinite(x), x, 0).astype(np.float64)
+        # (the fp32 instruction's bound where a tile was computed again: 16 roundings per 16 k)
+        allowed = (K + 24) * 2.0 ** -24 * (np.abs(finite(A)) @ np.abs(finite(B))) + 2.0 ** -149 * K
+        assert np.all(np.abs(out - expected)[fine] <= allowed[fine])
+
+
+@pytest.mark.gpu
+def test_batch_scope_is_one_launch_of_split_tiles():
+    from gpu_util import DeviceArray
+    M, N, K, n = 640, 640, 640, 5
+    rng = np.random.RandomState(2)
+    A, B = rng.randint(-8, 9, (n, M, K)).astype(np.float32), rng.randint(-8, 9, (n, K, N)).astype(np.float32)
+    dA, dB, dC = DeviceArray(A), DeviceArray(B), DeviceArray(np.zeros((n, M, N), np.float32))
+    w = runtime.wrappers()
+    assert w.tiramisu_hip_batch_begin() == 0
+    for i in range(n):
+        w.tiramisu_hip_sgemm(dA.ptr + 4 * i * M * K, dB.ptr + 4 * i * K * N, dC.ptr + 4 * i * M * N, M, N, K, 1.0, 0.0, 0, 0, 0, 0, 0, 0, False, False)
+    assert w.tiramisu_hip_batch_end() == 0
+    assert np.array_equal(dC.download(), A.astype(np.float64) @ B.astype(np.float64))

@@ -20,6 +20,7 @@
 #include "../../include/tiramisu_hip_wrappers.h"
 #include "kernels/gemm_mfma.hip.h"
 #include "kernels/gemm_mfma_f64.hip.h"
+#include "kernels/gemm_mfma_split.hip.h"
 #include "kernels/target_gfx950.h"
 
 namespace {
@@ -211,6 +212,44 @@ void launch_small(bool vec_ok, const float *A, const float *B, float *C, int M, 
     else launch_small_slice<AK, BK_, BM, BN, 64>(edge, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
 
+// A kernel whose LDS exceeds the 64 KiB that a launch gets without asking (once per device and kernel: `asked` is the kernel's).
+void allow_lds(const void *kernel, int bytes, std::atomic<unsigned long long> &asked, const char *fn) {
+    if (bytes <= 64 * 1024) return;
+    int device = 0;
+    check(hipGetDevice(&device), fn);
+    const unsigned long long bit = 1ull << (device & 63);
+    if (asked.load() & bit) return;
+    check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes), fn);
+    asked.fetch_or(bit);
+}
+
+// fp32 operands as three bf16 parts each (kernels/gemm_mfma_split.hip.h)
+template <class CFG>
+void launch_split(const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc, float alpha, float beta) {
+    const int tiles = ((M + CFG::BM - 1) / CFG::BM) * ((N + CFG::BN - 1) / CFG::BN);
+    if (active_batch) {
+        static std::atomic<unsigned long long> asked{0};
+        allow_lds((const void *)tgemm::sgemm_split_batched_kernel<CFG>, CFG::LDS_BYTES, asked, "tiramisu_hip_sgemm");
+        hipLaunchKernelGGL((tgemm::sgemm_split_batched_kernel<CFG>), dim3(tiles, 1, active_batch_count), dim3(CFG::NT), CFG::LDS_BYTES, current_stream,
+                           *active_batch, M, N, K, lda, ldb, ldc, alpha, beta);
+    } else {
+        static std::atomic<unsigned long long> asked{0};
+        allow_lds((const void *)tgemm::sgemm_split_kernel<CFG>, CFG::LDS_BYTES, asked, "tiramisu_hip_sgemm");
+        hipLaunchKernelGGL((tgemm::sgemm_split_kernel<CFG>), dim3(tiles), dim3(CFG::NT), CFG::LDS_BYTES, current_stream, A, B, C, M, N, K, lda, ldb, ldc,
+                           alpha, beta);
+    }
+    check(hipGetLastError(), "tiramisu_hip_sgemm");
+}
+template <bool AK, bool BK_>
+void dispatch_split(int edge, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc, float alpha, float beta) {
+    const bool whole = ttarget::split_whole(edge, M, N, K);
+    if (edge == 64) launch_split<typename tgemm::split_config<64, AK, BK_, false>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else if (edge == 128 && whole) launch_split<typename tgemm::split_config<128, AK, BK_, false>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else if (edge == 128) launch_split<typename tgemm::split_config<128, AK, BK_, true>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else if (whole) launch_split<typename tgemm::split_config<256, AK, BK_, false>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else launch_split<typename tgemm::split_config<256, AK, BK_, true>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+}
+
 // Few C tiles but a long reduction (a batch of 64 rows against wide weights, as in recurrent
 // cells): 64x32 tiles, 8 groups of wavefronts share the K range of each tile and reduce through
 // LDS, and up to four K-slices are requested ahead (the launch is latency-bound).
@@ -382,13 +421,18 @@ void *static_scratch_here() {
 template <bool AK, bool BK_>
 void dispatch_edge(bool vec_ok, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb,
                    long ldc, float alpha, float beta) {
-    const int bm = tile_for(M, N);
+    const int bm = tile_for(M, N), problems = active_batch ? active_batch_count : 1;
     const bool edge = !(vec_ok && M % bm == 0 && N % bm == 0 && K % (bm == 64 ? 32 : 16) == 0);   // K-slice of the tile
-    if (bm == 64 || M < 32 || N < 32) {
-        const ttarget::small_tile t = ttarget::small_tile_for(M, N, K, active_batch ? active_batch_count : 1, !edge);
-        if (t == ttarget::TILE_64x32) return launch_small<AK, BK_, 64, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-        if (t == ttarget::TILE_32) return launch_small<AK, BK_, 32, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    }
+    ttarget::small_tile t = ttarget::TILE_64;
+    if (bm == 64 || M < 32 || N < 32) t = ttarget::small_tile_for(M, N, K, problems, !edge);
+    const int tile_m = t == ttarget::TILE_64 ? bm : t == ttarget::TILE_64x32 ? 64 : 32, tile_n = t == ttarget::TILE_64 ? bm : 32;
+    // (a slice of 32 k is guarded like any other: the small tiles look at theirs themselves)
+    const bool guarded = t == ttarget::TILE_64 ? edge : !(vec_ok && M % tile_m == 0 && N % tile_n == 0 && K % ttarget::small_tile_slice(K) == 0);
+    if (lda >= 4 && lda < ttarget::SPLIT_LD_LIMIT && ldb >= 4 && ldb < ttarget::SPLIT_LD_LIMIT)
+        if (const int split = ttarget::split_tile_for(M, N, K, problems, tile_m, tile_n, guarded))
+            return dispatch_split<AK, BK_>(split, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    if (t == ttarget::TILE_64x32) return launch_small<AK, BK_, 64, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    if (t == ttarget::TILE_32) return launch_small<AK, BK_, 32, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     if (edge) dispatch_tile<AK, BK_, true>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     else dispatch_tile<AK, BK_, false>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
@@ -397,17 +441,8 @@ template <class S, bool A_KFAST, bool B_NFAST>
 void launch_dgemm_kernel(const double *A, const double *B, double *C, int M, int N, int K, long sam, long sak, long sbk, long sbn, long ldc,
                                 double alpha, double beta) {
     auto kernel = tgemm64::dgemm_kernel<S, A_KFAST, B_NFAST>;
-    // the large tile's two LDS stages exceed the 64 KiB that a launch gets without asking (once per device)
     static std::atomic<unsigned long long> asked{0};
-    if (S::LDS_BYTES > 64 * 1024) {
-        int device = 0;
-        check(hipGetDevice(&device), "tiramisu_hip_dgemm");
-        const unsigned long long bit = 1ull << (device & 63);
-        if (!(asked.load() & bit)) {
-            check(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS_BYTES), "tiramisu_hip_dgemm");
-            asked.fetch_or(bit);
-        }
-    }
+    allow_lds((const void *)kernel, S::LDS_BYTES, asked, "tiramisu_hip_dgemm");
     const unsigned tiles = (unsigned)(((M + S::BM - 1) / S::BM) * ((N + S::BN - 1) / S::BN));
     hipLaunchKernelGGL(kernel, dim3(tiles), dim3(S::NT), S::LDS_BYTES, current_stream, A, B, C, M, N, K, sam, sak, sbk, sbn, ldc, alpha, beta);
     check(hipGetLastError(), "tiramisu_hip_dgemm");

@@ -62,6 +62,55 @@ inline small_tile small_tile_for(long M, long N, long K, long problems, bool who
 // 14.4; with one row 1 x 142339 x 20 17.8 (one thread per element), 18.2, 10.2.
 inline int small_tile_slice(long K) { return K <= 32 ? 32 : 64; }
 
+// C tiles of the kernels that split fp32 operands into bf16 parts (gemm_mfma_split.hip.h), and when they replace the fp32 instruction.
+// Whole launches of both kinds are modelled like the tiles above: `fixed` microseconds and `first` per k for a round of tiles over the
+// compute units, `round` and `further` per k for each round after it; fitted at 64 ... 4096 k, up to sixteen rounds, uniform
+// random operands (rms error 3 to 8 %).  us measured with the fp32 instruction / split: 4096^3 946 / 607 (256 x 256),
+// 2048^3 136 / 97 (128 x 128), 4096 x 4096 x 128 43 / 33, 2048 x 2048 x 256 23.1 / 20.3, 1024^3 21.5 / 19.0 (64 x 64), guarded 3623 x 2943 x 920
+// 193 / 130, 1218 x 2748 x 611 50 / 37; and where the fp32 instruction stays: 1024 x 1024 x 256 8.2 / 8.8, 2048 x 2048 x 128
+// 14.8 / 14.9, 1520 x 3116 x 503 51 / 54.
+struct launch_model { int m, n; bool guarded; double fixed, round, first, further; };
+constexpr launch_model FP32_LAUNCHES[] = {
+    {256, 256, false, 11.0, 2.0, 0.2242, 0.23}, {192, 192, false, 9.2, 2.6, 0.1322, 0.132}, {128, 128, false, 4.9, 3.2, 0.0617, 0.0587},
+    {64, 64, false, 3.1, 0.7, 0.0175, 0.0157}, {64, 32, false, 3.3, 0.8, 0.0093, 0.0080}, {32, 32, false, 3.0, 0.5, 0.0061, 0.0043},
+    {128, 128, true, 6.7, 4.8, 0.0669, 0.0601}, {64, 64, true, 4.1, 1.1, 0.0206, 0.0165}, {64, 32, true, 4.4, 1.5, 0.0104, 0.0091},
+    {32, 32, true, 4.2, 0.8, 0.0073, 0.0048}};
+constexpr launch_model SPLIT_LAUNCHES[] = {
+    {256, 256, false, 10.1, 2.3, 0.135, 0.145}, {128, 128, false, 7.9, 5.8, 0.0380, 0.0404}, {64, 64, false, 5.3, 3.5, 0.0132, 0.0121},
+    {256, 256, true, 12.1, 2.3, 0.130, 0.145}, {128, 128, true, 9.2, 8.7, 0.0360, 0.0405}};
+inline double modelled(const launch_model &l, long M, long N, long K, long problems) {
+    const long tiles = ((M + l.m - 1) / l.m) * ((N + l.n - 1) / l.n) * problems;
+    const double more = (double)((tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS - 1);
+    return l.fixed + more * l.round + K * (l.first + more * l.further);
+}
+// k of a slice; LDS of a workgroup (two stages of three planes, or of eight wavefronts' own slices)
+constexpr int split_slice(int edge) { return edge == 128 ? 32 : 16; }
+constexpr int split_operand_words(int edge, bool kmajor) {
+    return edge == 64 ? 64 * 16 + (kmajor ? 0 : 64) : 3 * (split_slice(edge) / 8) * 4 * (kmajor ? edge + 128 / split_slice(edge) : edge + 16);
+}
+constexpr int split_lds_bytes(int edge, bool a_kmajor, bool b_kmajor) {
+    return 2 * 4 * (edge == 64 ? 8 : 1) * (split_operand_words(edge, a_kmajor) + split_operand_words(edge, b_kmajor));
+}
+// leading dimensions: four elements of a row at least, offsets within a tile in 32 bits
+constexpr long SPLIT_LD_LIMIT = 1L << 22;
+constexpr bool split_whole(int edge, long M, long N, long K) { return M % edge == 0 && N % edge == 0 && K % split_slice(edge) == 0; }
+// The edge of the split tile that takes an M x N x K product from fp32 tiles of m x n (guarded or not), 0: none.  Where the fp32
+// tiles are 32 wide, four groups of wavefronts add four partial sums: only the eight of the 64 x 64 tile are at least as close
+// to 64 bits.  Below 96 k the two are equally close, and little is gained.
+inline int split_tile_for(long M, long N, long K, long problems, int m, int n, bool guarded) {
+    if (M < 64 || N < 64 || K < 96) return 0;
+    double best = 0;
+    for (const launch_model &l : FP32_LAUNCHES)
+        if (l.m == m && l.n == n && l.guarded == guarded) best = 0.95 * modelled(l, M, N, K, problems);
+    int edge = 0;
+    for (const launch_model &l : SPLIT_LAUNCHES) {
+        if (l.guarded == split_whole(l.m, M, N, K) || (n == 32 && l.m != 64)) continue;
+        const double cost = modelled(l, M, N, K, problems);
+        if (cost < best) { best = cost; edge = l.m; }
+    }
+    return edge;
+}
+
 // C tiles of the bf16-input kernels.  What the loops over K of a launch take is modelled as `fixed` microseconds (start, first
 // slices) plus, for every 32 k of whole slices, `first` for the first round of tiles over the compute units and `further` for
 // each round after it.  Reading and writing C is left out: it takes every tile the same (64 MiB in and out at 4096 x 4096 20 us),
