@@ -50,6 +50,8 @@
 //                      of a tile; launch it with ceil(ST_TH / (ST_W*ST_RPT_EDGE - 2*ST_R*ST_RAD))
 //                      workgroups per boundary tile)
 //   ST_EXPR            expression of the new value in terms of ST_AT(dy, dx)
+//   ST_SHIFTS          1: the expression reads columns left or right of a cell and the radius is 1 (default 0): the values of
+//                      the adjacent lanes are fetched ahead of the step's barrier
 //   ST_NAME_EDGE       name of the kernel for the tiles that touch the fixed boundary
 //   ST_STREAM          bit 0: staging loads carry the non-temporal hint, bit 1: the stores of the tile centre do
 //   ST_GX, ST_GY       number of tiles along x and y
@@ -79,6 +81,14 @@
 #define ST_GLOBAL_LOAD1(p) (*(p))
 #define ST_GLOBAL_STORE4(p, v, stream) do { if (stream) __builtin_nontemporal_store((v), (p)); else *(p) = (v); } while (0)
 #define ST_GLOBAL_STORE1(p, v) (*(p) = (v))
+#define ST_GLOBAL_LOAD4_ANY(p) (*reinterpret_cast<const st_f4_any *>(p))
+#define ST_GLOBAL_STORE4_ANY(p, v, stream) do { if (stream) __builtin_nontemporal_store((v), reinterpret_cast<st_f4_any *>(p)); else *reinterpret_cast<st_f4_any *>(p) = (v); } while (0)
+#define ST_KEEP(a, b) asm volatile("" : "+v"(a), "+v"(b))
+#endif
+// a quad that begins at any cell (rows of a length that is not a multiple of four)
+#ifndef ST_GLOBAL_LOAD4_ANY
+#define ST_GLOBAL_LOAD4_ANY(p) (st_f4{ST_GLOBAL_LOAD1(p), ST_GLOBAL_LOAD1((p) + 1), ST_GLOBAL_LOAD1((p) + 2), ST_GLOBAL_LOAD1((p) + 3)})
+#define ST_GLOBAL_STORE4_ANY(p, v, stream) do { for (int e_ = 0; e_ < 4; e_++) ST_GLOBAL_STORE1((p) + e_, (v)[e_]); } while (0)
 #endif
 
 #define ST_HY (ST_R * ST_RAD)                       /* halo rows */
@@ -99,12 +109,20 @@
     float *__restrict__ dst_prev = ST_MODE == 2 ? ST_PLANE((src_plane + ST_R - 1) & 1) : nullptr;              \
     const float *fixed_other = ST_PLANE(ST_MODE == 3 ? src_plane : 1 - src_plane);
 
+#ifndef ST_SHIFTS
+#define ST_SHIFTS 0
+#endif
+#ifndef ST_KEEP
+#define ST_KEEP(a, b) ((void)0)
+#endif
+
 #ifndef TIRAMISU_AMD_STENCIL2D_REGS_COMMON
 #define TIRAMISU_AMD_STENCIL2D_REGS_COMMON
 #ifdef ST_HOST_MODEL
 typedef float st_f4 __attribute__((vector_size(16)));
 #else
 typedef float st_f4 __attribute__((ext_vector_type(4)));
+typedef float st_f4_any __attribute__((ext_vector_type(4), aligned(4)));
 #endif
 
 // lane i receives lane i-1's value; lane 0, which has no such neighbour, reads 0 (its cells next to the region's
@@ -135,11 +153,22 @@ __device__ __forceinline__ st_f4 st_load_quad(const float *plane, int gy, int gx
         const st_f4 a = ST_GLOBAL_LOAD4(reinterpret_cast<const st_f4 *>(plane + (in ? (size_t)gy * NX + gx : (size_t)0)), false);
         return in ? a : v;
     }
-    const bool row_in = !CHECK || (gy >= 0 && gy < NY);
+    // Rows at any alignment: the same 16-byte instruction loads from any multiple of four bytes (one load per cell: 1030 x 1030, 9
+    // steps, 22.5 us; so 15.6).  Where the plane ends inside the quad it is moved to the row's last four cells and shifted.
+    if (!CHECK) return ST_GLOBAL_LOAD4_ANY(plane + (size_t)gy * NX + gx);
+    if (NX >= 4) {
+        const bool in = gy >= 0 && gy < NY && gx >= 0 && gx < NX;
+        const int at = gx < NX - 4 ? gx : NX - 4, behind = gx - at;
+        const st_f4 a = ST_GLOBAL_LOAD4_ANY(plane + (in ? (size_t)gy * NX + at : (size_t)0));
+        const st_f4 one = {a[1], a[2], a[3], 0.f}, two = {a[2], a[3], 0.f, 0.f}, three = {a[3], 0.f, 0.f, 0.f};
+        const st_f4 q = behind <= 0 ? a : behind == 1 ? one : behind == 2 ? two : three;
+        return in ? q : v;
+    }
+    const bool row_in = gy >= 0 && gy < NY;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         const int xx = gx + e;
-        const bool in = row_in && (!CHECK || (xx >= 0 && xx < NX));
+        const bool in = row_in && xx >= 0 && xx < NX;
         const float a = ST_GLOBAL_LOAD1(plane + (in ? (size_t)gy * NX + xx : (size_t)0));
         v[e] = in ? a : 0.f;
     }
@@ -190,10 +219,12 @@ __device__ __forceinline__ void ST_CAT(ST_NAME, _sweep)(const float *__restrict_
                 if (EDGE && (gy < WY0 || gy > WY1)) continue;
                 if ((ST_NX % 4 == 0) && (!EDGE || (gx >= WX0 && gx + 3 <= WX1))) {
                     ST_GLOBAL_STORE4(reinterpret_cast<st_f4 *>(to + (size_t)gy * ST_NX + gx), cur[r], (ST_STREAM & 2) != 0);
+                } else if (!EDGE || (gx >= WX0 && gx + 3 <= WX1)) {
+                    ST_GLOBAL_STORE4_ANY(to + (size_t)gy * ST_NX + gx, cur[r], (ST_STREAM & 2) != 0);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++)
-                        if (!EDGE || (gx + e >= WX0 && gx + e <= WX1)) ST_GLOBAL_STORE1(to + (size_t)gy * ST_NX + gx + e, cur[r][e]);
+                        if (gx + e >= WX0 && gx + e <= WX1) ST_GLOBAL_STORE1(to + (size_t)gy * ST_NX + gx + e, cur[r][e]);
                 }
             }
         }
@@ -209,6 +240,20 @@ __device__ __forceinline__ void ST_CAT(ST_NAME, _sweep)(const float *__restrict_
             *slot(parity, wave, 0, i) = cur[i];
             *slot(parity, wave, 1, i) = cur[RPT - ST_RAD + i];
         }
+        // The adjacent lanes' cells next to each of my quads, ahead of the barrier.  A lane shift takes the vector ALU twice as long as an
+        // add (1.8 against 1.0 ns per SIMD, as any operand that does not come from the lane's own registers), and an add that has one
+        // folded in stops the adds of the other wavefronts from being issued in pairs with it; here they fill the time in
+        // which the wavefronts wait for each other and for the LDS (8192 x 8192, launches of 11, 9 and 12 steps 160, 129 and 179 us
+        // with the shifts folded into the adds, 136, 115 and 170 so).  The empty statement keeps the compiler from folding them.
+        float from_left[RPT], from_right[RPT];
+        if (ST_SHIFTS) {
+#pragma unroll
+            for (int r = 0; r < RPT; r++) {
+                from_left[r] = st_from_left(cur[r][3]);
+                from_right[r] = st_from_right(cur[r][0]);
+                ST_KEEP(from_left[r], from_right[r]);
+            }
+        }
         if (ST_RAD > 0) __syncthreads();
         // my rows with ST_RAD rows of the neighbouring wavefronts above and below
         st_f4 ext[RPT + 2 * ST_RAD];
@@ -222,11 +267,11 @@ __device__ __forceinline__ void ST_CAT(ST_NAME, _sweep)(const float *__restrict_
 #pragma unroll
         for (int r = 0; r < RPT; r++) {
             // Old value at row r + dy, column e + dx of the quad (columns -RAD .. 3 + RAD): columns outside the quad
-            // come from the adjacent lane.  The shift is written where the value is used, once per use: the compiler
-            // folds a lane shift into the add that consumes it (v_add_f32_dpp) only when the two are a few
-            // instructions apart, and a shift folded that way costs no instruction.
+            // come from the adjacent lane: fetched above (ST_SHIFTS), or by a shift that is written where the value is used,
+            // once per use, so that the compiler folds it into the add that consumes it (v_add_f32_dpp).
             auto old_at = [&](int dy, int col) -> float {
                 const st_f4 &row = ext[r + ST_RAD + dy];
+                if (ST_SHIFTS && r + dy >= 0 && r + dy < RPT && (col < 0 || col > 3)) return col < 0 ? from_left[r + dy] : from_right[r + dy];
                 return col < 0 ? st_from_left(row[4 + col]) : col > 3 ? st_from_right(row[col - 4]) : row[col];
             };
             const bool row_in = !EDGE || (gy0 + r >= ST_Y0 && gy0 + r <= ST_Y1);

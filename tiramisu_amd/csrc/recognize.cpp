@@ -318,6 +318,8 @@ bool emit_stencil(context &ctx, const node_ptr &root, const node_ptr &time_loop,
     dev.fct = f;
     dev.device = true;
     const std::string point_text = dev.print(point);
+    // the cells left and right of a thread's quads take registers: with them the compiler is held to 128, two workgroups per compute unit
+    const bool sideways = radius == 1 && std::any_of(taps.begin(), taps.end(), [](const std::pair<long, long> &t) { return t.second != 0; });
     std::map<std::pair<int, int>, std::pair<kernel, kernel>> by_steps;   // (steps, mode) -> (interior tiles, tiles on the fixed boundary)
     std::ostringstream host;
     // one launch per chunk: the boundary slices ride behind the interior tiles (TIRAMISU_STENCIL_MERGE=0: two launches)
@@ -350,12 +352,13 @@ bool emit_stencil(context &ctx, const node_ptr &root, const node_ptr &time_loop,
               << "\n#define ST_Y0 " << lo[1] << "\n#define ST_Y1 " << hi[1] << "\n#define ST_X0 " << lo[2] << "\n#define ST_X1 " << hi[2]
               << "\n#define ST_GX " << GX << "\n#define ST_GY " << GY << "\n#define ST_IBX0 " << bx0 << "\n#define ST_IBX1 " << bx1
               << "\n#define ST_IBY0 " << by0 << "\n#define ST_IBY1 " << by1 << "\n#define ST_W " << WAVES
-              << "\n#define ST_MERGE " << (merge ? 1 : 0) << "\n#define ST_XCD " << env_int("TIRAMISU_STENCIL_XCD", 1) << "\n#define ST_OCC " << env_int("TIRAMISU_STENCIL_OCCUPANCY", 0) << "\n#define ST_STREAM " << env_int("TIRAMISU_STENCIL_STREAM", 2)
+              << "\n#define ST_MERGE " << (merge ? 1 : 0) << "\n#define ST_XCD " << env_int("TIRAMISU_STENCIL_XCD", 1) << "\n#define ST_OCC " << env_int("TIRAMISU_STENCIL_OCCUPANCY", sideways && ch.steps > 1 ? 4 : 0) << "\n#define ST_STREAM " << env_int("TIRAMISU_STENCIL_STREAM", 2)
               << "\n#define ST_RPT " << ROWS << "\n#define ST_RPT_EDGE " << rows_edge << "\n#define ST_R " << ch.steps << "\n#define ST_MODE " << ch.mode << "\n#define ST_RAD " << radius
+              << "\n#define ST_SHIFTS " << (sideways ? 1 : 0)
               << "\n#define ST_EXPR " << point_text << "\n#include \"stencil2d_regs.hip.h\"\n"
               << "#undef ST_NAME\n#undef ST_NAME_EDGE\n#undef ST_NY\n#undef ST_NX\n#undef ST_Y0\n#undef ST_Y1\n#undef ST_X0\n#undef ST_X1\n"
               << "#undef ST_GX\n#undef ST_GY\n#undef ST_IBX0\n#undef ST_IBX1\n#undef ST_IBY0\n#undef ST_IBY1\n#undef ST_W\n#undef ST_OCC\n#undef ST_STREAM\n"
-              << "#undef ST_MERGE\n#undef ST_XCD\n#undef ST_RPT\n#undef ST_RPT_EDGE\n#undef ST_R\n#undef ST_MODE\n#undef ST_RAD\n#undef ST_EXPR\n";
+              << "#undef ST_MERGE\n#undef ST_XCD\n#undef ST_RPT\n#undef ST_RPT_EDGE\n#undef ST_R\n#undef ST_MODE\n#undef ST_RAD\n#undef ST_SHIFTS\n#undef ST_EXPR\n";
             k.source = s.str();            // both kernels come from the one inclusion
             ke.source = "";
             for (kernel *q : {&k, &ke}) {
