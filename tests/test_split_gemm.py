@@ -159,3 +159,48 @@ def test_batch_scope_is_one_launch_of_split_tiles():
         w.tiramisu_hip_sgemm(dA.ptr + 4 * i * M * K, dB.ptr + 4 * i * K * N, dC.ptr + 4 * i * M * N, M, N, K, 1.0, 0.0, 0, 0, 0, 0, 0, 0, False, False)
     assert w.tiramisu_hip_batch_end() == 0
     assert np.array_equal(dC.download(), A.astype(np.float64) @ B.astype(np.float64))
+
+
+def conv_expected(x, w, bias):
+    """Convolution plus bias and the sum of the magnitudes, in float64, image by image (x padded)."""
+    n, ci, hp, wp = x.shape
+    co, h = w.shape[0], hp - 2
+    out, size = (np.empty((n, co, h, h)) for _ in range(2))
+    w2 = w.reshape(co, -1).astype(np.float64)
+    for i in range(n):
+        cols = np.stack([x[i, :, ky:ky + h, kx:kx + h] for ky in range(3) for kx in range(3)], 1).reshape(ci * 9, h * h).astype(np.float64)
+        with np.errstate(all="ignore"):
+            out[i] = (w2 @ cols).reshape(co, h, h) + bias[:, None, None]
+            size[i] = (np.abs(w2) @ np.abs(cols)).reshape(co, h, h) + np.abs(bias)[:, None, None]
+    return out, size
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["whole", "uniform", "special"])
+def test_windowed_convolution(kind):
+    from gpu_util import DeviceArray
+    name, shape = "conv2d_9x32x64x128", (9, 32, 64, 128)
+    p = runtime.load(PROGRAMS, name)
+    how = [k["how"] for k in p.manifest["kernels"]]
+    assert any("three bf16 parts" in s and "sliding window" in s and "cut into" in s for s in how)
+    n, ci, co, h = shape
+    rng = np.random.RandomState(3)
+    x, w, bias = np.zeros((n, ci, h + 2, h + 2), np.float32), rng.uniform(-1, 1, (co, ci, 3, 3)).astype(np.float32), rng.uniform(-1, 1, co).astype(np.float32)
+    x[:, :, 1:-1, 1:-1] = rng.uniform(-1, 1, (n, ci, h, h))
+    if kind == "whole":
+        x, w, bias = (np.round(8 * v).astype(np.float32) for v in (x, w, bias))
+    if kind == "special":        # in a whole tile, in a piece, and small numbers
+        x[0, 5, 40, 40], x[8, 31, 128, 100], x[4] = np.inf, np.nan, x[4] * np.float32(2.0 ** -126)
+    d = [DeviceArray(v) for v in (x, w, bias, np.zeros((n, co, h, h), np.float32))]
+    p(*[v.buffer() for v in d])
+    out = d[3].download()
+    expected, size = conv_expected(x, w, bias)
+    relu = np.where(np.isnan(expected), 0.0, np.maximum(expected, 0))
+    if kind == "whole":
+        assert np.array_equal(out, relu)
+        return
+    fine = np.isfinite(expected)
+    K = ci * 9
+    allowed = (K + 24) * 2.0 ** -24 * size + 2.0 ** -149 * K if kind == "special" else (6 / 16 * K / 2 + 24) * 2.0 ** -24 * size + 2.0 ** -25 * size
+    assert np.all(np.abs(out - relu)[fine] <= allowed[fine])
+    assert np.array_equal(np.isinf(out), expected == np.inf)

@@ -94,6 +94,8 @@ constexpr int split_lds_bytes(int edge, bool a_kmajor, bool b_kmajor) {
 // leading dimensions: four elements of a row at least, offsets within a tile in 32 bits
 constexpr long SPLIT_LD_LIMIT = 1L << 22;
 constexpr bool split_whole(int edge, long M, long N, long K) { return M % edge == 0 && N % edge == 0 && K % split_slice(edge) == 0; }
+// ... of a workgroup of the windowed convolution on split operands (gemm_mfma_window_split.hip.h): three planes of 16-byte granules
+constexpr long window_split_lds_bytes(long rows, long taps, long window) { return 3 * 16 * (rows * (taps | 1) + 1 + window); }
 // The edge of the split tile that takes an M x N x K product from fp32 tiles of m x n (guarded or not), 0: none.  Where the fp32
 // tiles are 32 wide, four groups of wavefronts add four partial sums: only the eight of the 64 x 64 tile are at least as close
 // to 64 bits.  Below 96 k the two are equally close, and little is gained.

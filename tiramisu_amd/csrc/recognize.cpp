@@ -1285,6 +1285,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     int win_splits = 1;                  // pieces that each tile of the last, incomplete round is cut into
     long win_grid = 0, win_scratch_floats = 0, win_counters = 0;
     int win_resident = 1;                // workgroups that share a compute unit
+    bool win_split = false;              // operands split into bf16 parts (kernels/gemm_mfma_window_split.hip.h)
     std::string window_call_head;
     if (!bf16 && !with_consumer && lit && operands.size() == 1 && operands[0].first.linear && operands[0].first.kmajor &&
         !operands[0].second.linear && GK.dims.size() >= 2 && GK.literal && GN.literal && Ml % BM == 0 && Nl % BN == 0 && WGK == 1 &&
@@ -1337,10 +1338,23 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
             if (windowed) {
                 // as many workgroups as the chip holds take tiles from a queue; the tiles left over after the last
                 // full round of the grid are cut along the channel blocks into short pieces that fill the end
-                const long tiles = (Ml / BM) * (Nl / BN), blocks = win_channels / win_cb;
+                const long tiles = (Ml / BM) * (Nl / BN);
                 // two workgroups per compute unit when their LDS fits: one's tile boundaries (epilogue stores, the wait
                 // for the first block) are covered by the other's matrix instructions
                 win_resident = 2 * (2 * stage_bytes + 64) <= ttarget::LDS_BYTES_PER_CU ? env_int("TIRAMISU_MFMA_WINDOW_RESIDENT", 2) : 1;
+                // On the bf16 matrix cores a tile's start and end weigh more: for tiles of 256 positions with 32 channels or more, and more
+                // of them than two for every compute unit (32 images of 112 x 112, 64 to 64 channels 266 -> 181 us; one of 28 x 28 with tiles
+                // of 64 positions 13.6 -> 21, 12 of 40 x 40 with 16 channels 16.4 -> 17.2)
+                win_split = BM == 64 && BN == 256 && WGM == 1 && WGN == 4 && win_channels % 8 == 0 && win_channels >= 32 && tiles > 2 * ttarget::COMPUTE_UNITS &&
+                            lda_lit < (1L << 22) && 2 * (ttarget::window_split_lds_bytes(BM, win_taps, need) + 64) <= ttarget::LDS_BYTES_PER_CU &&
+                            !backend_option("TIRAMISU_MFMA_NO_SPLIT_OPERANDS") && !backend_option("TIRAMISU_MFMA_WINDOW_CB") &&
+                            !backend_option("TIRAMISU_MFMA_WINDOW_AHEAD") && env_int("TIRAMISU_MFMA_WINDOW_XCD_QUEUES", 1) != 0;
+                if (win_split) {
+                    win_cb = 8;
+                    win_floats = (int)need;
+                    win_resident = env_int("TIRAMISU_MFMA_WINDOW_RESIDENT", 2);
+                }
+                const long blocks = win_channels / win_cb;
                 win_grid = std::min<long>(tiles, (long)ttarget::COMPUTE_UNITS * win_resident);
                 const long rest = tiles % win_grid;
                 if (rest > 0 && tiles > win_grid && !backend_option("TIRAMISU_MFMA_NO_TAIL_SPLIT")) win_splits = (int)std::min<long>(std::min<long>(blocks, 2 * win_grid / rest), 16);
@@ -1544,13 +1558,14 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         body << bf16_config_text(bf16_direct, BM, BK, WGM, WGN, bf16_stages, edge);
     } else {
         body << "    extern __shared__ __attribute__((aligned(16))) float _lds[];\n";
-        if (split_edge) body << "    typedef tgemm::split_config<" << split_edge << ", " << (operands[0].first.kmajor ? "true" : "false") << ", " << (operands[0].second.kmajor ? "true" : "false")
+        if (win_split) body << "    typedef tgemm::config_window<" << BM << ", " << BN << ", " << WGM << ", " << WGN << "> CFG;\n";
+        else if (split_edge) body << "    typedef tgemm::split_config<" << split_edge << ", " << (operands[0].first.kmajor ? "true" : "false") << ", " << (operands[0].second.kmajor ? "true" : "false")
                              << ", " << (edge ? "true" : "false") << ">::type CFG;\n";
         else body << "    typedef " << cfg << " CFG;\n";
     }
     body << "    const int _M = " << dev.print(Me) << ", _N = " << dev.print(Ne) << ", _K = " << dev.print(Ke) << ";\n";
     body << "    int _tm, _tn;\n    tgemm::tile_of_block((_M + CFG::BM - 1) / CFG::BM, (_N + CFG::BN - 1) / CFG::BN, _tm, _tn);\n";
-    if (!split_edge) body << "    tgemm::accumulators<CFG> _acc;\n    _acc.clear();\n" << consumer_loads_text.str();
+    if (!split_edge && !win_split) body << "    tgemm::accumulators<CFG> _acc;\n    _acc.clear();\n" << consumer_loads_text.str();
     int term = 0, ktab_words = 0;
     std::string split_call_head;
     const std::string kname = "_kernel_" + std::to_string(ctx.next_kernel_id());
@@ -1593,8 +1608,9 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
             for (int p : GN.dims) pre << " + (long)" << U.dims[p].kvar << " * " << dev.print(o.second.coef.at(p));
             pre << ";\n    }\n};\n";
             std::ostringstream call;
-            call << "    tgemm::contraction_window<CFG, " << win_cb << ", " << win_taps << ", " << win_floats << ", " << env_int("TIRAMISU_MFMA_WINDOW_AHEAD", 2) << ", " << win_splits << ", " << (env_int("TIRAMISU_MFMA_WINDOW_XCD_QUEUES", 1) ? "true" : "false") << ", " << kname << "_taps>("
-                 << o.first.buf->get_name() << " + (" << dev.print(o.first.base) << "), " << dev.print(o.first.ld) << ", " << o.second.buf->get_name() << " + ("
+            if (win_split) call << "    tgemm::contraction_window_split<CFG, " << win_taps << ", " << win_floats << ", " << win_splits << ", " << kname << "_taps>(";
+            else call << "    tgemm::contraction_window<CFG, " << win_cb << ", " << win_taps << ", " << win_floats << ", " << env_int("TIRAMISU_MFMA_WINDOW_AHEAD", 2) << ", " << win_splits << ", " << (env_int("TIRAMISU_MFMA_WINDOW_XCD_QUEUES", 1) ? "true" : "false") << ", " << kname << "_taps>(";
+            call << o.first.buf->get_name() << " + (" << dev.print(o.first.base) << "), " << dev.print(o.first.ld) << ", " << o.second.buf->get_name() << " + ("
                  << dev.print(o.second.base) << "), " << win_x_elements << "L, " << kname << "_pos(), " << win_chan_stride << "L, " << win_channels
                  << ", _M, _N, _tail_scratch, _lds, ";
             window_call_head = call.str();
@@ -1740,7 +1756,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     }
     const std::string epi_args = two_pass ? "_epi_value, _epi_store" : "_epi";
     if (windowed) {
-        body << window_call_head << epi_args << ");\n";
+        body << window_call_head << (two_pass || !win_split ? epi_args : "[](int, int, float _sum) { return _sum; }, _epi") << ");\n";
     } else if (split_edge) {
         body << split_call_head << (two_pass ? epi_args : "[](int, int, float _sum) { return _sum; }, _epi") << ");\n";
     } else {
@@ -1754,7 +1770,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     k.name = kname;
     bool any_gather = false;
     for (auto &o : operands) any_gather = any_gather || !o.first.linear || !o.second.linear;
-    k.how = std::string("mfma-contraction: ") + (bf16 ? (bf16_direct ? "v_mfma_f32_32x32x16_bf16, slices loaded straight into LDS (through registers where an operand begins at an odd element), " : "v_mfma_f32_32x32x16_bf16, ") : split_edge ? "v_mfma_f32_32x32x16_bf16 on the three bf16 parts of every fp32 operand element, " : "v_mfma_f32_32x32x2_f32, ") + (windowed ? "implicit GEMM, sliding window of " + std::to_string(win_taps) + " taps staged in LDS by blocks of " + std::to_string(win_cb) + " channels, " :
+    k.how = std::string("mfma-contraction: ") + (bf16 ? (bf16_direct ? "v_mfma_f32_32x32x16_bf16, slices loaded straight into LDS (through registers where an operand begins at an odd element), " : "v_mfma_f32_32x32x16_bf16, ") : split_edge || win_split ? "v_mfma_f32_32x32x16_bf16 on the three bf16 parts of every fp32 operand element, " : "v_mfma_f32_32x32x2_f32, ") + (windowed ? "implicit GEMM, sliding window of " + std::to_string(win_taps) + " taps staged in LDS by blocks of " + std::to_string(win_cb) + " channels, " :
                                                                                       any_gather ? "implicit GEMM (gathered operand), " : "") + "M " +
             std::to_string(Mg.size()) + " dim(s) x N " + std::to_string(Ng.size()) + " x K " + std::to_string(Kg.size()) + ", tile " +
             std::to_string(BM) + "x" + std::to_string(BN) + "x" + std::to_string(BK) + (edge ? ", guarded edges" : ", whole tiles") + ", " +
@@ -1839,7 +1855,8 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         else if (bf16) k.lds_bytes = std::to_string(bf16_stages * (BK / 8) * (BM + BN) * 4 * 4);
         else if (ktab_words) k.lds_bytes = std::to_string(2 * (rowA + rowB) * 4 + ktab_words * 4);
         if (with_consumer) k.lds_bytes = std::to_string(std::stol(k.lds_bytes) + BM * (BN + 1) * 4);
-        if (windowed) k.lds_bytes = std::to_string(2 * ((long)win_cb * (win_taps * BM + 32) + (long)win_cb * win_floats) * 4);
+        if (win_split) k.lds_bytes = std::to_string(ttarget::window_split_lds_bytes(BM, win_taps, win_floats));
+        else if (windowed) k.lds_bytes = std::to_string(2 * ((long)win_cb * (win_taps * BM + 32) + (long)win_cb * win_floats) * 4);
     }
     std::ostringstream src;
     src << pre.str();
@@ -1882,7 +1899,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     k.source = src.str();
     add_include_once(ctx, "#include \"gemm_mfma.hip.h\"");
     if (bf16) add_include_once(ctx, "#include \"gemm_mfma_bf16.hip.h\"");
-    if (windowed) add_include_once(ctx, "#include \"gemm_mfma_window.hip.h\"");
+    if (windowed) add_include_once(ctx, win_split ? "#include \"gemm_mfma_window_split.hip.h\"" : "#include \"gemm_mfma_window.hip.h\"");
     if (split_edge) add_include_once(ctx, "#include \"gemm_mfma_split.hip.h\"");
     if (bf16_direct) {
         host << "        if ((" << addresses << ") % 4 == 0) {\n" << launch_text(k, "            ") << "        } else {\n"
