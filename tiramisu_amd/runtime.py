@@ -100,6 +100,8 @@ class Buffer:
         return ctypes.byref(self.raw)
 
 
+HIP_STREAM_LEGACY = 1        # hipStreamLegacy: the null stream, by a handle that is not null
+
 _wrappers = None
 
 
@@ -221,8 +223,7 @@ class Program:
         """Arguments: ``Buffer`` objects, numpy arrays (host buffers) or torch tensors (host or GPU buffers by where
         they live).  With a GPU tensor among them the function's kernels run on torch's current stream of that
         tensor's device, in order with the torch work around the call (the runtime's stream of the calling thread is
-        put back afterwards); when that is torch's default stream the call waits for it first and for its own
-        kernels afterwards."""
+        put back afterwards); when that is torch's default stream the call waits for its kernels before it returns."""
         bufs, torch_stream = [], None
         for a in args:
             if isinstance(a, Buffer):
@@ -240,19 +241,18 @@ class Program:
             self.check(bufs)
         if torch_stream is None:
             rc = self.fn(*[b.pointer() for b in bufs])
-        elif torch_stream == 0:
-            # torch's default stream is the device's null stream, and its handle, 0, means the calling thread's own
-            # default stream to tiramisu_hip_set_stream: the call is ordered by waiting on both sides instead
-            import torch
-            torch.cuda.current_stream().synchronize()
-            rc = self.fn(*[b.pointer() for b in bufs])
-            wrappers().tiramisu_hip_stream_synchronize(0)
         else:
+            # torch's default stream is the device's null stream.  Its handle, 0, means the calling thread's own default stream to
+            # tiramisu_hip_set_stream; HIP's other name for it does not.  On it the kernels follow the torch work before the call
+            # without a wait on the host (one wait less: a convolution of 8 images of 112 x 112 from 3 to 64 channels 40 -> 37.5 us,
+            # from 64 to 64, 32 images, 204 -> 196)
             w = wrappers()
             before = w.tiramisu_hip_get_stream()
-            w.tiramisu_hip_set_stream(torch_stream)
+            w.tiramisu_hip_set_stream(torch_stream or HIP_STREAM_LEGACY)
             try:
                 rc = self.fn(*[b.pointer() for b in bufs])
+                if torch_stream == 0:
+                    w.tiramisu_hip_stream_synchronize(0)
             finally:
                 w.tiramisu_hip_set_stream(before)
         if rc != 0:
