@@ -115,11 +115,15 @@ static inline float model_load1(const void *p) { record_load(p, 1); return 0.f; 
 #define ST_RAD 1
 #define ST_EXPR (ST_AT(0, 0) + ST_AT(-1, 0) + ST_AT(1, 0) + ST_AT(0, -1) + ST_AT(0, 1))
 
-// the fused form: 8 wavefronts x 11 rows, boundary slices of 5 rows per thread
+// the fused form: 8 wavefronts x 11 rows, boundary slices of 5 rows per thread, or what the compile line says
+#ifndef MODEL_ROWS
+#define MODEL_ROWS 11
+#define MODEL_ROWS_EDGE 5
+#endif
 #define ST_NAME model_fused
 #define ST_NAME_EDGE model_fused_edge
-#define ST_RPT 11
-#define ST_RPT_EDGE 5
+#define ST_RPT MODEL_ROWS
+#define ST_RPT_EDGE MODEL_ROWS_EDGE
 #include "../../tiramisu_amd/csrc/kernels/stencil2d_regs.hip.h"
 #undef ST_NAME
 #undef ST_NAME_EDGE
@@ -138,9 +142,9 @@ static inline float model_load1(const void *p) { record_load(p, 1); return 0.f; 
 
 // One launch of `steps` steps in `mode` reading plane `src_plane` (of the pair; mode 2 reads the third plane).
 static void run_launch(int ny, int nx, int steps, int mode, int src_plane) {
-    const int waves = 8, rows = mode == 3 ? 4 : 11;
+    const int waves = 8, rows = mode == 3 ? 4 : MODEL_ROWS;
     const tstencil::launch_geometry g = tstencil::plan_launch(ny, nx, 1, ny - 2, 1, nx - 2, 1, steps, waves, rows);
-    if (g.rows_edge != (mode == 3 ? 2 : 5)) {
+    if (g.rows_edge != (mode == 3 ? 2 : MODEL_ROWS_EDGE)) {
         // the emitter would compile another instance of the kernel (whole rows per thread in the slices): not modelled
         return;
     }
@@ -230,7 +234,7 @@ int main(int argc, char **argv) {
         for (int nx : widths) {
             const int ny = n;
             for (int r = 1; r <= r_hi; r++) {
-                if (88 - 2 * r <= 0) break;
+                if (8 * MODEL_ROWS - 2 * r < tstencil::MIN_TILE_ROWS) break;
                 for (int mode = 0; mode <= 3; mode++) {
                     if ((mode == 0 || mode == 1) && r % 2 == 0) continue;
                     if (mode == 2 && r < 2) continue;

@@ -12,12 +12,14 @@ import os
 import shutil
 import subprocess
 
+import pytest
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 MODEL = os.path.join(ROOT, "tests", "host_models", "stencil_address_model.cpp")
 
 
-def build_model(source, out):
-    subprocess.run(["g++", "-std=c++17", "-O2", "-Wno-unknown-pragmas", "-o", out, source], check=True)
+def build_model(source, out, *defines):
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wno-unknown-pragmas", *defines, "-o", out, source], check=True)
 
 
 def test_every_load_and_store_of_the_stencil_kernel_is_in_bounds_and_owed(tmp_path):
@@ -27,6 +29,17 @@ def test_every_load_and_store_of_the_stencil_kernel_is_in_bounds_and_owed(tmp_pa
     print(r.stdout[-2000:])
     assert r.returncode == 0, r.stdout[-2000:]
     assert " 0 failure(s)" in r.stdout
+
+
+@pytest.mark.parametrize("rows,rows_edge", [(2, 1), (2, 2), (3, 3), (4, 2), (5, 5), (6, 3), (7, 7), (8, 4), (10, 5)])
+def test_fewer_rows_per_thread(tmp_path, rows, rows_edge):
+    """The strips that the plan gives to small planes: planes of one tile to several, with and without interior tiles,
+    every number of steps down to tiles of the fewest rows."""
+    exe = str(tmp_path / "model")
+    build_model(MODEL, exe, "-DMODEL_ROWS=%d" % rows, "-DMODEL_ROWS_EDGE=%d" % rows_edge)
+    for lo, hi in ((5, 40), (530, 532)):
+        r = subprocess.run([exe, str(lo), str(hi), "12"], stdout=subprocess.PIPE, text=True)
+        assert r.returncode == 0 and " 0 failure(s)" in r.stdout, r.stdout[-2000:]
 
 
 def test_the_model_reports_broken_indexing(tmp_path):

@@ -301,11 +301,12 @@ bool emit_stencil(context &ctx, const node_ptr &root, const node_ptr &time_loop,
     const long T0 = lo[0], T1 = hi[0];
     const long steps = T1 - T0 + 1;
     // region staged by one workgroup: WAVES*ROWS rows by 256 columns (kernels/stencil2d_regs.hip.h)
-    // fused launches: 8 wavefronts x 11 rows (a sweep over both put the optimum there); a single step out of place
-    // streams, and 4 rows per thread keep more workgroups and loads in flight
-    const int WAVES = env_int("TIRAMISU_STENCIL_WAVES", 8), ROWS = env_int("TIRAMISU_STENCIL_ROWS", planar ? 4 : 11);
-    if (WAVES < 1 || WAVES > 16 || ROWS < radius || ROWS > 32) return false;
-    const int LH = WAVES * ROWS, LW = 256;
+    // fused launches: 8 wavefronts x 11 rows (a sweep over both put the optimum there), fewer where the plane is small
+    // (plan_rows); a single step out of place streams, and 4 rows per thread keep more workgroups and loads in flight
+    const int WAVES = env_int("TIRAMISU_STENCIL_WAVES", 8), MAX_ROWS = env_int("TIRAMISU_STENCIL_ROWS", planar ? 4 : 11);
+    const bool forced_rows = env_int("TIRAMISU_STENCIL_ROWS", -1) == env_int("TIRAMISU_STENCIL_ROWS", -2);   // set, to whatever
+    if (WAVES < 1 || WAVES > 16 || MAX_ROWS < radius || MAX_ROWS > 32) return false;
+    const int LH = WAVES * MAX_ROWS, LW = 256;
     // most steps of one launch; a launch between the two planes takes the largest odd number below.  12: the final
     // launch writes two planes and has HBM time to cover one step more than the 11 of the others
     const int rcap = tstencil::step_cap(env_int("TIRAMISU_STENCIL_STEPS", 12), radius, LH);
@@ -337,6 +338,7 @@ bool emit_stencil(context &ctx, const node_ptr &root, const node_ptr &time_loop,
             kernel k, ke;
             k.name = "_kernel_" + std::to_string(ctx.next_kernel_id());
             ke.name = "_kernel_" + std::to_string(ctx.next_kernel_id());
+            const int ROWS = planar || forced_rows ? MAX_ROWS : tstencil::plan_rows(NY, NX, lo[1], hi[1], lo[2], hi[2], radius, ch.steps, WAVES, MAX_ROWS);
             const tstencil::launch_geometry g = tstencil::plan_launch(NY, NX, lo[1], hi[1], lo[2], hi[2], radius, ch.steps, WAVES, ROWS);
             const int TH = g.tile_rows, TW = g.tile_columns, rows_edge = g.rows_edge, TH_edge = g.slice_rows, edge_sub = g.slices;
             const long GX = g.tiles_x, GY = g.tiles_y, bx0 = g.ibx0, bx1 = g.ibx1, by0 = g.iby0, by1 = g.iby1;

@@ -46,12 +46,19 @@ inline std::vector<chunk> plan_time_loop(long first_step, long steps, int rcap, 
     if (planar) {
         chunks.push_back({first_step, 1, 3});
     } else if (temp_plane) {
-        // the final launch's length: the one that needs the fewest launches (the longest of those)
+        // the final launch's length: the one that needs the fewest launches and, if it can be had, none of a single
+        // step, whose traffic and launch cost as much as three steps' (the longest of those)
         int best = 2;
         size_t best_n = 0;
+        bool best_single = true;
         for (int fin = (int)std::min<long>(rcap, steps - 1); fin >= 2; fin--) {
-            const size_t n = odd_chunks(first_step, steps - fin).size();
-            if (best_n == 0 || n < best_n) { best = fin; best_n = n; }
+            const std::vector<chunk> head = odd_chunks(first_step, steps - fin);
+            const bool single = head.back().steps == 1;
+            if (best_n == 0 || head.size() < best_n || (head.size() == best_n && best_single && !single)) {
+                best = fin;
+                best_n = head.size();
+                best_single = single;
+            }
         }
         chunks = odd_chunks(first_step, steps - best);
         chunks.back().mode = 1;
@@ -99,6 +106,23 @@ inline launch_geometry plan_launch(long NY, long NX, long y0, long y1, long x0, 
     g.slice_rows = waves * g.rows_edge - 2 * g.halo_rows;
     g.slices = (g.tile_rows + g.slice_rows - 1) / g.slice_rows;
     return g;
+}
+
+// Rows per thread of one launch: at most `rows`, and as few as keep the launch within WHOLE_CHIP workgroups and a tile
+// at MIN_TILE_ROWS rows.  A thread walks its rows one after the other in every step, so a plane whose tiles leave
+// compute units idle (or whose chip holds the workgroups of shorter strips at once) takes as long as one strip: 11 rows
+// everywhere against this rule 18.8 -> 16.9 us (64^2 x 24), 19.3 -> 16.1 (500^2 x 20), 15.3 -> 12.7 (1030^2 x 9),
+// 33.6 -> 31.4 (2001^2 x 16).  512 is two workgroups of 8 wavefronts on each of 256 compute units: allowed 768, 2001^2 x 16
+// takes 38.7, and 256 gives 33.7.  Tiles of 8 rows and more only: 200^2 x 13 10.4 instead of 9.5, 300^2 x 8 8.7 instead of 8.1.
+constexpr int MIN_TILE_ROWS = 4;
+constexpr long WHOLE_CHIP = 512;
+inline int plan_rows(long NY, long NX, long y0, long y1, long x0, long x1, int radius, int steps, int waves, int rows) {
+    for (int fewer = std::max(2, radius); fewer < rows; fewer++) {
+        if (waves * fewer - 2 * steps * radius < MIN_TILE_ROWS) continue;
+        const launch_geometry g = plan_launch(NY, NX, y0, y1, x0, x1, radius, steps, waves, fewer);
+        if (g.interior + g.edge_tiles * g.slices <= WHOLE_CHIP) return fewer;
+    }
+    return rows;
 }
 
 }  // namespace tstencil
