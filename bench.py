@@ -41,6 +41,7 @@ import numpy as np  # noqa: E402
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
 FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix
 BF16_MFMA_PEAK_TFLOPS = 2500.0
+SPLIT_MFMA_PEAK_TFLOPS = BF16_MFMA_PEAK_TFLOPS / 6   # fp32 products as six products of bf16 parts
 FP32_VALU_PEAK_TFLOPS = 157.3  # MI355X vector fp32 (256 CUs x 128 lanes x 2 flops x 2.4 GHz): what a kernel without MFMA is priced against
 FP32_VALU_PLAIN_TFLOPS = 39.3  # 256 CUs x 64 lanes x 2.4 GHz x 1 flop: separate adds and multiplies, one per lane and clock (no FMA:
                                # the stencil's value must round as the un-fused program's; packed fp32 is not used on this pool)
@@ -300,6 +301,11 @@ def bench_heat2d(steps, warmup, with_cpu):
     return out
 
 
+def matrix_peak(name, kernel, peak_tflops):
+    """The rate that the matrix instructions of a function's kernel can reach; peak_tflops: with the ordinary ones."""
+    return SPLIT_MFMA_PEAK_TFLOPS if "three bf16 parts" in kernel_descriptions(name).get(kernel, "") else peak_tflops
+
+
 def bench_sgemm(M, steps, warmup, with_cpu):
     from tiramisu_amd import runtime
     from oracle import build as oracle_build
@@ -319,12 +325,13 @@ def bench_sgemm(M, steps, warmup, with_cpu):
     dom = max(prof.items(), key=lambda kv: kv[1][0] * kv[1][1])
     kernel_ms, basis = launch_duration(prof, dom[0], ms)
     achieved = flop / (kernel_ms * 1e-3) / 1e12
+    peak = matrix_peak(name, dom[0], FP32_MFMA_PEAK_TFLOPS)
     out = {
         "value": flop / (ms * 1e-3) / 1e9, "unit": "GFLOP/s", "ms_per_step": ms, "warmup_extra_steps": EXTRA_WARMUP.get("last", 0),
-        "roofline": {"bound": "mfma", "achieved": achieved, "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / FP32_MFMA_PEAK_TFLOPS, "traffic": (kernel_traffic(name, dom[0]) or {}).get("bytes"),
+        "roofline": {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
+                     "frac": achieved / peak, "traffic": (kernel_traffic(name, dom[0]) or {}).get("bytes"),
                      "kernel": dom[0], "kernel_ms": kernel_ms, "kernel_ms_basis": basis, "kernel_ms_between_events": dom[1][0],
-                     "frac_between_events": flop / (dom[1][0] * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS},
+                     "frac_between_events": flop / (dom[1][0] * 1e-3) / 1e12 / peak},
     }
     if with_cpu:
         cpu = runtime.Program(oracle_build.cpu_program_library(PROGRAMS, name), name, needs_gpu_runtime=False)
@@ -467,6 +474,7 @@ def _generic_bench(name, host_arrays, flop, peak_tflops, steps, warmup, with_cpu
     dom_flop = flop * dominant_flop_share / dom[1][1]   # flops of an average launch of the dominant kernel
     kernel_ms, basis = launch_duration(prof, dom[0], ms)
     achieved = dom_flop / (kernel_ms * 1e-3) / 1e12
+    peak_tflops = matrix_peak(name, dom[0], peak_tflops)
     out = {"value": flop / (ms * 1e-3) / 1e9, "unit": "GFLOP/s", "ms_per_step": ms, "warmup_extra_steps": EXTRA_WARMUP.get("last", 0),
            "roofline": {"bound": "mfma", "achieved": achieved, "peak": peak_tflops, "unit": "TFLOP/s",
                         "frac": achieved / peak_tflops, "traffic": (kernel_traffic(name, dom[0]) or {}).get("bytes"),
