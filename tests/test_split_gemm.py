@@ -3,8 +3,9 @@ and on the GPU every tile, whole and guarded, in every layout, through the libra
 
 Exactness: products and sums of small whole numbers are exact.  Accuracy: with uniform operands a sum of K products rounds its
 accumulator once per matrix instruction, six per sixteen k, each time by at most 2^-24 of the sum of the magnitudes so far; the
-products left out are at most 2^-25 of theirs.  |error| <= (6/16 K 2^-24 / 2 + 2^-25) sum |a b| therefore bounds every element (on
-average half the accumulator's final value is there when it is rounded), with a few more roundings for partial sums, alpha and beta."""
+products left out are below 2^-24 of theirs.  |error| <= (6/16 K 2^-24 / 2 + 2^-24) sum |a b| therefore bounds every element (on
+average half the accumulator's final value is there when it is rounded), with a few more roundings for partial sums, alpha and beta.
+One product per sum: see test_one_product_per_sum."""
 import ctypes
 import os
 import subprocess
@@ -64,7 +65,7 @@ def test_rule(rule):
 
 
 def bound(A, B, K):
-    return (6 / 16 * K / 2 + 24) * 2.0 ** -24 * (np.abs(A) @ np.abs(B)) + 2.0 ** -25 * (np.abs(A) @ np.abs(B))
+    return (6 / 16 * K / 2 + 24) * 2.0 ** -24 * (np.abs(A) @ np.abs(B)) + 2.0 ** -24 * (np.abs(A) @ np.abs(B))
 
 
 def operands(rng, M, N, K, tA, tB, pad, kind):
@@ -105,6 +106,45 @@ def test_library_call(rule, M, N, K, edge, tA, tB):
             assert np.array_equal(out[:, :N], expected)
         else:
             assert np.all(np.abs(out[:, :N] - expected) <= bound(a, b, K))
+
+
+# Sums of one product each: the parts of both operands show one by one.
+#   random   the five smaller products add up to at most 2^-7 of the product before the largest joins them: their roundings are
+#            below 5 2^-31 of it, 2^-5 units in the last place.  Then one rounding, half a unit, and what is left out, below
+#            2^-24 of the product: less than a unit.
+#   others   the product has 24 significant bits at most, of 24 times one (all three parts of one operand) or of 12 times
+#            12 (hA*hB, hA*mB, mA*hB, mA*mB): exact, and every partial sum with it.
+LONE = ("random", "long times one", "one times long", "half times half")
+
+
+def lone_operands(rng, kind, a_shape, b_shape):
+    """Positive numbers for the two operands."""
+    draw = {"random": lambda s: rng.uniform(0.5, 2, s), "long": lambda s: rng.randint(1 << 22, 1 << 23, s) * 2 + 1,
+            "one": lambda s: 2.0 ** rng.randint(-20, 20, s), "half": lambda s: rng.randint(1 << 10, 1 << 11, s) * 2 + 1}
+    names = ("random", "random") if kind == "random" else kind.split(" times ")
+    return [draw[n](s).astype(np.float32) for n, s in zip(names, (a_shape, b_shape))]
+
+
+def check_lone(out, expected, kind):
+    if kind == "random":
+        assert np.all(np.abs(out - expected) <= (1.5 + 2.0 ** -5) * np.spacing(expected.astype(np.float32)))
+    else:
+        assert np.array_equal(out, expected)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K,edge", SIZES)
+def test_one_product_per_sum(rule, M, N, K, edge, tA, tB):
+    assert rule.split_tile(M, N, K) == edge
+    rng = np.random.RandomState(K)
+    for kind in LONE:
+        at = rng.permutation(M) % K                       # (M > K: every k has its rows)
+        values, b = lone_operands(rng, kind, M, (K, N))
+        a = np.zeros((M, K), np.float32)
+        a[np.arange(M), at] = values
+        out = call(np.ascontiguousarray(a.T) if tA else a, np.ascontiguousarray(b.T) if tB else b, np.zeros((M, N), np.float32), M, N, K, 1.0, 0.0, tA, tB)
+        check_lone(out, values[:, None].astype(np.float64) * b[at], kind)
 
 
 @pytest.mark.gpu
@@ -201,6 +241,29 @@ def test_windowed_convolution(kind):
         return
     fine = np.isfinite(expected)
     K = ci * 9
-    allowed = (K + 24) * 2.0 ** -24 * size + 2.0 ** -149 * K if kind == "special" else (6 / 16 * K / 2 + 24) * 2.0 ** -24 * size + 2.0 ** -25 * size
+    allowed = (K + 24) * 2.0 ** -24 * size + 2.0 ** -149 * K if kind == "special" else (6 / 16 * K / 2 + 24) * 2.0 ** -24 * size + 2.0 ** -24 * size
     assert np.all(np.abs(out - relu)[fine] <= allowed[fine])
     assert np.array_equal(np.isinf(out), expected == np.inf)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", LONE)
+def test_windowed_convolution_of_one_product_per_sum(kind):
+    from gpu_util import DeviceArray
+    n, ci, co, h = 9, 32, 64, 128
+    p = runtime.load(PROGRAMS, "conv2d_9x32x64x128")
+    rng = np.random.RandomState(4)
+    x = np.zeros((n, ci, h + 2, h + 2), np.float32)
+    values, x[:, :, 1:-1, 1:-1] = lone_operands(rng, kind, ci * 9, (n, ci, h, h))
+    dx, dbias, dout = DeviceArray(x), DeviceArray(np.zeros(co, np.float32)), DeviceArray(np.zeros((n, co, h, h), np.float32))
+    places = np.concatenate([rng.permutation(ci * 9), rng.permutation(ci * 9)])
+    for first in range(0, ci * 9, co):                    # every input channel and tap has an output channel
+        at = places[first:first + co]
+        w = np.zeros((co, ci * 9), np.float32)
+        w[np.arange(co), at] = values[at]
+        dw = DeviceArray(w.reshape(co, ci, 3, 3))
+        p(dx.buffer(), dw.buffer(), dbias.buffer(), dout.buffer())
+        out = dout.download()
+        for o in range(co):
+            c, ky, kx = at[o] // 9, at[o] % 9 // 3, at[o] % 3
+            check_lone(out[:, o], x[:, c, ky:ky + h, kx:kx + h].astype(np.float64) * values[at[o]], kind)

@@ -4,13 +4,17 @@
 // A float has 24 significant bits, a bf16 number 8 and the same exponents.  With h = bf16(x), m = bf16(x - h), l = x - h - m
 // (both differences are exact) l has at most 8 significant bits again: x = h + m + l.  A product is then nine products of
 // bf16 numbers, which the matrix cores form exactly and add in fp32.  The six of them down to 2^-18 of the largest are taken,
-//     hA*hB, hA*mB, mA*hB, mA*mB, hA*lB, lA*hB;
-// the other three together are at most 2^-25 of the product, less than one fp32 multiplication rounds by, and they are zero
-// wherever the product has 24 significant bits or fewer (products of small whole numbers stay exact).
+//     mA*mB, hA*mB, hA*lB, lA*hB, mA*hB, hA*hB;
+// the other three together are below 2^-24 of the product (they come near it: both operands 1 + 2^-8 - 2^-17), as much as one fp32
+// multiplication may round by, and they are zero wherever the product has 24 significant bits or fewer (products of small whole
+// numbers stay exact).  The largest comes last: a sum that one product dominates is then rounded at its full size once.  One product
+// alone is within 1.45 units in the last place, 0.39 rms (fp32 instruction 0.5 and 0.29; with the largest first, rounded again
+// by each of the five that follow, 3.4 and 0.60).  The order of the five costs nothing in accuracy; in this one neighbours share an operand
+// where they can, which the power limit rewards (4096^3 582 to 598 us; smallest first 609 to 620, largest first 602 to 617).
 // v_mfma_f32_32x32x16_bf16 does sixteen times the work of v_mfma_f32_32x32x2_f32 per cycle, so that six of it take 3/8 of the
 // fp32 instruction's time; and an accumulator is rounded six times per sixteen k instead of eight times or more, which is why
 // the error against 64 bits is smaller (uniform random operands, 2-norm: 4096^3 1.00e-6 against 1.15e-6, with partial sums
-// 2048^3 4.9e-7 against 8.1e-7, 1024^3 1.9e-7 against 4.1e-7).
+// 2048^3 4.9e-7 against 8.1e-7, 1024^3 1.7e-7 against 4.1e-7).
 //
 // What three bf16 numbers cannot hold is multiplied by the fp32 instruction.  Operands are scaled by 2^16 on the way (exactly;
 // the sums are scaled back), so that the last part of the smallest fp32 number, 2^-149, is still a bf16 number, 2^-133.  What is
@@ -54,8 +58,8 @@ __device__ __forceinline__ void split_pair(const split_constants &c, float a, fl
     b -= __builtin_bit_cast(float, part[1] & c.high);
     part[2] = split_pack(a, b);
 }
-// The products taken: part of A, part of B.
-constexpr int SPLIT_A[6] = {0, 0, 1, 1, 0, 2}, SPLIT_B[6] = {0, 1, 0, 1, 2, 0};
+// The products taken: part of A, part of B; and the parts in the order in which they are needed.
+constexpr int SPLIT_A[6] = {1, 0, 0, 2, 1, 0}, SPLIT_B[6] = {1, 1, 2, 0, 0, 0}, SPLIT_READ[3] = {1, 0, 2};
 
 // Takes the scale out of the sums of the wavefront's rows from m0 and columns from n0; whether one that is in C is not finite.
 template <class CFG>
@@ -282,7 +286,8 @@ __device__ __forceinline__ void tile_accumulate_split(accumulators<CFG> &acc, co
     auto read = [&](int stage, split_x8 (&fa)[3][TM], split_x8 (&fb)[3][TN]) {
         const int kq = 2 * wk + h;
 #pragma unroll
-        for (int p = 0; p < 3; p++) {
+        for (int o = 0; o < 3; o++) {
+            const int p = SPLIT_READ[o];
 #pragma unroll
             for (int i = 0; i < TM; i++) fa[p][i] = opA::read(stage_a(stage), p, wm * CFG::WM + i * 32 + l32, kq);
 #pragma unroll

@@ -130,7 +130,8 @@ __device__ __forceinline__ void contraction_window_split(const float *__restrict
             const int off = h && !odd ? TAP_OFFSETS::at(odd ? 0 : 2 * st + 1) : TAP_OFFSETS::at(2 * st);
             split_x8 fa[3][TM], fb[3][TN];
 #pragma unroll
-            for (int s = 0; s < 3; s++) {
+            for (int o = 0; o < 3; o++) {
+                const int s = SPLIT_READ[o];
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
                     const int own = (wm * CFG::WM + i * 32 + l32) * ROW + h + 2 * st, at = odd && h ? BM * ROW : own;
