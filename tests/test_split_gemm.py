@@ -84,6 +84,33 @@ def call(A, B, C, M, N, K, alpha, beta, tA, tB, offset=0):
     return dC.download()[offset:].reshape(C.shape)
 
 
+def test_lanes_that_share_lds_without_a_barrier_are_ordered(tmp_path):
+    """64 x 64 tiles pass a slice from lane to lane through LDS without a barrier of the workgroup.  Seen per thread the addresses stored to
+    and read from differ, so only a fence keeps the compiler from moving one across the other: in what it makes of the kernel, every
+    run of stores to LDS stands between two fences."""
+    source, ir = tmp_path / "waves.hip", tmp_path / "waves.ll"
+    source.write_text('#include "gemm_mfma_split.hip.h"\n' + "".join(
+        "template __global__ void tgemm::sgemm_split_kernel<tgemm::config_waves<%s, %s>>(const float *, const float *, float *, int, int, int, long, long, long,"
+        " float, float);\n" % layout for layout in (("true", "false"), ("false", "true"))))
+    subprocess.run([build.HIPCC] + build.HIP_FLAGS + ["-w", "--cuda-device-only", "-S", "-emit-llvm", "-I" + os.path.join(build.CSRC, "kernels"), str(source), "-o", str(ir)], check=True)
+    runs, before = 0, None                # the last fence ("fence") or access to LDS ("load", "store") of the block
+    for line in ir.read_text().splitlines():
+        text = line.strip()
+        if line[:1] not in (" ", "\t") and before is not None:
+            assert before != "store", "a block ends behind stores"
+            before = None
+        elif text.startswith("fence "):
+            before = "fence"
+        elif "addrspace(3)" in text and text.startswith("store "):
+            assert before in ("fence", "store"), text
+            runs += before == "fence"
+            before = "store"
+        elif "addrspace(3)" in text and " = load " in text:
+            assert before != "store", text
+            before = "load"
+    assert runs >= 2 * 3                  # the first slice, two stages of the loop, in two kernels
+
+
 SIZES = [(704, 1088, 528, 64), (1408, 2560, 416, 128), (1219, 2747, 611, 128), (1300, 2690, 450, 128), (2560, 3584, 208, 256), (2701, 3915, 99, 256)]
 
 

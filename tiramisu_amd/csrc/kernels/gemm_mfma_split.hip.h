@@ -372,6 +372,13 @@ struct config_waves {
     static_assert(LDS_BYTES == ttarget::split_lds_bytes(BM, A_KMAJOR, B_KMAJOR), "two stages of every wavefront's slices");
 };
 
+// Between the accesses of a wavefront's lanes to LDS that only they use: what was written or read before is done for what is written or
+// read behind.  The LDS executes a wavefront's accesses in order, so this holds the compiler alone and is no instruction.
+__device__ __forceinline__ void wave_lds_in_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // One operand's X x 16 slice of one wavefront, in fp32.
 template <int X, bool KMAJOR>
 struct wave_operand {
@@ -465,8 +472,10 @@ __device__ __forceinline__ void tile_accumulate_waves(accumulators<CFG> &acc, co
         opB::load(B, n0, s * BK, atb, rb);
     };
     auto store = [&](int stage) {
+        wave_lds_in_order();                 // the lanes have read what the stage held
         opA::store(lds + stage * CFG::WAVE_WORDS, ra);
         opB::store(lds + stage * CFG::WAVE_WORDS + CFG::A_WORDS, rb);
+        wave_lds_in_order();                 // the lanes read what the others stored
     };
     // A slice is four tile products; while the matrix cores work on one, the vector ALUs split the block of 32 rows or columns that
     // the next one needs, requested from LDS one product earlier: column block 1, row block 1, then the first row and
