@@ -37,7 +37,7 @@ def test_sgemm_on_gpu_tensors_default_and_side_stream():
     C = torch.randint(-5, 5, (M, N), generator=g).float()
     scal = np.array([3.0, 2.0], np.float32)
     expected = 3.0 * (A.double() @ B.double()) + 2.0 * C.double()
-    # torch's default stream: the call waits on both sides
+    # torch's default stream: the call waits on both sides (test_calls_on_the_default_stream_... has torch work in flight)
     dA, dB, dC = A.cuda(), B.cuda(), C.cuda()
     print("default stream", flush=True)
     prog(scal, dA, dB, dC)
@@ -57,6 +57,61 @@ def test_sgemm_on_gpu_tensors_default_and_side_stream():
     # a tensor in the wrong memory is refused before anything is launched
     with pytest.raises(ValueError):
         prog(scal, A, dB, dC)
+
+
+@pytest.mark.gpu
+def test_calls_on_the_default_stream_follow_torch_work_and_keep_the_threads_stream():
+    import threading
+    import torch
+    M, N, K = 128, 192, 96
+    prog = runtime.load(PROGRAMS, "sgemm_%dx%dx%d" % (M, N, K))
+    w, call, seen = runtime.wrappers(), prog.fn, []
+    prog.fn = lambda *p: (seen.append(w.tiramisu_hip_get_stream()), call(*p))[1]
+    scal, eye = np.array([1.0, 0.0], np.float32), torch.eye(K, N, device="cuda")
+    big = torch.zeros(4096, 4096, device="cuda")
+
+    def follow(i):
+        A, C = torch.zeros(M, K, device="cuda"), torch.zeros(M, N, device="cuda")
+        torch.cuda.synchronize()
+        y = big
+        for _ in range(10):                              # milliseconds of torch work, then the input
+            y = y @ big
+        A += y[:M, :K] + float(i + 1)
+        done = torch.cuda.Event()
+        done.record()
+        in_flight = not done.query()
+        prog(scal, A, eye, C)
+        result = C * 1.0
+        assert torch.all(result[:, :K] == i + 1) and torch.all(result[:, K:] == 0)
+        return in_flight
+
+    follow(0)                                            # (loads the library's kernels)
+    print("torch work in flight", flush=True)
+    before = w.tiramisu_hip_get_stream()
+    assert follow(1) and seen[-1] == before == w.tiramisu_hip_get_stream()
+    own = w.tiramisu_hip_stream_create()
+    w.tiramisu_hip_set_stream(own)                       # a stream that the caller gave the runtime
+    follow(2)
+    assert seen[-1] == own == w.tiramisu_hip_get_stream()
+    w.tiramisu_hip_set_stream(None)
+    w.tiramisu_hip_stream_destroy(own)
+    print("two threads", flush=True)
+    failed, calls = [], len(seen)
+
+    def repeat(first):
+        try:
+            for i in range(first, first + 5):
+                follow(i)
+        except BaseException as e:
+            failed.append(e)
+
+    threads = [threading.Thread(target=repeat, args=(10 * t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    assert set(seen[calls:]) == {before}            # the handle that names each thread's own default stream
 
 
 @pytest.mark.gpu

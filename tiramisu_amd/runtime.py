@@ -223,7 +223,8 @@ class Program:
         """Arguments: ``Buffer`` objects, numpy arrays (host buffers) or torch tensors (host or GPU buffers by where
         they live).  With a GPU tensor among them the function's kernels run on torch's current stream of that
         tensor's device, in order with the torch work around the call (the runtime's stream of the calling thread is
-        put back afterwards); when that is torch's default stream the call waits for its kernels before it returns."""
+        put back afterwards); when that is torch's default stream they run on the runtime's stream of the calling
+        thread, and the call waits for torch's default stream first and for its own kernels afterwards."""
         bufs, torch_stream = [], None
         for a in args:
             if isinstance(a, Buffer):
@@ -241,18 +242,26 @@ class Program:
             self.check(bufs)
         if torch_stream is None:
             rc = self.fn(*[b.pointer() for b in bufs])
-        else:
-            # torch's default stream is the device's null stream.  Its handle, 0, means the calling thread's own default stream to
-            # tiramisu_hip_set_stream; HIP's other name for it does not.  On it the kernels follow the torch work before the call
-            # without a wait on the host (one wait less: a convolution of 8 images of 112 x 112 from 3 to 64 channels 40 -> 37.5 us,
-            # from 64 to 64, 32 images, 204 -> 196)
+        elif torch_stream == 0:
+            # torch's default stream is the device's null stream, and its handle, 0, means the calling thread's own default
+            # stream to tiramisu_hip_set_stream; HIP's other name for it does not.  The kernels stay on the thread's stream, so that
+            # calls from several threads overlap (two threads of a 1.33 ms pass each 2.2 ms a round; on the null stream, one
+            # after the other, 2.7), ordered by a wait on both sides.  The runtime waits: torch's synchronize() costs 3 us more.
             w = wrappers()
             before = w.tiramisu_hip_get_stream()
-            w.tiramisu_hip_set_stream(torch_stream or HIP_STREAM_LEGACY)
+            w.tiramisu_hip_set_stream(HIP_STREAM_LEGACY)
+            try:
+                w.tiramisu_hip_stream_synchronize(0)
+            finally:
+                w.tiramisu_hip_set_stream(before)
+            rc = self.fn(*[b.pointer() for b in bufs])
+            w.tiramisu_hip_stream_synchronize(0)
+        else:
+            w = wrappers()
+            before = w.tiramisu_hip_get_stream()
+            w.tiramisu_hip_set_stream(torch_stream)
             try:
                 rc = self.fn(*[b.pointer() for b in bufs])
-                if torch_stream == 0:
-                    w.tiramisu_hip_stream_synchronize(0)
             finally:
                 w.tiramisu_hip_set_stream(before)
         if rc != 0:
