@@ -11,6 +11,7 @@ int main()
     generate(1408, 2560, 416);     // 128x128, whole
     generate(1219, 2747, 611);     // 128x128, rows at every alignment, everything ends inside a tile
     generate(2560, 3584, 208);     // 256x256, whole
+    generate(2560, 3584, 210);     // 256x256, guarded in K only
     generate(2701, 3915, 99);      // 256x256, guarded, three k in the last slice
     return 0;
 }

@@ -24,41 +24,47 @@ def rule(tmp_path_factory):
     """split_tile_for of kernels/target_gfx950.h, preceded by the fp32 tile that the library call would take."""
     d = tmp_path_factory.mktemp("rule")
     (d / "rule.cpp").write_text('''#include "%s"
-extern "C" int fp32_tile(long M, long N, long K, int *m, int *n) {
-    const int bm = ttarget::square_tile_for(M, N);
-    bool edge = !(M %% bm == 0 && N %% bm == 0 && K %% (bm == 64 ? 32 : 16) == 0);
-    *m = *n = bm;
-    if (bm == 64 || M < 32 || N < 32) {
-        const ttarget::small_tile t = ttarget::small_tile_for(M, N, K, 1, !edge);
-        if (t != ttarget::TILE_64) { *m = t == ttarget::TILE_64x32 ? 64 : 32; *n = 32; edge = !(M %% *m == 0 && N %% *n == 0 && K %% ttarget::small_tile_slice(K) == 0); }
-    }
-    return edge;
+extern "C" int fp32_tile(long M, long N, long K, int aligned, int *m, int *n) {
+    const ttarget::fp32_tiles t = ttarget::library_tiles_for(M, N, K, 1, aligned);
+    *m = t.m;
+    *n = t.n;
+    return t.guarded;
 }
-extern "C" int split_tile(long M, long N, long K) {
-    int m, n;
-    const int edge = fp32_tile(M, N, K, &m, &n);
-    return ttarget::split_tile_for(M, N, K, 1, m, n, edge);
+extern "C" int split_tile(long M, long N, long K, int aligned) {
+    const ttarget::fp32_tiles t = ttarget::library_tiles_for(M, N, K, 1, aligned);
+    return ttarget::split_tile_for(M, N, K, 1, t.m, t.n, t.guarded);
+}
+extern "C" double fp32_model(long M, long N, long K, int m, int n, int guarded) {
+    for (const ttarget::launch_model &l : ttarget::FP32_LAUNCHES)
+        if (l.m == m && l.n == n && l.guarded == (bool)guarded) return ttarget::modelled(l, M, N, K, 1);
+    return 0;
 }
 ''' % os.path.join(build.CSRC, "kernels", "target_gfx950.h"))
     subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-o", str(d / "rule.so"), str(d / "rule.cpp")], check=True)
     lib = ctypes.CDLL(str(d / "rule.so"))
-    for f in (lib.split_tile, lib.fp32_tile):
-        f.argtypes = [ctypes.c_long] * 3 + ([ctypes.POINTER(ctypes.c_int)] * 2 if f is lib.fp32_tile else [])
+    sizes, out = [ctypes.c_long] * 3, [ctypes.POINTER(ctypes.c_int)] * 2
+    lib.split_tile.argtypes, lib.fp32_tile.argtypes = sizes + [ctypes.c_int], sizes + [ctypes.c_int] + out
+    lib.fp32_model.argtypes, lib.fp32_model.restype = sizes + [ctypes.c_int] * 3, ctypes.c_double
     return lib
 
 
 def test_rule(rule):
     for M, N, K, edge in ((4096, 4096, 4096, 256), (2048, 2048, 2048, 128), (1024, 1024, 1024, 64), (4096, 4096, 95, 0), (63, 4096, 4096, 0),
-                          (4096, 63, 4096, 0), (512, 512, 512, 0), (64, 64, 4096, 0), (4097, 4096, 96, 256)):
-        assert rule.split_tile(M, N, K) == edge, (M, N, K)
+                          (4096, 63, 4096, 0), (512, 512, 512, 0), (64, 64, 4096, 0), (4097, 4096, 96, 256),
+                          # a square tile of 256 or 192 that K asks to guard: the library's fp32 tiles are 64 x 64
+                          (4096, 4096, 1000, 256), (4096, 4096, 4095, 256), (3072, 3072, 3000, 128), (3840, 3840, 500, 256)):
+        assert rule.split_tile(M, N, K, True) == edge, (M, N, K)
+    assert rule.split_tile(4096, 4096, 4096, False) == 256
     m, n = ctypes.c_int(), ctypes.c_int()
     rng = np.random.RandomState(1)
     for _ in range(3000):
         M, N, K = (int(v) for v in np.exp(rng.uniform(np.log(16), np.log(5000), 3)))
         if rng.rand() < 0.5:
             M, N, K = (max(64, v // 64 * 64) for v in (M, N, K))
-        edge = rule.split_tile(M, N, K)
-        rule.fp32_tile(M, N, K, m, n)
+        aligned = rng.rand() < 0.7
+        edge = rule.split_tile(M, N, K, aligned)
+        guarded = rule.fp32_tile(M, N, K, aligned, m, n)
+        assert rule.fp32_model(M, N, K, m, n, guarded) > 0            # every tile that the library launches has its figures
         if edge:      # sizes that the kernels' loads require; as many partial sums as the fp32 tile's four, or more
             assert min(M, N) >= 64 and K >= 96 and (n.value != 32 or edge == 64)
             assert edge != 64 or (M % 64 == 0 and N % 64 == 0 and K % 16 == 0)
@@ -111,14 +117,15 @@ def test_lanes_that_share_lds_without_a_barrier_are_ordered(tmp_path):
     assert runs >= 2 * 3                  # the first slice, two stages of the loop, in two kernels
 
 
-SIZES = [(704, 1088, 528, 64), (1408, 2560, 416, 128), (1219, 2747, 611, 128), (1300, 2690, 450, 128), (2560, 3584, 208, 256), (2701, 3915, 99, 256)]
+SIZES = [(704, 1088, 528, 64), (1408, 2560, 416, 128), (1219, 2747, 611, 128), (1300, 2690, 450, 128), (2560, 3584, 208, 256), (2701, 3915, 99, 256),
+         (2560, 3584, 210, 256)]        # (all but K a multiple of the tile)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("M,N,K,edge", SIZES)
 def test_library_call(rule, M, N, K, edge, tA, tB):
-    assert rule.split_tile(M, N, K) == edge
+    assert rule.split_tile(M, N, K, True) == rule.split_tile(M, N, K, False) == edge
     rng = np.random.RandomState(M + K)
     for kind, pad, offset, alpha, beta in (("whole", 0, 0, 2.0, 3.0), ("uniform", 3 if edge != 64 else 4, 1 if M % 2 else 4, 1.0, 0.0)):
         A, B = operands(rng, M, N, K, tA, tB, pad, kind)
@@ -163,7 +170,7 @@ def check_lone(out, expected, kind):
 @pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("M,N,K,edge", SIZES)
 def test_one_product_per_sum(rule, M, N, K, edge, tA, tB):
-    assert rule.split_tile(M, N, K) == edge
+    assert rule.split_tile(M, N, K, True) == rule.split_tile(M, N, K, False) == edge
     rng = np.random.RandomState(K)
     for kind in LONE:
         at = rng.permutation(M) % K                       # (M > K: every k has its rows)

@@ -421,19 +421,14 @@ void *static_scratch_here() {
 template <bool AK, bool BK_>
 void dispatch_edge(bool vec_ok, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb,
                    long ldc, float alpha, float beta) {
-    const int bm = tile_for(M, N), problems = active_batch ? active_batch_count : 1;
-    const bool edge = !(vec_ok && M % bm == 0 && N % bm == 0 && K % (bm == 64 ? 32 : 16) == 0);   // K-slice of the tile
-    ttarget::small_tile t = ttarget::TILE_64;
-    if (bm == 64 || M < 32 || N < 32) t = ttarget::small_tile_for(M, N, K, problems, !edge);
-    const int tile_m = t == ttarget::TILE_64 ? bm : t == ttarget::TILE_64x32 ? 64 : 32, tile_n = t == ttarget::TILE_64 ? bm : 32;
-    // (a slice of 32 k is guarded like any other: the small tiles look at theirs themselves)
-    const bool guarded = t == ttarget::TILE_64 ? edge : !(vec_ok && M % tile_m == 0 && N % tile_n == 0 && K % ttarget::small_tile_slice(K) == 0);
+    const int problems = active_batch ? active_batch_count : 1;
+    const ttarget::fp32_tiles t = ttarget::library_tiles_for(M, N, K, problems, vec_ok);
     if (lda >= 4 && lda < ttarget::SPLIT_LD_LIMIT && ldb >= 4 && ldb < ttarget::SPLIT_LD_LIMIT)
-        if (const int split = ttarget::split_tile_for(M, N, K, problems, tile_m, tile_n, guarded))
+        if (const int split = ttarget::split_tile_for(M, N, K, problems, t.m, t.n, t.guarded))
             return dispatch_split<AK, BK_>(split, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    if (t == ttarget::TILE_64x32) return launch_small<AK, BK_, 64, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    if (t == ttarget::TILE_32) return launch_small<AK, BK_, 32, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    if (edge) dispatch_tile<AK, BK_, true>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    if (t.m == 64 && t.n == 32) return launch_small<AK, BK_, 64, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    if (t.m == 32) return launch_small<AK, BK_, 32, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    if (t.guarded) dispatch_tile<AK, BK_, true>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     else dispatch_tile<AK, BK_, false>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
 

@@ -62,6 +62,21 @@ inline small_tile small_tile_for(long M, long N, long K, long problems, bool who
 // 14.4; with one row 1 x 142339 x 20 17.8 (one thread per element), 18.2, 10.2.
 inline int small_tile_slice(long K) { return K <= 32 ? 32 : 64; }
 
+// The fp32 tiles of a library product; `aligned`: rows and operands begin at multiples of 16 bytes.  (A slice of 32 k is guarded like
+// any other.  256 x 256 and 192 x 192 come whole only: where K or the alignment asks for guards, 64 x 64 take their place.)
+struct fp32_tiles { int m, n; bool guarded; };
+inline fp32_tiles library_tiles_for(long M, long N, long K, long problems, bool aligned) {
+    const int edge = square_tile_for(M, N);
+    const bool guarded = !(aligned && M % edge == 0 && N % edge == 0 && K % (edge == 64 ? 32 : 16) == 0);
+    if (edge == 64 || M < 32 || N < 32) {
+        const small_tile t = small_tile_for(M, N, K, problems, !guarded);
+        const int m = t == TILE_64x32 ? 64 : 32;
+        if (t != TILE_64) return {m, 32, !(aligned && M % m == 0 && N % 32 == 0 && K % small_tile_slice(K) == 0)};
+    }
+    if (guarded && edge > 128) return {64, 64, true};
+    return {edge, edge, guarded};
+}
+
 // C tiles of the kernels that split fp32 operands into bf16 parts (gemm_mfma_split.hip.h), and when they replace the fp32 instruction.
 // Whole launches of both kinds are modelled like the tiles above: `fixed` microseconds and `first` per k for a round of tiles over the
 // compute units, `round` and `further` per k for each round after it; fitted at 64 ... 4096 k, up to sixteen rounds, uniform
@@ -69,12 +84,16 @@ inline int small_tile_slice(long K) { return K <= 32 ? 32 : 64; }
 // 2048^3 136 / 97 (128 x 128), 4096 x 4096 x 128 43 / 33, 2048 x 2048 x 256 23.1 / 20.3, 1024^3 21.5 / 19.0 (64 x 64), guarded 3623 x 2943 x 920
 // 193 / 130, 1218 x 2748 x 611 50 / 37; and where the fp32 instruction stays: 1024 x 1024 x 256 8.2 / 8.8, 2048 x 2048 x 128
 // 14.8 / 14.9, 1520 x 3116 x 503 51 / 54.
+// Tiles of 256 and 192 that are guarded, which divide M and N but not K (programs, which also read C; fp32 / split): 4096 x 4096 x 1000
+// 257 / 179, x 250 90 / 73, 3072 x 6144 x 1000 294 / 264; left: 3072 x 3072 x 250 51 / 55, x 2030 283 / 291, 3072 x 6144 x 250 97 / 114.
+// Library calls, whose fp32 tiles are then 64 x 64: 4096 x 4096 x 1000 316 / 180, x 4095 1115 / 620, 3072 x 3072 x 3000 469 / 386, x 100 31 / 28.
 struct launch_model { int m, n; bool guarded; double fixed, round, first, further; };
 constexpr launch_model FP32_LAUNCHES[] = {
     {256, 256, false, 11.0, 2.0, 0.2242, 0.23}, {192, 192, false, 9.2, 2.6, 0.1322, 0.132}, {128, 128, false, 4.9, 3.2, 0.0617, 0.0587},
     {64, 64, false, 3.1, 0.7, 0.0175, 0.0157}, {64, 32, false, 3.3, 0.8, 0.0093, 0.0080}, {32, 32, false, 3.0, 0.5, 0.0061, 0.0043},
     {128, 128, true, 6.7, 4.8, 0.0669, 0.0601}, {64, 64, true, 4.1, 1.1, 0.0206, 0.0165}, {64, 32, true, 4.4, 1.5, 0.0104, 0.0091},
-    {32, 32, true, 4.2, 0.8, 0.0073, 0.0048}};
+    {32, 32, true, 4.2, 0.8, 0.0073, 0.0048},
+    {256, 256, true, 17.0, 17.0, 0.2275, 0.231}, {192, 192, true, 7.8, 2.0, 0.130, 0.1323}};       // (generated code only: library_tiles_for)
 constexpr launch_model SPLIT_LAUNCHES[] = {
     {256, 256, false, 10.1, 2.3, 0.135, 0.145}, {128, 128, false, 7.9, 5.8, 0.0380, 0.0404}, {64, 64, false, 5.3, 3.5, 0.0132, 0.0121},
     {256, 256, true, 12.1, 2.3, 0.130, 0.145}, {128, 128, true, 9.2, 8.7, 0.0360, 0.0405}};
@@ -98,7 +117,8 @@ constexpr bool split_whole(int edge, long M, long N, long K) { return M % edge =
 constexpr long window_split_lds_bytes(long rows, long taps, long window) { return 3 * 16 * (rows * (taps | 1) + 1 + window); }
 // The edge of the split tile that takes an M x N x K product from fp32 tiles of m x n (guarded or not), 0: none.  Where the fp32
 // tiles are 32 wide, four groups of wavefronts add four partial sums: only the eight of the 64 x 64 tile are at least as close
-// to 64 bits.  Below 96 k the two are equally close, and little is gained.
+// to 64 bits.  Below 96 k the two are equally close, and little is gained.  Tiles without a row above (64 x 256: a result of at most
+// 64 rows, very wide) keep the fp32 instruction.
 inline int split_tile_for(long M, long N, long K, long problems, int m, int n, bool guarded) {
     if (M < 64 || N < 64 || K < 96) return 0;
     double best = 0;
