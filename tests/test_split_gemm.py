@@ -197,8 +197,9 @@ def test_program(M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(704, 1088, 528), (1219, 2747, 611), (2560, 3584, 208)])
-def test_numbers_that_three_parts_do_not_hold(M, N, K):
+@pytest.mark.parametrize("M,N,K", [(704, 1088, 528), (1219, 2747, 611), (2560, 3584, 208), (2701, 3915, 99)])
+@pytest.mark.parametrize("transposed", [False, True])         # (each operand in both layouts)
+def test_numbers_that_three_parts_do_not_hold(M, N, K, transposed):
     rng = np.random.RandomState(5)
     A, B = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N)))
     A[3, 5], A[M - 1, K - 1], A[70, 0], B[7, 9] = np.inf, np.nan, 2.0 ** 120, -np.inf
@@ -209,7 +210,8 @@ def test_numbers_that_three_parts_do_not_hold(M, N, K):
     with np.errstate(all="ignore"):
         expected = A.astype(np.float64) @ B.astype(np.float64)
         fp32 = expected.astype(np.float32)
-        out = call(A, B, np.zeros((M, N), np.float32), M, N, K, 1.0, 0.0, False, False)
+        a, b = (np.ascontiguousarray(x.T) for x in (A, B)) if transposed else (A, B)
+        out = call(a, b, np.zeros((M, N), np.float32), M, N, K, 1.0, 0.0, transposed, transposed)
         assert np.array_equal(np.isnan(out), np.isnan(fp32))
         # (a sum of fp32 numbers may overflow where the exact one does not: only near the largest number, which no element is)
         assert np.array_equal(np.isinf(out), np.isinf(fp32)) and np.array_equal(np.sign(out[np.isinf(out)]), np.sign(fp32[np.isinf(out)]))

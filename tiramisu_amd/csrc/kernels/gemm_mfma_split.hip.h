@@ -19,7 +19,9 @@
 // What three bf16 numbers cannot hold is multiplied by the fp32 instruction.  Operands are scaled by 2^16 on the way (exactly;
 // the sums are scaled back), so that the last part of the smallest fp32 number, 2^-149, is still a bf16 number, 2^-133.  What is
 // left are infinities, NaNs and numbers that overflow, from 2^111 on, or whose products do: they all show as sums that are
-// not finite, and a wavefront that finds one computes its part of the tile again from global memory (recompute_fp32).
+// not finite, and a wavefront that finds one computes its part of the tile again from global memory (recompute_fp32): 4096^3 with one row
+// of NaN 1150 us, with operands of 2^60, whose every product overflows, 2030 (bound by the L2; 600 without, 960 with the fp32 instruction),
+// 1024^3 38 (18; 20).
 //
 // What bounds it: at 4096^3 the power limit (620 us on random operands, 470 on zeros, 948 with the fp32 instruction), on small tiles the
 // vector work of the split, seven instructions per element, each done once per tile (1024^3 17 us, 20.5 before).
@@ -115,40 +117,64 @@ struct split_source {
         const f32x4 none = {0.f, 0.f, 0.f, 0.f};
         return k < KE ? shifted_down(v, max(x - (XE - 4), 0)) : none;
     }
-    // the four elements (x, k .. k + 3), zero behind KE
-    __device__ __forceinline__ f32x4 fetch(int x, int k) const {
+    // the four elements (x0 + x, k0 + k + i ..), `at` = place(x0, x, k), i uniform: all there (WHOLE), or zero behind KE
+    template <bool WHOLE>
+    __device__ __forceinline__ f32x4 four(int x0, int k0, int k, int i, uint32_t at) const {
+        const float *const scalar = base + (KMAJOR ? (long)x0 * ld + k0 : (long)k0 * ld + x0);
+        auto element = [&](const float *from, int d) {          // d k further
+            return reinterpret_cast<const char *>(from) + (at + 4u * (uint32_t)(KMAJOR ? d : d * (int)ld));
+        };
         f32x4 v;
+        if (WHOLE && KMAJOR) {
+            const f32x4_u q = *reinterpret_cast<const f32x4_u *>(element(scalar + i, 0));
+            return f32x4{q[0], q[1], q[2], q[3]};
+        }
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int xx = EDGE ? min(x, XE - 1) : x, kk = min(k + e, KE - 1);
-            v[e] = base[KMAJOR ? (long)xx * ld + kk : (long)kk * ld + xx];
-            if (k + e >= KE) v[e] = 0.f;
+        for (int e = i; e < i + 4; e++) {
+            const int last = KE - 1 - k0 - k;                     // (negative where k0 + k lies behind KE)
+            if (WHOLE) v[e - i] = *reinterpret_cast<const float *>(element(scalar + (long)e * ld, 0));
+            else v[e - i] = *reinterpret_cast<const float *>(element(scalar, min(e, last)));
+            if (!WHOLE && e > last) v[e - i] = 0.f;
         }
         return v;
     }
 };
 
 // The wavefront's part of a tile with the fp32 instruction, operands straight from global memory: of the slices first, first + step, ...
-// of BK k the k in [from, from + count).
+// of BK k the k in [from, from + 16), eight of them on each half of the wavefront, so that a row is read 64 bytes at a time.
 template <class CFG, class SRCA, class SRCB>
-__device__ __forceinline__ void recompute_fp32(accumulators<CFG> &acc, const SRCA &A, const SRCB &B, int K, int m0, int n0, int first, int step, int from, int count) {
+__device__ __forceinline__ void recompute_fp32(accumulators<CFG> &acc, const SRCA &A, const SRCB &B, int K, int m0, int n0, int first, int step, int from) {
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
-    acc.clear();
-    for (int s = first; s * CFG::BK < K; s += step)
-#pragma unroll 1
-        for (int k = s * CFG::BK + from; k < s * CFG::BK + from + count && k < K; k += 8) {
-            f32x4 a[CFG::TM], b[CFG::TN];
+    uint32_t ata[CFG::TM], atb[CFG::TN];
 #pragma unroll
-            for (int i = 0; i < CFG::TM; i++) a[i] = A.fetch(m0 + i * 32 + l32, k + 4 * h);
+    for (int i = 0; i < CFG::TM; i++) ata[i] = A.place(m0, i * 32 + l32, 8 * h);
 #pragma unroll
-            for (int j = 0; j < CFG::TN; j++) b[j] = B.fetch(n0 + j * 32 + l32, k + 4 * h);
+    for (int j = 0; j < CFG::TN; j++) atb[j] = B.place(n0, j * 32 + l32, 8 * h);
+    auto slice = [&](int k, auto whole) {
+        constexpr bool WHOLE = decltype(whole)::value;
+        f32x4 a[2][CFG::TM], b[2][CFG::TN];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+#pragma unroll
+            for (int i = 0; i < CFG::TM; i++) a[q][i] = A.template four<WHOLE>(m0, k, 8 * h, 4 * q, ata[i]);
+#pragma unroll
+            for (int j = 0; j < CFG::TN; j++) b[q][j] = B.template four<WHOLE>(n0, k, 8 * h, 4 * q, atb[j]);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; q++)
 #pragma unroll
             for (int e = 0; e < 4; e++)
 #pragma unroll
                 for (int i = 0; i < CFG::TM; i++)
 #pragma unroll
-                    for (int j = 0; j < CFG::TN; j++) acc.t[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][e], b[j][e], acc.t[i][j], 0, 0, 0);
-        }
+                    for (int j = 0; j < CFG::TN; j++)
+                        acc.t[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][i][e], b[q][j][e], acc.t[i][j], 0, 0, 0);
+    };
+    acc.clear();
+    int k = first * CFG::BK + from;
+#pragma unroll 1
+    for (; k + 16 <= K; k += step * CFG::BK) slice(k, std::true_type());
+    if (CFG::EDGE && k < K) slice(k, std::false_type());
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
@@ -353,7 +379,7 @@ __device__ __forceinline__ void tile_accumulate_split(accumulators<CFG> &acc, co
     }
     m0 += wm * CFG::WM;
     n0 += wn * CFG::WN;
-    if (__any(unscale(acc, M, N, m0, n0))) recompute_fp32(acc, A, B, K, m0, n0, 0, 1, wk * 16, 16);
+    if (__any(unscale(acc, M, N, m0, n0))) recompute_fp32(acc, A, B, K, m0, n0, 0, 1, wk * 16);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
@@ -534,7 +560,7 @@ __device__ __forceinline__ void tile_accumulate_waves(accumulators<CFG> &acc, co
             }
         }
     }
-    if (__any(unscale(acc, M, N, m0, n0))) recompute_fp32(acc, A, B, K, m0, n0, wave, W, 0, BK);
+    if (__any(unscale(acc, M, N, m0, n0))) recompute_fp32(acc, A, B, K, m0, n0, wave, W, 0);
 }
 
 // The sums of the wavefronts, added in their order; each finishes its SHARE of the tile's quads.  value and store as in tile_epilogue.

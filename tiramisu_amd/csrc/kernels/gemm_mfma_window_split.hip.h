@@ -14,7 +14,7 @@
 //
 // 32 images of 112 x 112, 64 to 64 channels: 242 us with the fp32 instruction, 181 so; matrix cores 58 % busy at the 1.8 GHz that
 // the power limit leaves.  The error against 64 bits is smaller (gemm_mfma_split.hip.h), and sums that are not finite are
-// computed again with the fp32 instruction.
+// computed again with the fp32 instruction (operands of 2^60, every sum: 454 us a call, 198 without, 276 with that instruction alone).
 //
 // Requirements (checked by the emitter): those of contraction_window, and whole blocks of 8 channels.  Work distribution, pieces of
 // the last tiles and their hand-over are contraction_window's.
@@ -156,16 +156,14 @@ __device__ __forceinline__ void contraction_window_split(const float *__restrict
         acc.clear();
 #pragma unroll 1
         for (int c = first * CB; c < end * CB; c += 2)
-#pragma unroll 1
-            for (int tap = 0; tap < TAPS; tap++) {
-                int off = 0;
 #pragma unroll
-                for (int q = 0; q < TAPS; q++) off = q == tap ? TAP_OFFSETS::at(q) : off;
+            for (int tap = 0; tap < TAPS; tap++) {
+                if (tap % 9 == 0) __builtin_amdgcn_sched_barrier(0);       // nine taps' operands at a time
                 float a[TM], b[TN];
 #pragma unroll
                 for (int i = 0; i < TM; i++) a[i] = A[(long)(p.m0 + wm * CFG::WM + i * 32 + l32) * lda + (long)(c + h) * TAPS + tap];
 #pragma unroll
-                for (int j = 0; j < TN; j++) b[j] = X[p.f0 + fp[j] + (long)(c + h) * chan_stride + off];
+                for (int j = 0; j < TN; j++) b[j] = X[p.f0 + fp[j] + (long)(c + h) * chan_stride + TAP_OFFSETS::at(tap)];
 #pragma unroll
                 for (int i = 0; i < TM; i++)
 #pragma unroll
