@@ -82,13 +82,13 @@ def test_cpu_generated_code_matches_oracle(n, steps):
 
 # ---------------------------------------------------------------- GPU parity
 
-def run_on_gpu(n, steps, planes):
+def run_on_gpu(n, steps, planes, programs=PROGRAMS):
     w = runtime.wrappers()
     nbytes = planes.nbytes
     dev = w.tiramisu_hip_malloc(nbytes)
     w.tiramisu_hip_memcpy_to_device(dev, planes.ctypes.data, nbytes)
     name = "heat2d_%dx%d" % (n, steps)
-    prog = runtime.load(PROGRAMS, name)
+    prog = runtime.load(programs, name)
     prog(runtime.Buffer.from_device(dev, planes.shape, np.float32))
     w.tiramisu_hip_stream_synchronize(0)
     out = np.empty_like(planes)
@@ -116,6 +116,16 @@ def test_gpu_boundaries_of_both_planes_are_respected(n, steps):
     planes = rng.uniform(0, 1, (2, n, n)).astype(np.float32)
     expected = ref.heat2d(planes[0], steps, boundary_other=planes[1])
     out = run_on_gpu(n, steps, planes.copy())
+    assert np.array_equal(out, expected)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,steps", [(67, 23), (203, 15), (1367, 23), (1631, 12)])
+def test_gpu_short_strips_match_oracle(n, steps):
+    rng = np.random.RandomState(n)
+    planes = rng.uniform(0, 1, (2, n, n)).astype(np.float32)
+    expected = ref.heat2d(planes[0], steps, boundary_other=planes[1])
+    out = run_on_gpu(n, steps, planes.copy(), os.path.join(ROOT, "tests", "programs"))
     assert np.array_equal(out, expected)
 
 
