@@ -5,7 +5,11 @@ Exactness: products and sums of small whole numbers are exact.  Accuracy: with u
 accumulator once per matrix instruction, six per sixteen k, each time by at most 2^-24 of the sum of the magnitudes so far; the
 products left out are below 2^-24 of theirs.  |error| <= (6/16 K 2^-24 / 2 + 2^-24) sum |a b| therefore bounds every element (on
 average half the accumulator's final value is there when it is rounded), with a few more roundings for partial sums, alpha and beta.
-One product per sum: see test_one_product_per_sum."""
+One product per sum: see test_one_product_per_sum.
+
+The whole result, by the 2-norm: each rounding is off by 2^-23 / sqrt(12) of the accumulator's size on average, and that size grows with
+the root of k: 6/16 K roundings come to sqrt(3/16 K / 12) 2^-23 = sqrt(K) / 8 2^-23 of the result.  Twice that, and 2^-24 for the products left
+out, is allowed: at most 8e-7 at the sizes here, where any one of the six products missing is off by 2e-6 (see test_missing_products)."""
 import ctypes
 import os
 import subprocess
@@ -74,6 +78,35 @@ def bound(A, B, K):
     return (6 / 16 * K / 2 + 24) * 2.0 ** -24 * (np.abs(A) @ np.abs(B)) + 2.0 ** -24 * (np.abs(A) @ np.abs(B))
 
 
+def distance(out, expected):
+    return np.linalg.norm(out - expected) / np.linalg.norm(expected)
+
+
+def allowed_distance(K):
+    return 2 * K ** 0.5 / 8 * 2.0 ** -23 + 2.0 ** -24
+
+
+def test_missing_products():
+    """Five of the six products, in 64 bits: every one that is left out shows in the distance that the tests allow."""
+    def bf16(x):
+        u = x.astype(np.float32).view(np.uint32).astype(np.uint64)
+        return ((u + 0x7fff + ((u >> 16) & 1)) & 0xffff0000).astype(np.uint32).view(np.float32)
+
+    def parts(x):
+        h = bf16(x)
+        m = bf16(x - h)
+        return [p.astype(np.float64) for p in (h, m, x - h - m)]
+
+    rng = np.random.RandomState(6)
+    K = max([s[2] for s in SIZES] + [32 * 9])
+    A, B = (parts(rng.uniform(-1, 1, s).astype(np.float32)) for s in ((64, K), (K, 64)))
+    six = [(0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (2, 0)]
+    expected = sum(A) @ sum(B)
+    assert distance(sum(A[i] @ B[j] for i, j in six), expected) < 2.0 ** -24
+    for left_out in six:
+        assert distance(sum(A[i] @ B[j] for i, j in six if (i, j) != left_out), expected) > 1.5 * allowed_distance(K)
+
+
 def operands(rng, M, N, K, tA, tB, pad, kind):
     def one(rows, cols):
         full = np.full((rows, cols + pad), np.nan, np.float32)       # what lies between the rows must not matter
@@ -140,6 +173,7 @@ def test_library_call(rule, M, N, K, edge, tA, tB):
             assert np.array_equal(out[:, :N], expected)
         else:
             assert np.all(np.abs(out[:, :N] - expected) <= bound(a, b, K))
+            assert distance(out[:, :N], expected) <= allowed_distance(K)
 
 
 # Sums of one product each: the parts of both operands show one by one.
@@ -279,6 +313,9 @@ def test_windowed_convolution(kind):
     K = ci * 9
     allowed = (K + 24) * 2.0 ** -24 * size + 2.0 ** -149 * K if kind == "special" else (6 / 16 * K / 2 + 24) * 2.0 ** -24 * size + 2.0 ** -24 * size
     assert np.all(np.abs(out - relu)[fine] <= allowed[fine])
+    if kind == "uniform":
+        positive = expected > 0                           # (the others are zero)
+        assert distance(out[positive], expected[positive]) <= allowed_distance(K)
     assert np.array_equal(np.isinf(out), expected == np.inf)
 
 
