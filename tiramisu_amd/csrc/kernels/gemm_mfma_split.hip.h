@@ -4,13 +4,14 @@
 // A float has 24 significant bits, a bf16 number 8 and the same exponents.  With h = bf16(x), m = bf16(x - h), l = x - h - m
 // (both differences are exact) l has at most 8 significant bits again: x = h + m + l.  A product is then nine products of
 // bf16 numbers, which the matrix cores form exactly and add in fp32.  The six of them down to 2^-18 of the largest are taken,
-//     mA*mB, hA*mB, hA*lB, lA*hB, mA*hB, hA*hB;
+//     mA*mB, mA*hB, lA*hB, hA*lB, hA*mB, hA*hB;
 // the other three together are below 2^-24 of the product (they come near it: both operands 1 + 2^-8 - 2^-17), as much as one fp32
 // multiplication may round by, and they are zero wherever the product has 24 significant bits or fewer (products of small whole
 // numbers stay exact).  The largest comes last: a sum that one product dominates is then rounded at its full size once.  One product
 // alone is within 1.45 units in the last place, 0.39 rms (fp32 instruction 0.5 and 0.29; with the largest first, rounded again
 // by each of the five that follow, 3.4 and 0.60).  The order of the five costs nothing in accuracy; in this one neighbours share an operand
-// where they can, which the power limit rewards (4096^3 582 to 598 us; smallest first 609 to 620, largest first 602 to 617).
+// where they can, which the power limit rewards (4096^3 590 us; smallest first 609, largest first 602; a convolution 64 to 64 channels, which
+// waits for the parts from LDS, 170.5, 173 and 169).
 // v_mfma_f32_32x32x16_bf16 does sixteen times the work of v_mfma_f32_32x32x2_f32 per cycle, so that six of it take 3/8 of the
 // fp32 instruction's time; and an accumulator is rounded six times per sixteen k instead of eight times or more, which is why
 // the error against 64 bits is smaller (uniform random operands, 2-norm: 4096^3 1.00e-6 against 1.15e-6, with partial sums
@@ -23,8 +24,8 @@
 // of NaN 1150 us, with operands of 2^60, whose every product overflows, 2030 (bound by the L2; 600 without, 960 with the fp32 instruction),
 // 1024^3 38 (18; 20).
 //
-// What bounds it: at 4096^3 the power limit (620 us on random operands, 470 on zeros, 948 with the fp32 instruction), on small tiles the
-// vector work of the split, seven instructions per element, each done once per tile (1024^3 17 us, 20.5 before).
+// What bounds it: at 4096^3 the power limit (596 to 625 us on random operands, machines differ, 470 on zeros; 948 to 964 with the fp32 instruction), on small tiles the
+// vector work of the split, seven instructions per element, each done once per tile (1024^3 17 to 19 us, 20.6 to 22.5 with the fp32 instruction).
 #ifndef TIRAMISU_AMD_GEMM_MFMA_SPLIT_HIP_H
 #define TIRAMISU_AMD_GEMM_MFMA_SPLIT_HIP_H
 #include "gemm_mfma.hip.h"
@@ -61,7 +62,7 @@ __device__ __forceinline__ void split_pair(const split_constants &c, float a, fl
     part[2] = split_pack(a, b);
 }
 // The products taken: part of A, part of B; and the parts in the order in which they are needed.
-constexpr int SPLIT_A[6] = {1, 0, 0, 2, 1, 0}, SPLIT_B[6] = {1, 1, 2, 0, 0, 0}, SPLIT_READ[3] = {1, 0, 2};
+constexpr int SPLIT_A[6] = {1, 1, 2, 0, 0, 0}, SPLIT_B[6] = {1, 0, 0, 2, 1, 0}, SPLIT_READ[3] = {1, 0, 2};
 
 // Takes the scale out of the sums of the wavefront's rows from m0 and columns from n0; whether one that is in C is not finite.
 template <class CFG>

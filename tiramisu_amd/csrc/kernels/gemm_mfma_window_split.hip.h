@@ -10,9 +10,9 @@
 // workgroups of four wavefronts share a compute unit and cover each other's splitting, barriers and epilogues.  LDS accesses
 // are free of bank conflicts: lanes store and read granules of neighbouring positions, and rows of A lie an odd number of
 // granules apart.  (One workgroup of eight wavefronts with two stages, 512 positions and one barrier per block, the split dealt out
-// between the matrix instructions: 229 us instead of 181 for the case below; it needs more registers than there are.)
+// between the matrix instructions: 229 us where this form took 181; it needs more registers than there are.)
 //
-// 32 images of 112 x 112, 64 to 64 channels: 242 us with the fp32 instruction, 181 so; matrix cores 58 % busy at the 1.8 GHz that
+// 32 images of 112 x 112, 64 to 64 channels: 250 us with the fp32 instruction, 172 so (median launches); matrix cores 58 % busy at the 1.8 GHz that
 // the power limit leaves.  The error against 64 bits is smaller (gemm_mfma_split.hip.h), and sums that are not finite are
 // computed again with the fp32 instruction (operands of 2^60, every sum: 454 us a call, 198 without, 276 with that instruction alone).
 //
