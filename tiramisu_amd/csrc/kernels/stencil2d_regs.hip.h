@@ -243,8 +243,8 @@ __device__ __forceinline__ void ST_CAT(ST_NAME, _sweep)(const float *__restrict_
         // The adjacent lanes' cells next to each of my quads, ahead of the barrier.  A lane shift takes the vector ALU twice as long as an
         // add (1.8 against 1.0 ns per SIMD, as any operand that does not come from the lane's own registers), and an add that has one
         // folded in stops the adds of the other wavefronts from being issued in pairs with it; here they fill the time in
-        // which the wavefronts wait for each other and for the LDS (8192 x 8192, launches of 11, 9 and 12 steps 160, 129 and 179 us
-        // with the shifts folded into the adds, 136, 115 and 170 so).  The empty statement keeps the compiler from folding them.
+        // which the wavefronts wait for each other and for the LDS (8192 x 8192, median launches of 11, 9 and 12 steps 165, 131 and 180 us
+        // with the shifts folded into the adds, 139 to 146, 119 to 121 and 176 to 178 so).  The empty statement keeps the compiler from folding them.
         float from_left[RPT], from_right[RPT];
         if (ST_SHIFTS) {
 #pragma unroll

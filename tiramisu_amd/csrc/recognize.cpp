@@ -1345,7 +1345,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
                 // for the first block) are covered by the other's matrix instructions
                 win_resident = 2 * (2 * stage_bytes + 64) <= ttarget::LDS_BYTES_PER_CU ? env_int("TIRAMISU_MFMA_WINDOW_RESIDENT", 2) : 1;
                 // On the bf16 matrix cores a tile's start and end weigh more: for tiles of 256 positions with 32 channels or more, and more
-                // of them than two for every compute unit (32 images of 112 x 112, 64 to 64 channels 266 -> 181 us; one of 28 x 28 with tiles
+                // of them than two for every compute unit (32 images of 112 x 112, 64 to 64 channels 250 -> 172 us in the kernel; one of 28 x 28 with tiles
                 // of 64 positions 13.6 -> 21, 12 of 40 x 40 with 16 channels 16.4 -> 17.2)
                 win_split = BM == 64 && BN == 256 && WGM == 1 && WGN == 4 && win_channels % 8 == 0 && win_channels >= 32 && tiles > 2 * ttarget::COMPUTE_UNITS &&
                             lda_lit < (1L << 22) && 2 * (ttarget::window_split_lds_bytes(BM, win_taps, need) + 64) <= ttarget::LDS_BYTES_PER_CU &&

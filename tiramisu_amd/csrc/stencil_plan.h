@@ -1,6 +1,6 @@
 // How the stencil emitter cuts a time loop into launches and a launch into workgroups: plain integer arithmetic,
 // shared by the emitter (recognize.cpp), which prints the result as the macros of kernels/stencil2d_regs.hip.h, and by
-// the host-side model of that kernel's loads and stores (tests/programs/stencil_address_model.cpp).
+// the host-side model of that kernel's loads and stores (tests/host_models/stencil_address_model.cpp).
 #ifndef TIRAMISU_AMD_STENCIL_PLAN_H
 #define TIRAMISU_AMD_STENCIL_PLAN_H
 #include <algorithm>
