@@ -143,6 +143,8 @@ void tiramisu_hip_parallel_for(int32_t first, int32_t last, void (*body)(int32_t
  * block out again while that work still runs. */
 int tiramisu_hip_set_stream(void *stream);
 void *tiramisu_hip_get_stream(void);
+/* Waits for the device's null stream (other libraries' default stream), whatever the calling thread's current one. */
+int tiramisu_hip_null_stream_synchronize(void);
 /* A new stream that does not synchronise with the default stream (default priority), for callers that overlap
  * calls; destroy waits for the stream's work and, if it is the calling thread's current stream, restores the
  * per-thread default stream.  Scratch blocks that the runtime keeps per (thread, stream) stay allocated until

@@ -856,6 +856,11 @@ int tiramisu_hip_set_stream(void *stream) {
 
 void *tiramisu_hip_get_stream(void) { return (void *)current_stream; }
 
+int tiramisu_hip_null_stream_synchronize(void) {
+    check(hipStreamSynchronize(hipStreamLegacy), __FUNCTION__);
+    return 0;
+}
+
 void *tiramisu_hip_stream_create(void) {
     hipStream_t s;
     check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), __FUNCTION__);   // default priority

@@ -100,8 +100,6 @@ class Buffer:
         return ctypes.byref(self.raw)
 
 
-HIP_STREAM_LEGACY = 1        # hipStreamLegacy: the null stream, by a handle that is not null
-
 _wrappers = None
 
 
@@ -244,16 +242,11 @@ class Program:
             rc = self.fn(*[b.pointer() for b in bufs])
         elif torch_stream == 0:
             # torch's default stream is the device's null stream, and its handle, 0, means the calling thread's own default
-            # stream to tiramisu_hip_set_stream; HIP's other name for it does not.  The kernels stay on the thread's stream, so that
-            # calls from several threads overlap (two threads of a 1.33 ms pass each 2.2 ms a round; on the null stream, one
-            # after the other, 2.7), ordered by a wait on both sides.  The runtime waits: torch's synchronize() costs 3 us more.
+            # stream to tiramisu_hip_set_stream.  The kernels stay on the thread's stream, so that calls from several threads
+            # overlap (two threads of a 1.33 ms pass each 2.0 to 2.2 ms a round; on the null stream, one after the other, 2.7),
+            # ordered by a wait on both sides.  The runtime waits: torch's synchronize() costs 3 us more.
             w = wrappers()
-            before = w.tiramisu_hip_get_stream()
-            w.tiramisu_hip_set_stream(HIP_STREAM_LEGACY)
-            try:
-                w.tiramisu_hip_stream_synchronize(0)
-            finally:
-                w.tiramisu_hip_set_stream(before)
+            w.tiramisu_hip_null_stream_synchronize()
             rc = self.fn(*[b.pointer() for b in bufs])
             w.tiramisu_hip_stream_synchronize(0)
         else:
