@@ -212,6 +212,19 @@ def test_gpu_sizes_that_end_inside_a_tile(M, N, K, what, programs_dir):
         assert np.array_equal(d[2].download(), exact, equal_nan=True), infinite
 
 
+TILES = [(1793, 3842, 514, "tile 128x256x64, guarded edges"), (1921, 2562, 578, "tile 192x128x64, guarded edges"),
+         (673, 3202, 1090, "tile 96x128x64, guarded edges"), (1473, 642, 514, "tile 64x128x64, guarded edges"), (33, 66, 194, "tile 32x64x64, guarded edges"),
+         (2000, 1500, 1010, "tile 128x128x32, guarded edges, slices in pairs"), (3842, 3970, 1278, "tile 256x256x32, guarded edges, slices in pairs"),
+         (1920, 2560, 1024, "tile 192x128x64, whole tiles")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,what", TILES)
+def test_gpu_tiles_between_the_squares(M, N, K, what, programs_dir):
+    """The tiles between the squares of 256, 128 and 64, and slices in pairs, at their remainders: exact as above."""
+    test_gpu_sizes_that_end_inside_a_tile(M, N, K, what, programs_dir)
+
+
 VIEWS = [("a_backwards", 200, 150, 100), ("b_backwards", 200, 150, 100), ("a_backwards_whole", 128, 192, 128), ("b_backwards_whole", 128, 192, 128),
          ("b_overlapping", 66, 30, 50)]
 

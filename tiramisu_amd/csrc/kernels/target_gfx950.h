@@ -134,32 +134,44 @@ inline int split_tile_for(long M, long N, long K, long problems, int m, int n, b
 }
 
 // C tiles of the bf16-input kernels.  What the loops over K of a launch take is modelled as `fixed` microseconds (start, first
-// slices) plus, for every 32 k of whole slices, `first` for the first round of tiles over the compute units and `further` for
-// each round after it.  Reading and writing C is left out: it takes every tile the same (64 MiB in and out at 4096 x 4096 20 us),
-// so the model only orders the tiles.  It is fitted to whole launches of 32 ... 4096 k with a tenth of the chip's tiles up to
-// sixteen rounds: 300 x 260 x 3000 takes 13.0 us with 64 x 64 (14.1 modelled) and 21.6 with 128 x 128 (19.9), 1000 x 750 x 500
-// 5.6 and 8.0 (4.7, 6.6), 2000 x 1500 x 1000 15.6 with 128 x 128 and 18.0 with 64 x 64 (9.3, 14.3), 3000 x 2700 x 4000 82 with
-// 256 x 256 and 109 with 128 x 128 (78, 95), 4096 x 3072 x 32, half of a slice of the 64 x 64 tiles, 17.3 with 128 x 128 and
-// 20.5 with 64 x 64 (4.6, 5.7).
+// slices) plus, for every 32 k of whole stages, `first` for the first round of tiles over the compute units and `further` for
+// each round after it.  Reading and writing C is left out: it takes every tile about the same (1.07 us per million elements),
+// so the model only orders the tiles.  It is fitted to whole launches of 100 sizes of 32 ... 4096 rows, columns and k (rms error
+// 8 to 12 %).  A stage of the LDS ring holds `slices` slices of `k`: with 64 k a row of A is read 128 bytes at a time, a whole line
+// of the L1, and there is one barrier for twice the work (4096^3 125 -> 121 us, 2000 x 1500 x 1000 15.3 -> 14.2); slices of 32 in
+// more stages start earlier and pad less.
+// The tiles between the squares of 256, 128 and 64 are for results that those cover badly: 1500 x 1000 x 3000 are 96 tiles of 128 x 128
+// (34 us) or 384 of 64 x 64, two rounds (28), but 192 of 64 x 128 (22); 1798 x 3830 x 3428 88 us with 128 x 128, 56 with 128 x 256;
+// 1908 x 2550 x 858 27 and 20 with 192 x 128; 682 x 3212 x 1114 19 and 14.4 with 96 x 128; 417 x 396 x 3318 20 with 64 x 64 and 15 with 32 x 64.
+// A tile is taken from `from` to `to` k.  Up to 512 k the squares keep the figures they were fitted with there: the tiles between them
+// would give less than a microsecond, and the model errs by as much (805 x 1240 x 306 6.5 us with 64 x 64, 6.7 with 64 x 128).
 // Direct tiles load their slices straight into LDS; the others serve rows of an odd number of elements and other operands that
 // those loads cannot address.
 struct bf16_tile {
-    int edge, k, waves_m, waves_n, stages;
+    int m, n, k, slices, waves_m, waves_n, stages;
     bool direct;
+    int from, to;
     double fixed, first, further;
 };
-constexpr bf16_tile BF16_TILES[] = {{256, 32, 4, 2, 4, true, 9.0, 0.55, 0.85}, {128, 32, 2, 4, 4, true, 3.9, 0.17, 0.28},
-                                    {64, 64, 2, 2, 3, true, 2.8, 0.12, 0.12},
-                                    {128, 64, 2, 2, 2, false, 8.0, 0.42, 0.4}, {64, 64, 2, 2, 2, false, 3.5, 0.19, 0.195}};
-constexpr bf16_tile BF16_TILE_ANY_SIZE = BF16_TILES[4];    // sizes known at run time only
+constexpr int ANY_K = 0x7fffffff;
+constexpr bf16_tile BF16_TILES[] = {
+    {256, 256, 32, 1, 4, 2, 4, true, 0, 512, 9.0, 0.55, 0.85}, {128, 128, 32, 1, 2, 4, 4, true, 0, 512, 3.9, 0.17, 0.28},
+    {64, 64, 64, 1, 2, 2, 3, true, 0, 512, 2.8, 0.12, 0.12}, {32, 64, 64, 1, 1, 2, 3, true, 192, 512, 2.7, 0.104, 0.092},
+    {256, 256, 32, 1, 4, 2, 4, true, 513, ANY_K, 9.0, 0.58, 0.85}, {256, 256, 32, 2, 4, 2, 2, true, 513, ANY_K, 9.5, 0.555, 0.85},
+    {128, 256, 64, 1, 2, 4, 3, true, 513, ANY_K, 6.2, 0.326, 0.51}, {192, 128, 64, 1, 2, 4, 3, true, 513, ANY_K, 5.6, 0.283, 0.386},
+    {128, 128, 32, 1, 2, 4, 4, true, 513, ANY_K, 3.9, 0.251, 0.295}, {128, 128, 32, 2, 2, 4, 3, true, 513, ANY_K, 4.4, 0.227, 0.349},
+    {96, 128, 64, 1, 1, 4, 3, true, 513, ANY_K, 5.8, 0.188, 0.285}, {64, 128, 64, 1, 2, 2, 3, true, 513, ANY_K, 4.1, 0.167, 0.179},
+    {64, 64, 64, 1, 2, 2, 3, true, 513, ANY_K, 3.35, 0.132, 0.117}, {32, 64, 64, 1, 1, 2, 3, true, 513, ANY_K, 3.2, 0.114, 0.090},
+    {128, 128, 64, 1, 2, 2, 2, false, 0, ANY_K, 8.0, 0.42, 0.4}, {64, 64, 64, 1, 2, 2, 2, false, 0, ANY_K, 3.5, 0.19, 0.195}};
+constexpr bf16_tile BF16_TILE_ANY_SIZE = BF16_TILES[sizeof(BF16_TILES) / sizeof(BF16_TILES[0]) - 1];    // sizes known at run time only
 
 inline bf16_tile bf16_tile_for(long M, long N, long K, bool direct) {
     const bf16_tile *best = nullptr;
     double best_cost = 0;
     for (const bf16_tile &c : BF16_TILES) {
-        if (c.direct != direct) continue;
-        const long tiles = ((M + c.edge - 1) / c.edge) * ((N + c.edge - 1) / c.edge), rounds = (tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS;
-        const double cost = c.fixed + ((K + c.k - 1) / c.k * c.k / 32) * (c.first + (rounds - 1) * c.further);
+        if (c.direct != direct || K < c.from || K > c.to) continue;
+        const long tiles = ((M + c.m - 1) / c.m) * ((N + c.n - 1) / c.n), rounds = (tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS, stage = c.k * c.slices;
+        const double cost = c.fixed + ((K + stage - 1) / stage * stage / 32) * (c.first + (rounds - 1) * c.further);
         if (!best || cost < best_cost) { best = &c; best_cost = cost; }
     }
     return *best;

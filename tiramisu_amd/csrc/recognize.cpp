@@ -1202,7 +1202,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     if (const char *e = backend_option("TIRAMISU_MFMA_PAD")) PADX = std::atoi(e);
     if (const char *e = backend_option("TIRAMISU_MFMA_WGK")) WGK = std::atoi(e);
     bool bf16_edge = false, bf16_direct = false;
-    int bf16_stages = 2;                 // of the LDS ring
+    int bf16_stages = 2, bf16_slices = 1;        // of the LDS ring; slices of a stage
     if (bf16) {
         // the tile whose launch is modelled fastest (kernels/target_gfx950.h); rows of an even number of elements are
         // loaded straight into LDS (32-bit offsets from an operand's first row: operands below 2 GiB, walked forwards; rows
@@ -1228,8 +1228,10 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         }
         bf16_direct = lit && dword_rows && small_enough && forwards;
         const ttarget::bf16_tile tile = lit ? ttarget::bf16_tile_for(Ml, Nl, Kl, bf16_direct) : ttarget::BF16_TILE_ANY_SIZE;
-        BM = BN = tile.edge;
-        BK = tile.k;
+        BM = tile.m;
+        BN = tile.n;
+        BK = tile.k * tile.slices;
+        bf16_slices = tile.slices;
         WGM = tile.waves_m;
         WGN = tile.waves_n;
         bf16_stages = tile.stages;
@@ -1547,9 +1549,9 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
                             std::to_string(WGM) + ", " + std::to_string(WGN) + ", " + (operands[0].first.kmajor ? "true" : "false") + ", " +
                             (operands[0].second.kmajor ? "true" : "false") + ", " + (edge ? "true" : "false") + ", " + std::to_string(PADX) + ", " + std::to_string(WGK) + ", " + std::to_string(DEPTH) + ">";
     const int NT = 64 * WGM * WGN * WGK;
-    auto bf16_config_text = [](bool direct, int tile, int k, int waves_m, int waves_n, int stages, bool guarded) {
+    auto bf16_config_text = [](bool direct, int m, int n, int k, int waves_m, int waves_n, int stages, bool guarded) {
         std::ostringstream os;
-        os << "    typedef tgemm::config_bf16" << (direct ? "_direct<" : "<") << tile << ", " << tile << ", " << k << ", " << waves_m << ", " << waves_n;
+        os << "    typedef tgemm::config_bf16" << (direct ? "_direct<" : "<") << m << ", " << n << ", " << k << ", " << waves_m << ", " << waves_n;
         if (direct) os << ", " << stages;
         os << (guarded ? ", true" : ", false") << "> CFG;\n";
         return os.str();
@@ -1557,7 +1559,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     if (bf16) {
         body << "    extern __shared__ __attribute__((aligned(16))) uint32_t _lds[];\n";
         // slices go straight from global memory into an LDS ring where they can
-        body << bf16_config_text(bf16_direct, BM, BK, WGM, WGN, bf16_stages, edge);
+        body << bf16_config_text(bf16_direct, BM, BN, BK, WGM, WGN, bf16_stages, edge);
     } else {
         body << "    extern __shared__ __attribute__((aligned(16))) float _lds[];\n";
         if (win_split) body << "    typedef tgemm::config_window<" << BM << ", " << BN << ", " << WGM << ", " << WGN << "> CFG;\n";
@@ -1775,7 +1777,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     k.how = std::string("mfma-contraction: ") + (bf16 ? (bf16_direct ? "v_mfma_f32_32x32x16_bf16, slices loaded straight into LDS (through registers where an operand begins at an odd element), " : "v_mfma_f32_32x32x16_bf16, ") : split_edge || win_split ? "v_mfma_f32_32x32x16_bf16 on the three bf16 parts of every fp32 operand element, " : "v_mfma_f32_32x32x2_f32, ") + (windowed ? "implicit GEMM, sliding window of " + std::to_string(win_taps) + " taps staged in LDS by blocks of " + std::to_string(win_cb) + " channels, " :
                                                                                       any_gather ? "implicit GEMM (gathered operand), " : "") + "M " +
             std::to_string(Mg.size()) + " dim(s) x N " + std::to_string(Ng.size()) + " x K " + std::to_string(Kg.size()) + ", tile " +
-            std::to_string(BM) + "x" + std::to_string(BN) + "x" + std::to_string(BK) + (edge ? ", guarded edges" : ", whole tiles") + ", " +
+            std::to_string(BM) + "x" + std::to_string(BN) + "x" + std::to_string(BK / bf16_slices) + (edge ? ", guarded edges" : ", whole tiles") + (bf16_slices > 1 ? ", slices in pairs, " : ", ") +
             std::to_string(operands.size()) + " product term(s)" + (has_init ? ", fused initialisation" : "") + (has_epi ? ", fused epilogue" : "") +
             (with_consumer ? ", " + std::to_string(xs.size()) + " point-wise statement(s) of the following nest fused (" + std::to_string(G) + " column group(s) per unit, " +
                                  std::to_string(dead.size()) + " temporaries kept in registers)" : "") +
@@ -1883,14 +1885,14 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         const ttarget::bf16_tile t = ttarget::bf16_tile_for(Ml, Nl, Kl, false);
         unaligned = k;
         unaligned.name = kname + "_unaligned";
-        unaligned.grid[0] = std::to_string(((Ml + t.edge - 1) / t.edge) * ((Nl + t.edge - 1) / t.edge));
+        unaligned.grid[0] = std::to_string(((Ml + t.m - 1) / t.m) * ((Nl + t.n - 1) / t.n));
         unaligned.block[0] = std::to_string(64 * t.waves_m * t.waves_n);
-        unaligned.lds_bytes = std::to_string(t.stages * (t.k / 8) * 2 * t.edge * 4 * 4);
+        unaligned.lds_bytes = std::to_string(t.stages * (t.k / 8) * (t.m + t.n) * 4 * 4);
         std::string text = body.str();
         auto replace_all = [&](const std::string &from, const std::string &to) {
             for (size_t at = text.find(from); at != std::string::npos; at = text.find(from, at + to.size())) text.replace(at, from.size(), to);
         };
-        replace_all(bf16_config_text(true, BM, BK, WGM, WGN, bf16_stages, edge), bf16_config_text(false, t.edge, t.k, t.waves_m, t.waves_n, t.stages, true));
+        replace_all(bf16_config_text(true, BM, BN, BK, WGM, WGN, bf16_stages, edge), bf16_config_text(false, t.m, t.n, t.k * t.slices, t.waves_m, t.waves_n, t.stages, true));
         replace_all("tile_accumulate_bf16_direct<CFG>", "tile_accumulate_bf16<CFG>");
         print_kernel(unaligned, text);
         std::set<std::string> operand_buffers;
