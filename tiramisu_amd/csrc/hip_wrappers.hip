@@ -780,6 +780,7 @@ int tiramisu_hip_dgemm(double *A, double *B, double *C, uint64_t M, uint64_t N, 
     switch (tgemm64::tile_for((long)M, (long)N, (long)K)) {
     case tgemm64::TILE_128: launch(tgemm64::shape_128()); break;
     case tgemm64::TILE_96: launch(tgemm64::shape_96()); break;
+    case tgemm64::TILE_96_SHARED: launch(tgemm64::shape_96_shared()); break;
     case tgemm64::TILE_64: launch(tgemm64::shape_64()); break;
     case tgemm64::TILE_32: launch(tgemm64::shape_32()); break;
     case tgemm64::TILE_32_SHARED: K <= 32 ? launch(tgemm64::shape_32_short()) : launch(tgemm64::shape_32_shared()); break;

@@ -6,15 +6,14 @@
 // tiles of 16 x 16 per wavefront.  K is walked in slices of BK: the slice's A and B parts go from
 // global memory to registers (8-byte loads, the thread-to-element mapping chosen so that consecutive lanes follow
 // the operand's unit stride), from there to one of two LDS stages as [k][m] and [k][n], and each k-step (4) of a slice reads
-// TM + TN operand fragments for TM * TN matrix instructions.  The next slice's global loads are issued before the
-// current slice is multiplied and stored to the other stage after it: one barrier per slice.
+// TM + TN operand fragments for TM * TN matrix instructions.  A slice is stored to its stage while the one before it is multiplied,
+// two slices after its loads were issued, and a step's fragments are read during the step before: one barrier per slice, ahead of its last step.
 //
 // What bounds it: with tiles enough, the fp64 matrix instruction (64 cycles each, so LDS is never short); with few, the chain of
-// one tile's slices, each a trip to memory, two LDS accesses and a barrier.  Hence tiles from 128 x 128 down to 16 x 16, and, in
-// tiles that cannot fill the chip, groups of wavefronts that share a slice's k (WGK).  us before and after (before: 128 x 128,
-// 64 x 64 or 32 x 32 by the number of tiles, slices of 16, every element guarded in all slices and in the epilogue):
-//   1500 x 1430 x 250 62 -> 33, 2000 x 1100 x 700 112 -> 78, 1000^3 62 -> 48, 500^3 15.6 -> 11.6, 64 x 2048 x 512 14.8 -> 8.2,
-//   180^3 7.6 -> 5.2, 16 x 16 x 2000 47 -> 14.3; 2048^3 314 (55 TFLOP/s) either way.
+// one tile's slices, each a trip to memory, two LDS accesses and a barrier.  Hence tiles from 128 x 128 down to 16 x 16, and groups
+// of wavefronts that share a slice's k (WGK).  us of a launch with loads one slice ahead, fragments read by the step that multiplies them and fewer
+// such groups -> now: 1500 x 1430 x 250 33.6 -> 30.8, 2000 x 1100 x 700 77.5 -> 67, 1500 x 1430 x 1000 107 -> 93, 1000^3 49 -> 46.5, 500^3 11.4 -> 10.4,
+// 2048^3 310 (55 TFLOP/s), 200 x 300 x 1000 9.6 either way.
 //
 // Instruction layout (one wavefront): lane l supplies A[row l % 16][k l / 16] and B[k l / 16][column l % 16];
 // its four results are rows l / 16 + 0, 4, 8, 12 of column l % 16.
@@ -31,8 +30,11 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 // BK: the k of a slice.  PAD of 2 doubles: rows lie 4 words apart modulo the 64 banks, so the 16 k that the consecutive lanes of
 // a k-contiguous operand store fall on different banks.
 // WGK groups of wavefronts each multiply 1 / WGK of a slice's k for the same tile; their sums are added through LDS.
-template <int TM_, int TN_, int WGM_, int WGN_, int BK_, int WGK_ = 1, int PAD = 2>
+// AHEAD: the pipeline below; without it a slice is loaded and stored around the one that is multiplied, in the registers that two workgroups
+// of the largest tiles have to a compute unit (2048^3 with 128 x 128 tiles 314 us; with the pipeline, which spills there, 349 to 513 by layout).
+template <int TM_, int TN_, int WGM_, int WGN_, int BK_, int WGK_ = 1, bool AHEAD_ = true, int PAD = 2>
 struct shape {
+    static constexpr bool AHEAD = AHEAD_;
     static constexpr int TM = TM_, TN = TN_, WGM = WGM_, WGN = WGN_, BK = BK_, WGK = WGK_;
     static constexpr int NT = 64 * WGM * WGN * WGK;
     static constexpr int RESIDENT = WGK == 1 ? 2 : 1;                        // workgroups that share a compute unit
@@ -50,22 +52,27 @@ struct shape {
 
 // The tiles, and the one whose launch is modelled fastest: `fixed` microseconds (start, the last store), `round` for every round of
 // tiles over the compute units (first slice, epilogue), and per k `first` for a round that a compute unit has to itself or
-// `further` for each of several, whichever is more.  Fits to whole launches of 16 ... 2048 in each size (measured / modelled:
+// `further` for each of several, whichever is more.  Fits to whole launches of 16 ... 2048 in each size, before the pipeline (measured / modelled:
 // 1500 x 1430 x 250 32.5 / 34.1 with 32 x 32, 34.3 / 34.7 with 96 x 96, 46 / 47 with 128 x 128; x 1000 114 / 120, 107 / 108,
 // 155 / 155; 2080 x 4832 x 32 25 / 29, 30 / 29, 27 / 29; 1000^3 48 / 46 with 64 x 64, 55 / 55 with 32 x 32; 700 x 900 x 1000 45.5 / 42.1 without and 42.4 / 41.9 with
 // shared slices; 200 x 300 x 1000 9.7 / 8.6 with 16 x 16, 18.6 / 18 with 32 x 32).
-enum tile { TILE_128, TILE_96, TILE_64, TILE_32, TILE_32_SHARED, TILE_16, TILES };
-typedef shape<4, 2, 2, 4, 16> shape_128;             // 2 x 4 wavefronts: two per SIMD cover each other's waits
-typedef shape<3, 3, 2, 2, 16> shape_96;
+// Tiles of 96 x 96 that fit the chip in a round leave each SIMD one wavefront: with slices of 32 k shared by two groups it has two. They take the place of
+// tiles whose sums are of one part (with the pipeline: 2000 x 1100 x 700 67 against 78 with 96 x 96, 1500 x 1430 x 1000 93 and 108, x 250 30.7 and 33 with
+// 32 x 32, 1120 x 1965 x 256 30.7 and 31.9, error against 64 bits and more 0.75 of it), not of those of four or eight, which are closer: 64 x 64 without
+// shared slices, faster where its tiles are several rounds (1960 x 1449 x 466 57 and 75), has twice their error.
+enum tile { TILE_128, TILE_96, TILE_64, TILE_32, TILE_32_SHARED, TILE_16, TILES, TILE_96_SHARED };
+typedef shape<4, 2, 2, 4, 16, 1, false> shape_128;   // 2 x 4 wavefronts: two per SIMD cover each other's waits
+typedef shape<3, 3, 2, 2, 16, 1, false> shape_96;
+typedef shape<3, 3, 2, 2, 32, 2> shape_96_shared;
 typedef shape<2, 2, 2, 2, 64, 4> shape_64;
 typedef shape<1, 1, 2, 2, 16> shape_32;              // eight workgroups to a compute unit: short reductions, many tiles
 typedef shape<1, 1, 2, 2, 64, 4> shape_32_shared;
-typedef shape<1, 1, 1, 1, 128, 8> shape_16;
+typedef shape<1, 1, 1, 1, 128, 8, false> shape_16;      // (241 x 288 x 1344 16.5 us; with the pipeline 16.8)
 // For at most 32 k, which two groups hold sixteen each of, as in the slices above (the sums are the same ones): the other groups'
 // wavefronts only cost their start.  us of a call with 32 x 32 tiles without shared slices, with all groups, with two:
 // 384 x 512 x 32 3.9, 4.2, 3.9; 345 x 533 x 11 3.8, 4.3, 4.0; 1184 x 160 x 32 3.8, 4.3, 3.9.
 typedef shape<1, 1, 2, 2, 32, 2> shape_32_short;
-typedef shape<1, 1, 1, 1, 32, 2> shape_16_short;
+typedef shape<1, 1, 1, 1, 32, 2, false> shape_16_short;
 
 inline tile tile_for(long M, long N, long K) {
     static const struct { int edge; double fixed, round, first, further; } model[TILES] = {
@@ -80,6 +87,8 @@ inline tile tile_for(long M, long N, long K) {
         const double cost = model[i].fixed + rounds * model[i].round + (double)K * slope;
         if (i == 0 || cost < best_cost) { best = i; best_cost = cost; }
     }
+    const bool one_part = best == TILE_128 || best == TILE_96 || best == TILE_32;
+    if (one_part && ((M + 95) / 96) * ((N + 95) / 96) <= ttarget::COMPUTE_UNITS && 7.7 + 0.083 * (double)K < 0.9 * best_cost) return TILE_96_SHARED;
     return (tile)best;
 }
 
@@ -155,32 +164,60 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_SIMD) dgemm_kernel(const d
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
 
+    // One slice is multiplied while the next travels: the other stage is filled from registers during the first k-step and its
+    // successor asked for; a k-step's operands are read from LDS during the step before it, the first of a slice behind the one barrier,
+    // which lies before the last step, so that its matrix instructions cover the reads.
+    constexpr int KS = BK / 4 / S::WGK;
+    static_assert(KS % 2 == 0, "k-steps of a wavefront in pairs: the registers of a slice's first step are free in its last");
+    double fa[2][TM], fb[2][TN];
+    auto read = [&](int stage, int ks, int buf) {
+        const double *la = lds64 + stage * S::STAGE + wm * (16 * TM) + l16;
+        const double *lb = lds64 + stage * S::STAGE + BK * S::A_ROW + wn * (16 * TN) + l16;
+        const int k = 4 * (wk * KS + ks) + kq;
+#pragma unroll
+        for (int i = 0; i < TM; i++) fa[buf][i] = la[k * S::A_ROW + 16 * i];
+#pragma unroll
+        for (int j = 0; j < TN; j++) fb[buf][j] = lb[k * S::B_ROW + 16 * j];
+    };
     const int slices = (K + BK - 1) / BK;
     if (slices > 0) {
         load_slice(0);
         store_slice(0);
+        if (S::AHEAD && slices > 1) load_slice(BK);
     }
     __syncthreads();
+    if (S::AHEAD && slices > 0) read(0, 0, 0);
     for (int s = 0; s < slices; s++) {
         const int stage = s & 1;
-        if (s + 1 < slices) load_slice((s + 1) * BK);
-        const double *la = lds64 + stage * S::STAGE + wm * (16 * TM) + l16;
-        const double *lb = lds64 + stage * S::STAGE + BK * S::A_ROW + wn * (16 * TN) + l16;
 #pragma unroll
-        for (int ks = 0; ks < BK / 4 / S::WGK; ks++) {
-            double fa[TM], fb[TN];
-            const int k = 4 * (wk * (BK / 4 / S::WGK) + ks) + kq;
-#pragma unroll
-            for (int i = 0; i < TM; i++) fa[i] = la[k * S::A_ROW + 16 * i];
-#pragma unroll
-            for (int j = 0; j < TN; j++) fb[j] = lb[k * S::B_ROW + 16 * j];
+        for (int ks = 0; ks < KS; ks++) {
+            const int buf = ks & 1;
+            if (!S::AHEAD) {
+                if (ks == 0 && s + 1 < slices) load_slice((s + 1) * BK);
+                read(stage, ks, buf);
+            } else if (ks == 0 && s + 1 < slices) {
+                store_slice(stage ^ 1);
+                if (s + 2 < slices) load_slice((s + 2) * BK);
+            }
+            if (!S::AHEAD) {
+            } else if (ks + 1 < KS) {
+                read(stage, ks + 1, buf ^ 1);
+            } else {
+                __builtin_amdgcn_sched_barrier(0);
+                __syncthreads();
+                if (s + 1 < slices) read(stage ^ 1, 0, buf ^ 1);
+            }
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i], fb[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[buf][i], fb[buf][j], acc[i][j], 0, 0, 0);
+            // (one matrix instruction to a step: the step's reads stay ahead of it; 500^3 10.7 us without, 10.4 so)
+            if constexpr (TM * TN == 1 && S::WGM * S::WGN > 1) __builtin_amdgcn_sched_barrier(0);
         }
-        if (s + 1 < slices) store_slice(stage ^ 1);
-        __syncthreads();
+        if (!S::AHEAD) {
+            if (s + 1 < slices) store_slice(stage ^ 1);
+            __syncthreads();
+        }
     }
 
     if (S::WGK > 1) {
