@@ -145,6 +145,11 @@ int tiramisu_hip_set_stream(void *stream);
 void *tiramisu_hip_get_stream(void);
 /* Waits for the device's null stream (other libraries' default stream), whatever the calling thread's current one. */
 int tiramisu_hip_null_stream_synchronize(void);
+/* Calls a generated function (extern "C" int f(halide_buffer_t *...)) of up to eight arguments, all in GPU memory.  `description` holds for
+ * every argument the code and the bits of its type, the number of its dimensions and their extents, outermost first.  `stream`: the kernels
+ * run there, and the thread's stream is put back; NULL (another library's default stream): they run on the thread's own stream, and the call
+ * waits for the device's null stream first and for that stream afterwards.  Returns what the function returns, -1 for more arguments. */
+int tiramisu_hip_call(void *function, int32_t arguments, const uint64_t *pointers, const int32_t *description, void *stream);
 /* A new stream that does not synchronise with the default stream (default priority), for callers that overlap
  * calls; destroy waits for the stream's work and, if it is the calling thread's current stream, restores the
  * per-thread default stream.  Scratch blocks that the runtime keeps per (thread, stream) stay allocated until

@@ -868,6 +868,61 @@ int tiramisu_hip_null_stream_synchronize(void) {
     return 0;
 }
 
+// (the buffer layout that generated functions take: host glue of hip_backend.cpp)
+struct call_dimension { int32_t min, extent, stride; uint32_t flags; };
+struct call_buffer {
+    uint64_t device;
+    const void *device_interface;
+    uint8_t *host;
+    uint64_t flags;
+    struct { uint8_t code, bits; uint16_t lanes; } type;
+    int32_t dimensions;
+    call_dimension *dim;
+    void *padding;
+};
+
+int tiramisu_hip_call(void *function, int32_t arguments, const uint64_t *pointers, const int32_t *description, void *stream) {
+    constexpr int MOST = 8, MOST_DIMENSIONS = 8;
+    if (arguments < 1 || arguments > MOST) return -1;
+    call_buffer b[MOST];
+    call_dimension dims[MOST][MOST_DIMENSIONS];
+    for (int i = 0; i < arguments; i++) {
+        const int32_t code = *description++, bits = *description++, nd = *description++;
+        if (nd > MOST_DIMENSIONS) return -1;
+        int64_t stride = 1;
+        for (int d = 0; d < nd; d++) {                       // innermost first, as the buffers are described
+            dims[i][d] = {0, description[nd - 1 - d], (int32_t)stride, 0};
+            stride *= dims[i][d].extent;
+        }
+        description += nd;
+        b[i] = {pointers[i], nullptr, nullptr, 0, {(uint8_t)code, (uint8_t)bits, 1}, nd, dims[i], nullptr};
+    }
+    typedef call_buffer *p;
+    auto call = [&]() -> int {
+        switch (arguments) {
+        case 1: return ((int (*)(p))function)(b);
+        case 2: return ((int (*)(p, p))function)(b, b + 1);
+        case 3: return ((int (*)(p, p, p))function)(b, b + 1, b + 2);
+        case 4: return ((int (*)(p, p, p, p))function)(b, b + 1, b + 2, b + 3);
+        case 5: return ((int (*)(p, p, p, p, p))function)(b, b + 1, b + 2, b + 3, b + 4);
+        case 6: return ((int (*)(p, p, p, p, p, p))function)(b, b + 1, b + 2, b + 3, b + 4, b + 5);
+        case 7: return ((int (*)(p, p, p, p, p, p, p))function)(b, b + 1, b + 2, b + 3, b + 4, b + 5, b + 6);
+        default: return ((int (*)(p, p, p, p, p, p, p, p))function)(b, b + 1, b + 2, b + 3, b + 4, b + 5, b + 6, b + 7);
+        }
+    };
+    if (stream) {
+        const hipStream_t before = current_stream;
+        tiramisu_hip_set_stream(stream);
+        const int rc = call();
+        tiramisu_hip_set_stream((void *)before);
+        return rc;
+    }
+    tiramisu_hip_null_stream_synchronize();
+    const int rc = call();
+    tiramisu_hip_stream_synchronize(0);
+    return rc;
+}
+
 void *tiramisu_hip_stream_create(void) {
     hipStream_t s;
     check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), __FUNCTION__);   // default priority
