@@ -169,6 +169,30 @@ inline split_tile any_split_tile_for(long M, long N, long K, long problems, int 
     return tile;
 }
 
+// C tiles of a product with a gathered operand and at most 64 rows (an implicit GEMM: a convolution whose window is not staged in LDS; fp32
+// instruction).  With few columns a launch is bound by the chain of a tile's slices, so four groups of wavefronts share slices of 64 k; with
+// 32 rows or fewer a tile of 64 is half padding.  Modelled as whole launches: `fixed` microseconds, `round` for every round of tiles over the
+// compute units, and per k `first` or rounds times `further`, whichever is more; fitted to 44 convolutions of 3 ... 64 channels, 5 ... 64 filters
+// and 64 ... 300000 positions (rms error 9 to 14 %).  us of a launch with the tile of before (64 x 256 from 65536 columns on, else 64 x 64)
+// and with the one chosen: 2 images of 40 x 40, 64 to 48 channels 14.0, 6.5 (32 x 32); 3 of 24 x 24, 41 to 6 9.0, 4.7; 1 of 96 x 96, 44 to 15 10.7, 6.9 (32 x 64);
+// 32 of 100 x 100, 16 to 16 59, 35 (32 x 128); 7 of 96 x 96, 24 to 16 20.5, 12.2; 8 of 92 x 92, 40 to 50 53, 38 (64 x 64); 29 of 56 x 56, 46 to
+// 35 59, 46 (64 x 128); 8 of 112 x 112, 3 to 64 12.1, 11.4; of the 44 none slower, 0.71 of the time in the geometric mean.
+struct gathered_tile { int m, n, k, waves_m, waves_n, groups; double fixed, round, first, further; };
+constexpr gathered_tile GATHERED_TILES[] = {
+    {32, 32, 64, 1, 1, 4, 2.5, 0.66, 0.0056, 0.0047}, {32, 64, 64, 1, 2, 4, 1.8, 1.7, 0.0092, 0.0085}, {32, 128, 16, 1, 4, 1, 1.0, 1.7, 0.027, 0.0174},
+    {64, 64, 32, 2, 2, 1, 2.15, 0.96, 0.0178, 0.0177}, {64, 128, 16, 2, 2, 1, 1.9, 1.4, 0.0395, 0.0313}};
+inline gathered_tile gathered_tile_for(long M, long N, long K) {
+    const gathered_tile *best = nullptr;
+    double best_cost = 0;
+    for (const gathered_tile &c : GATHERED_TILES) {
+        const long tiles = ((M + c.m - 1) / c.m) * ((N + c.n - 1) / c.n);
+        const double rounds = (double)((tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS), slope = rounds * c.further > c.first ? rounds * c.further : c.first;
+        const double cost = c.fixed + rounds * c.round + (double)K * slope;
+        if (!best || cost < best_cost) { best = &c; best_cost = cost; }
+    }
+    return *best;
+}
+
 // C tiles of the bf16-input kernels.  What the loops over K of a launch take is modelled as `fixed` microseconds (start, first
 // slices) plus, for every 32 k of whole stages, `first` for the first round of tiles over the compute units and `further` for
 // each round after it.  Reading and writing C is left out: it takes every tile about the same (1.07 us per million elements),

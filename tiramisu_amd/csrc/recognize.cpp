@@ -1376,6 +1376,21 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         }
     }
 
+    // short products with a gathered operand whose window is not staged: the tile that is modelled fastest (kernels/target_gfx950.h)
+    {
+        bool gathered = lit && !bf16 && !with_consumer && !batched && !windowed && operands.size() == 1 && WGK == 1 && Ml <= 64 && operands[0].first.linear &&
+                        !operands[0].second.linear;
+        for (const char *forced : {"TIRAMISU_MFMA_TILE", "TIRAMISU_MFMA_BM", "TIRAMISU_MFMA_BN", "TIRAMISU_MFMA_BK", "TIRAMISU_MFMA_WGM", "TIRAMISU_MFMA_WGN",
+                                   "TIRAMISU_MFMA_WGK", "TIRAMISU_MFMA_DEPTH", "TIRAMISU_MFMA_PAD", "TIRAMISU_MFMA_NO_SPLITK"})
+            if (backend_option(forced)) gathered = false;
+        if (gathered) {
+            const ttarget::gathered_tile t = ttarget::gathered_tile_for(Ml, Nl, Kl);
+            long v;
+            BM = t.m; BN = t.n; BK = t.k; WGM = t.waves_m; WGN = t.waves_n; WGK = t.groups;
+            edge = !(Ml % BM == 0 && Nl % BN == 0 && Kl % BK == 0 && literal_value(operands[0].first.ld, v) && v % 4 == 0 && multiple_of(operands[0].first.base, 4));
+        }
+    }
+
     // ---- kernel text
     c_printer dev;
     dev.fct = f;
