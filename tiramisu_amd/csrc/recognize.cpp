@@ -1171,6 +1171,37 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         // (4-layer LSTM cell, 64x2048x1024 per layer: 1.30 ms per pass against 1.55 ms)
         if ((long)products.size() * Kl >= 1024) { BK = 64; WGK = 4; DEPTH = 1; }
     }
+    // Several terms or a point-wise nest behind them (recurrent cells) on at most 64 rows: where tiles of 32x32 of all iterations of the parallel
+    // host loop are fewer than two for every compute unit, a launch is bound by the chain of one tile's slices and its tail, and four
+    // groups of wavefronts to a slice of 64 k, the next two in flight, shorten both (eight to one of 128 where the tile above has eight, never
+    // fewer partial sums: at 64 x 256, 40 steps, 274 us with eight, 262 with four).  LSTM passes with the tile above and so, us: 3 layers of
+    // 20 x 64, 4 steps 71, 56; 2 of 16 x 128, 10 steps 117, 83; 1 of 32 x 448, 12 steps 291, 116; 2 of 64 x 256, 40 steps 365, 274; 2 of 64 x 512,
+    // 12 steps 178, 134; 3 of them 191, 181; 4 of 48 x 480, 12 steps 384, 208; 4 of 64 x 384, 30 steps 378, 368.  4 of 64 x 512 are two tiles for
+    // every unit: 30 steps 424 with the tile above and 421 so, 100 steps 1286 and 1297, so there it stays.
+    bool cell = lit && !bf16 && BM == 64 && BN <= 64 && Ml <= 64 && (operands.size() > 1 || with_consumer);
+    for (auto &o : operands) cell = cell && o.first.linear && o.second.linear;
+    for (const char *forced : {"TIRAMISU_MFMA_TILE", "TIRAMISU_MFMA_BM", "TIRAMISU_MFMA_BN", "TIRAMISU_MFMA_BK", "TIRAMISU_MFMA_WGM", "TIRAMISU_MFMA_WGN",
+                               "TIRAMISU_MFMA_WGK", "TIRAMISU_MFMA_DEPTH", "TIRAMISU_MFMA_PAD", "TIRAMISU_MFMA_NO_SPLITK"})
+        if (backend_option(forced)) cell = false;
+    if (cell) {
+        // iterations of the host loop: the literal bounds of min(3, ...) and max(0, ...); where they say nothing, the tile above stays
+        std::function<bool(const expr &, op_t, long &)> bound = [&](const expr &e, op_t op, long &v) {
+            if (!e.is_defined()) return false;
+            if (literal_value(e, v)) return true;
+            if (e.get_expr_type() != e_op || e.get_op_type() != op || e.get_n_arg() != 2) return false;
+            long a, b;
+            const bool ha = bound(e.get_operand(0), op, a), hb = bound(e.get_operand(1), op, b);
+            v = ha && hb ? (op == o_min ? std::min(a, b) : std::max(a, b)) : ha ? a : b;
+            return ha || hb;
+        };
+        long first = 0, last = 0;
+        const bool known = !batched || (bound(fuse->batch_first, o_max, first) && bound(fuse->batch_last, o_min, last));
+        const long cells = std::max<long>(1, last - first + 1);
+        if (known && (Ml + 31) / 32 * ((Nl + 31) / 32) * cells < 2 * ttarget::COMPUTE_UNITS) {
+            const bool eight = WGK == 8;
+            BM = BN = 32; BK = eight ? 128 : 64; WGM = WGN = 1; WGK = eight ? 8 : 4; DEPTH = eight ? 1 : 2;
+        }
+    }
     // a plain product of few 64x64 tiles: smaller tiles whose groups of wavefronts share each slice, where they are modelled faster
     // (kernels/target_gfx950.h)
     bool plain = lit && !bf16 && !with_consumer && !batched && BM == 64 && BN == 64 && WGK == 1 && operands.size() == 1;
