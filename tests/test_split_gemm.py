@@ -216,6 +216,22 @@ def test_one_product_per_sum(rule, M, N, K, edge, tA, tB):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tA,tB", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(1000, 1500, 700), (446, 1497, 733), (1001, 1503, 703), (1344, 1024, 176)])
+def test_products_of_the_fp32_instruction_are_rounded_once(rule, M, N, K, tA, tB):
+    """Sizes whose fp32 tiles are 64 x 32 or 32 x 32: no square of the split operands has as many partial sums there, and six of nine partial
+    products would not do instead: one product alone, exact in 64 bits, comes out rounded to fp32 once, to nearest."""
+    assert rule.split_tile(M, N, K, True) == 0
+    rng = np.random.RandomState(K)
+    at = rng.permutation(M) % K
+    values, b = lone_operands(rng, "random", M, (K, N))
+    a = np.zeros((M, K), np.float32)
+    a[np.arange(M), at] = values
+    out = call(np.ascontiguousarray(a.T) if tA else a, np.ascontiguousarray(b.T) if tB else b, np.zeros((M, N), np.float32), M, N, K, 1.0, 0.0, tA, tB)
+    assert np.array_equal(out, (values[:, None].astype(np.float64) * b[at]).astype(np.float32))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [s[:3] for s in SIZES if s[0] != 1300])
 def test_program(M, N, K):
     name = "sgemm_%dx%dx%d" % (M, N, K)

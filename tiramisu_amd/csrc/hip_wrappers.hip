@@ -240,20 +240,14 @@ void launch_split(const float *A, const float *B, float *C, int M, int N, int K,
     }
     check(hipGetLastError(), "tiramisu_hip_sgemm");
 }
-template <bool AK, bool BK_, int BM, int BN>
-void launch_split_tile(const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc, float alpha, float beta) {
-    if (ttarget::split_whole(BM, BN, M, N, K))
-        launch_split<typename tgemm::split_config<BM, BN, AK, BK_, false>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    else
-        launch_split<typename tgemm::split_config<BM, BN, AK, BK_, true>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-}
 template <bool AK, bool BK_>
-void dispatch_split(ttarget::split_tile tile, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc, float alpha, float beta) {
-    if (tile.m == 64 && tile.n == 64) launch_split_tile<AK, BK_, 64, 64>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    else if (tile.m == 64) launch_split_tile<AK, BK_, 64, 96>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    else if (tile.m == 96) launch_split_tile<AK, BK_, 96, 64>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    else if (tile.m == 128) launch_split_tile<AK, BK_, 128, 128>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
-    else launch_split_tile<AK, BK_, 256, 256>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+void dispatch_split(int edge, const float *A, const float *B, float *C, int M, int N, int K, long lda, long ldb, long ldc, float alpha, float beta) {
+    const bool whole = ttarget::split_whole(edge, M, N, K);
+    if (edge == 64) launch_split<typename tgemm::split_config<64, AK, BK_, false>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else if (edge == 128 && whole) launch_split<typename tgemm::split_config<128, AK, BK_, false>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else if (edge == 128) launch_split<typename tgemm::split_config<128, AK, BK_, true>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else if (whole) launch_split<typename tgemm::split_config<256, AK, BK_, false>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
+    else launch_split<typename tgemm::split_config<256, AK, BK_, true>::type>(A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
 }
 
 // Few C tiles but a long reduction (a batch of 64 rows against wide weights, as in recurrent
@@ -430,7 +424,7 @@ void dispatch_edge(bool vec_ok, const float *A, const float *B, float *C, int M,
     const int problems = active_batch ? active_batch_count : 1;
     const ttarget::fp32_tiles t = ttarget::library_tiles_for(M, N, K, problems, vec_ok);
     if (lda >= 4 && lda < ttarget::SPLIT_LD_LIMIT && ldb >= 4 && ldb < ttarget::SPLIT_LD_LIMIT)
-        if (const ttarget::split_tile split = ttarget::any_split_tile_for(M, N, K, problems, t.m, t.n, t.guarded, AK && BK_ && (lda % 4 != 0 || ldb % 4 != 0)); split.m)
+        if (const int split = ttarget::split_tile_for(M, N, K, problems, t.m, t.n, t.guarded))
             return dispatch_split<AK, BK_>(split, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     if (t.m == 64 && t.n == 32) return launch_small<AK, BK_, 64, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);
     if (t.m == 32) return launch_small<AK, BK_, 32, 32>(vec_ok, A, B, C, M, N, K, lda, ldb, ldc, alpha, beta);

@@ -24,9 +24,6 @@
 // of NaN 1150 us, with operands of 2^60, whose every product overflows, 2030 (bound by the L2; 600 without, 960 with the fp32 instruction),
 // 1024^3 38 (18; 20).
 //
-// The small tiles hold one stage per wavefront (two until now: 1024^3 19.0 us, so 18.3); a product of 64 x 64 or 64 x 96 and the split before it take the issue slots
-// in turn: measured 17.5 ns for one v_mfma_f32_32x32x16_bf16 alone, 27 with the ten vector instructions that a product of 64 x 64 brings, 24 alone.
-//
 // What bounds it: at 4096^3 the power limit (596 to 625 us on random operands, machines differ, 470 on zeros; 948 to 964 with the fp32 instruction), on small tiles the
 // vector work of the split, seven instructions per element, each done once per tile (1024^3 17 to 19 us, 20.6 to 22.5 with the fp32 instruction).
 #ifndef TIRAMISU_AMD_GEMM_MFMA_SPLIT_HIP_H
@@ -274,7 +271,7 @@ struct config_split {
     static constexpr int LDS_BYTES = 2 * STAGE_FLOATS * 4;
     static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile must be made of 32x32 MFMA tiles");
     static_assert(BK == 16 * WGK, "one step per wavefront and slice");
-    static_assert(LDS_BYTES == ttarget::split_lds_bytes(BM, BN, A_KMAJOR, B_KMAJOR) && LDS_BYTES <= ttarget::LDS_BYTES_PER_CU, "two stages must fit");
+    static_assert(LDS_BYTES == ttarget::split_lds_bytes(BM, A_KMAJOR, B_KMAJOR) && LDS_BYTES <= ttarget::LDS_BYTES_PER_CU, "two stages must fit");
     static_assert(BK == ttarget::split_slice(BM), "slice");
     static_assert(WGK == 1 || (WGK - 1) * WGM * WGN * TM * TN * 16 * 64 <= 2 * STAGE_FLOATS, "LDS too small for the K reduction");
 };
@@ -387,23 +384,20 @@ __device__ __forceinline__ void tile_accumulate_split(accumulators<CFG> &acc, co
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
-// Small tiles (64 x 64, 64 x 96, 96 x 64): every wavefront of a workgroup multiplies the whole tile over its own k (slices of 16, dealt round
-// robin) and nothing is shared until the sums are added: no barrier in the loop, and every element is read from LDS and split once.
-template <int BM_, int BN_, bool A_KMAJOR_, bool B_KMAJOR_, bool EDGE_>
-struct config_small {
-    static constexpr int BM = BM_, BN = BN_, BK = 16, WAVES = 8;
-    static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_, EDGE = EDGE_;
+// 64 x 64 tiles (whole ones only): every wavefront of a workgroup multiplies the whole tile over its own k (slices of 16, dealt round robin) and
+// nothing is shared until the sums are added: no barrier in the loop, and every element is read from LDS and split once.
+template <bool A_KMAJOR_, bool B_KMAJOR_>
+struct config_waves {
+    static constexpr int BM = 64, BN = 64, BK = 16, WAVES = 8;
+    static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_, EDGE = false;
     static constexpr int NT = 64 * WAVES, TM = BM / 32, TN = BN / 32;
     static constexpr int A_WORDS = BM * BK + (A_KMAJOR ? 0 : 4 * BK), B_WORDS = BN * BK + (B_KMAJOR ? 0 : 4 * BK);
     static constexpr int WAVE_WORDS = A_WORDS + B_WORDS;
-    // the sums of all wavefronts where the LDS holds them, else of half of them at a time
-    static constexpr int SUMS_AT_ONCE = TM * TN > 4 ? WAVES / 2 : WAVES;
-    static constexpr int STAGING = WAVES * WAVE_WORDS * 4, SUMS = SUMS_AT_ONCE * TM * TN * 16 * 64 * 4;
+    static constexpr int STAGING = 2 * WAVES * WAVE_WORDS * 4, SUMS = WAVES * TM * TN * 16 * 64 * 4;
     static constexpr int LDS_BYTES = STAGING > SUMS ? STAGING : SUMS;
     static constexpr int QUADS = TM * TN * 4, SHARE = QUADS / WAVES;       // of four accumulator registers; those a wavefront finishes
-    static_assert(LDS_BYTES == ttarget::split_lds_bytes(BM, BN, A_KMAJOR, B_KMAJOR) && LDS_BYTES <= ttarget::LDS_BYTES_PER_CU, "a stage of every wavefront's slices");
+    static_assert(LDS_BYTES == ttarget::split_lds_bytes(BM, A_KMAJOR, B_KMAJOR), "two stages of every wavefront's slices");
 };
-template <bool A_KMAJOR, bool B_KMAJOR> using config_waves = config_small<64, 64, A_KMAJOR, B_KMAJOR, false>;
 
 // Between the accesses of a wavefront's lanes to LDS that only they use: what was written or read before is done for what is written or
 // read behind.  The LDS executes a wavefront's accesses in order, so this holds the compiler alone and is no instruction.
@@ -434,22 +428,21 @@ struct wave_operand {
             at[v] = src.place(x0, x, k);
         }
     }
-    template <class SRC, class LAST>
-    static __device__ __forceinline__ void load(const SRC &src, int x0, int k0, const uint32_t (&at)[NV], f32x4 (&regs)[NV], LAST last) {
+    template <class SRC>
+    static __device__ __forceinline__ void load(const SRC &src, int x0, int k0, const uint32_t (&at)[NV], f32x4 (&regs)[NV]) {
 #pragma unroll
         for (int v = 0; v < NV; v++) {
             int x, k;
             unit((threadIdx.x & 63) + 64 * v, x, k);
-            regs[v] = src.load(x0, x, k0, k, 0, at[v], last);
+            regs[v] = src.load(x0, x, k0, k, 0, at[v], std::false_type());
         }
     }
-    template <class SRC, class LAST>
-    static __device__ __forceinline__ void store(uint32_t *lds, const f32x4 (&regs)[NV], const SRC &src, int x0, int k0, LAST last) {
+    static __device__ __forceinline__ void store(uint32_t *lds, const f32x4 (&regs)[NV]) {
 #pragma unroll
         for (int v = 0; v < NV; v++) {
             int x, k;
             unit((threadIdx.x & 63) + 64 * v, x, k);
-            *reinterpret_cast<f32x4 *>(lds + word(x, k)) = src.finish(regs[v], x0 + x, k0 + k, last);
+            *reinterpret_cast<f32x4 *>(lds + word(x, k)) = regs[v];
         }
     }
     // the eight k of a lane's row
@@ -482,72 +475,58 @@ __device__ __forceinline__ void split_eight(const split_constants &sc, const flo
     for (int s = 0; s < 3; s++) out[s] = __builtin_bit_cast(split_x8, split_u4{w[s][0], w[s][1], w[s][2], w[s][3]});
 }
 
-// acc += the wavefront's share of A(m0.., :) * B(:, n0..) over K
+// acc += the wavefront's share of A(m0.., :) * B(:, n0..) over K, whole tiles and slices
 template <class CFG, class SRCA, class SRCB>
 __device__ __forceinline__ void tile_accumulate_waves(accumulators<CFG> &acc, const SRCA &A, const SRCB &B, int M, int N, int K, int m0, int n0, float *lds_) {
     typedef wave_operand<CFG::BM, CFG::A_KMAJOR> opA;
     typedef wave_operand<CFG::BN, CFG::B_KMAJOR> opB;
-    constexpr int TM = CFG::TM, TN = CFG::TN, W = CFG::WAVES, BK = CFG::BK, T = TM * TN, BLOCKS = TM + TN;
-    static_assert(TM >= 2 && TN >= 2 && BLOCKS <= T && (BLOCKS < T || T % 2 == 0), "a product for every block that is split, and its elements read into the other registers");
+    constexpr int TM = CFG::TM, TN = CFG::TN, W = CFG::WAVES, BK = CFG::BK, T = TM * TN;
+    static_assert(TM == 2 && TN == 2, "four tile products");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, h = lane >> 5;
-    // One stage of the wavefront's own: the LDS executes its accesses in order, so a slice may be stored as soon as the last read of the
-    // one before it has been issued.
-    uint32_t *lds = reinterpret_cast<uint32_t *>(lds_) + wave * CFG::WAVE_WORDS;
-    const int KT = (K + BK - 1) / BK;
+    uint32_t *lds = reinterpret_cast<uint32_t *>(lds_) + 2 * wave * CFG::WAVE_WORDS;      // two stages of the wavefront's own
+    const int KT = K / BK;
     const int mine = KT > wave ? (KT - wave + W - 1) / W : 0;     // the wavefront's slices: wave, wave + W, ...
     f32x4 ra[opA::NV], rb[opB::NV];
     uint32_t ata[opA::NV], atb[opB::NV];
     opA::place(A, m0, ata);
     opB::place(B, n0, atb);
     const split_constants sc;
-    // Guarded tiles: the wavefront's last slice comes first, which may hold the last k; behind the last number the first slice of K
-    // again.  Whole ones: in order, and the last slice again (see tile_accumulate_split).
-    auto slice_of = [&](int n) -> int { return !CFG::EDGE ? wave + min(n, mine - 1) * W : n == 0 ? wave + (mine - 1) * W : n < mine ? wave + (n - 1) * W : 0; };
-    auto load = [&](int n, auto last) {
-        const int s = slice_of(n);
-        opA::load(A, m0, s * BK, ata, ra, last);
-        opB::load(B, n0, s * BK, atb, rb, last);
+    // (behind its end the wavefront's last slice again: see tile_accumulate_split)
+    auto load = [&](int n) {
+        const int s = wave + min(n, mine - 1) * W;
+        opA::load(A, m0, s * BK, ata, ra);
+        opB::load(B, n0, s * BK, atb, rb);
     };
-    auto store = [&](int n, auto last) {
-        const int s = slice_of(n);
+    auto store = [&](int stage) {
         wave_lds_in_order();                 // the lanes have read what the stage held
-        opA::store(lds, ra, A, m0, s * BK, last);
-        opB::store(lds + CFG::A_WORDS, rb, B, n0, s * BK, last);
+        opA::store(lds + stage * CFG::WAVE_WORDS, ra);
+        opB::store(lds + stage * CFG::WAVE_WORDS + CFG::A_WORDS, rb);
         wave_lds_in_order();                 // the lanes read what the others stored
     };
-    typedef std::true_type yes;
-    typedef std::false_type no;
-    // A slice is T tile products, row by row; while the matrix cores work on one, the vector ALUs split the block of 32 rows or columns that
-    // a later one needs, requested from LDS one product earlier: column blocks 1 .., row blocks 1 .., then the first row and column
-    // block of the next slice.  Block number b of that order is split during product b.
-    auto read_block = [&](int b, float (&to)[8]) {
-        if (b < TN - 1) opB::read(lds + CFG::A_WORDS, (b + 1) * 32 + l32, h, to);
-        else if (b < BLOCKS - 2) opA::read(lds, (b - TN + 2) * 32 + l32, h, to);
-        else if (b == BLOCKS - 2) opA::read(lds, l32, h, to);
-        else opB::read(lds + CFG::A_WORDS, l32, h, to);
+    // A slice is four tile products; while the matrix cores work on one, the vector ALUs split the block of 32 rows or columns that
+    // the next one needs, requested from LDS one product earlier: column block 1, row block 1, then the first row and
+    // column block of the next slice.
+    auto read_block = [&](int block, int stage, float (&to)[8]) {       // row blocks 0, 1, column blocks 2, 3
+        const uint32_t *la = lds + stage * CFG::WAVE_WORDS;
+        if (block < TM) opA::read(la, block * 32 + l32, h, to);
+        else opB::read(la + CFG::A_WORDS, (block - TM) * 32 + l32, h, to);
     };
     split_x8 fa[TM][3], fb[TN][3];
-    float e[2][8];                           // elements on the way from LDS, by the parity of the block
-    auto slice = [&](int n) {                // slice n is multiplied, n + 1 stored, n + 2 loaded
+    float e[2][8];                           // elements on the way from LDS, by the parity of the tile product that splits them
+    auto slice = [&](int stage) {
         split_x8 na[3], nb[3];
 #pragma unroll
         for (int t = 0; t < T; t++) {
             const int i = t / TN, j = t % TN;
-            if (t + 1 < BLOCKS) {
-                if (t + 1 == BLOCKS - 2) {
-                    store(n + 1, no());
-                    load(n + 2, no());
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                read_block(t + 1, e[(t + 1) & 1]);
-            } else if (t + 1 == T) {
-                read_block(0, e[0]);         // (of the next slice)
-            }
-            if (t < TN - 1) split_eight(sc, e[t & 1], fb[t + 1]);
-            else if (t < BLOCKS - 2) split_eight(sc, e[t & 1], fa[t - TN + 2]);
-            else if (t == BLOCKS - 2) split_eight(sc, e[t & 1], na);
-            else if (t == BLOCKS - 1) split_eight(sc, e[t & 1], nb);
+            if (t == 0) read_block(1, stage, e[1]);
+            else if (t == 1) read_block(0, stage ^ 1, e[0]);
+            else if (t == 2) read_block(2, stage ^ 1, e[1]);
+            else read_block(3, stage ^ 1, e[0]);
+            if (t == 0) split_eight(sc, e[0], fb[1]);
+            else if (t == 1) split_eight(sc, e[1], fa[1]);
+            else if (t == 2) split_eight(sc, e[0], na);
+            else split_eight(sc, e[1], nb);
 #pragma unroll
             for (int c = 0; c < 6; c++) acc.t[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][SPLIT_A[c]], fb[j][SPLIT_B[c]], acc.t[i][j], 0, 0, 0);
 #pragma unroll
@@ -562,54 +541,41 @@ __device__ __forceinline__ void tile_accumulate_waves(accumulators<CFG> &acc, co
         for (int p = 0; p < 3; p++) { fa[0][p] = na[p]; fb[0][p] = nb[p]; }
     };
     if (mine > 0) {
-        load(0, yes());
-        store(0, yes());
-        load(1, no());
+        load(0);
+        store(0);
+        load(1);
         float e0[8], e1[8];
-        read_block(BLOCKS - 2, e0);
-        read_block(BLOCKS - 1, e1);
-        read_block(0, e[0]);
+        read_block(0, 0, e0);
+        read_block(TM, 0, e1);
+        read_block(TM + 1, 0, e[0]);
         split_eight(sc, e0, fa[0]);
         split_eight(sc, e1, fb[0]);
-        for (int n = 0; n < mine; n += 2) {  // (in pairs: the next slice's parts need not be moved)
-            slice(n);
-            if (n + 1 < mine) slice(n + 1);
+        for (int b = 0; b < mine; b += 2) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                if (b + u >= mine) break;
+                store(u ^ 1);
+                load(b + u + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                slice(u);
+            }
         }
     }
     if (__any(unscale(acc, M, N, m0, n0))) recompute_fp32(acc, A, B, K, m0, n0, wave, W, 0);
 }
 
-// The sums of the wavefronts, added in their order (of tiles whose sums the LDS does not hold at once: of wavefronts w and w + 4 first); each
-// finishes its SHARE of the tile's quads.  value and store as in tile_epilogue.
+// The sums of the wavefronts, added in their order; each finishes its SHARE of the tile's quads.  value and store as in tile_epilogue.
 template <class CFG, class VALUE, class STORE>
-__device__ __forceinline__ void tile_finish_waves(accumulators<CFG> &acc, int M, int N, int m0, int n0, float *lds, VALUE value, STORE store) {
-    constexpr int W = CFG::SUMS_AT_ONCE, Q = CFG::QUADS, SHARE = CFG::SHARE;
+__device__ __forceinline__ void tile_finish_waves(const accumulators<CFG> &acc, int m0, int n0, float *lds, VALUE value, STORE store) {
+    constexpr int W = CFG::WAVES, Q = CFG::QUADS, SHARE = CFG::SHARE;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, h = lane >> 5;
     f32x4 *slots = reinterpret_cast<f32x4 *>(lds);
-    auto write = [&](int w) {
-#pragma unroll
-        for (int q = 0; q < Q; q++) {
-            const f32x16 &t = acc.t[q / 4 / CFG::TN][q / 4 % CFG::TN];
-            slots[(w * Q + q) * 64 + lane] = f32x4{t[4 * (q % 4)], t[4 * (q % 4) + 1], t[4 * (q % 4) + 2], t[4 * (q % 4) + 3]};
-        }
-    };
     __syncthreads();                         // every wavefront has read its slices
-    if (W < CFG::WAVES) {
-        if (wave >= W) write(wave - W);
-        __syncthreads();
-        if (wave < W) {
 #pragma unroll
-            for (int q = 0; q < Q; q++) {
-                const f32x4 v = slots[(wave * Q + q) * 64 + lane];
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc.t[q / 4 / CFG::TN][q / 4 % CFG::TN][4 * (q % 4) + e] += v[e];
-            }
-            wave_lds_in_order();             // a wavefront writes where it has read
-            write(wave);
-        }
-    } else {
-        write(wave);
+    for (int q = 0; q < Q; q++) {
+        const f32x16 &t = acc.t[q / 4 / CFG::TN][q / 4 % CFG::TN];
+        slots[(wave * Q + q) * 64 + lane] = f32x4{t[4 * (q % 4)], t[4 * (q % 4) + 1], t[4 * (q % 4) + 2], t[4 * (q % 4) + 3]};
     }
     __syncthreads();
     f32x4 sum[SHARE];
@@ -627,16 +593,16 @@ __device__ __forceinline__ void tile_finish_waves(accumulators<CFG> &acc, int M,
             for (int e = 0; e < 4; e++) {
                 const int q = wave * SHARE + c;
                 const int row = m0 + (q / 4 / CFG::TN) * 32 + 8 * (q % 4) + 4 * h + e, col = n0 + (q / 4 % CFG::TN) * 32 + l32;
-                if (CFG::EDGE && (row >= M || col >= N)) continue;
                 if (pass == 0) sum[c][e] = value(row, col, sum[c][e]);
                 else store(row, col, sum[c][e]);
             }
 }
 
 // ---- a tile from the first load to the last store.  The tiles that are used, whichever of the two kinds they are:
-template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, bool GUARDED> struct split_config { typedef config_small<BM, BN, A_KMAJOR, B_KMAJOR, GUARDED> type; };
-template <bool AK, bool BK_, bool G> struct split_config<256, 256, AK, BK_, G> { typedef config_split<256, 256, 16, 2, 4, AK, BK_, G, 1, false> type; };
-template <bool AK, bool BK_, bool G> struct split_config<128, 128, AK, BK_, G> { typedef config_split<128, 128, 32, 2, 2, AK, BK_, G, 2, true> type; };
+template <int EDGE_LENGTH, bool A_KMAJOR, bool B_KMAJOR, bool GUARDED> struct split_config;
+template <bool AK, bool BK_, bool G> struct split_config<256, AK, BK_, G> { typedef config_split<256, 256, 16, 2, 4, AK, BK_, G, 1, false> type; };
+template <bool AK, bool BK_, bool G> struct split_config<128, AK, BK_, G> { typedef config_split<128, 128, 32, 2, 2, AK, BK_, G, 2, true> type; };
+template <bool AK, bool BK_> struct split_config<64, AK, BK_, false> { typedef config_waves<AK, BK_> type; };
 
 template <class CFG, class VALUE, class STORE>
 __device__ __forceinline__ void split_mainloop(const float *__restrict__ A, long lda, const float *__restrict__ B, long ldb, int M, int N, int K, int m0, int n0,
@@ -645,9 +611,9 @@ __device__ __forceinline__ void split_mainloop(const float *__restrict__ A, long
     acc.clear();
     const split_source<CFG::A_KMAJOR, CFG::EDGE> sa{A, lda, M, K};
     const split_source<CFG::B_KMAJOR, CFG::EDGE> sb{B, ldb, N, K};
-    if constexpr (CFG::BM < 128) {
+    if constexpr (CFG::BM == 64) {
         tile_accumulate_waves<CFG>(acc, sa, sb, M, N, K, m0, n0, lds);
-        tile_finish_waves<CFG>(acc, M, N, m0, n0, lds, value, store);
+        tile_finish_waves<CFG>(acc, m0, n0, lds, value, store);
     } else {
         tile_accumulate_split<CFG>(acc, sa, sb, M, N, K, m0, n0, lds);
         if (tile_reduce_k<CFG>(acc, lds)) tile_epilogue<CFG>(acc, M, N, m0, n0, value, store);

@@ -102,19 +102,17 @@ inline double modelled(const launch_model &l, long M, long N, long K, long probl
     const double more = (double)((tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS - 1);
     return l.fixed + more * l.round + K * (l.first + more * l.further);
 }
-// k of a slice; LDS of a workgroup: two stages of three planes, or a slice of each of eight wavefronts and afterwards their sums (all
-// at once, or those of four where a tile has six accumulators)
+// k of a slice; LDS of a workgroup (two stages of three planes, or of eight wavefronts' own slices)
 constexpr int split_slice(int edge) { return edge == 128 ? 32 : 16; }
 constexpr int split_operand_words(int edge, bool kmajor) {
-    return edge < 128 ? edge * 16 + (kmajor ? 0 : 64) : 3 * (split_slice(edge) / 8) * 4 * (kmajor ? edge + 128 / split_slice(edge) : edge + 16);
+    return edge == 64 ? 64 * 16 + (kmajor ? 0 : 64) : 3 * (split_slice(edge) / 8) * 4 * (kmajor ? edge + 128 / split_slice(edge) : edge + 16);
 }
-constexpr int split_lds_bytes(int m, int n, bool a_kmajor, bool b_kmajor) {
-    const int stage = split_operand_words(m, a_kmajor) + split_operand_words(n, b_kmajor), sums = (m * n > 64 * 64 ? 4 : 8) * m * n;
-    return 4 * (m >= 128 ? 2 * stage : 8 * stage > sums ? 8 * stage : sums);
+constexpr int split_lds_bytes(int edge, bool a_kmajor, bool b_kmajor) {
+    return 2 * 4 * (edge == 64 ? 8 : 1) * (split_operand_words(edge, a_kmajor) + split_operand_words(edge, b_kmajor));
 }
 // leading dimensions: four elements of a row at least, offsets within a tile in 32 bits
 constexpr long SPLIT_LD_LIMIT = 1L << 22;
-constexpr bool split_whole(int m, int n, long M, long N, long K) { return M % m == 0 && N % n == 0 && K % split_slice(m) == 0; }
+constexpr bool split_whole(int edge, long M, long N, long K) { return M % edge == 0 && N % edge == 0 && K % split_slice(edge) == 0; }
 // ... of a workgroup of the windowed convolution on split operands (gemm_mfma_window_split.hip.h): three planes of 16-byte granules
 constexpr long window_split_lds_bytes(long rows, long taps, long window) { return 3 * 16 * (rows * (taps | 1) + 1 + window); }
 // The edge of the split tile that takes an M x N x K product from fp32 tiles of m x n (guarded or not), 0: none.  Where the fp32
@@ -128,45 +126,11 @@ inline int split_tile_for(long M, long N, long K, long problems, int m, int n, b
         if (l.m == m && l.n == n && l.guarded == guarded) best = 0.95 * modelled(l, M, N, K, problems);
     int edge = 0;
     for (const launch_model &l : SPLIT_LAUNCHES) {
-        if (l.guarded == split_whole(l.m, l.n, M, N, K) || (n == 32 && l.m != 64)) continue;
+        if (l.guarded == split_whole(l.m, M, N, K) || (n == 32 && l.m != 64)) continue;
         const double cost = modelled(l, M, N, K, problems);
         if (cost < best) { best = cost; edge = l.m; }
     }
     return edge;
-}
-
-// The tiles whose wavefronts each multiply all of it (config_small), beyond the whole 64 x 64 ones above: guarded, and half as long again on
-// one side, which needs a fifth less vector work per product and often fits the chip where squares do not.  Eight partial sums, at least as
-// many as any fp32 tile has.  us measured with what a launch took before / with these: 1000 x 1500 x 700 (A transposed) 28.1 (752 tiles of 64 x 32
-// in three rounds) / 20.9 (256 of 64 x 96); 64 x 64 guarded takes 27.5 there, 128 x 128 32.5.  Fitted to 78 sizes of 64 ... 4096
-// rows and columns, 96 ... 4096 k (rms error 4 %).  They have to be better by a tenth: closer than that, launches of few k came out up to 12 %
-// slower (161 x 2725 x 253 7.9 / 8.9).  Where both operands lie along k in rows that are no multiples of 16 bytes (`split_rows`), the 64
-// bytes of a row that a load takes lie in two lines more often than the fp32 tiles' 256: there by 28 % (737 x 894 x 2361 36.8 / 36.1,
-// in the other three layouts 49 / 36; 1443 x 421 x 3347 50.6 / 52.0 and 71 / 53).
-constexpr launch_model SMALL_SPLIT_LAUNCHES[] = {
-    {64, 64, true, 6.6, 4.8, 0.0102, 0.0149}, {64, 96, false, 6.6, 4.2, 0.0145, 0.0190}, {96, 64, false, 6.6, 4.2, 0.0145, 0.0190},
-    {64, 96, true, 8.5, 6.7, 0.0139, 0.0196}, {96, 64, true, 8.5, 6.6, 0.0139, 0.0196}};
-struct split_tile { int m, n; };
-inline split_tile any_split_tile_for(long M, long N, long K, long problems, int m, int n, bool guarded, bool split_rows) {
-    if (M < 64 || N < 64 || K < 96) return {0, 0};
-    const int edge = split_tile_for(M, N, K, problems, m, n, guarded);
-    split_tile tile = {edge, edge};
-    double best = 0;
-    if (edge) {
-        for (const launch_model &l : SPLIT_LAUNCHES)
-            if (l.m == edge && l.guarded != split_whole(edge, edge, M, N, K)) best = modelled(l, M, N, K, problems);
-    } else {
-        for (const launch_model &l : FP32_LAUNCHES)
-            if (l.m == m && l.n == n && l.guarded == guarded) best = 0.95 * modelled(l, M, N, K, problems);
-    }
-    const double limit = (split_rows ? 0.7 : 0.9) * best;
-    double chosen = 0;
-    for (const launch_model &l : SMALL_SPLIT_LAUNCHES) {
-        if (l.guarded == split_whole(l.m, l.n, M, N, K)) continue;
-        const double cost = modelled(l, M, N, K, problems);
-        if (cost < limit && (chosen == 0 || cost < chosen)) { chosen = cost; tile = {l.m, l.n}; }
-    }
-    return tile;
 }
 
 // C tiles of a product with a gathered operand and at most 64 rows (an implicit GEMM: a convolution whose window is not staged in LDS; fp32

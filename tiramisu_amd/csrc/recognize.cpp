@@ -1279,28 +1279,24 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
 
     // a plain product whose operands are better split into bf16 parts (kernels/gemm_mfma_split.hip.h): whole tiles there need no
     // alignment.  Options that shape a tile keep the fp32 instruction, as TIRAMISU_MFMA_NO_SPLIT_OPERANDS does.
-    ttarget::split_tile split = {0, 0};
+    int split_edge = 0;
     {
         bool may = lit && !bf16 && !with_consumer && !batched && operands.size() == 1 && !backend_option("TIRAMISU_MFMA_NO_SPLIT_OPERANDS");
         for (const char *forced : {"TIRAMISU_MFMA_TILE", "TIRAMISU_MFMA_BM", "TIRAMISU_MFMA_BN", "TIRAMISU_MFMA_BK", "TIRAMISU_MFMA_WGM", "TIRAMISU_MFMA_WGN",
                                    "TIRAMISU_MFMA_WGK", "TIRAMISU_MFMA_DEPTH", "TIRAMISU_MFMA_PAD", "TIRAMISU_MFMA_NO_SPLITK"})
             if (backend_option(forced)) may = false;
-        bool along_k = true, split_rows = false;
         for (auto &o : operands)
             for (const operand_info *g : {&o.first, &o.second}) {
-                long v = 0;
+                long v;
                 may = may && g->linear && literal_value(g->ld, v) && v >= 4 && v < ttarget::SPLIT_LD_LIMIT;
-                along_k = along_k && g->kmajor;
-                split_rows = split_rows || v % 4 != 0;
             }
-        if (may) split = ttarget::any_split_tile_for(Ml, Nl, Kl, 1, BM, BN, edge, along_k && split_rows);
-        if (split.m) {
-            BM = split.m;
-            BN = split.n;
-            BK = split.m < 128 ? 64 : ttarget::split_slice(split.m);     // (of small tiles four wavefronts take 16 k each, in turn with the other four)
+        if (may) split_edge = ttarget::split_tile_for(Ml, Nl, Kl, 1, BM, BN, edge);
+        if (split_edge) {
+            BM = BN = split_edge;
+            BK = split_edge == 64 ? 64 : ttarget::split_slice(split_edge);     // (of 64 x 64 tiles four wavefronts take 16 k each, in turn with the other four)
             WGM = WGK = 1;
             WGN = 8;                          // (512 threads)
-            edge = !ttarget::split_whole(split.m, split.n, Ml, Nl, Kl);
+            edge = !ttarget::split_whole(split_edge, Ml, Nl, Kl);
         }
     }
 
@@ -1613,13 +1609,13 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     } else {
         body << "    extern __shared__ __attribute__((aligned(16))) float _lds[];\n";
         if (win_split) body << "    typedef tgemm::config_window<" << BM << ", " << BN << ", " << WGM << ", " << WGN << "> CFG;\n";
-        else if (split.m) body << "    typedef tgemm::split_config<" << split.m << ", " << split.n << ", " << (operands[0].first.kmajor ? "true" : "false") << ", " << (operands[0].second.kmajor ? "true" : "false")
+        else if (split_edge) body << "    typedef tgemm::split_config<" << split_edge << ", " << (operands[0].first.kmajor ? "true" : "false") << ", " << (operands[0].second.kmajor ? "true" : "false")
                              << ", " << (edge ? "true" : "false") << ">::type CFG;\n";
         else body << "    typedef " << cfg << " CFG;\n";
     }
     body << "    const int _M = " << dev.print(Me) << ", _N = " << dev.print(Ne) << ", _K = " << dev.print(Ke) << ";\n";
     body << "    int _tm, _tn;\n    tgemm::tile_of_block((_M + CFG::BM - 1) / CFG::BM, (_N + CFG::BN - 1) / CFG::BN, _tm, _tn);\n";
-    if (!split.m && !win_split) body << "    tgemm::accumulators<CFG> _acc;\n    _acc.clear();\n" << consumer_loads_text.str();
+    if (!split_edge && !win_split) body << "    tgemm::accumulators<CFG> _acc;\n    _acc.clear();\n" << consumer_loads_text.str();
     int term = 0, ktab_words = 0;
     std::string split_call_head;
     const std::string kname = "_kernel_" + std::to_string(ctx.next_kernel_id());
@@ -1643,7 +1639,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
             term++;
             continue;
         }
-        if (split.m) {
+        if (split_edge) {
             used_buffers.insert(o.first.buf->get_name());
             used_buffers.insert(o.second.buf->get_name());
             split_call_head = "    tgemm::split_mainloop<CFG>(" + o.first.buf->get_name() + " + (" + dev.print(o.first.base) + "), " + dev.print(o.first.ld) + ", " +
@@ -1811,7 +1807,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     const std::string epi_args = two_pass ? "_epi_value, _epi_store" : "_epi";
     if (windowed) {
         body << window_call_head << (two_pass || !win_split ? epi_args : "[](int, int, float _sum) { return _sum; }, _epi") << ");\n";
-    } else if (split.m) {
+    } else if (split_edge) {
         body << split_call_head << (two_pass ? epi_args : "[](int, int, float _sum) { return _sum; }, _epi") << ");\n";
     } else {
         if (WGK > 1) body << "    if (tgemm::tile_reduce_k<CFG>(_acc, _lds))\n    ";
@@ -1824,7 +1820,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     k.name = kname;
     bool any_gather = false;
     for (auto &o : operands) any_gather = any_gather || !o.first.linear || !o.second.linear;
-    k.how = std::string("mfma-contraction: ") + (bf16 ? (bf16_direct ? "v_mfma_f32_32x32x16_bf16, slices loaded straight into LDS (through registers where an operand begins at an odd element), " : "v_mfma_f32_32x32x16_bf16, ") : split.m || win_split ? "v_mfma_f32_32x32x16_bf16 on the three bf16 parts of every fp32 operand element, " : "v_mfma_f32_32x32x2_f32, ") + (windowed ? "implicit GEMM, sliding window of " + std::to_string(win_taps) + " taps staged in LDS by blocks of " + std::to_string(win_cb) + " channels, " :
+    k.how = std::string("mfma-contraction: ") + (bf16 ? (bf16_direct ? "v_mfma_f32_32x32x16_bf16, slices loaded straight into LDS (through registers where an operand begins at an odd element), " : "v_mfma_f32_32x32x16_bf16, ") : split_edge || win_split ? "v_mfma_f32_32x32x16_bf16 on the three bf16 parts of every fp32 operand element, " : "v_mfma_f32_32x32x2_f32, ") + (windowed ? "implicit GEMM, sliding window of " + std::to_string(win_taps) + " taps staged in LDS by blocks of " + std::to_string(win_cb) + " channels, " :
                                                                                       any_gather ? "implicit GEMM (gathered operand), " : "") + "M " +
             std::to_string(Mg.size()) + " dim(s) x N " + std::to_string(Ng.size()) + " x K " + std::to_string(Kg.size()) + ", tile " +
             std::to_string(BM) + "x" + std::to_string(BN) + "x" + std::to_string(BK / bf16_slices) + (edge ? ", guarded edges" : ", whole tiles") + (bf16_slices > 1 ? ", slices in pairs, " : ", ") +
@@ -1905,7 +1901,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         const int rowA = operands[0].first.kmajor ? (BK / 4) * (BM + PADX) * 4 : BK * BM;
         const int rowB = operands[0].second.kmajor ? (BK / 4) * (BN + PADX) * 4 : BK * BN;
         k.lds_bytes = std::to_string(2 * (rowA + rowB) * 4);
-        if (split.m) k.lds_bytes = std::to_string(ttarget::split_lds_bytes(split.m, split.n, operands[0].first.kmajor, operands[0].second.kmajor));
+        if (split_edge) k.lds_bytes = std::to_string(ttarget::split_lds_bytes(split_edge, operands[0].first.kmajor, operands[0].second.kmajor));
         else if (bf16) k.lds_bytes = std::to_string(bf16_stages * (BK / 8) * (BM + BN) * 4 * 4);
         else if (ktab_words) k.lds_bytes = std::to_string(2 * (rowA + rowB) * 4 + ktab_words * 4);
         if (with_consumer) k.lds_bytes = std::to_string(std::stol(k.lds_bytes) + BM * (BN + 1) * 4);
@@ -1954,7 +1950,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     add_include_once(ctx, "#include \"gemm_mfma.hip.h\"");
     if (bf16) add_include_once(ctx, "#include \"gemm_mfma_bf16.hip.h\"");
     if (windowed) add_include_once(ctx, win_split ? "#include \"gemm_mfma_window_split.hip.h\"" : "#include \"gemm_mfma_window.hip.h\"");
-    if (split.m) add_include_once(ctx, "#include \"gemm_mfma_split.hip.h\"");
+    if (split_edge) add_include_once(ctx, "#include \"gemm_mfma_split.hip.h\"");
     if (bf16_direct) {
         host << "        if ((" << addresses << ") % 4 == 0) {\n" << launch_text(k, "            ") << "        } else {\n"
              << launch_text(unaligned, "            ") << "        }\n    }\n";
