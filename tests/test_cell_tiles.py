@@ -31,3 +31,25 @@ def test_gpu(s, programs_dir):
     runtime.load(programs_dir, name_of(s))(*[q.buffer() for q in d])
     y, expected = d[3].download(), ref.lstm(w, b, x)
     assert np.max(np.abs(y - expected)) <= RTOL * np.max(np.abs(expected))
+
+
+GROUPS = [((64, 32, 16, 96), "tile 64x64x32"), ((64, 128, 4, 96), "tile 32x32x64")]
+
+
+@pytest.mark.parametrize("s,tile", GROUPS)
+def test_column_groups_stay_in_one_launch(s, tile, programs_dir):
+    """A product and the nest that adds its column groups are one kernel, also where tiles of 32 columns hold too few units of them."""
+    kernels = json.load(open(os.path.join(programs_dir, "build", "column_groups_%dx%dx%dx%d.o.json" % s)))["kernels"]
+    assert len(kernels) == 1 and tile in kernels[0]["how"] and "(%d column group(s) per unit, 1 temporaries kept in registers)" % s[2] in kernels[0]["how"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("s", [g[0] for g in GROUPS])
+def test_gpu_column_groups(s, programs_dir):
+    from gpu_util import DeviceArray
+    M, H, G, K = s
+    rng = np.random.RandomState(G)
+    a, w = rng.randint(-4, 5, (M, K)).astype(np.float32), rng.randint(-4, 5, (K, G * H)).astype(np.float32)
+    d = [DeviceArray(v) for v in (a, w, np.full((M, H), np.nan, np.float32))]
+    runtime.load(programs_dir, "column_groups_%dx%dx%dx%d" % s)(*[q.buffer() for q in d])
+    assert np.array_equal(d[2].download(), (a @ w).reshape(M, G, H).sum(1))

@@ -1149,6 +1149,14 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
             name_outer_dims(X);
         }
     }
+    // a consumer needs tiles that hold all column groups of their units: how many units a tile of `columns` holds, 0 where it cannot
+    auto units_of_tile = [&](int columns) -> int {
+        const int units = columns / G;
+        if (columns % G != 0 || units == 0 || UE % units != 0 || Nl % columns != 0) return 0;
+        for (auto &o : operands)
+            if (!o.second.linear || (!o.second.kmajor && units % 4 != 0)) return 0;
+        return units;
+    };
     int BM = 64, BN = 64, BK = 16, PADX = 1, WGM = 2, WGN = 2, WGK = 1, DEPTH = 1;
     if (lit) {
         if (Ml <= 64 && Nl >= 256 * 256) { BM = 64; BN = 256; WGM = 1; WGN = 4; }   // short, very wide (convolutions)
@@ -1178,7 +1186,9 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     // 20 x 64, 4 steps 71, 56; 2 of 16 x 128, 10 steps 117, 83; 1 of 32 x 448, 12 steps 291, 116; 2 of 64 x 256, 40 steps 365, 274; 2 of 64 x 512,
     // 12 steps 178, 134; 3 of them 191, 181; 4 of 48 x 480, 12 steps 384, 208; 4 of 64 x 384, 30 steps 378, 368.  4 of 64 x 512 are two tiles for
     // every unit: 30 steps 424 with the tile above and 421 so, 100 steps 1286 and 1297, so there it stays.
-    bool cell = lit && !bf16 && BM == 64 && BN <= 64 && Ml <= 64 && (operands.size() > 1 || with_consumer);
+    // (Tiles that hold no whole units of the consumer are not taken: sixteen groups of columns that W holds side by side are four units to 64
+    // columns, but two to 32, and its loads take four.)
+    bool cell = lit && !bf16 && BM == 64 && BN <= 64 && Ml <= 64 && (with_consumer ? units_of_tile(32) > 0 : operands.size() > 1);
     for (auto &o : operands) cell = cell && o.first.linear && o.second.linear;
     for (const char *forced : {"TIRAMISU_MFMA_TILE", "TIRAMISU_MFMA_BM", "TIRAMISU_MFMA_BN", "TIRAMISU_MFMA_BK", "TIRAMISU_MFMA_WGM", "TIRAMISU_MFMA_WGN",
                                "TIRAMISU_MFMA_WGK", "TIRAMISU_MFMA_DEPTH", "TIRAMISU_MFMA_PAD", "TIRAMISU_MFMA_NO_SPLITK"})
@@ -1300,14 +1310,8 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         }
     }
 
-    // a consumer needs tiles that hold all column groups of their units
-    int UB = 0;
-    if (with_consumer) {
-        UB = BN / G;
-        if (BN % G != 0 || UB == 0 || UE % UB != 0 || Nl % BN != 0) return reject(35);
-        for (auto &o : operands)
-            if (!o.second.linear || (!o.second.kmajor && UB % 4 != 0)) return reject(35);
-    }
+    const int UB = with_consumer ? units_of_tile(BN) : 0;
+    if (with_consumer && UB == 0) return reject(35);
 
     // ---- a gathered B operand that is a sliding window (the implicit GEMM of a convolution): k = (channel,
     // taps...) with the channel outermost, offset = f(position) + channel * stride + tap offset.  When the piece
