@@ -6,14 +6,15 @@
 // tiles of 16 x 16 per wavefront.  K is walked in slices of BK: the slice's A and B parts go from
 // global memory to registers (8-byte loads, the thread-to-element mapping chosen so that consecutive lanes follow
 // the operand's unit stride), from there to one of two LDS stages as [k][m] and [k][n], and each k-step (4) of a slice reads
-// TM + TN operand fragments for TM * TN matrix instructions.  A slice is stored to its stage while the one before it is multiplied,
-// two slices after its loads were issued, and a step's fragments are read during the step before: one barrier per slice, ahead of its last step.
+// TM + TN operand fragments for TM * TN matrix instructions.  In all but the tiles of 128, of 96 with slices of their own and of 16 (AHEAD) a slice is
+// stored to its stage while the one before it is multiplied, one slice after its loads were issued, and a step's fragments are read during the step
+// before: one barrier per slice, ahead of its last step.
 //
 // What bounds it: with tiles enough, the fp64 matrix instruction (64 cycles each, so LDS is never short); with few, the chain of
 // one tile's slices, each a trip to memory, two LDS accesses and a barrier.  Hence tiles from 128 x 128 down to 16 x 16, and groups
-// of wavefronts that share a slice's k (WGK).  us of a launch with loads one slice ahead, fragments read by the step that multiplies them and fewer
-// such groups -> now: 1500 x 1430 x 250 33.6 -> 30.8, 2000 x 1100 x 700 77.5 -> 67, 1500 x 1430 x 1000 107 -> 93, 1000^3 49 -> 46.5, 500^3 11.4 -> 10.4,
-// 2048^3 310 (55 TFLOP/s), 200 x 300 x 1000 9.6 either way.
+// of wavefronts that share a slice's k (WGK).  us of a library call among others (nothing transposed, C not read) with loads one slice ahead, fragments
+// read by the step that multiplies them and fewer such groups -> now: 1500 x 1430 x 250 31.1 -> 28.5, 2000 x 1100 x 700 75 -> 65, 1500 x 1430 x 1000
+// 106 -> 91, 1000^3 47.3 -> 44.2, 500^3 10.7 -> 10.0, 2048^3 314 -> 312 (55 TFLOP/s), 200 x 300 x 1000 8.9 either way.
 //
 // Instruction layout (one wavefront): lane l supplies A[row l % 16][k l / 16] and B[k l / 16][column l % 16];
 // its four results are rows l / 16 + 0, 4, 8, 12 of column l % 16.
@@ -52,14 +53,16 @@ struct shape {
 
 // The tiles, and the one whose launch is modelled fastest: `fixed` microseconds (start, the last store), `round` for every round of
 // tiles over the compute units (first slice, epilogue), and per k `first` for a round that a compute unit has to itself or
-// `further` for each of several, whichever is more.  Fits to whole launches of 16 ... 2048 in each size, before the pipeline (measured / modelled:
+// `further` for each of several, whichever is more.  Fits to whole launches of 16 ... 2048 in each size of the tiles without the pipeline (measured / modelled:
 // 1500 x 1430 x 250 32.5 / 34.1 with 32 x 32, 34.3 / 34.7 with 96 x 96, 46 / 47 with 128 x 128; x 1000 114 / 120, 107 / 108,
 // 155 / 155; 2080 x 4832 x 32 25 / 29, 30 / 29, 27 / 29; 1000^3 48 / 46 with 64 x 64, 55 / 55 with 32 x 32; 700 x 900 x 1000 45.5 / 42.1 without and 42.4 / 41.9 with
-// shared slices; 200 x 300 x 1000 9.7 / 8.6 with 16 x 16, 18.6 / 18 with 32 x 32).
+// shared slices; 200 x 300 x 1000 9.7 / 8.6 with 16 x 16, 18.6 / 18 with 32 x 32); the order stays as the pipeline found it, so that no size gets fewer
+// partial sums: 64 x 64 without shared slices, faster where its tiles are several rounds (1960 x 1449 x 466 57 and 75), has twice their error.
 // Tiles of 96 x 96 that fit the chip in a round leave each SIMD one wavefront: with slices of 32 k shared by two groups it has two. They take the place of
-// tiles whose sums are of one part (with the pipeline: 2000 x 1100 x 700 67 against 78 with 96 x 96, 1500 x 1430 x 1000 93 and 108, x 250 30.7 and 33 with
-// 32 x 32, 1120 x 1965 x 256 30.7 and 31.9, error against 64 bits and more 0.75 of it), not of those of four or eight, which are closer: 64 x 64 without
-// shared slices, faster where its tiles are several rounds (1960 x 1449 x 466 57 and 75), has twice their error.
+// tiles whose sums are of one part, not of those of four or eight, which are closer, where they are modelled faster than these are now (`present`, fitted to
+// 140 sizes on both sides of the line, rms error 3 to 6 %).  us of a call with the tile they replace / with them: 1504 x 1485 x 1664 171 / 143,
+// 2000 x 1100 x 700 75 / 65, 1600 x 1293 x 1216 125 / 106 (96 x 96), 1440 x 1431 x 736 74 / 67, 1500 x 1430 x 250 31.1 / 28.5 (32 x 32), error against 64 bits and
+// more 0.75 of it; left: 1664 x 1337 x 140 19.4 / 20.8, 1943 x 1135 x 170 22.5 / 23.4 (32 x 32).
 enum tile { TILE_128, TILE_96, TILE_64, TILE_32, TILE_32_SHARED, TILE_16, TILES, TILE_96_SHARED };
 typedef shape<4, 2, 2, 4, 16, 1, false> shape_128;   // 2 x 4 wavefronts: two per SIMD cover each other's waits
 typedef shape<3, 3, 2, 2, 16, 1, false> shape_96;
@@ -87,8 +90,14 @@ inline tile tile_for(long M, long N, long K) {
         const double cost = model[i].fixed + rounds * model[i].round + (double)K * slope;
         if (i == 0 || cost < best_cost) { best = i; best_cost = cost; }
     }
-    const bool one_part = best == TILE_128 || best == TILE_96 || best == TILE_32;
-    if (one_part && ((M + 95) / 96) * ((N + 95) / 96) <= ttarget::COMPUTE_UNITS && 7.7 + 0.083 * (double)K < 0.9 * best_cost) return TILE_96_SHARED;
+    if (((M + 95) / 96) * ((N + 95) / 96) > ttarget::COMPUTE_UNITS) return (tile)best;
+    static const struct { tile which; double fixed, round, first, further; } present[] = {
+        {TILE_128, 6.5, 2.7, 0.1467, 0.1467}, {TILE_96, 5.8, 2.0, 0.1002, 0.1002}, {TILE_32, 3.0, 0.1, 0.0235, 0.0118}};
+    for (const auto &p : present) {
+        const long e = model[best].edge, tiles = ((M + e - 1) / e) * ((N + e - 1) / e);
+        const double rounds = (double)((tiles + ttarget::COMPUTE_UNITS - 1) / ttarget::COMPUTE_UNITS);
+        if (p.which == best && 8.2 + 0.083 * (double)K < p.fixed + rounds * p.round + (double)K * (rounds * p.further > p.first ? rounds * p.further : p.first)) return TILE_96_SHARED;
+    }
     return (tile)best;
 }
 
