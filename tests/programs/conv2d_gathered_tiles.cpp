@@ -13,5 +13,7 @@ int main()
     generate(3, 15, 8, 91);       // 32x128
     generate(8, 40, 50, 92);      // 64x64
     generate(7, 11, 35, 67);      // 64x128
+    generate(1, 64, 64, 16);      // 32x32 where few 64x64 tiles would share slices between two groups
+    generate(4, 64, 64, 64);      // such 64x64 tiles, one for every compute unit
     return 0;
 }

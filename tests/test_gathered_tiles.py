@@ -11,7 +11,8 @@ from test_conv2d import make_inputs, name_of
 from tiramisu_amd import runtime
 
 CASES = [((2, 41, 33, 13), "tile 32x32x64, guarded"), ((1, 64, 32, 8), "tile 32x32x64, whole"), ((1, 44, 15, 96), "tile 32x64x64, guarded"),
-         ((3, 15, 8, 91), "tile 32x128x16, guarded"), ((8, 40, 50, 92), "tile 64x64x32, guarded"), ((7, 11, 35, 67), "tile 64x128x16, guarded")]
+         ((3, 15, 8, 91), "tile 32x128x16, guarded"), ((8, 40, 50, 92), "tile 64x64x32, guarded"), ((7, 11, 35, 67), "tile 64x128x16, guarded"),
+         ((1, 64, 64, 16), "tile 32x32x64, whole"), ((4, 64, 64, 64), "tile 64x64x64, whole")]
 
 
 @pytest.mark.parametrize("s,what", CASES)

@@ -145,13 +145,18 @@ struct gathered_tile { int m, n, k, waves_m, waves_n, groups; double fixed, roun
 constexpr gathered_tile GATHERED_TILES[] = {
     {32, 32, 64, 1, 1, 4, 2.5, 0.66, 0.0056, 0.0047}, {32, 64, 64, 1, 2, 4, 1.8, 1.7, 0.0092, 0.0085}, {32, 128, 16, 1, 4, 1, 1.0, 1.7, 0.027, 0.0174},
     {64, 64, 32, 2, 2, 1, 2.15, 0.96, 0.0178, 0.0177}, {64, 128, 16, 2, 2, 1, 1.9, 1.4, 0.0395, 0.0313}};
+// (whole 64 x 64 tiles whose slices of 64 k two groups share, a round of them)
+constexpr double GATHERED_TWO_GROUPS_FIXED = 1.6, GATHERED_TWO_GROUPS_PER_K = 0.0185;
+inline double modelled(const gathered_tile &c, long M, long N, long K) {
+    const long tiles = ((M + c.m - 1) / c.m) * ((N + c.n - 1) / c.n);
+    const double rounds = (double)((tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS), slope = rounds * c.further > c.first ? rounds * c.further : c.first;
+    return c.fixed + rounds * c.round + (double)K * slope;
+}
 inline gathered_tile gathered_tile_for(long M, long N, long K) {
     const gathered_tile *best = nullptr;
     double best_cost = 0;
     for (const gathered_tile &c : GATHERED_TILES) {
-        const long tiles = ((M + c.m - 1) / c.m) * ((N + c.n - 1) / c.n);
-        const double rounds = (double)((tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS), slope = rounds * c.further > c.first ? rounds * c.further : c.first;
-        const double cost = c.fixed + rounds * c.round + (double)K * slope;
+        const double cost = modelled(c, M, N, K);
         if (!best || cost < best_cost) { best = &c; best_cost = cost; }
     }
     return *best;

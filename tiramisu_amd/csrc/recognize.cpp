@@ -1228,9 +1228,11 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     }
     // at most one 64x64 tile per compute unit and a long reduction: two groups of wavefronts share each
     // (64-k) slice, so that every SIMD has two wavefronts to alternate between (1024^3: 20.6 us against 21.9)
+    bool two_groups = false;
     if (lit && !bf16 && BM == 64 && BN == 64 && WGK == 1 && Ml % 64 == 0 && Nl % 64 == 0 && Kl % 64 == 0 && Kl >= 512 &&
         (Ml / 64) * (Nl / 64) <= ttarget::COMPUTE_UNITS) {
         WGK = 2; BK = 64;
+        two_groups = true;
     }
     // a forced square tile starts from that tile's own defaults (no K groups, slices of 32 for 64x64, of 16 above)
     if (const char *e = backend_option("TIRAMISU_MFMA_TILE")) { BM = BN = std::atoi(e); PADX = BM == 256 ? 0 : 1; WGM = WGN = 2; WGK = 1; DEPTH = 1; BK = BM == 64 ? 32 : 16; }
@@ -1407,18 +1409,23 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         }
     }
 
-    // short products with a gathered operand whose window is not staged: the tile that is modelled fastest (kernels/target_gfx950.h)
+    // short products with a gathered operand whose window is not staged: the tile that is modelled fastest (kernels/target_gfx950.h), also in
+    // the place of 64x64 tiles that two groups share, if it has as many groups (1 image of 16 x 16, 64 to 64 channels 11.3 us with those, 5.5 with
+    // 32x32; 4 of 32 x 32 11.6, 5.8; 4 of 64 x 64 13.1 and 14.3: there they stay)
     {
-        bool gathered = lit && !bf16 && !with_consumer && !batched && !windowed && operands.size() == 1 && WGK == 1 && Ml <= 64 && operands[0].first.linear &&
+        bool gathered = lit && !bf16 && !with_consumer && !batched && !windowed && operands.size() == 1 && (WGK == 1 || two_groups) && Ml <= 64 && operands[0].first.linear &&
                         !operands[0].second.linear;
         for (const char *forced : {"TIRAMISU_MFMA_TILE", "TIRAMISU_MFMA_BM", "TIRAMISU_MFMA_BN", "TIRAMISU_MFMA_BK", "TIRAMISU_MFMA_WGM", "TIRAMISU_MFMA_WGN",
                                    "TIRAMISU_MFMA_WGK", "TIRAMISU_MFMA_DEPTH", "TIRAMISU_MFMA_PAD", "TIRAMISU_MFMA_NO_SPLITK"})
             if (backend_option(forced)) gathered = false;
         if (gathered) {
             const ttarget::gathered_tile t = ttarget::gathered_tile_for(Ml, Nl, Kl);
+            if (two_groups && (t.groups < 2 || ttarget::modelled(t, Ml, Nl, Kl) >= ttarget::GATHERED_TWO_GROUPS_FIXED + Kl * ttarget::GATHERED_TWO_GROUPS_PER_K)) gathered = false;
             long v;
-            BM = t.m; BN = t.n; BK = t.k; WGM = t.waves_m; WGN = t.waves_n; WGK = t.groups;
-            edge = !(Ml % BM == 0 && Nl % BN == 0 && Kl % BK == 0 && literal_value(operands[0].first.ld, v) && v % 4 == 0 && multiple_of(operands[0].first.base, 4));
+            if (gathered) {
+                BM = t.m; BN = t.n; BK = t.k; WGM = t.waves_m; WGN = t.waves_n; WGK = t.groups;
+                edge = !(Ml % BM == 0 && Nl % BN == 0 && Kl % BK == 0 && literal_value(operands[0].first.ld, v) && v % 4 == 0 && multiple_of(operands[0].first.base, 4));
+            }
         }
     }
 
