@@ -99,6 +99,21 @@ def test_tensor_calls_on_the_default_and_a_side_stream_and_what_is_refused():
 
 
 @pytest.mark.gpu
+def test_weights_held_as_parameters_take_the_one_entry():
+    import torch
+    p = runtime.load(PROGRAMS, "conv2d_2x8x64x16")
+    x, out = torch.ones(2, 8, 18, 18, device="cuda"), torch.zeros(2, 64, 16, 16, device="cuda")
+    layer = torch.nn.Conv2d(8, 64, 3).cuda()
+    with torch.no_grad():
+        layer.weight.fill_(0.25)
+        layer.bias.fill_(1.0)
+    calls, one_entry = [], p._call_of_tensors
+    p._call_of_tensors = lambda args: calls.append(one_entry(args)) or calls[-1]
+    p(x, layer.weight, layer.bias, out)
+    assert calls == [0] and torch.all(out == 8 * 9 * 0.25 + 1.0)
+
+
+@pytest.mark.gpu
 def test_tensor_calls_follow_torch_work_in_two_threads():
     import threading
     import torch

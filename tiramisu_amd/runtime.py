@@ -236,9 +236,9 @@ class Program:
         torch = sys.modules.get("torch")
         if torch is None or self.fn is not fn or len(args) != len(arguments):
             return None
-        tensor, pointers = torch.Tensor, []
+        kinds, pointers = (torch.Tensor, torch.nn.Parameter), []
         for a, (dtype, shape) in zip(args, arguments):
-            if type(a) is not tensor or _tensor_type(a.dtype) is not dtype or a.shape != shape or not a.is_cuda or not a.is_contiguous():
+            if type(a) not in kinds or _tensor_type(a.dtype) is not dtype or a.shape != shape or not a.is_cuda or not a.is_contiguous():
                 return None
             pointers.append(a.data_ptr())
         if 0 in pointers:
@@ -266,12 +266,6 @@ class Program:
         tensor's device, in order with the torch work around the call (the runtime's stream of the calling thread is
         put back afterwards); when that is torch's default stream they run on the runtime's stream of the calling
         thread, and the call waits for torch's default stream first and for its own kernels afterwards."""
-        if args and not isinstance(args[0], (Buffer, np.ndarray)) and self.of_tensors is not None:
-            rc = self._call_of_tensors(args)
-            if rc is not None:
-                if rc != 0:
-                    raise RuntimeError("Tiramisu function returned %d" % rc)
-                return rc
         bufs, torch_stream = [], None
         for a in args:
             if isinstance(a, Buffer):
@@ -279,6 +273,12 @@ class Program:
             elif isinstance(a, np.ndarray):
                 bufs.append(Buffer.from_numpy(a))
             elif type(a).__module__.split(".")[0] == "torch":
+                if not bufs and self.of_tensors is not None:
+                    rc = self._call_of_tensors(args)
+                    if rc is not None:
+                        if rc != 0:
+                            raise RuntimeError("Tiramisu function returned %d" % rc)
+                        return rc
                 bufs.append(Buffer.from_tensor(a))
                 if a.is_cuda and torch_stream is None:
                     import torch
