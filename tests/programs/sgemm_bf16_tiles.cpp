@@ -15,5 +15,8 @@ int main()
     generate(2000, 1500, 1010);   // 128 x 128, pairs: the last one begins its second slice
     generate(3842, 3970, 1278);   // 256 x 256, pairs
     generate(1920, 2560, 1024);   // whole tiles of 192 x 128
+    generate(3841, 3074, 1088);   // 256 x 256, pairs: 192 tiles, rows of A at whole lines
+    generate(2560, 3520, 1368);   // 256 x 256, slices one by one: 140 tiles
+    generate(4096, 2560, 640);    // 128 x 128: rows at multiples of 16 bytes
     return 0;
 }

@@ -215,13 +215,21 @@ def test_gpu_sizes_that_end_inside_a_tile(M, N, K, what, programs_dir):
 TILES = [(1793, 3842, 514, "tile 128x256x64, guarded edges"), (1921, 2562, 578, "tile 192x128x64, guarded edges"),
          (673, 3202, 1090, "tile 96x128x64, guarded edges"), (1473, 642, 514, "tile 64x128x64, guarded edges"), (33, 66, 194, "tile 32x64x64, guarded edges"),
          (2000, 1500, 1010, "tile 128x128x32, guarded edges, slices in pairs"), (3842, 3970, 1278, "tile 256x256x32, guarded edges, slices in pairs"),
-         (1920, 2560, 1024, "tile 192x128x64, whole tiles")]
+         (1920, 2560, 1024, "tile 192x128x64, whole tiles"),
+         # 192 tiles of 256 and rows of A at whole lines: pairs; 140 tiles: one by one; rows at 16 bytes: 128 x 128 rather than two rounds of 192 x 128
+         (3841, 3074, 1088, "tile 256x256x32, guarded edges, slices in pairs"), (2560, 3520, 1368, "tile 256x256x32, guarded edges, 1 product"),
+         (4096, 2560, 640, "tile 128x128x32, whole tiles, 1 product")]
+
+
+@pytest.mark.parametrize("M,N,K,what", TILES)
+def test_tiles_of_the_model(M, N, K, what, programs_dir):
+    assert what in how(programs_dir, name_of(M, N, K))
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,what", TILES)
 def test_gpu_tiles_between_the_squares(M, N, K, what, programs_dir):
-    """The tiles between the squares of 256, 128 and 64, and slices in pairs, at their remainders: exact as above."""
+    """The tiles between the squares of 256, 128 and 64, and slices in pairs or one by one, at their remainders: exact as above."""
     test_gpu_sizes_that_end_inside_a_tile(M, N, K, what, programs_dir)
 
 

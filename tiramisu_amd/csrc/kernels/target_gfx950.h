@@ -174,36 +174,49 @@ inline gathered_tile gathered_tile_for(long M, long N, long K) {
 // 1908 x 2550 x 858 27 and 20 with 192 x 128; 682 x 3212 x 1114 19 and 14.4 with 96 x 128; 417 x 396 x 3318 20 with 64 x 64 and 15 with 32 x 64.
 // A tile is taken from `from` to `to` k.  Up to 512 k the squares keep the figures they were fitted with there: the tiles between them
 // would give less than a microsecond, and the model errs by as much (805 x 1240 x 306 6.5 us with 64 x 64, 6.7 with 64 x 128).
+// Where the rows of both operands lie at multiples of 16 bytes, two workgroups with 128 x 128 tiles to a compute unit cover each other better
+// (`further_aligned`: 2328 x 3776 x 644 36.6 us, 3224 x 2688 x 592, as much work, 26.8); there they are ahead of several rounds of 192 x 128:
+// 4096 x 2560 x 640 26.1 and 28.5, 4035 x 2816 x 688 31.6 and 32.8, 3456 x 3264 x 600 30.9 and 31.1; not where their last round is a quarter of the
+// chip or less, which nothing covers: 2946 x 2752 x 584 27.0 and 26.1, 3000 x 3000 x 800 32.1 and 31.6.
+// Tiles of 256 x 256 load their slices in pairs where the launch asks most of the L1: one tile for every compute unit, or 180 of them and rows of A
+// that lie at whole lines (4096^3 122.5 -> 119.0 us, 4000 x 4000 x 1300 56.3 -> 55.3, 3840 x 3072 x 4096 99.1 -> 97.1).  With fewer two stages cover the way to
+// memory worse than four: 3000 x 2700 x 4000 82.8 us one by one and 88.6 in pairs, 2560 x 3520 x 1368 40.1 and 42.7, 3383 x 3956 x 2808 87.4 and 88.5, in several rounds
+// 7000 x 6000 x 3000 261 and 266.
 // Direct tiles load their slices straight into LDS; the others serve rows of an odd number of elements and other operands that
 // those loads cannot address.
 struct bf16_tile {
     int m, n, k, slices, waves_m, waves_n, stages;
     bool direct;
     int from, to;
-    double fixed, first, further;
+    double fixed, first, further, further_aligned;
 };
 constexpr int ANY_K = 0x7fffffff;
 constexpr bf16_tile BF16_TILES[] = {
-    {256, 256, 32, 1, 4, 2, 4, true, 0, 512, 9.0, 0.55, 0.85}, {128, 128, 32, 1, 2, 4, 4, true, 0, 512, 3.9, 0.17, 0.28},
-    {64, 64, 64, 1, 2, 2, 3, true, 0, 512, 2.8, 0.12, 0.12}, {32, 64, 64, 1, 1, 2, 3, true, 192, 512, 2.7, 0.104, 0.092},
-    {256, 256, 32, 1, 4, 2, 4, true, 513, ANY_K, 9.0, 0.58, 0.85}, {256, 256, 32, 2, 4, 2, 2, true, 513, ANY_K, 9.5, 0.555, 0.85},
-    {128, 256, 64, 1, 2, 4, 3, true, 513, ANY_K, 6.2, 0.326, 0.51}, {192, 128, 64, 1, 2, 4, 3, true, 513, ANY_K, 5.6, 0.283, 0.386},
-    {128, 128, 32, 1, 2, 4, 4, true, 513, ANY_K, 3.9, 0.251, 0.295}, {128, 128, 32, 2, 2, 4, 3, true, 513, ANY_K, 4.4, 0.227, 0.349},
-    {96, 128, 64, 1, 1, 4, 3, true, 513, ANY_K, 5.8, 0.188, 0.285}, {64, 128, 64, 1, 2, 2, 3, true, 513, ANY_K, 4.1, 0.167, 0.179},
-    {64, 64, 64, 1, 2, 2, 3, true, 513, ANY_K, 3.35, 0.132, 0.117}, {32, 64, 64, 1, 1, 2, 3, true, 513, ANY_K, 3.2, 0.114, 0.090},
-    {128, 128, 64, 1, 2, 2, 2, false, 0, ANY_K, 8.0, 0.42, 0.4}, {64, 64, 64, 1, 2, 2, 2, false, 0, ANY_K, 3.5, 0.19, 0.195}};
+    {256, 256, 32, 1, 4, 2, 4, true, 0, ANY_K, 9.0, 0.55, 0.85, 0.85}, {128, 128, 32, 1, 2, 4, 4, true, 0, 512, 3.9, 0.17, 0.28, 0.28},
+    {64, 64, 64, 1, 2, 2, 3, true, 0, 512, 2.8, 0.12, 0.12, 0.12}, {32, 64, 64, 1, 1, 2, 3, true, 192, 512, 2.7, 0.104, 0.092, 0.092},
+    {128, 256, 64, 1, 2, 4, 3, true, 513, ANY_K, 6.2, 0.326, 0.51, 0.51}, {192, 128, 64, 1, 2, 4, 3, true, 513, ANY_K, 5.6, 0.283, 0.386, 0.386},
+    {128, 128, 32, 1, 2, 4, 4, true, 513, ANY_K, 3.9, 0.251, 0.295, 0.24}, {128, 128, 32, 2, 2, 4, 3, true, 513, ANY_K, 4.4, 0.227, 0.349, 0.349},
+    {96, 128, 64, 1, 1, 4, 3, true, 513, ANY_K, 5.8, 0.188, 0.285, 0.285}, {64, 128, 64, 1, 2, 2, 3, true, 513, ANY_K, 4.1, 0.167, 0.179, 0.179},
+    {64, 64, 64, 1, 2, 2, 3, true, 513, ANY_K, 3.35, 0.132, 0.117, 0.117}, {32, 64, 64, 1, 1, 2, 3, true, 513, ANY_K, 3.2, 0.114, 0.090, 0.090},
+    {128, 128, 64, 1, 2, 2, 2, false, 0, ANY_K, 8.0, 0.42, 0.4, 0.4}, {64, 64, 64, 1, 2, 2, 2, false, 0, ANY_K, 3.5, 0.19, 0.195, 0.195}};
 constexpr bf16_tile BF16_TILE_ANY_SIZE = BF16_TILES[sizeof(BF16_TILES) / sizeof(BF16_TILES[0]) - 1];    // sizes known at run time only
 
-inline bf16_tile bf16_tile_for(long M, long N, long K, bool direct) {
+// `lda`, `ldb`: elements from one row of A, of B to the next, or what they are multiples of
+inline bf16_tile bf16_tile_for(long M, long N, long K, bool direct, long lda, long ldb) {
     const bf16_tile *best = nullptr;
     double best_cost = 0;
+    const bool aligned = lda % 8 == 0 && ldb % 8 == 0;
     for (const bf16_tile &c : BF16_TILES) {
         if (c.direct != direct || K < c.from || K > c.to) continue;
         const long tiles = ((M + c.m - 1) / c.m) * ((N + c.n - 1) / c.n), rounds = (tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS, stage = c.k * c.slices;
-        const double cost = c.fixed + ((K + stage - 1) / stage * stage / 32) * (c.first + (rounds - 1) * c.further);
+        const bool covered = aligned && tiles - (rounds - 1) * COMPUTE_UNITS > COMPUTE_UNITS / 4;
+        const double cost = c.fixed + ((K + stage - 1) / stage * stage / 32) * (c.first + (rounds - 1) * (covered ? c.further_aligned : c.further));
         if (!best || cost < best_cost) { best = &c; best_cost = cost; }
     }
-    return *best;
+    bf16_tile tile = *best;
+    const long tiles = ((M + tile.m - 1) / tile.m) * ((N + tile.n - 1) / tile.n);
+    if (tile.m == 256 && K > 512 && (tiles == COMPUTE_UNITS || (tiles >= 180 && lda % 64 == 0))) { tile.slices = 2; tile.stages = 2; }
+    return tile;
 }
 
 }  // namespace ttarget

@@ -7,6 +7,7 @@
 #include <unistd.h>
 #include <algorithm>
 #include <cstdlib>
+#include <numeric>
 #include <sstream>
 
 #include "hip_backend.h"
@@ -1254,6 +1255,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
         for (auto &o : operands)
             if (!o.first.linear || !o.second.linear || !o.first.kmajor || o.second.kmajor) return reject(25);
         bool aligned = true, dword_rows = true, small_enough = true, forwards = true;
+        long row_a = 0, row_b = 0;               // what the rows' lengths are multiples of
         for (auto &o : operands) {
             long v;
             for (const operand_info *g : {&o.first, &o.second}) {
@@ -1262,6 +1264,8 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
             }
             long lda = 0, ldb = 0;
             if (lit && literal_value(o.first.ld, lda) && literal_value(o.second.ld, ldb)) {
+                row_a = std::gcd(row_a, lda);
+                row_b = std::gcd(row_b, ldb);
                 // (a tile's rows and slices may reach behind the operand: their offsets must not wrap either)
                 if ((double)(Ml + 256) * lda * 2 >= 2147483648.0 || (double)(Kl + 256) * ldb * 2 >= 2147483648.0) small_enough = false;
                 if (lda <= 0 || ldb < Nl) forwards = false;
@@ -1270,7 +1274,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
             }
         }
         bf16_direct = lit && dword_rows && small_enough && forwards;
-        const ttarget::bf16_tile tile = lit ? ttarget::bf16_tile_for(Ml, Nl, Kl, bf16_direct) : ttarget::BF16_TILE_ANY_SIZE;
+        const ttarget::bf16_tile tile = lit ? ttarget::bf16_tile_for(Ml, Nl, Kl, bf16_direct, row_a, row_b) : ttarget::BF16_TILE_ANY_SIZE;
         BM = tile.m;
         BN = tile.n;
         BK = tile.k * tile.slices;
@@ -1939,7 +1943,7 @@ bool emit_contraction(context &ctx, const node_ptr &root, launch_plan &plan, con
     kernel unaligned;
     std::string addresses;
     if (bf16_direct) {
-        const ttarget::bf16_tile t = ttarget::bf16_tile_for(Ml, Nl, Kl, false);
+        const ttarget::bf16_tile t = ttarget::bf16_tile_for(Ml, Nl, Kl, false, 1, 1);
         unaligned = k;
         unaligned.name = kname + "_unaligned";
         unaligned.grid[0] = std::to_string(((Ml + t.m - 1) / t.m) * ((Nl + t.n - 1) / t.n));
