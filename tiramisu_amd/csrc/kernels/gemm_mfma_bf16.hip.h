@@ -274,7 +274,7 @@ __device__ __forceinline__ void tile_accumulate_bf16(accumulators<CFG> &acc, con
 // dword, so the last row itself is whole); columns of B behind N are the start of the next row and only reach columns of C
 // that nobody stores; so do rows of A behind M.  Only k behind the last one has to be zero: rows of B there are (behind
 // the end), and A, whose row simply goes on into the next, is masked in registers in the last slice.
-// (2000 x 1500 x 1000: 14.2 us with 128 x 128 tiles against 48.7 with guarded 64 x 64 tiles staged through registers; what bounds
+// (2000 x 1500 x 1000: 15.0 us a call with 128 x 128 tiles against 48.7 with guarded 64 x 64 tiles staged through registers; what bounds
 // it: operands of 512 KB per compute unit, 7 of the 11 us within the kernel, and C, 2.5;
 // 300 x 260 x 3000: 13.0 us with 64 x 64 tiles against 99.8.)
 template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int STAGES_, bool EDGE_ = false>

@@ -140,7 +140,7 @@ inline int split_tile_for(long M, long N, long K, long problems, int m, int n, b
 // and 64 ... 300000 positions (rms error 9 to 14 %).  us of a launch with the tile of before (64 x 256 from 65536 columns on, else 64 x 64)
 // and with the one chosen: 2 images of 40 x 40, 64 to 48 channels 14.0, 6.5 (32 x 32); 3 of 24 x 24, 41 to 6 9.0, 4.7; 1 of 96 x 96, 44 to 15 10.7, 6.9 (32 x 64);
 // 32 of 100 x 100, 16 to 16 59, 35 (32 x 128); 7 of 96 x 96, 24 to 16 20.5, 12.2; 8 of 92 x 92, 40 to 50 53, 38 (64 x 64); 29 of 56 x 56, 46 to
-// 35 59, 46 (64 x 128); 8 of 112 x 112, 3 to 64 12.1, 11.4; of the 44 none slower, 0.71 of the time in the geometric mean.
+// 35 59, 46 (64 x 128); 8 of 112 x 112, 3 to 64 13.3, 13.0; of the 44 none slower, 0.71 of the time in the geometric mean.
 struct gathered_tile { int m, n, k, waves_m, waves_n, groups; double fixed, round, first, further; };
 constexpr gathered_tile GATHERED_TILES[] = {
     {32, 32, 64, 1, 1, 4, 2.5, 0.66, 0.0056, 0.0047}, {32, 64, 64, 1, 2, 4, 1.8, 1.7, 0.0092, 0.0085}, {32, 128, 16, 1, 4, 1, 1.0, 1.7, 0.027, 0.0174},
@@ -167,7 +167,7 @@ inline gathered_tile gathered_tile_for(long M, long N, long K) {
 // each round after it.  Reading and writing C is left out: it takes every tile about the same (1.07 us per million elements),
 // so the model only orders the tiles.  It is fitted to whole launches of 100 sizes of 32 ... 4096 rows, columns and k (rms error
 // 8 to 12 %).  A stage of the LDS ring holds `slices` slices of `k`: with 64 k a row of A is read 128 bytes at a time, a whole line
-// of the L1, and there is one barrier for twice the work (4096^3 125 -> 121 us, 2000 x 1500 x 1000 15.3 -> 14.2); slices of 32 in
+// of the L1, and there is one barrier for twice the work (4096^3 122.5 -> 119.0 us, 2000 x 1500 x 1000 16.2 -> 15.0 a call); slices of 32 in
 // more stages start earlier and pad less.
 // The tiles between the squares of 256, 128 and 64 are for results that those cover badly: 1500 x 1000 x 3000 are 96 tiles of 128 x 128
 // (34 us) or 384 of 64 x 64, two rounds (28), but 192 of 64 x 128 (22); 1798 x 3830 x 3428 88 us with 128 x 128, 56 with 128 x 256;
